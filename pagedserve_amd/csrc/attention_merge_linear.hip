@@ -19,7 +19,7 @@
 // with atomic adds; the blocks of the first heads add the bias.  The sum over heads is
 // therefore made by the adds, in an order that differs from run to run within float rounding,
 // as for every product here whose k range is split over blocks.
-#include "gemm_bf16_common.h"
+#include "gemm_tile.h"
 
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
 

@@ -20,6 +20,15 @@ int ps_norm_gemm_fused(const NormPrologue& norm, const void* w, const float* bia
                        int n, int k, int ldc, int c_dtype, int epilogue, const KvScatter& scatter,
                        const void* w_packed, hipStream_t s);
 bool ps_gemm_nt_mfma_supported(const void* a, const void* w, int k, int lda, int dtype);
+bool ps_gemm_nt_f32_skinny_takes(const void* a, const void* w, int m, int n, int k, int lda,
+                                 int epilogue);
+int ps_gemm_nt_f32_skinny(const void* a, const void* w, const float* bias, void* c, int m, int n,
+                          int k, int lda, int ldc, int epilogue, const KvScatter& scatter,
+                          hipStream_t s);
+bool ps_gemm_nt_f32_tiled_supported(const void* a, const void* w, int m, int k, int lda);
+int ps_gemm_nt_f32_tiled(const void* a, const void* w, const float* bias, void* c, int m, int n,
+                         int k, int lda, int ldc, int epilogue, const KvScatter& scatter,
+                         hipStream_t s);
 bool ps_norm_gemm_fusable(const void* w, const NormPrologue& norm, int m, int n, int k, int dtype);
 
 // The size of the argument block, so that a caller that lays it out by hand can check that
@@ -116,8 +125,16 @@ extern "C" int ps_linear(const PsLinearArgs* p, void* stream) {
     lda = k;
     if (pack_norm) layouts |= 1;
   }
-  // Matrix cores when the operands allow 16-byte loads; in float only for many rows (the
-  // tile is 128 rows high), else the plain kernel.
+  if (p->dtype == PS_F32) {
+    if (ps_gemm_nt_f32_skinny_takes(a, p->w, m, n, k, lda, p->epilogue))
+      return ps_gemm_nt_f32_skinny(a, p->w, p->bias, p->c, m, n, k, lda, p->ldc, p->epilogue,
+                                   scatter, s);
+    if (ps_gemm_nt_f32_tiled_supported(a, p->w, m, k, lda))
+      return ps_gemm_nt_f32_tiled(a, p->w, p->bias, p->c, m, n, k, lda, p->ldc, p->epilogue, scatter,
+                                  s);
+  }
+  // Matrix cores when the operands allow 16-byte loads (in float what is left here are many rows
+  // of a k that is no multiple of 32, and up to 8 rows for the plain kernel).
   const bool mfma = ps_gemm_nt_mfma_supported(a, p->w, k, lda, p->dtype) &&
                     (p->dtype == PS_BF16 || m >= 96);
   if (mfma) {

@@ -1,10 +1,10 @@
 // Matrix products on the matrix cores (MFMA) of gfx950:  C[m, n] = epi(sum_k A[m, k] W[n, k] + b[n]).
 //
-// Two kernels (the tiled bfloat16 product for many rows with k a multiple of 64 is a file of
-// its own, gemm_tiled_bf16.hip; this file dispatches to it).
+// Two kernels (the tiled product for many rows whose k comes in whole pieces of 128 bytes is a file
+// of its own, gemm_tiled.hip, and so is the one of few float rows, gemm_skinny_f32.hip; this file
+// dispatches bfloat16 to the former).
 //
-// gemm_nt_tiled_kernel — many rows in float32, and bfloat16 shapes the other tiled kernel does
-//   not take.  128 x 128 outputs per 256-thread block, four waves in a 2 x 2 arrangement, each
+// gemm_nt_tiled_kernel — many rows of a k that the other tiled kernel does not take.  128 x 128 outputs per 256-thread block, four waves in a 2 x 2 arrangement, each
 //   wave 2 x 2 tiles of 32 x 32.  A and W tiles of 64 bytes of k per row go global ->
 //   registers -> LDS (two buffers, one barrier per k tile); every lane reads 16 bytes of k for
 //   its row from LDS.  For bfloat16 that is the operand of one v_mfma_f32_32x32x16_bf16; for

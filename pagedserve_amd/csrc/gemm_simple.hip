@@ -1,15 +1,14 @@
 // C[m, n] = epilogue(sum_k A[m, k] W[n, k] + bias[n]) with float multiply-adds.
 //
-// The true 32-bit matrix product of the engine (no reduced-precision matrix mode): every
-// product and every sum is an IEEE float operation, summed over k in ascending order inside
-// one thread, so a row's result does not depend on how many other rows the call has.  Also
-// the fallback of the bfloat16 path for shapes that the MFMA kernel refuses.
+// For shapes that the matrix-core kernels refuse (rows that cannot be loaded in pieces of 16 bytes),
+// in float and bfloat16: every product and every sum is an IEEE float operation, summed over k in
+// ascending order inside one thread.
 //
 // Tile: 64 x 64 outputs per 256-thread block, 16 k per stage through LDS, 4 x 4 outputs per
 // thread.  Any m, n, k and any row strides; loads are bounds-checked and zero-filled.
 //
-// Up to 16 rows of float (a decode step of the 32-bit path) take a second kernel: the tiled one
-// would run on n / 64 blocks that each walk the whole k in stages of 16, a few dozen blocks
+// Up to 8 rows of float (a decode step of the 32-bit path) may take a second kernel (where it is ahead
+// of the matrix cores: gemm_skinny_f32.hip): the tiled one would run on n / 64 blocks that each walk the whole k in stages of 16, a few dozen blocks
 // bound by the latency of hundreds of dependent trips (8 rows x 2304 x 768: 70 us).  Here a
 // wave owns a few output columns, its lanes stride over k with 16-byte loads of the weights
 // (each read once, as the step's bytes are the weights') and of the rows (which the caches
@@ -164,7 +163,7 @@ __global__ __launch_bounds__(256) void gemm_nt_f32_rows_kernel(
 }
 
 static bool rows_kernel_takes(const void* a, const void* w, int m, int k, int lda) {
-  return m >= 1 && m <= 16 && k % 4 == 0 && lda % 4 == 0 &&
+  return m >= 1 && m <= 8 && k % 4 == 0 && lda % 4 == 0 &&
          (reinterpret_cast<uintptr_t>(a) & 15u) == 0 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
 }
 
@@ -185,13 +184,10 @@ static int launch_f32_rows(const void* a, const void* w, const float* bias, void
       if (cols == 4) PS_LAUNCH_FR(EPI, 4, 4);                 \
       else if (cols == 2) PS_LAUNCH_FR(EPI, 4, 2);            \
       else PS_LAUNCH_FR(EPI, 4, 1);                           \
-    } else if (m <= 8) {                                      \
+    } else {                                                  \
       if (cols == 4) PS_LAUNCH_FR(EPI, 8, 4);                 \
       else if (cols == 2) PS_LAUNCH_FR(EPI, 8, 2);            \
       else PS_LAUNCH_FR(EPI, 8, 1);                           \
-    } else {                                                  \
-      if (cols >= 2) PS_LAUNCH_FR(EPI, 16, 2);                \
-      else PS_LAUNCH_FR(EPI, 16, 1);                          \
     }                                                         \
   } while (0)
   switch (epilogue) {

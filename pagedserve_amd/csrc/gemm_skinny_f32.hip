@@ -1,0 +1,213 @@
+// Matrix product of few float rows (decode steps and short prompt portions of the 32-bit path) on
+// the matrix cores of gfx950, in true 32-bit (v_mfma_f32_16x16x4_f32):
+//   C[m, n] = epi(sum_k A[m, k] W[n, k] + b[n]),   k a multiple of 4, any m and n.
+//
+// Bound by reading W once, and at these sizes by the one trip to memory that this takes: like the
+// bfloat16 product for few rows, a block owns 16 NT weight rows and MB blocks of 16 rows of A, its
+// waves take turns along k in steps of 32 values (128 bytes of every row), operands go straight from
+// memory to the matrix cores, UNROLL steps asked for together, and the waves' partial tiles are summed
+// in LDS in a fixed order.  Rows of A beyond MB blocks go to further blocks (grid z), which read the
+// same weights out of the L2.  k may be split over blocks; those partial sums are added with float
+// atomics into the stream (residual epilogue only).  A lane's 16 bytes of k are the same for both
+// operands, so that which four values an instruction multiplies does not matter.
+//
+// Measured with weights from memory, before (the plain kernel, or up to 16 rows one dot product per
+// wave and column) and after, in us: 64 x 2304 x 768 88 / 10.2, 64 x 768 x 3072 338 / 9.5, 32 x 768 x
+// 768 89 / 5.7, 200 x 768 x 768 34 / 9.8, 16 x 3072 x 768 8.6 / 6.1, 8 x 768 x 3072 7.1 / 5.7,
+// 16 x 50257 x 768 68 / 48 (its weights alone are 30 at the rate of a copy).
+#include "common.h"
+#include "linear.h"
+#include "pagedserve_hip.h"
+
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
+
+#define SF_STEP 32    // values of k per step of a wave: 128 bytes of every row
+
+template <int EPI, int MB, int NT, int UNROLL, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void gemm_nt_skinny_f32_kernel(
+    const float* __restrict__ a, const float* __restrict__ w, const float* __restrict__ bias,
+    float* __restrict__ c, int m, int n, int k, int lda, int ldc, int k_chunk, int k_splits,
+    KvScatter scatter) {
+  __shared__ float partial[NT][WAVES][MB][4][64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // the same in every lane: scalar
+  const int n0 = blockIdx.x * 16 * NT;
+  const int split = blockIdx.y;
+  const int row0 = blockIdx.z * (MB * 16);
+  const int k_begin = split * k_chunk;
+  const int k_end = k_begin + k_chunk < k ? k_begin + k_chunk : k;
+  const int sub = lane & 15;
+  const int group = lane >> 4;
+  const float* w_ptr[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    const int row = n0 + j * 16 + sub < n ? n0 + j * 16 + sub : n - 1;
+    w_ptr[j] = w + (int64_t)row * k;
+  }
+  const float* a_ptr[MB];
+#pragma unroll
+  for (int b = 0; b < MB; ++b) {
+    const int row = row0 + b * 16 + sub < m ? row0 + b * 16 + sub : m - 1;
+    a_ptr[b] = a + (int64_t)row * lda;
+  }
+  // an accumulator for each of a lane's four values of k: short chains, whose rounding errors stay
+  // small and whose instructions do not wait for each other
+  f32x4 acc[NT][MB][4];
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+#pragma unroll
+    for (int b = 0; b < MB; ++b)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[j][b][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  // wave `wave` takes the steps wave, wave + WAVES, ... of the block's range; UNROLL of them are
+  // asked for together
+  for (int k0 = k_begin + wave * SF_STEP; k0 < k_end; k0 += WAVES * UNROLL * SF_STEP) {
+    f32x4 wf[UNROLL][NT][2], xf[UNROLL][MB][2];
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int kk = k0 + u * WAVES * SF_STEP + h * 16 + group * 4;
+        const bool there = kk < k_end;      // (k is a multiple of 4: a piece is whole or absent)
+        // unconditional loads from a clamped place, zeroed afterwards: loads under a branch
+        // would not be issued together
+        const int at = there ? kk : k_begin;
+#pragma unroll
+        for (int j = 0; j < NT; ++j) wf[u][j][h] = *reinterpret_cast<const f32x4*>(w_ptr[j] + at);
+#pragma unroll
+        for (int b = 0; b < MB; ++b) xf[u][b][h] = *reinterpret_cast<const f32x4*>(a_ptr[b] + at);
+        if (!there) {
+#pragma unroll
+          for (int j = 0; j < NT; ++j) wf[u][j][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int b = 0; b < MB; ++b) xf[u][b][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+      }
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int b = 0; b < MB; ++b)
+              acc[j][b][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[u][j][h][i], xf[u][b][h][i],
+                                                                  acc[j][b][i], 0, 0, 0);
+  }
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+#pragma unroll
+    for (int b = 0; b < MB; ++b)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) partial[j][wave][b][i][lane] =
+            (acc[j][b][0][i] + acc[j][b][1][i]) + (acc[j][b][2][i] + acc[j][b][3][i]);
+  __syncthreads();
+
+  // element i of a 16 x 16 accumulator: weight row (lane / 16) * 4 + i, activation row lane % 16;
+  // 16 consecutive threads finish one run of 16 columns
+  for (int e = threadIdx.x; e < NT * MB * 256; e += 64 * WAVES) {
+    const int col_in = e & 15;
+    const int row_in = (e >> 4) & 15;
+    const int b = (e >> 8) % MB;
+    const int j = (e >> 8) / MB;
+    const int col = n0 + j * 16 + col_in;
+    const int row = row0 + b * 16 + row_in;
+    if (col >= n || row >= m) continue;
+    const int i = col_in & 3;
+    const int at = (col_in >> 2) * 16 + row_in;
+    float v = 0.f;
+#pragma unroll
+    for (int p = 0; p < WAVES; ++p) v += partial[j][p][b][i][at];
+    if (bias != nullptr && split == 0) v += bias[col];
+    float* dst = c + (int64_t)row * ldc + col;
+    if (EPI == PS_EPI_RESIDUAL) {
+      if (k_splits > 1) unsafeAtomicAdd(dst, v);
+      else *dst += v;
+    } else {
+      v = apply_activation<EPI>(v);
+      *dst = v;
+      if (EPI == PS_EPI_NONE) kv_scatter_store<float>(scatter, row, col, v);
+    }
+  }
+}
+
+// --------------------------------------------------------------------------------- host
+// Whether this kernel takes the product (a row of either operand in pieces of 16 bytes), and is the
+// fastest that does.  The lines, with weights from memory, in us:
+// - Up to 8 rows one dot product per wave and column (gemm_simple.hip) is ahead while the weights are
+//   few (8 x 768 x 768 4.2 against 4.9) and level at very many columns; up to 4 rows always but
+//   where k is long and can be split (4 x 1024 x 4096 9.8 against 8.4).
+// - Residual epilogue, k split: 200 x 768 x 3072 24.3 against 25.2 for the tiled kernel, 300 rows 33 against
+//   28; 300 x 768 x 768 11.4 against 11.5; wide models sooner (32 x 1600 x 6400 25.4 against 25.2).
+// - Otherwise up to 64 rows and one round of loads (32 x 4096 x 1024 12.2 against 17.3, 64 rows 17.1
+//   against 17.4; 32 x 4800 x 1600 24.0 against 22.7; 100 x 2304 x 768 13.1 against 11.8), and not
+//   the output head beyond 16 rows (32 x 50257 x 768 71 against 68).
+// - A k that is no multiple of 32, which the tiled kernel does not take, up to 768 rows: there it
+//   meets the one that does (gemm_mfma.hip).
+bool ps_gemm_nt_f32_skinny_takes(const void* a, const void* w, int m, int n, int k, int lda,
+                                 int epilogue) {
+  if (k % 4 != 0 || lda % 4 != 0 || (reinterpret_cast<uintptr_t>(a) & 15u) != 0 ||
+      (reinterpret_cast<uintptr_t>(w) & 15u) != 0)
+    return false;
+  const bool residual = epilogue == PS_EPI_RESIDUAL;
+  const int64_t weights = (int64_t)n * k;
+  if (m <= 4) return residual && k >= 4096;
+  if (m <= 8) return weights > (1 << 20) && n < 64 * 256;
+  if (m <= 16) return true;
+  if (k % SF_STEP != 0) return m < 768;
+  if (residual) return (int64_t)m * n <= 160000 && weights < 6000000;
+  return n < 64 * 256 && (k <= 768 ? m <= 64 : k <= 1024 && m <= 32);
+}
+
+template <int EPI>
+static int launch_skinny_f32(const void* a, const void* w, const float* bias, void* c, int m, int n,
+                             int k, int lda, int ldc, const KvScatter& scatter, hipStream_t s) {
+  const int row_blocks = (m + 15) / 16;
+  int k_splits = 1, k_chunk = k;
+#define PS_LAUNCH_SF(MB, NT, UNROLL, WAVES)                                                         \
+  hipLaunchKernelGGL((gemm_nt_skinny_f32_kernel<EPI, MB, NT, UNROLL, WAVES>),                       \
+                     dim3((n + 16 * NT - 1) / (16 * NT), k_splits, (row_blocks + MB - 1) / MB),     \
+                     dim3(64 * WAVES), 0, s, (const float*)a, (const float*)w, bias, (float*)c, m,  \
+                     n, k, lda, ldc, k_chunk, k_splits, scatter)
+  if (EPI == PS_EPI_RESIDUAL && m > 16) {
+    // ranges of one round of four waves' loads (32 x 768 x 3072: 7.2 us with ranges of 384, 8.7 with 768)
+    k_splits = (k + 4 * 3 * SF_STEP - 1) / (4 * 3 * SF_STEP);
+    k_chunk = ((k + k_splits - 1) / k_splits + SF_STEP - 1) / SF_STEP * SF_STEP;
+    k_splits = (k + k_chunk - 1) / k_chunk;
+    PS_LAUNCH_SF(2, 1, 3, 4);
+  } else if (m <= 16) {
+    // (up to 1,024 k stay in one block: no atomics)
+    if (EPI == PS_EPI_RESIDUAL && k > 1024) {
+      k_splits = (k + 8 * 3 * SF_STEP - 1) / (8 * 3 * SF_STEP);
+      k_chunk = ((k + k_splits - 1) / k_splits + SF_STEP - 1) / SF_STEP * SF_STEP;
+      k_splits = (k + k_chunk - 1) / k_chunk;
+    }
+    if (n >= 64 * 256) PS_LAUNCH_SF(1, 2, 3, 8);
+    else if (k_chunk <= 8 * 3 * SF_STEP) PS_LAUNCH_SF(1, 1, 3, 8);
+    else PS_LAUNCH_SF(1, 1, 4, 8);
+  } else if (k > 8 * 3 * SF_STEP) PS_LAUNCH_SF(1, 1, 4, 8);
+  else if (m <= 32) PS_LAUNCH_SF(2, 1, 3, 8);
+  else PS_LAUNCH_SF(2, 2, 3, 8);
+#undef PS_LAUNCH_SF
+  PS_CHECK_LAUNCH("ps_linear(skinny, float)");
+  return 0;
+}
+
+int ps_gemm_nt_f32_skinny(const void* a, const void* w, const float* bias, void* c, int m, int n,
+                          int k, int lda, int ldc, int epilogue, const KvScatter& scatter,
+                          hipStream_t s) {
+#define PS_SKINNY_CASE(EPI) \
+  case EPI: return launch_skinny_f32<EPI>(a, w, bias, c, m, n, k, lda, ldc, scatter, s)
+  switch (epilogue) {
+    PS_SKINNY_CASE(PS_EPI_NONE);
+    PS_SKINNY_CASE(PS_EPI_GELU_TANH);
+    PS_SKINNY_CASE(PS_EPI_GELU_ERF);
+    PS_SKINNY_CASE(PS_EPI_RELU2);
+    PS_SKINNY_CASE(PS_EPI_RESIDUAL);
+    default: ps_set_error("ps_linear: unknown epilogue %d", epilogue); return 1;
+  }
+#undef PS_SKINNY_CASE
+}

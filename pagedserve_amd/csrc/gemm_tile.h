@@ -1,5 +1,5 @@
-// What the tiled bfloat16 products share: vector types, the fast GELU of a bfloat16 result, and
-// the epilogue that takes a wave's 32 x 32 accumulators to memory.
+// What the tiled products share: vector types, a step of the matrix cores, the fast GELU of a
+// bfloat16 result, and the epilogue that takes a wave's 32 x 32 accumulators to memory.
 #pragma once
 
 #include "common.h"
@@ -9,8 +9,31 @@
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16;
 
-#define TB_BK 64     // values of k per stage
+#define TB_BK 64     // bfloat16 values of k per stage
 #define TB_ROW 128   // bytes per row and stage
+
+typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_t;
+
+// One step of the matrix cores on 16 bytes of k per lane, into ACCS accumulators whose sum is the
+// result.  bfloat16: the operand of one v_mfma_f32_32x32x16_bf16.  float: the four values feed four
+// v_mfma_f32_32x32x2_f32, true 32-bit products and sums (both operands use the same assignment of k
+// to lanes and instructions, which is all a dot product needs), which take turns in the accumulators:
+// with four of them the chains are a quarter as long and have half the rounding error, and no
+// instruction waits for the one before.
+template <int ACCS>
+__device__ inline void mma_step(bf16_t, const u32x4_t& a, const u32x4_t& w, f32x16 (&acc)[ACCS]) {
+  static_assert(ACCS == 1, "one instruction per step");
+  acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                   __builtin_bit_cast(bf16x8, w), acc[0], 0, 0, 0);
+}
+template <int ACCS>
+__device__ inline void mma_step(float, const u32x4_t& a, const u32x4_t& w, f32x16 (&acc)[ACCS]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    acc[i % ACCS] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+        __builtin_bit_cast(float, (uint32_t)a[i]), __builtin_bit_cast(float, (uint32_t)w[i]),
+        acc[i % ACCS], 0, 0, 0);
+}
 
 typedef const __attribute__((address_space(1))) void* global_ptr_t;
 typedef __attribute__((address_space(3))) void* lds_ptr_t;

@@ -1,16 +1,17 @@
-// Tiled bfloat16 matrix product for many rows (prompt portions) on gfx950:
-//   C[m, n] = epi(sum_k A[m, k] W[n, k] + b[n]),   k a multiple of 64.
+// Tiled matrix product for many rows (prompt portions) on gfx950, in bfloat16 or in true 32-bit:
+//   C[m, n] = epi(sum_k A[m, k] W[n, k] + b[n]),   rows of k in whole pieces of 128 bytes.
 //
 // Operand tiles go from global memory straight into LDS (global_load_lds_dwordx4: no trip
-// through registers), several k tiles ahead of the one being multiplied.  A stage holds 64
-// values of k (128 bytes) of every row of the block's A and W tiles.  One load instruction of
+// through registers), several k tiles ahead of the one being multiplied.  A stage holds 128
+// bytes (64 bfloat16 or 32 float values of k) of every row of the block's A and W tiles.  One load instruction of
 // a wave fills 1024 contiguous bytes of LDS, eight rows; which 16-byte piece of its row a
 // lane fetches is chosen so that piece c of row r lands in slot c ^ ((r >> 1) & 7) of the
 // row.  With that, the 16 lanes that read one k piece of 16 consecutive rows for an MFMA
 // operand touch every LDS bank once.
 //
 // Four waves in a 2 x 2 arrangement; a wave owns WM x WN accumulators of 32 x 32
-// (v_mfma_f32_32x32x16_bf16, float accumulation), so a block makes 64 WM x 64 WN outputs.
+// (v_mfma_f32_32x32x16_bf16 or v_mfma_f32_32x32x2_f32, float accumulation), so a block makes 64 WM x
+// 64 WN outputs.
 // With KW = 2 the two waves of a row of the arrangement share one accumulator of 32 columns
 // instead and take every other k tile each; the block meets once per pair of tiles, and the
 // two sums meet in LDS at the end.  A block then makes 64 x 32 outputs: twice as many blocks
@@ -28,7 +29,7 @@
 #include "linear.h"
 #include "pagedserve_hip.h"
 
-#include "gemm_bf16_common.h"
+#include "gemm_tile.h"
 
 // Wait until at most `pending` of this wave's loads are in flight, then meet the other waves.
 // The asm statements are compiler barriers for memory as well: LDS reads stay behind them.
@@ -49,13 +50,15 @@ __device__ inline void wait_ahead_and_sync(int ahead) {
   else wait_loads_and_sync<(MOST >= 6 ? 6 : 0) * LOADS>();
 }
 
-template <int WM, int WN, int STAGES, typename TOut, int EPI, int KW = 1>
-__global__ __launch_bounds__(256) void gemm_nt_bf16_tiled_kernel(
-    const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, const float* __restrict__ bias,
+template <typename T, int WM, int WN, int STAGES, typename TOut, int EPI, int KW = 1>
+__global__ __launch_bounds__(256) void gemm_nt_ring_kernel(
+    const T* __restrict__ a, const T* __restrict__ w, const float* __restrict__ bias,
     TOut* __restrict__ c, int m, int n, int k, int lda, int ldc, int tiles_m, int tiles_n,
     int row_major, int k_splits, int k_chunk, KvScatter scatter) {
   static_assert(KW == 1 || (KW == 2 && WM == 1 && WN == 1), "k halves go with one accumulator per wave");
   constexpr int BM = 64 * WM, BN = 64 * WN / KW;
+  constexpr int BK = TB_ROW / (int)sizeof(T);     // values of k per stage
+  constexpr int PIECE = 16 / (int)sizeof(T);      // values of k in 16 bytes
   constexpr int STAGE_BYTES = (BM + BN) * TB_ROW;
   constexpr int LOADS_A = BM / 32;   // load instructions per wave and stage (8 rows each)
   constexpr int LOADS_W = BN / 32;
@@ -86,10 +89,10 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_tiled_kernel(
   const int m0 = tile_m * BM;
   const int n0 = tile_n * BN;
   const int k_begin = split * k_chunk;
-  const int k_tiles = ((k_begin + k_chunk < k ? k_begin + k_chunk : k) - k_begin) / TB_BK;
+  const int k_tiles = ((k_begin + k_chunk < k ? k_begin + k_chunk : k) - k_begin) / BK;
 
   // ---- loads: lane l of a load instruction fills slot l % 8 of row l / 8 of its eight rows
-  const bf16_t* src[LOADS];
+  const T* src[LOADS];
   int dst[LOADS];
 #pragma unroll
   for (int j = 0; j < LOADS; ++j) {
@@ -99,11 +102,11 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_tiled_kernel(
     const int piece = (lane & 7) ^ ((tile_row >> 1) & 7);
     if (is_a) {
       const int row = m0 + tile_row < m ? m0 + tile_row : m - 1;
-      src[j] = a + (int64_t)row * lda + k_begin + piece * 8;
+      src[j] = a + (int64_t)row * lda + k_begin + piece * PIECE;
       dst[j] = group * 8 * TB_ROW;
     } else {
       const int row = n0 + tile_row < n ? n0 + tile_row : n - 1;
-      src[j] = w + (int64_t)row * k + k_begin + piece * 8;
+      src[j] = w + (int64_t)row * k + k_begin + piece * PIECE;
       dst[j] = (BM + group * 8) * TB_ROW;
     }
   }
@@ -111,17 +114,21 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_tiled_kernel(
     unsigned char* stage = lds + (kt % STAGES) * STAGE_BYTES;
 #pragma unroll
     for (int j = 0; j < LOADS; ++j)
-      __builtin_amdgcn_global_load_lds((global_ptr_t)(src[j] + (int64_t)kt * TB_BK),
+      __builtin_amdgcn_global_load_lds((global_ptr_t)(src[j] + (int64_t)kt * BK),
                                        (lds_ptr_t)(stage + dst[j]), 16, 0, 0);
   };
 
-  f32x16 acc[WM][WN];
+  // (128 x 128 tiles have registers for two accumulators of a float sum)
+  constexpr int ACCS = sizeof(T) == 2 ? 1 : (WM * WN == 4 ? 2 : 4);
+  f32x16 sums[WM][WN][ACCS];
 #pragma unroll
   for (int i = 0; i < WM; ++i)
 #pragma unroll
     for (int j = 0; j < WN; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+      for (int p = 0; p < ACCS; ++p)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sums[i][j][p][e] = 0.f;
 
   // ---- operands: lane l reads the 16 bytes of k piece 2 s + l / 32 of row l % 32
   const int key = (lane >> 1) & 7;   // ((row >> 1) & 7) of every row this lane reads
@@ -138,11 +145,10 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_tiled_kernel(
   // lone block took 800 cycles, of which the matrix instructions are 128.  LDS reads come back
   // in the order of issue: waiting until READS are left in flight leaves exactly the next
   // step's.
-  typedef unsigned int tb_u32x4 __attribute__((ext_vector_type(4)));
   constexpr int READS = WM + WN;    // LDS reads of one k step
-  tb_u32x4 fa[2][WM], fw[2][WN];
+  u32x4_t fa[2][WM], fw[2][WN];
   const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_ptr_t)lds;
-  auto fetch = [&](int kt, int s, tb_u32x4* da, tb_u32x4* dw) {
+  auto fetch = [&](int kt, int s, u32x4_t* da, u32x4_t* dw) {
     const uint32_t stage = lds_base + (uint32_t)((kt % STAGES) * STAGE_BYTES);
     const uint32_t slot = (uint32_t)(((2 * s + (lane >> 5)) ^ key) << 4);
 #pragma unroll
@@ -158,7 +164,7 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_tiled_kernel(
                    : "v"(stage + (uint32_t)(w_row + j * 32 * TB_ROW) + slot)
                    : "memory");
   };
-  constexpr int STEPS = TB_BK / 16;
+  constexpr int STEPS = TB_ROW / 32;   // 16 bytes of k from each half of the wave
   static_assert(STEPS % 2 == 0, "the operand buffers alternate per step");
 
   if constexpr (KW == 2) {
@@ -182,7 +188,7 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_tiled_kernel(
       if (kt < k_tiles) {
         // all four steps' operands are asked for at once and used as they arrive (reads come
         // back in the order of issue): one trip to LDS per tile stands open, not one per step
-        tb_u32x4 ga[STEPS], gw[STEPS];
+        u32x4_t ga[STEPS], gw[STEPS];
 #pragma unroll
         for (int s = 0; s < STEPS; ++s) fetch(kt, s, &ga[s], &gw[s]);
 #pragma unroll
@@ -193,9 +199,7 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_tiled_kernel(
           else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
           asm volatile("" : "+v"(ga[s]));
           asm volatile("" : "+v"(gw[s]));
-          acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              *reinterpret_cast<const bf16x8*>(&ga[s]), *reinterpret_cast<const bf16x8*>(&gw[s]),
-              acc[0][0], 0, 0, 0);
+          mma_step(T{}, ga[s], gw[s], sums[0][0]);
         }
       }
     }
@@ -238,15 +242,24 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_tiled_kernel(
   #pragma unroll
         for (int i = 0; i < WM; ++i)
   #pragma unroll
-          for (int j = 0; j < WN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                *reinterpret_cast<const bf16x8*>(&fa[s & 1][i]),
-                *reinterpret_cast<const bf16x8*>(&fw[s & 1][j]), acc[i][j], 0, 0, 0);
+          for (int j = 0; j < WN; ++j) mma_step(T{}, fa[s & 1][i], fw[s & 1][j], sums[i][j]);
       }
     }
   }
 
-  // ---- epilogue (gemm_bf16_common.h): each wave turns its accumulators through a region of
+  f32x16 acc[WM][WN];
+#pragma unroll
+  for (int i = 0; i < WM; ++i)
+#pragma unroll
+    for (int j = 0; j < WN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        acc[i][j][e] = ACCS == 1   ? sums[i][j][0][e]
+                       : ACCS == 2 ? sums[i][j][0][e] + sums[i][j][1 % ACCS][e]
+                                   : (sums[i][j][0][e] + sums[i][j][1 % ACCS][e]) +
+                                         (sums[i][j][2 % ACCS][e] + sums[i][j][3 % ACCS][e]);
+
+  // ---- epilogue (gemm_tile.h): each wave turns its accumulators through a region of
   // LDS of its own and stores rows in aligned pieces
   static_assert(4 * 32 * (WN * 32 + 8) * 4 + (KW - 1) * 2 * 16 * 64 * 4 <= STAGES * STAGE_BYTES,
                 "the epilogue reuses the stages");
@@ -277,11 +290,12 @@ bool ps_gemm_nt_bf16_tiled_supported(const void* a, const void* w, int m, int k,
          (reinterpret_cast<uintptr_t>(a) & 15u) == 0 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
 }
 
-template <int WM, int WN, int STAGES, typename TOut, int KW = 1>
+template <typename T, int WM, int WN, int STAGES, typename TOut, int KW = 1>
 static int launch_variant(const void* a, const void* w, const float* bias, void* c, int m, int n,
                           int k, int lda, int ldc, int epilogue, const KvScatter& scatter,
                           hipStream_t s) {
   constexpr int BM = 64 * WM, BN = 64 * WN / KW;
+  constexpr int BK = TB_ROW / (int)sizeof(T);
   const int tiles_m = (m + BM - 1) / BM;
   const int tiles_n = (n + BN - 1) / BN;
   // what one XCD's run of tiles fetches into its L2, in rows of k values
@@ -292,17 +306,26 @@ static int launch_variant(const void* a, const void* w, const float* bias, void*
   // Few tiles with a long k leave most of the chip idle: where partial sums can be added in
   // place (residual epilogue) k is split over blocks.  Float atomics are slow, so this pays
   // only while the output is small.
+  // float products keep the matrix cores sixteen times as long, so there the adds weigh less: as many
+  // ranges of a long k as leave at most three blocks per compute unit (with one range and with this
+  // many: 330 x 1024 x 4096 50 and 43 us, 1024 x 768 x 3072 60 and 56; but 1024 x 768 x 768 18 and 28)
   int k_splits = 1;
-  if (epilogue == PS_EPI_RESIDUAL && tiles_m * tiles_n <= ps_compute_units() / 4 && k >= 2048) {
+  if (sizeof(T) == 4) {
+    if (epilogue == PS_EPI_RESIDUAL && k > 1024) {
+      k_splits = 3 * ps_compute_units() / (tiles_m * tiles_n);
+      if (k_splits > k / 256) k_splits = k / 256;
+      if (k_splits < 1) k_splits = 1;
+    }
+  } else if (epilogue == PS_EPI_RESIDUAL && tiles_m * tiles_n <= ps_compute_units() / 4 && k >= 2048) {
     k_splits = ps_compute_units() / (tiles_m * tiles_n);
     if (k_splits > k / 256) k_splits = k / 256;
   }
-  int k_chunk = (k / TB_BK + k_splits - 1) / k_splits * TB_BK;
+  int k_chunk = (k / BK + k_splits - 1) / k_splits * BK;
   k_splits = (k + k_chunk - 1) / k_chunk;
   dim3 grid(tiles_m * tiles_n * k_splits);
 #define PS_LAUNCH_TB(EPI)                                                                     \
-  hipLaunchKernelGGL((gemm_nt_bf16_tiled_kernel<WM, WN, STAGES, TOut, EPI, KW>), grid, dim3(256), 0, \
-                     s, (const bf16_t*)a, (const bf16_t*)w, bias, (TOut*)c, m, n, k, lda, ldc, \
+  hipLaunchKernelGGL((gemm_nt_ring_kernel<T, WM, WN, STAGES, TOut, EPI, KW>), grid, dim3(256), 0, \
+                     s, (const T*)a, (const T*)w, bias, (TOut*)c, m, n, k, lda, ldc, \
                      tiles_m, tiles_n, row_major, k_splits, k_chunk, scatter)
   switch (epilogue) {
     case PS_EPI_NONE: PS_LAUNCH_TB(PS_EPI_NONE); break;
@@ -313,7 +336,7 @@ static int launch_variant(const void* a, const void* w, const float* bias, void*
     default: ps_set_error("ps_linear: unknown epilogue %d", epilogue); return 1;
   }
 #undef PS_LAUNCH_TB
-  PS_CHECK_LAUNCH("ps_linear(tiled, bfloat16)");
+  PS_CHECK_LAUNCH("ps_linear(tiled)");
   return 0;
 }
 
@@ -328,17 +351,17 @@ static int launch_tiled_bf16(const void* a, const void* w, const float* bias, vo
   const int64_t tiles_128_64 = (int64_t)((m + 127) / 128) * ((n + 63) / 64);
   const int units = ps_compute_units();
   if (m > 64 && tiles_128 >= 3 * units)
-    return launch_variant<2, 2, 2, TOut>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
+    return launch_variant<bf16_t, 2, 2, 2, TOut>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
   // 128 x 64: three stages while two blocks per unit hold them all (1100 x 3072 x 1024 with
   // weights from memory: 16.1 against 17.7 us), two stages, which let a third block in, beyond
   if (m > 64 && tiles_128_64 >= units + units / 2 && tiles_128_64 <= 2 * units)
-    return launch_variant<2, 1, 3, TOut>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
+    return launch_variant<bf16_t, 2, 1, 3, TOut>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
   if (m > 64 && tiles_128_64 >= units + units / 2)
-    return launch_variant<2, 1, 2, TOut>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
+    return launch_variant<bf16_t, 2, 1, 2, TOut>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
   // a long k with a block per compute unit: four stages of 128 x 64 (2048 x 1024 x 4096 with
   // weights from memory: 34.7 us against 37.8 for 64 x 64 tiles)
   if (m > 64 && k >= 2048 && tiles_128_64 >= units)
-    return launch_variant<2, 1, 4, TOut>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
+    return launch_variant<bf16_t, 2, 1, 4, TOut>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
   // 64 x 64 tiles.  What a compute unit has in flight decides how long a k tile takes to
   // arrive from memory.  Many blocks fill a unit by their number and keep two stages, which
   // lets five of them in; up to two blocks per unit get four stages each.  That also holds for
@@ -362,13 +385,13 @@ static int launch_tiled_bf16(const void* a, const void* w, const float* bias, vo
   // steps of operands at once instead of one step ahead changes nothing, and eight waves on a
   // tile of 64 x 64, four for the even and four for the odd k tiles, gain a third of this.
   if ((2 * tiles_64 <= units || (k >= 2048 && 16 * tiles_64 <= 9 * units)) && k_tiles > 2)
-    return launch_variant<1, 1, 6, TOut, 2>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
+    return launch_variant<bf16_t, 1, 1, 6, TOut, 2>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
   if ((tiles_64 <= 2 * units && k_tiles > 2) || k >= 2048)
-    return launch_variant<1, 1, 4, TOut>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
+    return launch_variant<bf16_t, 1, 1, 4, TOut>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
   // up to three blocks per unit: three stages each (544 x 4096 x 1024: 15.9 against 18.2 us)
   if (tiles_64 <= 3 * units && k_tiles > 2)
-    return launch_variant<1, 1, 3, TOut>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
-  return launch_variant<1, 1, 2, TOut>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
+    return launch_variant<bf16_t, 1, 1, 3, TOut>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
+  return launch_variant<bf16_t, 1, 1, 2, TOut>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
 }
 
 int ps_gemm_nt_bf16_tiled(const void* a, const void* w, const float* bias, void* c, int m, int n,
@@ -377,4 +400,37 @@ int ps_gemm_nt_bf16_tiled(const void* a, const void* w, const float* bias, void*
   if (c_dtype == PS_F32)
     return launch_tiled_bf16<float>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
   return launch_tiled_bf16<bf16_t>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
+}
+
+// The same product in true 32-bit.  Its matrix instructions take sixteen times as long per value of
+// k, so that small tiles keep the matrix cores as busy as large ones would and balance better over
+// the compute units: 64 x 64 (three stages, or two where more than two blocks share a unit: 100 x 4800 x
+// 1600 36 us with three and 44 with two, 2048 x 4096 x 1024 162 and 155), or 64 x 32 where those leave
+// half of the units without a block (100 x 2304 x 768 11.9 against 18.5).  Only many rounds of blocks
+// make larger tiles worth their uneven last round: 128 x 64 from six of 64 x 64 per unit (2048 x 4800 x
+// 1600 272 against 282), 128 x 128 from four of its own (4096 x 4096 x 1024 283 against 300; with three, 4096 x
+// 3072 x 768, 200 against 175).  With weights from memory, the kernel that did this before (128 x 128
+// tiles; below 96 rows the plain kernel) and this one, in us: 2048 x 2304 x 768 110 / 75, 2048 x 3072 x
+// 768 120 / 95 (102 TFLOP/s; the library's 4096-cubed product reaches 139), 300 x 2304 x 768 65 / 19,
+// 544 x 768 x 768 35 / 12, 330 x 1024 x 4096 60 / 43, 64 x 50257 x 768 201 / 70, 4096 x 3072 x 768 172 / 175.
+bool ps_gemm_nt_f32_tiled_supported(const void* a, const void* w, int m, int k, int lda) {
+  return m > 16 && k % (TB_ROW / 4) == 0 && lda % 4 == 0 &&
+         (reinterpret_cast<uintptr_t>(a) & 15u) == 0 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
+}
+
+int ps_gemm_nt_f32_tiled(const void* a, const void* w, const float* bias, void* c, int m, int n,
+                         int k, int lda, int ldc, int epilogue, const KvScatter& scatter,
+                         hipStream_t s) {
+  const int64_t tiles_64 = (int64_t)((m + 63) / 64) * ((n + 63) / 64);
+  const int units = ps_compute_units();
+  const bool splits_k = epilogue == PS_EPI_RESIDUAL && k > 1024;
+  if (2 * tiles_64 <= units && !splits_k)
+    return launch_variant<float, 1, 1, 4, float, 2>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
+  if (tiles_64 <= 2 * units)
+    return launch_variant<float, 1, 1, 3, float>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
+  if ((int64_t)((m + 127) / 128) * ((n + 127) / 128) >= 4 * units)
+    return launch_variant<float, 2, 2, 2, float>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
+  if (tiles_64 >= 6 * units)
+    return launch_variant<float, 2, 1, 2, float>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
+  return launch_variant<float, 1, 1, 2, float>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
 }

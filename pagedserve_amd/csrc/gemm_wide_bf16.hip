@@ -3,7 +3,7 @@
 //
 // At the rate of the matrix cores a compute unit has to feed them 2 KB of operands per 32 x 32
 // x 16 product; LDS delivers 128 bytes per cycle and the vector cache 64.  The kernel in
-// gemm_tiled_bf16.hip brings both operands through LDS and reuses each fragment twice, which
+// gemm_tiled.hip brings both operands through LDS and reuses each fragment twice, which
 // fills the LDS path at half the matrix cores' rate.  Here a block is four waves side by side
 // along n: a wave owns 32 WM rows x 64 columns, the block 32 WM x 256.  The rows of A are
 // shared by the four waves and go through LDS (straight from global memory, three k tiles in
@@ -23,9 +23,7 @@
 // flight.
 #include <type_traits>
 
-#include "gemm_bf16_common.h"
-
-typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_t;
+#include "gemm_tile.h"
 
 #define GW_WN 2          // 32-column fragments per wave
 #define GW_BN 256        // columns per block
@@ -61,7 +59,7 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_wide_kernel(
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // the same in every lane: scalar
-  // every XCD works on a contiguous run of tiles (see gemm_tiled_bf16.hip)
+  // every XCD works on a contiguous run of tiles (see gemm_tiled.hip)
   const int blocks = gridDim.x;
   const int per_xcd = blocks / 8;
   int tile = blockIdx.x;

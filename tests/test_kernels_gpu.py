@@ -154,6 +154,33 @@ def test_gemm_nt(dtype, m, n, k, epilogue):
     torch.testing.assert_close(out.double(), expected, atol=atol * 2, rtol=rtol)
 
 
+# Float rows on either side of the lines between the kernels (4 / 8 / 16 / 32 / 64 rows, one round of loads,
+# k a multiple of 32 or not, k split or not), with columns and a k that end inside a tile, a step and a round.
+@pytest.mark.parametrize("m,n,k", [(4, 100, 4096), (5, 2100, 516), (8, 1400, 772), (9, 37, 4), (16, 16400, 100), (16, 50, 1028),
+                                   (17, 70, 36), (32, 130, 768), (33, 310, 768), (64, 95, 736), (32, 77, 1024), (65, 200, 800),
+                                   (20, 60, 3104), (100, 1500, 3072), (230, 1040, 768), (70, 90, 100), (800, 40, 68),
+                                   (65, 33, 32), (129, 4200, 64), (300, 65, 2080)])
+@pytest.mark.parametrize("epilogue", ["none", "gelu_tanh", "residual"])
+def test_gemm_of_float_rows(m, n, k, epilogue):
+    from pagedserve_amd.ops import kernels
+
+    a = _rand((m + 1, k + 4), torch.float32, 15)[:m, :k]      # (rows further apart than k)
+    w = _rand((n, k), torch.float32, 16, 1.0 / math.sqrt(k))
+    bias = _rand((n,), torch.float32, 17)
+    expected = a.double() @ w.double().t() + bias.double()
+    wide = _rand((m + 1, n + 3), torch.float32, 18)
+    before, out = wide.clone(), wide[:m, :n]
+    if epilogue == "gelu_tanh":
+        expected = F.gelu(expected, approximate="tanh")
+    elif epilogue == "residual":
+        expected = before[:m, :n].double() + expected
+    kernels.gemm_nt(a, w, bias, out, epilogue=epilogue)
+    # a sum of k products of size 1 / sqrt(k) in float: each of k additions rounds at most 2^-24 of a sum
+    # that stays near 1 in size, errors adding like a walk
+    torch.testing.assert_close(out.double(), expected, atol=2e-6 * math.sqrt(k) / 8 + 4e-6, rtol=4e-6)
+    assert torch.equal(wide[:, n:], before[:, n:]) and torch.equal(wide[m:], before[m:])
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_gemm_float_logits_and_strided_views(dtype):
     """bfloat16 operands with float output (the head), inputs and outputs that are column
