@@ -46,7 +46,8 @@ struct DecodeLds {
 
 // The work of one block: token n of the list, one head, one range of its keys.  The caller
 // provides the block's LDS (the kernel below its own; a kernel that runs blocks of several
-// kinds in one launch a share of what all of them need).
+// kinds in one launch a share of what all of them need).  `context` (one split only): the head's
+// finished values go there, into LDS, for the caller to go on with, instead of to `out`.
 template <typename T, int LPK, int AD_WAVES, int AD_UNROLL, bool NT>
 __device__ __forceinline__ void attention_decode_block(
     DecodeLds<AD_WAVES>& lds, const int n, const int head, const int split,
@@ -56,7 +57,7 @@ __device__ __forceinline__ void attention_decode_block(
     const int* __restrict__ tok_item, const int* __restrict__ tok_pos,
     const int* __restrict__ tables, int table_width, int heads, int kv_heads, int head_dim,
     int page_size, int page_shift, int num_pages, float scale_log2, int window, int splits,
-    const AttnExtras extra) {
+    const AttnExtras extra, T* context = nullptr) {
   constexpr int GROUPS = 64 / LPK;               // keys per wave load
   constexpr int KEYS_PER_WAVE = GROUPS * AD_UNROLL;
   float (&s_acc)[AD_WAVES][256] = lds.acc;
@@ -234,7 +235,9 @@ __device__ __forceinline__ void attention_decode_block(
     block_l += s_ml[w][1] * c;
     if (d < head_dim) value += s_acc[w][d] * c;
   }
-  if (splits == 1 && out != nullptr) {
+  if (context != nullptr) {
+    if (d < head_dim) context[d] = from_float<T>(value / block_l * gate_factor(extra, t, head));
+  } else if (splits == 1 && out != nullptr) {
     if (d < head_dim)
       out[(int64_t)t * out_stride + (int64_t)head * head_dim + d] =
           from_float<T>(value / block_l * gate_factor(extra, t, head));

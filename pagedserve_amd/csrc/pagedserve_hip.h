@@ -199,6 +199,19 @@ int ps_attention_merge_linear(const float* partial, int64_t partial_floats, cons
                               const void* w_packed, const float* bias, float* residual,
                               int64_t ld_res, int n, int tiles_per_block, void* stream);
 
+// Decode attention and output projection in one launch, for up to 64 tokens of items 0 .. count - 1
+// (token t is item t) and heads of 64 or 128, bfloat16:  residual[t, :] += context of token t  W^T +
+// bias, W [n, heads * head_dim] in its packed copy.  One block per (token, head, part of the
+// columns): `parts` parts, each of which repeats the attention; `waves` (4, 8 or 16) to a block.
+int ps_attention_decode_linear(const void* q, int64_t q_stride, const void* k_pool,
+                               const void* v_pool, const int* tok_pos, const int* tables,
+                               int table_width, int count, int heads, int kv_heads, int head_dim,
+                               int page_size, int num_pages, float scale, int window,
+                               const float* sink, const float* gate, int64_t gate_ld, float softcap,
+                               const float* logistic, float logistic_norm, const void* w_packed,
+                               const float* bias, float* residual, int64_t ld_res, int n, int parts,
+                               int waves, void* stream);
+
 // ps_attention_decode for callers that cannot allocate device memory: code under HIP graph
 // capture, tight serving loops, harnesses that forbid hipMalloc.  It has no counterpart in the
 // reference.  The partial results of the key ranges go into a device array that is part of the

@@ -107,6 +107,10 @@ _SIGNATURES = {
                                     c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
                                     c_int, c_int, c_float, c_int, c_int, c_int, c_void_p, c_float, c_void_p, c_float, c_int,
                                     c_void_p],
+    "ps_attention_decode_linear": [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int,
+                                   c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_void_p, c_void_p,
+                                   c_int64, c_float, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_int64,
+                                   c_int, c_int, c_int, c_void_p],
     "ps_attention_merge_linear": [c_void_p, c_int64, c_void_p, c_int, c_int, c_int, c_int, c_void_p,
                                   c_void_p, c_void_p, c_int64, c_int, c_int, c_void_p],
     "ps_attention_tiled_f32": [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_void_p,
@@ -897,6 +901,46 @@ def attention_decode_partial(q, k_pool, v_pool, partial, tok_item, tok_pos, tabl
           float(scale), int(window), int(splits), int(waves), _check_sink(sink, heads),
           _check_cap(softcap), *_check_logistic(logistic, heads), dtype_code(q.dtype), _stream())
     return count
+
+
+def decode_linear_supported(dtype, tokens, head_dim, packed) -> bool:
+    """Whether ``attention_decode_linear`` takes a step: bfloat16, up to 64 single-token items, heads
+    of 64 or 128, and the packed copy of the output projection's matrix."""
+    return dtype == torch.bfloat16 and packed is not None and 1 <= tokens <= 64 and head_dim in (64, 128)
+
+
+def attention_decode_linear(q, k_pool, v_pool, tok_pos, tables, heads, scale, w, packed, bias, residual, parts, waves,
+                            window=0, sink=None, gate=None, softcap=0.0, logistic=None):
+    """residual[t] += (decode attention of token t, which is item t) w^T + bias, in one launch; ``packed`` is
+    ``pack_decode_weight(w)``.  ``parts``: into how many parts the columns are dealt, one block per (token,
+    head, part); ``waves``: 4, 8 or 16 to a block."""
+    _check(q, "q", torch.bfloat16, 2)
+    pages, kv_heads, page_size, head_dim = _check_pools(k_pool, v_pool, q.dtype)
+    q_stride = _rows(q, "q")
+    tokens = q.shape[0]
+    if q.shape[1] != heads * head_dim:
+        raise KernelError("attention: q rows must hold heads x head_dim values")
+    _check_step_index(None, tok_pos, tables, tokens, direct_items=True)
+    _check(residual, "residual", torch.float32, 2)
+    _check(w, "w", torch.bfloat16, 2)
+    n, k = w.shape
+    if k != heads * head_dim or residual.shape[1] != n or residual.shape[0] < tokens:
+        raise KernelError(f"attention_decode_linear: w {tuple(w.shape)} and residual {tuple(residual.shape)} do not "
+                          f"fit {tokens} rows of {heads} heads of {head_dim}")
+    if packed is None or packed.dtype != torch.bfloat16 or not packed.is_contiguous() \
+            or packed.numel() != -(-n // 16) * 16 * k:
+        raise KernelError("attention_decode_linear: the packed copy does not belong to w")
+    if bias is not None:
+        _check(bias, "bias", torch.float32, 1)
+        if bias.numel() != n or not bias.is_contiguous():
+            raise KernelError("attention_decode_linear: bias does not match n")
+    gate_ptr, gate_ld = _check_gate(gate, tokens, heads)
+    _call("ps_attention_decode_linear", q.data_ptr(), q_stride, k_pool.data_ptr(), v_pool.data_ptr(),
+          tok_pos.data_ptr(), tables.data_ptr(), tables.shape[1], tokens, heads, kv_heads, head_dim, page_size, pages,
+          float(scale), int(window), _check_sink(sink, heads), gate_ptr, gate_ld, _check_cap(softcap),
+          *_check_logistic(logistic, heads), packed.data_ptr(), _ptr(bias), residual.data_ptr(),
+          _rows(residual, "residual"), n, int(parts), int(waves), _stream())
+    return residual
 
 
 def attention_merge_linear(partial, count, heads, head_dim, splits, w, packed, bias, residual, tok_list=None,

@@ -373,12 +373,22 @@ class Attention(Mixer):
             # a head size that the split-KV kernel does not take: every token, decoded ones
             # too, goes to the kernel that takes all sizes
             singles = 0
+        if residual is not None and singles == tokens and kernels.decode_linear_supported(
+                self.dtype, tokens, self.head_dim, self.out_packed):
+            shape = self._one_launch_decode(singles, ctx.max_kv_len)
+            if shape is not None:
+                # a decode step over some hundreds of keys: attention and output projection in one launch
+                kernels.attention_decode_linear(q, cache.k_pool, cache.v_pool, ctx.positions, tables, self.heads,
+                                                self.scale, self.out_weight, self.out_packed, self.out_bias, residual,
+                                                *shape, window=self.span, sink=sink, gate=gates,
+                                                softcap=self.score_cap, logistic=self.logistic)
+                return
         merged_splits = 0
         if residual is not None and gates is None and singles == tokens and kernels.merge_linear_supported(
                 self.dtype, tokens, self.head_dim, self.out_packed):
             merged_splits = self._merged_splits(singles, ctx.max_kv_len)
         if merged_splits:
-            # a decode step of few tokens over long contexts: the key ranges are merged inside
+            # a decode step of few tokens over longer contexts: the key ranges are merged inside
             # the output projection, which is split over the heads: no launch for the merge
             splits = merged_splits
             partial = self._range_records(ctx)
@@ -490,6 +500,50 @@ class Attention(Mixer):
         """Most keys that a query of a step sees whose longest request has ``max_kv_len``."""
         limit = self.window or self.chunk
         return min(max_kv_len, limit) if limit else max_kv_len
+
+    def _one_launch_decode(self, count: int, max_kv_len: int):
+        """(parts, waves) for the kernel that does attention and output projection of a decode step in
+        one launch, or ``None`` where two launches are as fast: ``parts`` blocks per (token, head) pair, each
+        with all keys and a part of the columns, blocks of ``waves`` waves.  (us for attention and
+        projection together, keys and weights from memory, two launches and one; keys in units of 64
+        dimensions.)
+
+        * The keys of a pair go through one compute unit: up to 1,024 of them that costs less than a
+          second launch (1, 8 and 16 requests of 12 heads over 144 keys 8.6 / 5.9, 9.2 / 7.7 and 11.0 / 8.4, over
+          540 keys 9.7 / 8.3, 13.6 / 10.5 and 16.4 / 12.3, over 1,000 keys 9.7 / 9.5, 14.8 / 12.6 and
+          19.1 / 15.4); beyond, ranges are ahead (over 2,000 keys 10.2 / 13.8 and 18.3 / 18.9) unless the
+          pairs fill half of the units, where the two-launch path has few ranges or none either (23.9
+          / 20.5 with 12 requests).
+        * Parts until the blocks come to one per unit.  Up to 128 keys blocks of four waves are over
+          soonest and two or three of them share a unit (16 requests over 40 keys 8.6 / 7.0 in 3 parts, 8.0
+          with one block of 16 waves); up to 512 keys eight waves take them in one round of loads, beyond or without
+          parts sixteen.
+        * Between one and one and a half pairs per unit, up to 512 keys: four waves, two parts (24
+          requests over 270 keys 15.5 / 12.7; over 1,000 keys 23.6 / 24.5).
+        * Not where a block would take in more than 128 KB of weights, nor beyond some 330,000
+          atomic adds (8 requests of 25 heads at width 1,600 over 144 keys: 11.7 / 13.5).  An engine whose
+          requests never see 128 keys (a toy's bound, a tiny window) keeps the two launches, whose number
+          the tests of recorded steps count on."""
+        pairs = count * self.heads
+        units = kernels.compute_units()
+        keys = self._visible(max_kv_len) * self.head_dim // 64
+        if 2 * pairs > 3 * units or pairs * self.width > 330_000 or keys < 128:
+            return None
+        if keys <= 128:
+            parts, waves = max(1, min(12, (5 * units + pairs) // (2 * pairs))), 4
+        elif pairs > units:
+            if keys > 512:
+                return None
+            parts, waves = 2, 4
+        else:
+            if keys > 1024 and (2 * pairs < units or keys >= 4096):
+                return None
+            parts = min(8, units // pairs)
+            waves = 8 if parts > 1 and keys <= 512 else 16
+        parts = min(parts, -(-self.width // 16))
+        if self.width * self.head_dim * 2 > 131072 * parts:
+            return None
+        return parts, waves
 
     def _range_records(self, ctx):
         """Scratch for one record per (token, head, key range): always asked for at its largest

@@ -1161,6 +1161,52 @@ def test_linear_takes_the_wide_product_for_long_k():
     assert torch.equal(v_pool.view(torch.int16), v_ref.view(torch.int16))
 
 
+@pytest.mark.parametrize("heads,kv_heads,head_dim,page_size,width", [(12, 12, 64, 16, 768), (4, 2, 128, 12, 200), (3, 1, 64, 8, 40),
+                                                                     (6, 6, 128, 16, 1000)])
+@pytest.mark.parametrize("count", [1, 3, 16, 20])
+@pytest.mark.parametrize("parts,waves", [(1, 4), (1, 16), (2, 8), (3, 16), (7, 4)])
+@pytest.mark.parametrize("window", [0, 33, -32])
+def test_attention_with_the_output_projection_in_one_launch(heads, kv_heads, head_dim, page_size, width, count, parts, waves,
+                                                            window):
+    """residual + gated capped softmax(q K^T) V W^T + bias in float64 over the gathered pages: contexts around page
+    edges, more tiles of columns than a round of weights holds and fewer than waves, a width that ends inside a tile,
+    rows beyond the count untouched; with and without bias, gate, sink and cap."""
+    from pagedserve_amd.ops import kernels
+
+    dtype = torch.bfloat16
+    if parts > -(-width // 16):
+        pytest.skip("more parts than tiles of columns")
+    contexts = [1, 700, 16, 17, 31, 33, 128, 512, 15, 64, 2, 300, 90, 257, 1000, 48, 129, 8, 65, 1100][:count]
+    k_pool, v_pool, tables = _paged_fixture(dtype, contexts, kv_heads, head_dim, page_size, 411)
+    q = _rand((count, heads * head_dim), dtype, 412)
+    w = _rand((width, heads * head_dim), dtype, 413, 1.0 / math.sqrt(heads * head_dim))
+    packed = kernels.pack_decode_weight(w)
+    tok_item = torch.arange(count, dtype=torch.int32, device="cuda")
+    tok_pos = torch.tensor([c - 1 for c in contexts], dtype=torch.int32, device="cuda")
+    scale = head_dim ** -0.5
+    start = _rand((count + 2, width), torch.float32, 415)
+    assert kernels.decode_linear_supported(dtype, count, head_dim, packed)
+    for bias, sink, gate, cap in ((_rand((width,), torch.float32, 414), None, None, 0.0),
+                                  (None, _rand((heads,), torch.float32, 416), _rand((count, heads), torch.float32, 417), 2.0)):
+        # the same kernel's parts, launched one after the other, are tested on their own: their result in float64
+        context = torch.empty((count, heads * head_dim), dtype=dtype, device="cuda")
+        kernels.attention_rowwise(q, k_pool, v_pool, context, tok_item, tok_pos, tables, heads, scale, window, sink=sink,
+                                  gate=gate, softcap=cap)
+        if sink is None and window == 0:
+            context = _attention_expected(q, k_pool, v_pool, tables, tok_item, tok_pos, heads, scale).to(dtype)
+        expected = start[:count].double() + context.double() @ w.double().t()
+        if bias is not None:
+            expected += bias.double()
+        residual = start.clone()
+        kernels.attention_decode_linear(q, k_pool, v_pool, tok_pos, tables, heads, scale, w, packed, bias, residual, parts,
+                                        waves, window=window, sink=sink, gate=gate, softcap=cap)
+        # each context value is a bfloat16 on either side, here and there one step (2^-8 of it) apart: of sums of
+        # heads * head_dim products of size 1 / sqrt(heads * head_dim) some 2^-9 of the context's size (at most 4)
+        torch.testing.assert_close(residual[:count].double(), expected, atol=1e-2, rtol=5e-4)
+        assert float((residual[:count].double() - expected).norm() / (expected - start[:count].double()).norm()) < 3e-3
+        assert torch.equal(residual[count:], start[count:])
+
+
 @pytest.mark.parametrize("heads,kv_heads,head_dim,page_size", [(12, 12, 64, 16), (4, 2, 128, 12), (2, 1, 256, 16), (3, 3, 192, 8),
                                                                (5, 5, 64, 16)])
 @pytest.mark.parametrize("count", [1, 2, 3, 5, 8, 16])
