@@ -381,6 +381,12 @@ int ps_gla_output(const float* o, const float* w, float eps, const float* gate, 
 // logits[r, :vocab] = cap * tanh(logits[r, :vocab] / cap), rows ld floats apart.
 int ps_softcap(float* logits, int64_t ld, int rows, int vocab, float cap, void* stream);
 
+// dst[i] = src[i] for `words` 32-bit words, either side device memory or pinned host memory under
+// the address that ps_host_address gives for it.  The host may reuse or read the memory once an
+// event recorded behind the launch has happened.
+int ps_copy_words(const void* src, void* dst, int64_t words, void* stream);
+int ps_host_address(void* host, void** address);
+
 // ---- selective state-space mixer -------------------------------------------------------------
 // state: [slots, channels, states + taps - 1] float per request: the recurrence's numbers of a
 // channel and behind them its last taps - 1 raw inputs, oldest first.

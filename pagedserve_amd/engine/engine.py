@@ -14,6 +14,7 @@ only on (tokens, items, wanted rows), so a captured HIP graph of a decode step s
 valid from step to step.
 """
 
+import weakref
 from dataclasses import dataclass, field
 from typing import Hashable, List, Optional, Sequence
 
@@ -69,6 +70,14 @@ class _ReplayPlan:
         self.items = items
 
 
+def _drain(stream, *buffers):
+    """An engine is gone: its buffers are given back once its stream is through with them."""
+    try:
+        stream.synchronize()
+    except RuntimeError:       # (the device is gone with the process, or the work on it failed)
+        pass
+
+
 class StepError(ValueError):
     """A step that the engine refuses before anything ran."""
 
@@ -109,7 +118,8 @@ class Engine:
         capacity = ((7 + 2 * max(1, len(self.query_tiles))) * max_step_tokens + 5 * max_requests + 1
                     + len(groups) * max_requests * self.table_width + 16)
         self._meta_device = torch.empty(capacity, dtype=torch.int32, device=self.device)
-        self._meta_host = [torch.empty(capacity, dtype=torch.int32, pin_memory=True) for _ in range(2)]
+        self._meta_words = [kernels.HostWords(capacity) for _ in range(2)]
+        self._meta_host = [words.tensor for words in self._meta_words]
         self._meta_events = [torch.cuda.Event(), torch.cuda.Event()]
         self._meta_pending = [False, False]
         self._meta_owner = [None, None]   # replay plan whose constant arrays a buffer holds
@@ -118,18 +128,18 @@ class Engine:
         # chosen tokens: one per wanted row, and a step wants at most one row per token
         self._tokens = torch.zeros(max(max_requests, max_step_tokens), dtype=torch.int32,
                                    device=self.device)
-        self._tokens_host = [torch.zeros(self._tokens.numel(), dtype=torch.int32, pin_memory=True)
-                             for _ in range(2)]
+        self._tokens_words = [kernels.HostWords(self._tokens.numel()) for _ in range(2)]
+        self._tokens_host = [words.tensor for words in self._tokens_words]
         self._tokens_ready = [torch.cuda.Event(), torch.cuda.Event()]
         self._tokens_turn = 0
-        from ..ops import kernels
-
         self._top_choice = kernels.TopChoice(min(self._tokens.numel(), 64), self.device)
         self.tokens_chosen_by_head = 0   # greedy steps (launched or recorded) without a sampling launch
         self._carried_rows = 0    # rows of the last step whose chosen tokens a step may carry on
         # The engine's work runs on a stream of its own (default priority): a capture cannot
         # record from the default stream.
         self.stream = torch.cuda.Stream(device=self.device)
+        # the pinned buffers, which kernels access without the allocator's knowledge, outlive the work on them
+        weakref.finalize(self, _drain, self.stream, self._meta_words, self._tokens_words)
         # a part that looks at host values of a step cannot be replayed
         self.use_graphs = use_graphs and getattr(model, "graph_safe", False)
         self.max_graphs = 48     # recorded layouts kept; the least recently replayed goes first
@@ -446,8 +456,7 @@ class Engine:
         slot_index = np.asarray(slot_list, dtype=np.int64)
         for group in range(groups):
             section(f"tables{group}").reshape(items, width)[:] = cache.table_arrays[group][slot_index]
-        device = self._meta_device
-        device[:cursor].copy_(self._meta_host[turn][:cursor], non_blocking=True)
+        self._meta_words[turn].to_device(self._meta_device, cursor)
         self._meta_events[turn].record()
         self._meta_pending[turn] = True
         self._last_layout = (offsets, cursor)
@@ -493,7 +502,7 @@ class Engine:
             self._tokens_turn ^= 1
             rows = output.tokens.numel()
             output.host_tokens = self._tokens_host[turn][:rows]
-            output.host_tokens.copy_(output.tokens, non_blocking=True)
+            self._tokens_words[turn].from_device(output.tokens, rows)
             output.ready = self._tokens_ready[turn]
             output.ready.record()
             self._carried_rows = rows
@@ -648,7 +657,7 @@ class Engine:
             sections["uniform"].view(np.float32)[:] = [b for _, b in select]
         for group in range(len(cache.groups)):
             sections[f"tables{group}"][:] = cache.table_arrays[group][slots]
-        self._meta_device[:plan.used].copy_(self._meta_host[turn][:plan.used], non_blocking=True)
+        self._meta_words[turn].to_device(self._meta_device, plan.used)
         self._meta_events[turn].record()
         self._meta_pending[turn] = True
         plan.graph.launch()

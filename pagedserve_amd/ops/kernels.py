@@ -94,6 +94,8 @@ _SIGNATURES = {
                        c_int, c_float, c_int, c_void_p],
     "ps_gla_output": [c_void_p, c_void_p, c_float, c_void_p, c_int64, c_void_p, c_int64, c_int,
                       c_int, c_int, c_int, c_void_p],
+    "ps_copy_words": [c_void_p, c_void_p, c_int64, c_void_p],
+    "ps_host_address": [c_void_p, c_void_p],
     "ps_softcap": [c_void_p, c_int64, c_int, c_int, c_float, c_void_p],
     "ps_attention_decode": [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_void_p,
                             c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
@@ -2242,6 +2244,35 @@ def softcap(logits, cap):
         _call("ps_softcap", logits.data_ptr(), _rows(logits, "logits"), logits.shape[0], logits.shape[1],
               float(cap), _stream())
     return logits
+
+
+class HostWords:
+    """A pinned int32 buffer that kernels read and write themselves.  The copy engine's path holds a small
+    step up for tens of microseconds; a kernel's own access to the host's memory costs a launch and the trip.
+
+    The allocator does not see these accesses: whoever owns the buffer keeps it until they are through."""
+
+    def __init__(self, count: int):
+        self.tensor = torch.zeros(count, dtype=torch.int32, pin_memory=True)
+        address = c_void_p()
+        _call("ps_host_address", self.tensor.data_ptr(), ctypes.cast(ctypes.pointer(address), c_void_p))
+        self.address = address.value
+
+    def _check_range(self, device_words, count):
+        _check(device_words, "device words", torch.int32, 1)
+        if not (0 <= count <= self.tensor.numel() and count <= device_words.numel() and device_words.is_contiguous()):
+            raise KernelError(f"{count} words do not fit a host buffer of {self.tensor.numel()} and a contiguous device "
+                              f"buffer of {device_words.numel()}")
+
+    def to_device(self, target, count: int):
+        """target[:count] = the buffer's first ``count`` words, on the current stream."""
+        self._check_range(target, count)
+        _call("ps_copy_words", self.address, target.data_ptr(), count, _stream())
+
+    def from_device(self, source, count: int):
+        """The buffer's first ``count`` words = source[:count], on the current stream."""
+        self._check_range(source, count)
+        _call("ps_copy_words", source.data_ptr(), self.address, count, _stream())
 
 
 def sample(logits, inv_temperature, uniform, out):

@@ -1,5 +1,6 @@
 """The engine against the plain implementation under every way of cutting the work."""
 
+import ctypes
 import json
 import os
 import subprocess
@@ -372,3 +373,56 @@ def test_greedy_tokens_are_the_argmax_of_the_logits(folders, live):
     assert engine.graph_summary()["graph_replays"] >= 4
     torch.cuda.synchronize()
     assert int(engine._top_choice.keys.abs().sum()) == 0 and int(engine._top_choice.ticket.abs().sum()) == 0
+
+
+@pytest.mark.parametrize("count", [0, 1, 3, 4, 1023, 1024, 1025, 70001])
+@pytest.mark.parametrize("offset", [0, 1, 2])
+def test_words_between_host_memory_and_the_device(count, offset):
+    """Whole and ragged pieces, device buffers that do not start at 16 bytes, words behind the last one untouched;
+    what the host writes between two copies is seen by the second; ordinary memory is refused."""
+    from pagedserve_amd.ops import kernels
+
+    words = kernels.HostWords(70016)
+    device = torch.full((70016 + offset,), -7, dtype=torch.int32, device="cuda")[offset:]
+    for turn in range(2):
+        words.tensor[:] = torch.arange(70016, dtype=torch.int32) * (turn + 3) - 50000
+        device.fill_(-7)
+        words.to_device(device, count)
+        torch.cuda.synchronize()
+        assert torch.equal(device[:count].cpu(), words.tensor[:count]) and int((device[count:] != -7).sum()) == 0
+        device += 1
+        expected = words.tensor.clone()
+        expected[:count] += 1
+        words.from_device(device, count)
+        torch.cuda.synchronize()
+        assert torch.equal(words.tensor, expected)
+    with pytest.raises(kernels.KernelError):
+        words.to_device(device[:3], 4)
+    with pytest.raises(kernels.KernelError):
+        words.to_device(device.float(), 4)
+    if count == 1 and offset == 0:
+        plain = torch.zeros(64, dtype=torch.int32)
+        with pytest.raises(kernels.KernelError):
+            kernels._call("ps_host_address", plain.data_ptr(),
+                          ctypes.cast(ctypes.pointer(ctypes.c_void_p()), ctypes.c_void_p))
+        torch.cuda.synchronize()
+
+
+def test_an_engine_that_goes_with_work_in_flight_waits_for_it(tmp_path):
+    """The pinned buffers of an engine are accessed by kernels: they are given back when its stream is through."""
+    import gc
+    import weakref
+
+    from pagedserve_amd.engine import Engine, StepEntry
+    from pagedserve_amd.model import random_model
+
+    model, config = random_model({"architectures": ["GPT2LMHeadModel"], "n_layer": 2, "n_embd": 64, "n_head": 4,
+                                  "n_inner": 256, "vocab_size": 512, "n_positions": 128, "layer_norm_epsilon": 1e-5,
+                                  "activation_function": "gelu_new", "eos_token_id": None}, dtype="bfloat16")
+    engine = Engine(model, num_pages=32, page_size=8, max_requests=2, max_step_tokens=64)
+    for step in range(4):
+        out = engine.step([StepEntry("a", [5 + step], [0])], greedy=True)
+    stream, gone = engine.stream, weakref.ref(engine)
+    del engine, out
+    gc.collect()
+    assert gone() is None and stream.query()
