@@ -8,10 +8,16 @@
 // One pass over the stream's rows, every piece optional:
 //   h <- h + factor * column_scale * y + rows + bias;   zero <- 0 (may be y);
 //   normed <- h / sqrt(mean(h^2) + eps) * gamma;   normed2 <- the same * gamma2
-// (column_scale: a float per column, null for ones).  A block of 256 threads per token.
-#define STREAM_HELD 8      // numbers of a row that a thread may hold
-template <typename T>
-__global__ __launch_bounds__(256) void stream_step_kernel(
+// (column_scale: a float per column, null for ones).  A block per token.
+//
+// A decode step's launch is bound by its trips to memory.  HELD numbers of a row to a thread, all of
+// their operands asked for at once: an operand that is not there is stood in for by the row itself (a
+// load under a branch would wait for the ones before it) and not used.  With few tokens a thread takes
+// one column.  A product's sum added, normed and cleared, with 256 threads to a row and a trip per operand before and
+// now, in us: 8 x 768 4.0 / 3.2, 8 x 4096 10.5 / 4.3, 2048 x 768 8.3 / 7.0, 2048 x 1600 17.4 / 15.0.  HELD = 0:
+// rows longer than a block holds.
+template <typename T, int HELD>
+__global__ __launch_bounds__(1024) void stream_step_kernel(
     float* __restrict__ h, const float* y, float factor, const float* __restrict__ column_scale,
     const float* __restrict__ rows, const float* __restrict__ bias, const float* __restrict__ gamma, float eps,
     T* __restrict__ normed, const float* __restrict__ gamma2, T* __restrict__ normed2, float* zero, int width) {
@@ -19,38 +25,45 @@ __global__ __launch_bounds__(256) void stream_step_kernel(
   const int64_t t = blockIdx.x;
   float* row = h + t * width;
   float sum = 0.f;
-  if (width <= 256 * STREAM_HELD) {
-    // rows that a block holds in registers, with the scales asked for beside them: one trip to
-    // memory and no second reading of the row
-    float held[STREAM_HELD], scale[STREAM_HELD], scale2[STREAM_HELD];
+  if constexpr (HELD > 0) {
+    const float* y_row = y != nullptr ? y + t * width : row;
+    const float* rows_row = rows != nullptr ? rows + t * width : row;
+    const float* column = column_scale != nullptr ? column_scale : row;
+    const float* bias_row = bias != nullptr ? bias : row;
+    const float* scale_row = gamma != nullptr ? gamma : row;
+    const float* scale2_row = gamma2 != nullptr ? gamma2 : row;
+    float held[HELD], vy[HELD], vc[HELD], vr[HELD], vb[HELD], scale[HELD], scale2[HELD];
 #pragma unroll
-    for (int i = 0; i < STREAM_HELD; ++i) {
-      const int d = threadIdx.x + 256 * i;
-      held[i] = scale[i] = scale2[i] = 0.f;
-      if (d < width) {
-        float v = row[d];
-        if (gamma != nullptr) scale[i] = gamma[d];
-        if (gamma2 != nullptr) scale2[i] = gamma2[d];
-        if (y != nullptr) v = fmaf(column_scale ? factor * column_scale[d] : factor, y[t * width + d], v);
-        if (rows != nullptr) v += rows[t * width + d];
-        if (bias != nullptr) v += bias[d];
-        held[i] = v;
-      }
+    for (int i = 0; i < HELD; ++i) {
+      const int at = threadIdx.x + blockDim.x * i;
+      const int d = at < width ? at : width - 1;
+      held[i] = row[d];
+      vy[i] = y_row[d];
+      vc[i] = column[d];
+      vr[i] = rows_row[d];
+      vb[i] = bias_row[d];
+      scale[i] = scale_row[d];
+      scale2[i] = scale2_row[d];
     }
 #pragma unroll
-    for (int i = 0; i < STREAM_HELD; ++i) {
-      const int d = threadIdx.x + 256 * i;
+    for (int i = 0; i < HELD; ++i) {
+      const int d = threadIdx.x + blockDim.x * i;
+      float v = held[i];
+      if (y != nullptr) v = fmaf(column_scale != nullptr ? factor * vc[i] : factor, vy[i], v);
+      if (rows != nullptr) v += vr[i];
+      if (bias != nullptr) v += vb[i];
       if (d < width) {
-        if (y != nullptr || rows != nullptr || bias != nullptr) row[d] = held[i];
+        if (y != nullptr || rows != nullptr || bias != nullptr) row[d] = v;
         if (zero != nullptr) zero[t * width + d] = 0.f;
+        sum = fmaf(v, v, sum);
       }
-      sum = fmaf(held[i], held[i], sum);
+      held[i] = v;
     }
     if (gamma == nullptr) return;
     const float inv = 1.0f / sqrtf(block_sum(sum, scratch) / (float)width + eps);
 #pragma unroll
-    for (int i = 0; i < STREAM_HELD; ++i) {
-      const int d = threadIdx.x + 256 * i;
+    for (int i = 0; i < HELD; ++i) {
+      const int d = threadIdx.x + blockDim.x * i;
       if (d < width) {
         normed[t * width + d] = from_float<T>(held[i] * inv * scale[i]);
         if (gamma2 != nullptr) normed2[t * width + d] = from_float<T>(held[i] * inv * scale2[i]);
@@ -140,12 +153,28 @@ extern "C" int ps_stream_step(float* h, const float* y, float factor, const floa
   PS_REQUIRE(out_dtype == PS_F32 || out_dtype == PS_BF16, "ps_stream_step: unknown dtype %d", out_dtype);
   if (tokens == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
-  if (out_dtype == PS_F32)
-    hipLaunchKernelGGL(stream_step_kernel<float>, dim3(tokens), dim3(256), 0, s, h, y, factor,
-                       column_scale, rows, bias, gamma, eps, (float*)normed, gamma2, (float*)normed2, zero, width);
-  else
-    hipLaunchKernelGGL(stream_step_kernel<bf16_t>, dim3(tokens), dim3(256), 0, s, h, y, factor,
-                       column_scale, rows, bias, gamma, eps, (bf16_t*)normed, gamma2, (bf16_t*)normed2, zero, width);
+  // few rows wait for their trips to memory: a thread per column; many rows fill the chip anyway and
+  // run as blocks of four waves
+  int threads = width >= 1024 ? 1024 : (width + 63) / 64 * 64;
+  if (tokens > 256 && width <= 256 * 8) threads = 256;
+  const int held = (width + threads - 1) / threads;
+#define PS_LAUNCH_SS(T, HELD)                                                                          \
+  hipLaunchKernelGGL((stream_step_kernel<T, HELD>), dim3(tokens), dim3(threads), 0, s, h, y, factor, \
+                     column_scale, rows, bias, gamma, eps, (T*)normed, gamma2, (T*)normed2, zero, width)
+#define PS_LAUNCH_SS_T(T)                   \
+  do {                                      \
+    if (held <= 1) PS_LAUNCH_SS(T, 1);      \
+    else if (held == 2) PS_LAUNCH_SS(T, 2); \
+    else if (held == 3) PS_LAUNCH_SS(T, 3); \
+    else if (held == 4) PS_LAUNCH_SS(T, 4); \
+    else if (held <= 6) PS_LAUNCH_SS(T, 6); \
+    else if (held <= 8) PS_LAUNCH_SS(T, 8); \
+    else PS_LAUNCH_SS(T, 0);                \
+  } while (0)
+  if (out_dtype == PS_F32) PS_LAUNCH_SS_T(float);
+  else PS_LAUNCH_SS_T(bf16_t);
+#undef PS_LAUNCH_SS_T
+#undef PS_LAUNCH_SS
   PS_CHECK_LAUNCH("ps_stream_step");
   return 0;
 }

@@ -20,7 +20,7 @@
 // STREAMS is a template argument so that every loop over the copies is unrolled and a
 // thread's loads of one column (the copies and y) leave together, without a branch between
 // them.  u waits in LDS (width floats) for the row's sum of squares.
-template <typename TOut, int STREAMS>
+template <typename TOut, int STREAMS, bool writes>
 __global__ __launch_bounds__(HS_THREADS) void hyper_step_kernel(
     float* __restrict__ X, const float* __restrict__ y, const float* __restrict__ mix,
     const float* __restrict__ out_w, const float* __restrict__ in_w,
@@ -29,25 +29,31 @@ __global__ __launch_bounds__(HS_THREADS) void hyper_step_kernel(
   extern __shared__ float s_u[];
   __shared__ float red[16];
   const int t = blockIdx.x;
-  const bool writes = y != nullptr;
   const bool reads = normed != nullptr;
-  // the few weights: every thread reads them itself (the same addresses in all lanes: scalar loads)
+  float* row = X + (int64_t)t * STREAMS * width;
+  // the few weights: every thread reads them itself (the same addresses in all lanes: scalar loads),
+  // without a branch, which would make the copies' loads wait for them: where nothing is read the row
+  // stands in for the weights
+  const float* in_from = reads ? in_w : row;
   float w_mix[STREAMS][STREAMS], w_out[STREAMS], w_in[STREAMS];
 #pragma unroll
   for (int a = 0; a < STREAMS; ++a) {
-    w_out[a] = writes ? out_w[a] : 0.f;
-    w_in[a] = reads ? in_w[a] : 0.f;
+    w_in[a] = in_from[a];
+    w_out[a] = 0.f;
+    if constexpr (writes) w_out[a] = out_w[a];
 #pragma unroll
-    for (int b = 0; b < STREAMS; ++b) w_mix[a][b] = writes ? mix[a * STREAMS + b] : (a == b ? 1.f : 0.f);
+    for (int b = 0; b < STREAMS; ++b) {
+      w_mix[a][b] = 0.f;
+      if constexpr (writes) w_mix[a][b] = mix[a * STREAMS + b];
+    }
   }
   float sumsq = 0.f;
-  float* row = X + (int64_t)t * STREAMS * width;
   // what one column needs; returns its u
   auto column = [&](const int col) -> float {
     float x[STREAMS];
 #pragma unroll
     for (int s = 0; s < STREAMS; ++s) x[s] = row[(int64_t)s * width + col];
-    if (writes) {
+    if constexpr (writes) {
       const float yv = y[(int64_t)t * width + col];
       float nx[STREAMS];
 #pragma unroll
@@ -114,9 +120,14 @@ extern "C" int ps_hyper_step(float* x, const float* y, const float* mix, const f
   // anyway and run faster as blocks of four waves that walk their row
   int threads = width >= HS_THREADS ? HS_THREADS : (width + 63) / 64 * 64;
   if (tokens > 256 && threads > 256) threads = 256;
-#define PS_LAUNCH_HS(TOut, S)                                                                     \
-  hipLaunchKernelGGL((hyper_step_kernel<TOut, S>), dim3(tokens), dim3(threads), lds, s, x, y,     \
-                     mix, out_w, in_w, gamma, eps, (TOut*)normed, zero, width)
+#define PS_LAUNCH_HSW(TOut, S, WRITES)                                                            \
+  hipLaunchKernelGGL((hyper_step_kernel<TOut, S, WRITES>), dim3(tokens), dim3(threads), lds, s, x, \
+                     y, mix, out_w, in_w, gamma, eps, (TOut*)normed, zero, width)
+#define PS_LAUNCH_HS(TOut, S)                       \
+  do {                                              \
+    if (y != nullptr) PS_LAUNCH_HSW(TOut, S, true); \
+    else PS_LAUNCH_HSW(TOut, S, false);             \
+  } while (0)
 #define PS_LAUNCH_HS_T(TOut)                         \
   switch (streams) {                                 \
     case 1: PS_LAUNCH_HS(TOut, 1); break;            \
@@ -135,6 +146,7 @@ extern "C" int ps_hyper_step(float* x, const float* y, const float* mix, const f
   }
 #undef PS_LAUNCH_HS_T
 #undef PS_LAUNCH_HS
+#undef PS_LAUNCH_HSW
   PS_CHECK_LAUNCH("ps_hyper_step");
   return 0;
 }
