@@ -25,6 +25,9 @@ bool ps_gemm_nt_f32_skinny_takes(const void* a, const void* w, int m, int n, int
 int ps_gemm_nt_f32_skinny(const void* a, const void* w, const float* bias, void* c, int m, int n,
                           int k, int lda, int ldc, int epilogue, const KvScatter& scatter,
                           hipStream_t s);
+bool ps_norm_gemm_f32_fusable(const void* w, const NormPrologue& norm, int m, int n, int k);
+int ps_norm_gemm_f32_fused(const NormPrologue& norm, const void* w, const float* bias, void* c, int m,
+                           int n, int k, int ldc, int epilogue, const KvScatter& scatter, hipStream_t s);
 bool ps_gemm_nt_f32_tiled_supported(const void* a, const void* w, int m, int k, int lda);
 int ps_gemm_nt_f32_tiled(const void* a, const void* w, const float* bias, void* c, int m, int n,
                          int k, int lda, int ldc, int epilogue, const KvScatter& scatter,
@@ -113,6 +116,8 @@ extern "C" int ps_linear(const PsLinearArgs* p, void* stream) {
       return ps_norm_gemm_fused(norm, p->w, p->bias, p->c, m, n, k, p->ldc, p->c_dtype,
                                 p->epilogue, scatter, p->w_packed, s);
     }
+    if (p->dtype == PS_F32 && ps_norm_gemm_f32_fusable(p->w, norm, m, n, k))
+      return ps_norm_gemm_f32_fused(norm, p->w, p->bias, p->c, m, n, k, p->ldc, p->epilogue, scatter, s);
     PS_REQUIRE(p->norm_out != nullptr, "ps_linear: scratch for the normed rows is needed");
     PS_REQUIRE(p->ldh == k, "ps_linear: unfused norm needs dense rows (ldh %d, k %d)", p->ldh, k);
     const bool pack_norm = decode_rows && k % 64 == 0 && k <= 2048 &&

@@ -181,6 +181,34 @@ def test_gemm_of_float_rows(m, n, k, epilogue):
     assert torch.equal(wide[:, n:], before[:, n:]) and torch.equal(wide[m:], before[m:])
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 33, 4), (3, 192, 64), (8, 100, 772), (9, 2304, 768), (16, 50, 1024), (16, 31, 100),
+                                   (5, 8192, 260), (16, 8200, 128), (17, 40, 768), (4, 48, 1028)])
+@pytest.mark.parametrize("rms", [False, True])
+def test_norm_in_front_of_a_product_of_float_rows(m, n, k, rms):
+    """Fused up to 16 rows, 8,192 columns and a k of 1,024, two launches beyond; rows picked by an index."""
+    from pagedserve_amd.ops import kernels
+
+    h = _rand((m + 3, k), torch.float32, 331, 2.0) + 0.5
+    gamma = 1.0 + _rand((k,), torch.float32, 332, 0.2)
+    beta = None if rms else _rand((k,), torch.float32, 333, 0.2)
+    w = _rand((n, k), torch.float32, 334, 1.0 / math.sqrt(k))
+    bias = _rand((n,), torch.float32, 335)
+    picked = torch.randperm(m + 3, generator=torch.Generator().manual_seed(1))[:m].to(torch.int32).cuda()
+    for rows in (None, picked):
+        x = (h[:m] if rows is None else h[rows.long()]).double()
+        centred = x if rms else x - x.mean(-1, keepdim=True)
+        normed = centred * torch.rsqrt((centred * centred).mean(-1, keepdim=True) + 1e-5) * gamma.double()
+        if beta is not None:
+            normed = normed + beta.double()
+        scratch = torch.empty((m + 3, k), dtype=torch.float32, device="cuda")
+        out = torch.full((m, n), float("nan"), device="cuda")
+        source = h[:m].contiguous() if rows is None else h
+        kernels.linear(kernels.PendingNorm(source, gamma, beta, 1e-5, rms, scratch, rows=rows), w, bias, out)
+        # (the bounds of test_gemm_of_float_rows, and the norm's own handful of roundings)
+        torch.testing.assert_close(out.double(), normed @ w.double().t() + bias.double(),
+                                   atol=2e-6 * math.sqrt(k) / 8 + 8e-6, rtol=8e-6)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_gemm_float_logits_and_strided_views(dtype):
     """bfloat16 operands with float output (the head), inputs and outputs that are column
