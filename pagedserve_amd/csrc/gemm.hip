@@ -116,10 +116,17 @@ extern "C" int ps_linear(const PsLinearArgs* p, void* stream) {
       return ps_norm_gemm_fused(norm, p->w, p->bias, p->c, m, n, k, p->ldc, p->c_dtype,
                                 p->epilogue, scatter, p->w_packed, s);
     }
-    if (p->dtype == PS_F32 && ps_norm_gemm_f32_fusable(p->w, norm, m, n, k))
-      return ps_norm_gemm_f32_fused(norm, p->w, p->bias, p->c, m, n, k, p->ldc, p->epilogue, scatter, s);
     PS_REQUIRE(p->norm_out != nullptr, "ps_linear: scratch for the normed rows is needed");
     PS_REQUIRE(p->ldh == k, "ps_linear: unfused norm needs dense rows (ldh %d, k %d)", p->ldh, k);
+    // every block of the fused kernel reads the rows: an output that lies over them, as a residual may,
+    // has to wait for the norm's own launch
+    const char* rows_begin = (const char*)p->norm_h;
+    const char* c_begin = (const char*)p->c;
+    const bool apart = p->epilogue != PS_EPI_RESIDUAL &&
+                       (c_begin + ((int64_t)(m - 1) * p->ldc + n) * 4 <= rows_begin ||
+                        rows_begin + (int64_t)m * k * 4 <= c_begin);
+    if (p->dtype == PS_F32 && apart && ps_norm_gemm_f32_fusable(p->w, norm, m, n, k))
+      return ps_norm_gemm_f32_fused(norm, p->w, p->bias, p->c, m, n, k, p->ldc, p->epilogue, scatter, s);
     const bool pack_norm = decode_rows && k % 64 == 0 && k <= 2048 &&
                            p->norm_out_rows >= padded_rows &&
                            ps_gemm_nt_mfma_skinny(p->norm_out, p->w, m, n, k, k, p->dtype, p->epilogue);

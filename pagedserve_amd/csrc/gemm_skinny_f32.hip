@@ -298,7 +298,6 @@ int ps_norm_gemm_f32_fused(const NormPrologue& norm, const void* w, const float*
     PS_SNF_CASE(PS_EPI_GELU_TANH);
     PS_SNF_CASE(PS_EPI_GELU_ERF);
     PS_SNF_CASE(PS_EPI_RELU2);
-    PS_SNF_CASE(PS_EPI_RESIDUAL);
     default: ps_set_error("ps_linear: unknown epilogue %d", epilogue); return 1;
   }
 #undef PS_SNF_CASE

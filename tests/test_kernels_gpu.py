@@ -209,6 +209,24 @@ def test_norm_in_front_of_a_product_of_float_rows(m, n, k, rms):
                                    atol=2e-6 * math.sqrt(k) / 8 + 8e-6, rtol=8e-6)
 
 
+@pytest.mark.parametrize("epilogue", ["residual", "none"])
+def test_a_product_of_float_rows_over_the_rows_that_its_norm_reads(epilogue):
+    """The output replaces (or is added to) the rows in front of the norm: the norm runs before the first
+    store, however small the call."""
+    from pagedserve_amd.ops import kernels
+
+    m, k = 8, 768
+    h = _rand((m, k), torch.float32, 341, 2.0)
+    gamma = 1.0 + _rand((k,), torch.float32, 342, 0.2)
+    w = _rand((k, k), torch.float32, 343, 1.0 / math.sqrt(k))
+    x = h.double()
+    normed = x * torch.rsqrt((x * x).mean(-1, keepdim=True) + 1e-5) * gamma.double()
+    expected = normed @ w.double().t() + (x if epilogue == "residual" else 0.0)
+    kernels.linear(kernels.PendingNorm(h, gamma, None, 1e-5, True, torch.empty_like(h)), w, None, h, epilogue=epilogue)
+    # (the bounds of test_norm_in_front_of_a_product_of_float_rows)
+    torch.testing.assert_close(h.double(), expected, atol=2e-6 * math.sqrt(k) / 8 + 8e-6, rtol=8e-6)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_gemm_float_logits_and_strided_views(dtype):
     """bfloat16 operands with float output (the head), inputs and outputs that are column
