@@ -20,6 +20,9 @@
 // STREAMS is a template argument so that every loop over the copies is unrolled and a
 // thread's loads of one column (the copies and y) leave together, without a branch between
 // them.  u waits in LDS (width floats) for the row's sum of squares.
+// The kernel waits on memory alone (two trips at few rows: the operands, then the store's way out; the bytes at
+// many).  Nothing that is optional stands behind a branch in front of the loads, which would make them wait
+// for what was asked for before: a row of 4 x 768 without and with it, 8 rows 3.3 / 3.85 us, 2,048 rows 13.4 / 15.3.
 template <typename TOut, int STREAMS, bool writes>
 __global__ __launch_bounds__(HS_THREADS) void hyper_step_kernel(
     float* __restrict__ X, const float* __restrict__ y, const float* __restrict__ mix,
