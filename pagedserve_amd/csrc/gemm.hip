@@ -118,13 +118,18 @@ extern "C" int ps_linear(const PsLinearArgs* p, void* stream) {
     }
     PS_REQUIRE(p->norm_out != nullptr, "ps_linear: scratch for the normed rows is needed");
     PS_REQUIRE(p->ldh == k, "ps_linear: unfused norm needs dense rows (ldh %d, k %d)", p->ldh, k);
-    // every block of the fused kernel reads the rows: an output that lies over them, as a residual may,
-    // has to wait for the norm's own launch
-    const char* rows_begin = (const char*)p->norm_h;
-    const char* c_begin = (const char*)p->c;
-    const bool apart = p->epilogue != PS_EPI_RESIDUAL &&
-                       (c_begin + ((int64_t)(m - 1) * p->ldc + n) * 4 <= rows_begin ||
-                        rows_begin + (int64_t)m * k * 4 <= c_begin);
+    // every block of the fused kernel reads the norm's operands while others store already: an output that
+    // lies over one of them (a residual, the rows in front of the norm, picked by an index or not) has to wait
+    // for the norm's own launch.  Rows that an index picks lie anywhere among the norm_h_rows.
+    const int64_t c_bytes = ((int64_t)(m - 1) * p->ldc + n) * 4;
+    auto over = [&](const void* operand, int64_t bytes) {
+      const uintptr_t c_begin = reinterpret_cast<uintptr_t>(p->c), begin = reinterpret_cast<uintptr_t>(operand);
+      return operand != nullptr && c_begin < begin + bytes && begin < c_begin + c_bytes;
+    };
+    const int64_t h_rows = p->norm_rows == nullptr ? m : p->norm_h_rows;
+    const bool apart = p->epilogue != PS_EPI_RESIDUAL && h_rows > 0 && !over(p->norm_h, h_rows * k * 4) &&
+                       !over(p->norm_rows, (int64_t)m * 4) && !over(p->gamma, (int64_t)k * 4) &&
+                       !over(p->beta, (int64_t)k * 4);
     if (p->dtype == PS_F32 && apart && ps_norm_gemm_f32_fusable(p->w, norm, m, n, k))
       return ps_norm_gemm_f32_fused(norm, p->w, p->bias, p->c, m, n, k, p->ldc, p->epilogue, scatter, s);
     const bool pack_norm = decode_rows && k % 64 == 0 && k <= 2048 &&

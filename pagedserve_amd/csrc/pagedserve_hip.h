@@ -40,7 +40,8 @@ int ps_gemm_nt(const void* a, const void* w, const float* bias, void* c, int m, 
 // A linear layer with what may be fused around it.
 //   * norm_h != null: the input rows are norm(norm_h[norm_rows ? norm_rows[r] : r]) * gamma
 //     (+ beta) instead of `a`; `norm_out` ([m, k] of `dtype`) is scratch for when the norm
-//     cannot be fused into the product (it is fused for bfloat16, m <= 16, k <= 1024);
+//     cannot be fused into the product (it is fused for m <= 16, k <= 1024; in float only where c lies
+//     over nothing that the norm reads);
 //   * k_pool != null: the output is [q | k | v] columns (q_cols, then kv_cols twice); besides
 //     being written to c, the k and v columns of row t are stored in the cache at the page
 //     slot of position tok_pos[t] of item tok_item[t] (what ps_kv_write does).
@@ -100,6 +101,9 @@ typedef struct PsLinearArgs {
   // the pages), so a kernel may leave them unwritten; they are unspecified afterwards.  The
   // tiled kernel for many rows does, which takes 40 % off what a prompt's QKV product writes.
   int scatter_only;
+  // With norm_rows: how many rows norm_h has; 0 where that is not known.  Known, a float norm and its
+  // product may run as one launch where c lies over none of those rows; else the norm runs first.
+  int norm_h_rows;
 } PsLinearArgs;
 
 int ps_linear(const PsLinearArgs* args, void* stream);

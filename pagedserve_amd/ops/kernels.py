@@ -344,7 +344,7 @@ class _LinearArgs(ctypes.Structure):
         ("norm_out_rows", c_int), ("c_layout", ctypes.POINTER(c_int)),
         ("top_tokens", c_void_p), ("top_keys", c_void_p), ("top_ticket", c_void_p),
         ("top_done", ctypes.POINTER(c_int)),
-        ("scatter_only", c_int),
+        ("scatter_only", c_int), ("norm_h_rows", c_int),
     ]
 
 
@@ -422,13 +422,13 @@ _MEMO_DONE = c_int(0)
 
 
 def _memo_key(x, out, scatter, a_packed, choose):
-    """What may differ between two calls of one call site, in two parts: the row count and
+    """What may differ between two calls of one call site, in two parts: the row counts and
     the addresses of the step's buffers and index arrays, which the same call site of another
     layer meets too, and the addresses that tell the site's own operands apart where it may be
     called with several (its norm's parameters; the cache pools, of which a block that runs
     twice in a step has two pairs).  Weights, bias and flags are the site's own and in neither."""
     if isinstance(x, PendingNorm):
-        step = (x.count, x.h.data_ptr(), _ptr(x.rows), x.scratch.data_ptr(), out.data_ptr())
+        step = (x.count, x.h.data_ptr(), x.h.shape[0], _ptr(x.rows), x.scratch.data_ptr(), out.data_ptr())
         site = (x.gamma.data_ptr(),)
     else:
         step = (x.shape[0], x.data_ptr(), x.stride(0), out.data_ptr(), a_packed)
@@ -452,7 +452,7 @@ def _field_ranges(names):
 # (the layers share the workspace and the index arrays).  All others are sizes, codes and flags.
 _SITE_FIELDS = ("w", "bias", "gamma", "beta", "k_pool", "v_pool", "w_packed")
 _STEP_FIELDS = ("a", "c", "m", "lda", "ldc", "norm_h", "norm_rows", "norm_out", "tok_item", "tok_pos",
-                "tables", "table_width", "a_packed", "c_rows", "norm_out_rows", "c_layout",
+                "tables", "table_width", "a_packed", "c_rows", "norm_out_rows", "norm_h_rows", "c_layout",
                 "top_tokens", "top_keys", "top_ticket", "top_done")
 _SITE_RANGES = _field_ranges(_SITE_FIELDS)
 _SIZE_RANGES = _field_ranges(name for name, _ in _LinearArgs._fields_
@@ -560,6 +560,7 @@ def linear(x, w, bias, out, epilogue="none", scatter=None, packed=None, a_packed
             _check(x.rows, "rows", torch.int32, 1)
         args.norm_h = x.h.data_ptr()
         args.norm_rows = _ptr(x.rows)
+        args.norm_h_rows = x.h.shape[0]
         args.gamma = x.gamma.data_ptr()
         args.beta = _ptr(x.beta)
         args.norm_out = x.scratch.data_ptr()

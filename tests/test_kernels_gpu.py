@@ -227,6 +227,28 @@ def test_a_product_of_float_rows_over_the_rows_that_its_norm_reads(epilogue):
     torch.testing.assert_close(h.double(), expected, atol=2e-6 * math.sqrt(k) / 8 + 8e-6, rtol=8e-6)
 
 
+@pytest.mark.parametrize("picked,over,fused", [([4, 5, 6, 7], 4, False), ([1, 9, 3, 4], 7, False), ([0, 1, 2, 3], 6, False),
+                                               ([9, 0, 5, 7], 10, True)])
+def test_a_product_of_float_rows_over_rows_that_an_index_picks(picked, over, fused):
+    """The output lies over some of the rows that the index may pick, behind as many as there are picked or not: the
+    norm runs in a launch of its own first, which leaves its rows in the scratch.  Behind the last row it does not."""
+    from pagedserve_amd.ops import kernels
+
+    m, k, rows = 4, 768, 10
+    room = _rand((rows + m, k), torch.float32, 344, 2.0)
+    h, out = room[:rows], room[over:over + m]
+    gamma = 1.0 + _rand((k,), torch.float32, 345, 0.2)
+    w = _rand((k, k), torch.float32, 346, 1.0 / math.sqrt(k))
+    index = torch.tensor(picked, dtype=torch.int32, device="cuda")
+    x = h[index.long()].double()
+    normed = x * torch.rsqrt((x * x).mean(-1, keepdim=True) + 1e-5) * gamma.double()
+    scratch = torch.full((m, k), float("nan"), device="cuda")
+    kernels.linear(kernels.PendingNorm(h, gamma, None, 1e-5, True, scratch, rows=index), w, None, out)
+    # (the bounds of test_norm_in_front_of_a_product_of_float_rows)
+    torch.testing.assert_close(out.double(), normed @ w.double().t(), atol=2e-6 * math.sqrt(k) / 8 + 8e-6, rtol=8e-6)
+    assert bool(scratch.isnan().all()) if fused else not bool(scratch.isnan().any())
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_gemm_float_logits_and_strided_views(dtype):
     """bfloat16 operands with float output (the head), inputs and outputs that are column
