@@ -5,16 +5,17 @@
 // Bound by reading W once, and at these sizes by the one trip to memory that this takes: like the
 // bfloat16 product for few rows, a block owns 16 NT weight rows and MB blocks of 16 rows of A, its
 // waves take turns along k in steps of 32 values (128 bytes of every row), operands go straight from
-// memory to the matrix cores, UNROLL steps asked for together, and the waves' partial tiles are summed
-// in LDS in a fixed order.  Rows of A beyond MB blocks go to further blocks (grid z), which read the
+// memory to the matrix cores, UNROLL steps asked for together (8 x 4096 x 1024 8.8 us where the compiler orders
+// the loads, 7.4 so), and the waves' partial tiles are summed in LDS in a fixed order.  Rows of A beyond MB blocks go to further blocks (grid z), which read the
 // same weights out of the L2.  k may be split over blocks; those partial sums are added with float
 // atomics into the stream (residual epilogue only).  A lane's 16 bytes of k are the same for both
 // operands, so that which four values an instruction multiplies does not matter.
 //
 // Measured with weights from memory, before (the plain kernel, or up to 16 rows one dot product per
-// wave and column) and after, in us: 64 x 2304 x 768 88 / 10.2, 64 x 768 x 3072 338 / 9.5, 32 x 768 x
-// 768 89 / 5.7, 200 x 768 x 768 34 / 9.8, 16 x 3072 x 768 8.6 / 6.1, 8 x 768 x 3072 7.1 / 5.7,
-// 16 x 50257 x 768 68 / 48 (its weights alone are 30 at the rate of a copy).
+// wave and column) and after, in us: 64 x 2304 x 768 88 / 9.7, 64 x 768 x 3072 338 / 9.5, 32 x 768 x
+// 768 89 / 5.4, 200 x 768 x 768 34 / 9.7, 16 x 3072 x 768 8.6 / 5.6, 8 x 768 x 3072 7.1 / 5.0,
+// 16 x 50257 x 768 68 / 46 (its weights alone are 30 at the rate of a copy).  Relative error against 64 bits: 16 x
+// 2304 x 768 9.3e-8 (the dot products 9.3e-8; with one accumulator per value of k 1.1e-7), 64 x 768 x 3072 1.0e-6 / 1.2e-7.
 #include "common.h"
 #include "linear.h"
 #include "pagedserve_hip.h"
@@ -22,6 +23,16 @@
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 
 #define SF_STEP 32    // values of k per step of a wave: 128 bytes of every row
+
+// The sum of N numbers in pairs, the pairs in pairs and so on.
+template <int N>
+__device__ inline float sum_in_pairs(float (&v)[N]) {
+#pragma unroll
+  for (int span = 1; span < N; span *= 2)
+#pragma unroll
+    for (int p = 0; p + span < N; p += 2 * span) v[p] += v[p + span];
+  return v[0];
+}
 
 // Sum the waves' partial tiles in a fixed order and finish the block's 16 NT columns of 16 MB rows.
 template <int EPI, int MB, int NT, int WAVES>
@@ -40,9 +51,10 @@ __device__ inline void skinny_f32_epilogue(float (&partial)[NT][WAVES][MB][4][64
     if (col >= n || row >= m) continue;
     const int i = col_in & 3;
     const int at = (col_in >> 2) * 16 + row_in;
-    float v = 0.f;
+    float of_wave[WAVES];
 #pragma unroll
-    for (int p = 0; p < WAVES; ++p) v += partial[j][p][b][i][at];
+    for (int p = 0; p < WAVES; ++p) of_wave[p] = partial[j][p][b][i][at];
+    float v = sum_in_pairs(of_wave);
     if (bias != nullptr && split == 0) v += bias[col];
     float* dst = c + (int64_t)row * ldc + col;
     if (EPI == PS_EPI_RESIDUAL) {
@@ -83,15 +95,17 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_nt_skinny_f32_kernel(
     const int row = row0 + b * 16 + sub < m ? row0 + b * 16 + sub : m - 1;
     a_ptr[b] = a + (int64_t)row * lda;
   }
-  // an accumulator for each of a lane's four values of k: short chains, whose rounding errors stay
-  // small and whose instructions do not wait for each other
-  f32x4 acc[NT][MB][4];
+  // an accumulator for each of a lane's four values of k, and for up to 16 rows two such fours that take
+  // turns: short chains, whose rounding errors stay small (with the sums in pairs behind them those of one dot
+  // product to a wave's 64 lanes) and whose instructions do not wait for each other
+  constexpr int SETS = MB == 1 ? 2 : 1;
+  f32x4 acc[NT][MB][4 * SETS];
 #pragma unroll
   for (int j = 0; j < NT; ++j)
 #pragma unroll
     for (int b = 0; b < MB; ++b)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[j][b][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int i = 0; i < 4 * SETS; ++i) acc[j][b][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // wave `wave` takes the steps wave, wave + WAVES, ... of the block's range; UNROLL of them are
   // asked for together
@@ -110,33 +124,41 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_nt_skinny_f32_kernel(
         for (int j = 0; j < NT; ++j) wf[u][j][h] = *reinterpret_cast<const f32x4*>(w_ptr[j] + at);
 #pragma unroll
         for (int b = 0; b < MB; ++b) xf[u][b][h] = *reinterpret_cast<const f32x4*>(a_ptr[b] + at);
+      }
+    // (without this the compiler asks for a few at a time, to use fewer registers)
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const bool there = k0 + u * WAVES * SF_STEP + h * 16 + group * 4 < k_end;
         if (!there) {
 #pragma unroll
           for (int j = 0; j < NT; ++j) wf[u][j][h] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int b = 0; b < MB; ++b) xf[u][b][h] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
-      }
-#pragma unroll
-    for (int u = 0; u < UNROLL; ++u)
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
           for (int j = 0; j < NT; ++j)
 #pragma unroll
             for (int b = 0; b < MB; ++b)
-              acc[j][b][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[u][j][h][i], xf[u][b][h][i],
-                                                                  acc[j][b][i], 0, 0, 0);
+              acc[j][b][(2 * u + h) % SETS * 4 + i] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                  wf[u][j][h][i], xf[u][b][h][i], acc[j][b][(2 * u + h) % SETS * 4 + i], 0, 0, 0);
+      }
   }
 #pragma unroll
   for (int j = 0; j < NT; ++j)
 #pragma unroll
     for (int b = 0; b < MB; ++b)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) partial[j][wave][b][i][lane] =
-            (acc[j][b][0][i] + acc[j][b][1][i]) + (acc[j][b][2][i] + acc[j][b][3][i]);
+      for (int i = 0; i < 4; ++i) {
+        float sums[4 * SETS];
+#pragma unroll
+        for (int p = 0; p < 4 * SETS; ++p) sums[p] = acc[j][b][p][i];
+        partial[j][wave][b][i][lane] = sum_in_pairs(sums);
+      }
   __syncthreads();
 
   skinny_f32_epilogue<EPI, MB, NT, WAVES>(partial, bias, c, m, n, ldc, n0, row0, split, k_splits, scatter);
@@ -145,7 +167,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_nt_skinny_f32_kernel(
 // The same for up to 16 rows with the norm of its input fused in front (whole k in one round of loads): while the
 // weights travel, each wave normalises up to two rows in registers (as norm_wave_kernel, elementwise.hip)
 // and leaves them in LDS, where the product reads its column operand.  One launch and one trip to memory
-// instead of two launches, in us: 1 x 2304 x 768 7.4 -> 5.2, 8 x 2304 x 768 8.7 -> 5.8, 16 x 2304 x 768
+// instead of two launches, in us: 1 x 2304 x 768 7.4 -> 5.3, 8 x 2304 x 768 8.7 -> 5.9, 16 x 2304 x 768
 // 11.6 -> 6.7, 8 x 4096 x 1024 16.9 -> 8.7.
 template <int EPI, int UNROLL>
 __global__ __launch_bounds__(512) void gemm_nt_skinny_norm_f32_kernel(
@@ -209,25 +231,19 @@ __global__ __launch_bounds__(512) void gemm_nt_skinny_norm_f32_kernel(
     for (int i = 0; i < PIECES; ++i) {
       const int col = (lane + i * 64) * 4;
       if (col >= k) continue;
-      float4 y;
-      y.x = v[i][0] * inv_std * g[i][0];
-      y.y = v[i][1] * inv_std * g[i][1];
-      y.z = v[i][2] * inv_std * g[i][2];
-      y.w = v[i][3] * inv_std * g[i][3];
-      if (shifts) {
-        y.x += b[i][0];
-        y.y += b[i][1];
-        y.z += b[i][2];
-        y.w += b[i][3];
-      }
-      *reinterpret_cast<float4*>(rows + r * STRIDE + col) = y;
+      f32x4 y;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        y[j] = shifts ? fmaf(v[i][j] * inv_std, g[i][j], b[i][j]) : v[i][j] * inv_std * g[i][j];
+      *reinterpret_cast<f32x4*>(rows + r * STRIDE + col) = y;
     }
   }
   __syncthreads();
   // (rows of LDS beyond m stay as they are: they only feed outputs that are never stored)
-  f32x4 acc[4];
+  constexpr int SETS = 3;     // (as above; the normed rows carry a rounding of their own)
+  f32x4 acc[4 * SETS];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < 4 * SETS; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int u = 0; u < UNROLL; ++u)
 #pragma unroll
@@ -237,11 +253,16 @@ __global__ __launch_bounds__(512) void gemm_nt_skinny_norm_f32_kernel(
       if (kk >= k) x = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[u][h][i], x[i], acc[i], 0, 0, 0);
+        acc[(2 * u + h) % SETS * 4 + i] =
+            __builtin_amdgcn_mfma_f32_16x16x4f32(wf[u][h][i], x[i], acc[(2 * u + h) % SETS * 4 + i], 0, 0, 0);
     }
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-    partial[0][wave][0][i][lane] = (acc[0][i] + acc[1][i]) + (acc[2][i] + acc[3][i]);
+  for (int i = 0; i < 4; ++i) {
+    float sums[4 * SETS];
+#pragma unroll
+    for (int p = 0; p < 4 * SETS; ++p) sums[p] = acc[p][i];
+    partial[0][wave][0][i][lane] = sum_in_pairs(sums);
+  }
   __syncthreads();
   skinny_f32_epilogue<EPI, 1, 1, WAVES>(partial, bias, c, m, n, ldc, n0, 0, 0, 1, scatter);
 }
@@ -329,8 +350,7 @@ static int launch_skinny_f32(const void* a, const void* w, const float* bias, vo
       k_chunk = ((k + k_splits - 1) / k_splits + SF_STEP - 1) / SF_STEP * SF_STEP;
       k_splits = (k + k_chunk - 1) / k_chunk;
     }
-    if (n >= 64 * 256) PS_LAUNCH_SF(1, 2, 3, 8);
-    else if (k_chunk <= 8 * 3 * SF_STEP) PS_LAUNCH_SF(1, 1, 3, 8);
+    if (k_chunk <= 8 * 3 * SF_STEP) PS_LAUNCH_SF(1, 1, 3, 8);
     else PS_LAUNCH_SF(1, 1, 4, 8);
   } else if (k > 8 * 3 * SF_STEP) PS_LAUNCH_SF(1, 1, 4, 8);
   else if (m <= 32) PS_LAUNCH_SF(2, 1, 3, 8);

@@ -209,6 +209,33 @@ def test_norm_in_front_of_a_product_of_float_rows(m, n, k, rms):
                                    atol=2e-6 * math.sqrt(k) / 8 + 8e-6, rtol=8e-6)
 
 
+@pytest.mark.parametrize("m,n,k,norm", [(5, 2304, 768, False), (16, 2304, 768, False), (16, 17000, 768, False), (8, 4096, 1024, False),
+                                        (16, 2100, 1600, False), (1, 2304, 768, True), (16, 2304, 768, True), (8, 4096, 1024, True),
+                                        (16, 1536, 512, True)])
+def test_float_products_of_few_rows_are_as_close_as_dot_products(m, n, k, norm):
+    """On the matrix cores, with a norm in front or without: no further from 64 bits than one dot product to a wave's
+    64 lanes, which is what four rows at a time take, behind a norm of its own (3 % for the draw of the errors)."""
+    from pagedserve_amd.ops import kernels
+
+    errors = [0.0, 0.0]
+    for seed in range(4):
+        h = _rand((m, k), torch.float32, 351 + seed)
+        w = _rand((n, k), torch.float32, 361 + seed, 1.0 / math.sqrt(k))
+        gamma, beta = 1.0 + _rand((k,), torch.float32, 371 + seed, 0.2), _rand((k,), torch.float32, 381 + seed)
+        x, exact = h, h.double()
+        if norm:
+            x = kernels.norm(h, gamma, beta, 1e-5, torch.empty_like(h))
+            exact = F.layer_norm(exact, (k,), gamma.double(), beta.double(), 1e-5)
+        exact = exact @ w.double().t()
+        out, dots = torch.empty((m, n), device="cuda"), torch.empty((m, n), device="cuda")
+        kernels.linear(kernels.PendingNorm(h, gamma, beta, 1e-5, False, torch.empty_like(h)) if norm else h, w, None, out)
+        for row in range(0, m, 4):
+            kernels.gemm_nt(x[row:row + 4], w, None, dots[row:row + 4])
+        for i, result in enumerate((out, dots)):
+            errors[i] += float((result.double() - exact).norm() / exact.norm()) / 4
+    assert errors[0] <= 1.03 * errors[1], errors
+
+
 @pytest.mark.parametrize("epilogue", ["residual", "none"])
 def test_a_product_of_float_rows_over_the_rows_that_its_norm_reads(epilogue):
     """The output replaces (or is added to) the rows in front of the norm: the norm runs before the first
