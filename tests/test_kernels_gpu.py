@@ -236,6 +236,21 @@ def test_float_products_of_few_rows_are_as_close_as_dot_products(m, n, k, norm):
     assert errors[0] <= 1.03 * errors[1], errors
 
 
+@pytest.mark.parametrize("m,n,k", [(1024, 768, 768), (1024, 1024, 1024), (1100, 1600, 1600), (1024, 1600, 6400), (540, 700, 2080)])
+def test_residual_products_of_many_float_rows_sum_short_chains(m, n, k):
+    """The residual product of 64 x 64 tiles takes whole k ranges; no chain of it is longer than 128 additions."""
+    from pagedserve_amd.ops import kernels
+
+    a = _rand((m, k), torch.float32, 391)
+    w = _rand((n, k), torch.float32, 392, 1.0 / math.sqrt(k))
+    out = torch.zeros((m, n), device="cuda")
+    kernels.gemm_nt(a, w, None, out, epilogue="residual")
+    exact = a.double() @ w.double().t()
+    # 128 additions to a sum that grows like a walk: sqrt(128 / 2) roundings of the sum's size, each 2^-24 at most
+    # and 0.41 of that in the mean square; 15 % for the sums behind the chains
+    assert float((out.double() - exact).norm() / exact.norm()) < 1.15 * 0.41 * 8 * 2.0 ** -24
+
+
 @pytest.mark.parametrize("epilogue", ["residual", "none"])
 def test_a_product_of_float_rows_over_the_rows_that_its_norm_reads(epilogue):
     """The output replaces (or is added to) the rows in front of the norm: the norm runs before the first
