@@ -151,7 +151,7 @@ extern "C" int ps_linear(const PsLinearArgs* p, void* stream) {
                                   s);
   }
   // Matrix cores when the operands allow 16-byte loads (in float what is left here are many rows
-  // of a k that is no multiple of 32, and up to 8 rows for the plain kernel).
+  // of a k that is no multiple of 32, and up to 16 rows for the plain kernel).
   const bool mfma = ps_gemm_nt_mfma_supported(a, p->w, k, lda, p->dtype) &&
                     (p->dtype == PS_BF16 || m >= 96);
   if (mfma) {

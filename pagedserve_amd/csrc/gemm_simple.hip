@@ -7,7 +7,7 @@
 // Tile: 64 x 64 outputs per 256-thread block, 16 k per stage through LDS, 4 x 4 outputs per
 // thread.  Any m, n, k and any row strides; loads are bounds-checked and zero-filled.
 //
-// Up to 8 rows of float (a decode step of the 32-bit path) may take a second kernel (where it is ahead
+// Up to 16 rows of float (a decode step of the 32-bit path) may take a second kernel (where it is ahead
 // of the matrix cores: gemm_skinny_f32.hip): the tiled one would run on n / 64 blocks that each walk the whole k in stages of 16, a few dozen blocks
 // bound by the latency of hundreds of dependent trips (8 rows x 2304 x 768: 70 us).  Here a
 // wave owns a few output columns, its lanes stride over k with 16-byte loads of the weights
@@ -92,7 +92,7 @@ __global__ __launch_bounds__(256) void gemm_nt_simple_kernel(
   }
 }
 
-// MR: rows held in registers (m <= MR); COLS: output columns per wave.  A lane walks k in
+// MR: rows held in registers, of which a block has the first, or at 9 to 16 rows the second eight; COLS: output columns per wave.  A lane walks k in
 // steps of 256 values and asks for 4 / COLS such steps of its COLS weight rows at once (four
 // 16-byte loads in flight whatever COLS is); the sums are formed in the order of k either way,
 // so the result does not depend on COLS.
@@ -105,6 +105,10 @@ __global__ __launch_bounds__(256) void gemm_nt_f32_rows_kernel(
   const int wave = threadIdx.x >> 6;
   const int col0 = (blockIdx.x * 4 + wave) * COLS;
   if (col0 >= n) return;
+  // (9 to 16 rows: the second eight are another block's)
+  a += (int64_t)blockIdx.y * MR * lda;
+  c += (int64_t)blockIdx.y * MR * ldc;
+  m -= blockIdx.y * MR;
   const float* w_row[COLS];
 #pragma unroll
   for (int j = 0; j < COLS; ++j) w_row[j] = w + (int64_t)(col0 + j < n ? col0 + j : n - 1) * k;
@@ -163,16 +167,16 @@ __global__ __launch_bounds__(256) void gemm_nt_f32_rows_kernel(
 }
 
 static bool rows_kernel_takes(const void* a, const void* w, int m, int k, int lda) {
-  return m >= 1 && m <= 8 && k % 4 == 0 && lda % 4 == 0 &&
+  return m >= 1 && m <= 16 && k % 4 == 0 && lda % 4 == 0 &&
          (reinterpret_cast<uintptr_t>(a) & 15u) == 0 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
 }
 
 static int launch_f32_rows(const void* a, const void* w, const float* bias, void* c, int m, int n,
                            int k, int lda, int ldc, int epilogue, hipStream_t s) {
 #define PS_LAUNCH_FR(EPI, MR, COLS)                                                              \
-  hipLaunchKernelGGL((gemm_nt_f32_rows_kernel<EPI, MR, COLS>), dim3((n + 4 * COLS - 1) / (4 * COLS)), \
-                     dim3(256), 0, s, (const float*)a, (const float*)w, bias, (float*)c, m, n, k, \
-                     lda, ldc)
+  hipLaunchKernelGGL((gemm_nt_f32_rows_kernel<EPI, MR, COLS>),                                   \
+                     dim3((n + 4 * COLS - 1) / (4 * COLS), (m + MR - 1) / MR), dim3(256), 0, s,  \
+                     (const float*)a, (const float*)w, bias, (float*)c, m, n, k, lda, ldc)
   // Columns per wave by the blocks they leave: a block of four waves per compute unit counts
   // for more than the reuse of the rows (8 x 768 x 3072 on 48 blocks of 4 columns a wave took
   // 31 us, twelve trips to memory one after the other).

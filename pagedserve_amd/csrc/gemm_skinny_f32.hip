@@ -270,9 +270,12 @@ __global__ __launch_bounds__(512) void gemm_nt_skinny_norm_f32_kernel(
 // --------------------------------------------------------------------------------- host
 // Whether this kernel takes the product (a row of either operand in pieces of 16 bytes), and is the
 // fastest that does.  The lines, with weights from memory, in us:
-// - Up to 8 rows one dot product per wave and column (gemm_simple.hip) is ahead while the weights are
-//   few (8 x 768 x 768 4.2 against 4.9) and level at very many columns; up to 4 rows always but
-//   where k is long and can be split (4 x 1024 x 4096 9.8 against 8.4).
+// - Up to 16 rows one dot product per wave and column (gemm_simple.hip) is ahead while the weights
+//   are few (8 x 768 x 768 4.2 against 4.7, 16 x 768 x 768 5.0 against 5.9, 16 x 64 x 256 3.1 against 5.3, 16 x
+//   1024 x 1024 5.6 against 6.8, 16 x 320 x 1280 4.7 against 5.6), and up to 8 level at very many columns; up to 4 rows
+//   always but where k is long and can be split (4 x 1024 x 4096 8.6 against 7.1).  Nine rows and more with the
+//   plain epilogue come here all the same: with a key/value scatter behind it the other kernel needs a second launch
+//   (2.5), and a product is the same bits with and without (16 x 192 x 64 3.3 here, 2.8 there).
 // - Residual epilogue, k split: 200 x 768 x 3072 24.3 against 25.2 for the tiled kernel, 300 rows 33 against
 //   28; 300 x 768 x 768 11.4 against 11.5; wide models sooner (32 x 1600 x 6400 25.4 against 25.2).
 // - Otherwise up to 64 rows and one round of loads (32 x 4096 x 1024 12.2 against 17.3, 64 rows 17.1
@@ -289,7 +292,7 @@ bool ps_gemm_nt_f32_skinny_takes(const void* a, const void* w, int m, int n, int
   const int64_t weights = (int64_t)n * k;
   if (m <= 4) return residual && k >= 4096;
   if (m <= 8) return weights > (1 << 20) && n < 64 * 256;
-  if (m <= 16) return true;
+  if (m <= 16) return weights > (1 << 20) || epilogue == PS_EPI_NONE;
   if (k % SF_STEP != 0) return m < 768;
   if (residual) return (int64_t)m * n <= 160000 && weights < 6000000;
   return n < 64 * 256 && (k <= 768 ? m <= 64 : k <= 1024 && m <= 32);

@@ -159,7 +159,9 @@ def test_gemm_nt(dtype, m, n, k, epilogue):
 @pytest.mark.parametrize("m,n,k", [(4, 100, 4096), (5, 2100, 516), (8, 1400, 772), (9, 37, 4), (16, 16400, 100), (16, 50, 1028),
                                    (17, 70, 36), (32, 130, 768), (33, 310, 768), (64, 95, 736), (32, 77, 1024), (65, 200, 800),
                                    (20, 60, 3104), (100, 1500, 3072), (230, 1040, 768), (70, 90, 100), (800, 40, 68),
-                                   (65, 33, 32), (129, 4200, 64), (300, 65, 2080)])
+                                   (65, 33, 32), (129, 4200, 64), (300, 65, 2080),
+                                   # 9 to 16 rows over few weights: two blocks to a wave's one, two or four columns
+                                   (9, 330, 772), (13, 1601, 640), (16, 3101, 320)])
 @pytest.mark.parametrize("epilogue", ["none", "gelu_tanh", "residual"])
 def test_gemm_of_float_rows(m, n, k, epilogue):
     from pagedserve_amd.ops import kernels
