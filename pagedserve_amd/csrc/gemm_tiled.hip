@@ -432,11 +432,12 @@ int ps_gemm_nt_bf16_tiled(const void* a, const void* w, const float* bias, void*
 // 1600 36 us with three and 44 with two, 2048 x 4096 x 1024 162 and 155), or 64 x 32 where those leave
 // half of the units without a block (100 x 2304 x 768 11.9 against 18.5).  Only many rounds of blocks
 // make larger tiles worth their uneven last round: 128 x 64 from six of 64 x 64 per unit (2048 x 4800 x
-// 1600 272 against 282), 128 x 128 from four of its own (4096 x 4096 x 1024 283 against 300; with three, 4096 x
-// 3072 x 768, 200 against 175).  With weights from memory, the kernel that did this before (128 x 128
+// 1600 272 against 282) and more than one row of them (128 x 50257 x 768 129 against 110, 128 x 50257 x 1600 237 against
+// 209), 128 x 128 from four of its own (4096 x 4096 x 1024 283 against 300; with three, 4096 x 3072 x 768, 200 against 175).  With weights from memory, the kernel that did this before (128 x 128
 // tiles; below 96 rows the plain kernel) and this one, in us: 2048 x 2304 x 768 110 / 75, 2048 x 3072 x
 // 768 120 / 95 (102 TFLOP/s; the library's 4096-cubed product reaches 139), 300 x 2304 x 768 65 / 19,
-// 544 x 768 x 768 35 / 12, 330 x 1024 x 4096 60 / 43, 64 x 50257 x 768 201 / 70, 4096 x 3072 x 768 172 / 175.
+// 544 x 768 x 768 35 / 12, 330 x 1024 x 4096 60 / 43, 64 x 50257 x 768 201 / 67, 96 x 50257 x 768 116 / 109, 4096 x 3072 x
+// 768 172 / 174.
 bool ps_gemm_nt_f32_tiled_supported(const void* a, const void* w, int m, int k, int lda) {
   return m > 16 && k % (TB_ROW / 4) == 0 && lda % 4 == 0 &&
          (reinterpret_cast<uintptr_t>(a) & 15u) == 0 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
@@ -454,7 +455,7 @@ int ps_gemm_nt_f32_tiled(const void* a, const void* w, const float* bias, void* 
     return launch_variant<float, 1, 1, 3, float>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
   if ((int64_t)((m + 127) / 128) * ((n + 127) / 128) >= 4 * units)
     return launch_variant<float, 2, 2, 2, float>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
-  if (tiles_64 >= 6 * units)
+  if (tiles_64 >= 6 * units && m > 128)
     return launch_variant<float, 2, 1, 2, float>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
   return launch_variant<float, 1, 1, 2, float>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
 }

@@ -161,7 +161,9 @@ def test_gemm_nt(dtype, m, n, k, epilogue):
                                    (20, 60, 3104), (100, 1500, 3072), (230, 1040, 768), (70, 90, 100), (800, 40, 68),
                                    (65, 33, 32), (129, 4200, 64), (300, 65, 2080),
                                    # 9 to 16 rows over few weights: two blocks to a wave's one, two or four columns
-                                   (9, 330, 772), (13, 1601, 640), (16, 3101, 320)])
+                                   (9, 330, 772), (13, 1601, 640), (16, 3101, 320),
+                                   # very many columns: one row of tiles of 64 or 128 rows, and two
+                                   (128, 50001, 64), (129, 50001, 64)])
 @pytest.mark.parametrize("epilogue", ["none", "gelu_tanh", "residual"])
 def test_gemm_of_float_rows(m, n, k, epilogue):
     from pagedserve_amd.ops import kernels
