@@ -174,7 +174,8 @@ __global__ __launch_bounds__(256) void norm_wave_kernel(
 // waves share a row and meet through LDS: one where rows are many, four where they are few and what
 // counts is the one trip to memory (then a thread holds one or two pieces).  Measured, in us, single
 // values per lane before and now: 64 x 768 3.3 / 2.85, 544 x 1024 3.7 / 3.1, 2048 x 768 4.5 / 4.2, 4096 x
-// 1600 11.9 / 10.6.  Rows of up to 256 values, a handful per lane either way, stay with norm_wave_kernel.
+// 1600 11.9 / 10.6.  Short rows, a handful of values per lane either way, stay with norm_wave_kernel (launch_norm
+// says up to where).
 template <typename T>
 __device__ inline void store4(T* out, const float* v);
 template <>
@@ -242,6 +243,54 @@ __global__ __launch_bounds__(256) void norm_vec_kernel(
   }
 }
 
+// norm_row_kernel: one block of four waves per row, the row held in registers (width <= 256 *
+// VPT), the two sums met through LDS.  For few wide rows that cannot be read in pieces of four: a
+// wave alone would hold 25 values per lane at 1,601 columns and ask for them one after the
+// other, four waves ask for 7 each (16 x 1601 3.6 us, a wave to a row 4.8).
+template <typename T, bool RMS, int VPT>
+__global__ __launch_bounds__(256) void norm_row_kernel(
+    const float* __restrict__ x, const int* __restrict__ rows, const float* __restrict__ gamma,
+    const float* __restrict__ beta, T* __restrict__ out, int width, float eps, int packed) {
+  __shared__ float scratch[16];
+  const int r = blockIdx.x;
+  const float* src = x + (int64_t)(rows ? rows[r] : r) * width;
+  float v[VPT], g[VPT], b[VPT];
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const int col = threadIdx.x + i * 256;
+    const int safe = col < width ? col : width - 1;
+    v[i] = src[safe];
+    g[i] = gamma[safe];
+    b[i] = (!RMS && beta != nullptr) ? beta[safe] : 0.f;
+  }
+  float sum = 0.f;
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    if ((int)threadIdx.x + i * 256 >= width) v[i] = 0.f;
+    sum += v[i];
+  }
+  float mean = 0.f;
+  if (!RMS) mean = block_sum(sum, scratch) / (float)width;
+  float sq = 0.f;
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const int col = threadIdx.x + i * 256;
+    const float c = col < width ? v[i] - mean : 0.f;
+    v[i] = c;
+    sq += c * c;
+  }
+  const float inv_std = 1.0f / sqrtf(block_sum(sq, scratch) / (float)width + eps);
+  T* dst = out + (int64_t)r * width;
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const int col = threadIdx.x + i * 256;
+    if (col >= width) continue;
+    const T y = from_float<T>(v[i] * inv_std * g[i] + b[i]);
+    if (packed) out[packed_offset(r, col, width)] = y;
+    else dst[col] = y;
+  }
+}
+
 template <typename T, bool RMS>
 __global__ void norm_block_kernel(const float* __restrict__ x, const int* __restrict__ rows,
                                   const float* __restrict__ gamma, const float* __restrict__ beta,
@@ -270,7 +319,11 @@ __global__ void norm_block_kernel(const float* __restrict__ x, const int* __rest
   }
 }
 
-#define NORM_FEW_ROWS 256   // up to here a block of four waves per row
+#define NORM_FEW_ROWS 256    // up to here a block of four waves per row, from the width on where that
+#define NORM_FEW_WIDTH 512   // is no slower than a wave that reads single values (64 x 320 3.2 against 3.0 us,
+                             // 64 x 512 3.15 against 3.25, 64 x 768 3.2 against 3.6)
+#define NORM_MANY_WIDTH 320  // the same for more rows, a wave to a row (300 x 260 3.15 against 3.05, 300 x 320 3.05
+                             // against 3.1, 300 x 768 3.2 against 3.6)
 
 template <typename T, bool RMS>
 static void launch_norm(const float* x, const int* rows, const float* gamma, const float* beta,
@@ -279,7 +332,8 @@ static void launch_norm(const float* x, const int* rows, const float* gamma, con
   const dim3 grid((n_rows + 3) / 4);
   const uintptr_t all = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(gamma) |
                         reinterpret_cast<uintptr_t>(beta) | reinterpret_cast<uintptr_t>(out);
-  if (width % 4 == 0 && width > 256 && width <= 2048 && (all & 15u) == 0) {
+  if (width % 4 == 0 && width >= (n_rows <= NORM_FEW_ROWS ? NORM_FEW_WIDTH : NORM_MANY_WIDTH) && width <= 2048 &&
+      (all & 15u) == 0) {
 #define PS_LAUNCH_NV(PIECES, WAVES)                                                               \
   hipLaunchKernelGGL((norm_vec_kernel<T, RMS, PIECES, WAVES>), WAVES == 1 ? grid : dim3(n_rows),  \
                      dim3(256), 0, s, x, rows, gamma, beta, (T*)out, n_rows, width, eps, packed)
@@ -292,6 +346,15 @@ static void launch_norm(const float* x, const int* rows, const float* gamma, con
     else if (width <= 1536) PS_LAUNCH_NV(6, 1);
     else PS_LAUNCH_NV(8, 1);
 #undef PS_LAUNCH_NV
+    return;
+  }
+  if (n_rows <= 64 && per_lane > 12 && per_lane <= 32) {
+#define PS_LAUNCH_NR(VPT)                                                                          \
+  hipLaunchKernelGGL((norm_row_kernel<T, RMS, VPT>), dim3(n_rows), dim3(256), 0, s, x, rows, gamma, \
+                     beta, (T*)out, width, eps, packed)
+    if (per_lane <= 16) PS_LAUNCH_NR(4);
+    else PS_LAUNCH_NR(8);
+#undef PS_LAUNCH_NR
     return;
   }
 #define PS_LAUNCH_NW(VPT)                                                                       \

@@ -102,6 +102,41 @@ def test_rmsnorm():
     torch.testing.assert_close(out.double(), expected, atol=2e-5, rtol=2e-5)
 
 
+# Either side of the lines between the norm kernels: 64 and 256 rows, 320, 512 and 2,048 columns, whole pieces of four
+# or not, every number of pieces to a lane, operands off 16 bytes.
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rms", [False, True])
+@pytest.mark.parametrize("rows,width", [(1, 516), (3, 2048), (8, 1028), (64, 508), (64, 769), (64, 1601), (65, 1602), (256, 512), (256, 1024),
+                                        (257, 320), (257, 512), (300, 516), (257, 768), (300, 1000), (257, 1028), (300, 1536),
+                                        (257, 1540), (300, 2048), (2, 2052), (257, 2052), (300, 316)])
+def test_norm_kernels_at_their_edges(dtype, rms, rows, width):
+    from pagedserve_amd.ops import kernels
+
+    # (values far from zero: a sum that takes a row's neighbours in, or leaves a piece out, shows)
+    x = _rand((rows + 2, width), torch.float32, 521, 2.0) + 3.0
+    gamma = 1.0 + _rand((width,), torch.float32, 522, 0.2)
+    beta = None if rms else _rand((width,), torch.float32, 523)
+    picked = torch.randperm(rows + 2, generator=torch.Generator().manual_seed(7))[:rows].to(torch.int32).cuda()
+    xd = x.double()
+    centred = xd if rms else xd - xd.mean(-1, keepdim=True)
+    expected = centred * torch.rsqrt((centred * centred).mean(-1, keepdim=True) + 1e-5) * gamma.double()
+    expected = expected if beta is None else expected + beta.double()
+    atol, rtol = _tol(dtype)
+    for index in (None, picked):
+        want = expected[:rows] if index is None else expected[picked.long()]
+        out = torch.full((rows + 1, width), -7.0, dtype=dtype, device="cuda")
+        kernels.norm(x[:rows] if index is None else x, gamma, beta, 1e-5, out, rows=index, rms=rms)
+        torch.testing.assert_close(out[:rows].double(), want, atol=atol, rtol=rtol)
+        assert bool((out[rows] == -7.0).all())
+        # the rows, and the result, 4 or 2 bytes off a whole piece
+        moved = torch.empty(x.numel() + 1, device="cuda")[1:].view_as(x)
+        moved.copy_(x)
+        for source, target in ((moved, torch.empty_like(out)),
+                               (x, torch.empty(out.numel() + 1, dtype=dtype, device="cuda")[1:].view_as(out))):
+            kernels.norm(source[:rows] if index is None else source, gamma, beta, 1e-5, target, rows=index, rms=rms)
+            torch.testing.assert_close(target[:rows].double(), want, atol=atol, rtol=rtol)
+
+
 # rows 1..64 take the skinny kernel in bfloat16, more rows the tiled one; k = 100 and 66 are
 # not multiples of 8 and fall to the plain kernel
 GEMM_SHAPES = [(1, 50, 64), (5, 1000, 96), (64, 2304, 768), (130, 70, 320), (33, 257, 100),
