@@ -505,30 +505,42 @@ class Attention(Mixer):
         """(parts, waves) for the kernel that does attention and output projection of a decode step in
         one launch, or ``None`` where two launches are as fast: ``parts`` blocks per (token, head) pair, each
         with all keys and a part of the columns, blocks of ``waves`` waves.  (us for attention and
-        projection together, keys and weights from memory, two launches and one; keys in units of 64
-        dimensions.)
+        projection together, keys and weights from memory, two launches and one; "keys" are those of the context
+        class, in units of 64 dimensions.)
 
         * The keys of a pair go through one compute unit: up to 1,024 of them that costs less than a
-          second launch (1, 8 and 16 requests of 12 heads over 144 keys 8.6 / 5.9, 9.2 / 7.7 and 11.0 / 8.4, over
-          540 keys 9.7 / 8.3, 13.6 / 10.5 and 16.4 / 12.3, over 1,000 keys 9.7 / 9.5, 14.8 / 12.6 and
-          19.1 / 15.4); beyond, ranges are ahead (over 2,000 keys 10.2 / 13.8 and 18.3 / 18.9) unless the
-          pairs fill half of the units, where the two-launch path has few ranges or none either (23.9
-          / 20.5 with 12 requests).
-        * Parts until the blocks come to one per unit.  Up to 128 keys blocks of four waves are over
-          soonest and two or three of them share a unit (16 requests over 40 keys 8.6 / 7.0 in 3 parts, 8.0
-          with one block of 16 waves); up to 512 keys eight waves take them in one round of loads, beyond or without
-          parts sixteen.
+          second launch (1, 8 and 16 requests of 12 heads over 144 keys 8.5 / 6.0, 9.3 / 7.7 and 11.1 / 8.4, over
+          400 keys 9.0 / 7.1, 11.9 / 9.3 and 14.9 / 11.0; one over 20 keys 7.8 / 4.3); beyond, ranges are ahead (1 and 8
+          over 2,000 keys 10.2 / 13.8 and 18.3 / 18.9) unless the pairs fill half of the units, where the two-launch
+          path has few ranges or none either (23.9 / 20.5 with 12 requests).
+        * Parts until the blocks come to one per unit, but four from 1,024 keys on, which every part reads again (one
+          request of 25 heads over 900 keys in 8, 4 and 3 parts 13.2, 10.9 and 10.7, two launches 12.6).  Up to 128
+          keys blocks of four waves are over soonest and two or three of them share a unit; up to 512 keys eight
+          waves take them in one round of loads, if the part's weights are one round too (512 columns: 3 of 25
+          heads at width 1,600 over 250 keys in 2 parts 10.2 with eight waves and 9.6 with sixteen, two launches
+          10.2); beyond, or without parts, sixteen.
         * Between one and one and a half pairs per unit, up to 512 keys: four waves, two parts (24
-          requests over 270 keys 15.5 / 12.7; over 1,000 keys 23.6 / 24.5).
-        * Not where a block would take in more than 128 KB of weights, nor beyond some 330,000
-          atomic adds (8 requests of 25 heads at width 1,600 over 144 keys: 11.7 / 13.5).  An engine whose
-          requests never see 128 keys (a toy's bound, a tiny window) keeps the two launches, whose number
-          the tests of recorded steps count on."""
+          requests of 12 heads over 270 keys 15.5 / 12.7; over 1,000 keys 23.6 / 24.5).
+        * Every pair's adds and weights count against it: not beyond 330,000 adds or 500,000 x 64 weights (32 requests of
+          8 heads of 128 over 20 keys 9.0 / 10.1; 16 of 16 heads of 64 within 128 9.6 / 9.5).  At widths over 1,024, where the
+          projection alone is well spread over the units, only while the pairs' weights come to under 200,000 x 64
+          values and, with several requests, the pairs fill at most half of the units, since above that the two
+          launches need no ranges (within 128 keys, 4, 6 and 8 requests of 25 heads at width 1,600: 9.4 / 9.1, 8.9 / 11.2
+          and 9.1 / 12.5, 6 and 8 of 20 heads at 1,280: 9.3 / 8.3 and 8.4 / 9.5; 3 and 4 of 16 heads of 128 at 2,048:
+          10.7 / 9.6 and 11.3 / 11.8).  Nor where a block would take in more than 128 KB of weights.
+        * Heads that share their keys change nothing: a block loads its group's keys again, but out of the cache, and
+          the kernel that loads them once per group needs a merge (24 requests of 16 heads over 2 within 128 and over
+          400 keys 13.2 / 9.7 and 16.3 / 14.1; 8 over 4 heads of 64, 8 and 32 heads over one and four: the same order)."""
         pairs = count * self.heads
         units = kernels.compute_units()
-        keys = self._visible(max_kv_len) * self.head_dim // 64
-        if 2 * pairs > 3 * units or pairs * self.width > 330_000 or keys < 128:
+        visible = self._visible(max_kv_len)
+        keys = visible * self.head_dim // 64
+        weights = pairs * self.width * self.head_dim // 64
+        if 2 * pairs > 3 * units or pairs * self.width > 330_000 or weights > 500_000:
             return None
+        if self.width > 1024 and count > 1 and (2 * pairs > units or weights >= 200_000):
+            return None
+        tiles = -(-self.width // 16)
         if keys <= 128:
             parts, waves = max(1, min(12, (5 * units + pairs) // (2 * pairs))), 4
         elif pairs > units:
@@ -538,9 +550,9 @@ class Attention(Mixer):
         else:
             if keys > 1024 and (2 * pairs < units or keys >= 4096):
                 return None
-            parts = min(8, units // pairs)
-            waves = 8 if parts > 1 and keys <= 512 else 16
-        parts = min(parts, -(-self.width // 16))
+            parts = min(4 if visible > 512 else 8, units // pairs)
+            waves = 8 if parts > 1 and visible <= 512 and -(-tiles // parts) <= 32 else 16
+        parts = min(parts, tiles)
         if self.width * self.head_dim * 2 > 131072 * parts:
             return None
         return parts, waves

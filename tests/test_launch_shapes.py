@@ -81,6 +81,39 @@ def test_documented_cases(monkeypatch):
     assert _part(12, window=256)._splits(32, 8192) == (1, 4)
 
 
+def test_attention_and_projection_in_one_launch(monkeypatch):
+    """Where a decode step takes the kernel that does both: short contexts as well (a window, an engine of few pages),
+    wide models only while pairs and weights are few, whatever the sizes within what the kernel takes."""
+    monkeypatch.setattr(kernels, "compute_units", lambda: 256)
+    for keys in (1, 20, 64, 127, 128):
+        assert _part(12)._one_launch_decode(1, keys) == (12, 4) and _part(12)._one_launch_decode(16, keys) == (3, 4)
+    assert _part(12, window=64)._one_launch_decode(8, 1024) == (7, 4)
+    assert _part(12)._one_launch_decode(8, 512) == (2, 8) and _part(12)._one_launch_decode(16, 1024) == (1, 16)
+    assert _part(12)._one_launch_decode(1, 1024) == (4, 16) and _part(12)._one_launch_decode(1, 2048) is None
+    assert _part(12)._one_launch_decode(24, 512) == (2, 4) and _part(12)._one_launch_decode(24, 1024) is None
+    # wide models
+    for keys in (128, 256, 512):
+        for count in (5, 6, 7, 8):
+            assert _part(25)._one_launch_decode(count, keys) is None
+        assert _part(25)._one_launch_decode(1, keys) and _part(25)._one_launch_decode(4, keys)
+        assert _part(20)._one_launch_decode(6, keys) and _part(20)._one_launch_decode(7, keys) is None
+        assert _part(16, 128)._one_launch_decode(3, keys) and _part(16, 128)._one_launch_decode(4, keys) is None
+    assert _part(25)._one_launch_decode(3, 256) == (3, 16)      # 34 tiles of columns in a part: two rounds of eight waves
+    assert _part(20)._one_launch_decode(3, 256) == (4, 8)
+    assert _part(8, 128)._one_launch_decode(28, 64) and _part(8, 128)._one_launch_decode(32, 64) is None
+    for units in (256, 304, 64):
+        monkeypatch.setattr(kernels, "compute_units", lambda: units)
+        for heads in (1, 2, 3, 12, 16, 25, 40, 96):
+            for head_dim in (64, 128):
+                for window in (0, 33, 300):
+                    part = _part(heads, head_dim, window)
+                    for count in range(1, 65):
+                        for keys in (1, 64, 128, 200, 256, 512, 1024, 2048, 8192):
+                            shape = part._one_launch_decode(count, keys)
+                            if shape is not None:
+                                assert 1 <= shape[0] <= -(-part.width // 16) and shape[1] in (4, 8, 16)
+
+
 def test_query_tiles_of_the_prefill_attention(monkeypatch):
     """Which of the tiled kernel's three tile sizes a step takes: 32 queries while tiles of 64
     leave half of the compute units without a block, 128 from three blocks per unit on (head

@@ -70,7 +70,8 @@ def test_real_sizes_match_plain(shape_models, name, dtype):
             # the decoded tokens came from replays of a recorded step
             summary = engine.graph_summary()
             assert summary["graph_replays"] >= 3 * 15 and not summary["capture_failures"], summary
-            assert max(summary["graph_nodes"].values()) > 5 * config["n_layer"]
+            # with every layer's launches: four where norms and attention share one with a product
+            assert max(summary["graph_nodes"].values()) >= 4 * config["n_layer"]
     print(name, dtype, {cut: f"{e / s:.2e}" for cut, (e, s, _) in worst.items()})
     del model
     torch.cuda.empty_cache()
