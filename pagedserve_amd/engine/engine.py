@@ -14,7 +14,6 @@ only on (tokens, items, wanted rows), so a captured HIP graph of a decode step s
 valid from step to step.
 """
 
-import weakref
 from dataclasses import dataclass, field
 from typing import Hashable, List, Optional, Sequence
 
@@ -68,14 +67,6 @@ class _ReplayPlan:
         self.logits = logits
         self.tokens = tokens
         self.items = items
-
-
-def _drain(stream, *buffers):
-    """An engine is gone: its buffers are given back once its stream is through with them."""
-    try:
-        stream.synchronize()
-    except RuntimeError:       # (the device is gone with the process, or the work on it failed)
-        pass
 
 
 class StepError(ValueError):
@@ -138,8 +129,6 @@ class Engine:
         # The engine's work runs on a stream of its own (default priority): a capture cannot
         # record from the default stream.
         self.stream = torch.cuda.Stream(device=self.device)
-        # the pinned buffers, which kernels access without the allocator's knowledge, outlive the work on them
-        weakref.finalize(self, _drain, self.stream, self._meta_words, self._tokens_words)
         # a part that looks at host values of a step cannot be replayed
         self.use_graphs = use_graphs and getattr(model, "graph_safe", False)
         self.max_graphs = 48     # recorded layouts kept; the least recently replayed goes first

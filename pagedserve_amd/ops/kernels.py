@@ -2248,13 +2248,18 @@ def softcap(logits, cap):
 
 
 class HostWords:
-    """A pinned int32 buffer that kernels read and write themselves.  The copy engine's path holds a small
-    step up for tens of microseconds; a kernel's own access to the host's memory costs a launch and the trip.
+    """A pinned int32 buffer that kernels read and write themselves.  The copy engine's path holds a step of
+    more than some 10 KB up by tens of microseconds; a kernel's own access to the host's memory costs a launch and
+    the trip.
 
-    The allocator does not see these accesses: whoever owns the buffer keeps it until they are through."""
+    The allocator does not see these accesses.  So one word is copied by the library's own means on every
+    stream that meets the buffer: the allocator then hands its memory out again only behind that stream's work
+    at the time when the buffer goes, and nobody has to wait for the work (a wait, in a finalizer, would break a
+    capture that is under way in the same thread)."""
 
     def __init__(self, count: int):
-        self.tensor = torch.zeros(count, dtype=torch.int32, pin_memory=True)
+        self.tensor = torch.empty(count, dtype=torch.int32, pin_memory=True)
+        self._streams = set()
         address = c_void_p()
         _call("ps_host_address", self.tensor.data_ptr(), ctypes.cast(ctypes.pointer(address), c_void_p))
         self.address = address.value
@@ -2264,16 +2269,21 @@ class HostWords:
         if not (0 <= count <= self.tensor.numel() and count <= device_words.numel() and device_words.is_contiguous()):
             raise KernelError(f"{count} words do not fit a host buffer of {self.tensor.numel()} and a contiguous device "
                               f"buffer of {device_words.numel()}")
+        stream = _stream()
+        if stream not in self._streams and self.tensor.numel():
+            device_words.new_empty(1).copy_(self.tensor[:1], non_blocking=True)
+            self._streams.add(stream)
+        return stream
 
     def to_device(self, target, count: int):
         """target[:count] = the buffer's first ``count`` words, on the current stream."""
-        self._check_range(target, count)
-        _call("ps_copy_words", self.address, target.data_ptr(), count, _stream())
+        stream = self._check_range(target, count)
+        _call("ps_copy_words", self.address, target.data_ptr(), count, stream)
 
     def from_device(self, source, count: int):
         """The buffer's first ``count`` words = source[:count], on the current stream."""
-        self._check_range(source, count)
-        _call("ps_copy_words", source.data_ptr(), self.address, count, _stream())
+        stream = self._check_range(source, count)
+        _call("ps_copy_words", source.data_ptr(), self.address, count, stream)
 
 
 def sample(logits, inv_temperature, uniform, out):

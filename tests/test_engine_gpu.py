@@ -408,21 +408,72 @@ def test_words_between_host_memory_and_the_device(count, offset):
         torch.cuda.synchronize()
 
 
-def test_an_engine_that_goes_with_work_in_flight_waits_for_it(tmp_path):
-    """The pinned buffers of an engine are accessed by kernels: they are given back when its stream is through."""
+def _toy_engine():
+    from pagedserve_amd.engine import Engine
+    from pagedserve_amd.model import random_model
+
+    model, _ = random_model({"architectures": ["GPT2LMHeadModel"], "n_layer": 2, "n_embd": 64, "n_head": 4,
+                             "n_inner": 256, "vocab_size": 512, "n_positions": 128, "layer_norm_epsilon": 1e-5,
+                             "activation_function": "gelu_new", "eos_token_id": None}, dtype="bfloat16")
+    return Engine(model, num_pages=32, page_size=8, max_requests=2, max_step_tokens=64)
+
+
+def test_an_engine_that_goes_with_work_in_flight_keeps_its_pinned_memory():
+    """The pinned buffers of an engine are accessed by kernels.  They are not handed to anyone else while its
+    stream still has work, and nobody waits for that."""
     import gc
     import weakref
 
-    from pagedserve_amd.engine import Engine, StepEntry
-    from pagedserve_amd.model import random_model
+    from pagedserve_amd.engine import StepEntry
 
-    model, config = random_model({"architectures": ["GPT2LMHeadModel"], "n_layer": 2, "n_embd": 64, "n_head": 4,
-                                  "n_inner": 256, "vocab_size": 512, "n_positions": 128, "layer_norm_epsilon": 1e-5,
-                                  "activation_function": "gelu_new", "eos_token_id": None}, dtype="bfloat16")
-    engine = Engine(model, num_pages=32, page_size=8, max_requests=2, max_step_tokens=64)
+    engine = _toy_engine()
     for step in range(4):
         out = engine.step([StepEntry("a", [5 + step], [0])], greedy=True)
+    torch.cuda.synchronize()
+    buffers = engine._meta_host + engine._tokens_host
+    mine = {(b.data_ptr(), b.numel()) for b in buffers}
     stream, gone = engine.stream, weakref.ref(engine)
-    del engine, out
+    # (as many free blocks as are asked for below: memory from the system would wait for the device)
+    spare = [torch.empty(count, dtype=torch.int32, pin_memory=True) for _, count in mine]
+    del spare
     gc.collect()
-    assert gone() is None and stream.query()
+    with torch.cuda.stream(stream):
+        torch.cuda._sleep(400_000_000)      # (a tenth of a second at least)
+        for words in engine._meta_words + engine._tokens_words:
+            words.from_device(engine._tokens, 1)
+    del engine, out, buffers, words
+    assert gone() is None
+    others = [torch.empty(count, dtype=torch.int32, pin_memory=True) for _, count in mine]
+    assert not stream.query(), "the work was over too soon for this test"
+    assert not {b.data_ptr() for b in others} & {address for address, _ in mine}
+    stream.synchronize()
+
+
+def test_an_engine_that_goes_inside_a_capture_leaves_it_whole():
+    """The collector may end an engine at any place, also between the launches that another one records."""
+    import gc
+    import weakref
+
+    from pagedserve_amd.engine import StepEntry
+    from pagedserve_amd.ops import kernels
+
+    engine = _toy_engine()
+    for step in range(3):
+        engine.step([StepEntry("a", [5 + step], [0])], greedy=True)
+    engine.ring = engine          # only the collector ends it
+    gone = weakref.ref(engine)
+    x = torch.randn(4, 64, device="cuda")
+    gamma, out = torch.ones(64, device="cuda"), torch.zeros(4, 64, device="cuda")
+    side, graph = torch.cuda.Stream(), kernels.StepGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        kernels.StepGraph.begin()
+        kernels.norm(x, gamma, None, 1e-5, out)
+        del engine
+        gc.collect()
+        graph.end()
+        graph.launch()
+    torch.cuda.synchronize()
+    assert gone() is None and graph.nodes == 1
+    torch.testing.assert_close(out, torch.nn.functional.layer_norm(x, (64,), gamma), atol=1e-5, rtol=1e-5)
+    graph.destroy()
