@@ -1337,7 +1337,7 @@ def test_attention_with_the_output_projection_in_one_launch(heads, kv_heads, hea
     assert kernels.decode_linear_supported(dtype, count, head_dim, packed)
     for bias, sink, gate, cap in ((_rand((width,), torch.float32, 414), None, None, 0.0),
                                   (None, _rand((heads,), torch.float32, 416), _rand((count, heads), torch.float32, 417), 2.0)):
-        # the same kernel's parts, launched one after the other, are tested on their own: their result in float64
+        # (the row-wise kernel is tested on its own; the formulas in float64 are in the test below)
         context = torch.empty((count, heads * head_dim), dtype=dtype, device="cuda")
         kernels.attention_rowwise(q, k_pool, v_pool, context, tok_item, tok_pos, tables, heads, scale, window, sink=sink,
                                   gate=gate, softcap=cap)
@@ -1354,6 +1354,53 @@ def test_attention_with_the_output_projection_in_one_launch(heads, kv_heads, hea
         torch.testing.assert_close(residual[:count].double(), expected, atol=1e-2, rtol=5e-4)
         assert float((residual[:count].double() - expected).norm() / (expected - start[:count].double()).norm()) < 3e-3
         assert torch.equal(residual[count:], start[count:])
+
+
+@pytest.mark.parametrize("heads,kv_heads,head_dim,page_size,width,parts,waves", [(12, 4, 64, 16, 768, 3, 4), (4, 1, 128, 12, 200, 2, 8),
+                                                                                 (16, 2, 64, 16, 1000, 1, 16)])
+@pytest.mark.parametrize("window", [0, 33, -32])
+@pytest.mark.parametrize("options", ["sink and cap", "gate", "logistic and gate"])
+def test_attention_and_projection_with_every_option_in_float64(heads, kv_heads, head_dim, page_size, width, parts, waves, window,
+                                                               options):
+    """The same against the formulas alone: a sink in the softmax's denominator, capped scores, a gate per head,
+    logistic weights over a fixed norm, windows and chunks of keys."""
+    from pagedserve_amd.ops import kernels
+
+    dtype, contexts = torch.bfloat16, [1, 300, 16, 33, 65, 128]
+    count, group, scale = len(contexts), heads // kv_heads, head_dim ** -0.5
+    k_pool, v_pool, tables = _paged_fixture(dtype, contexts, kv_heads, head_dim, page_size, 421)
+    q = _rand((count, heads * head_dim), dtype, 422)
+    w = _rand((width, heads * head_dim), dtype, 423, 1.0 / math.sqrt(heads * head_dim))
+    sink = _rand((heads,), torch.float32, 424) if "sink" in options else None
+    gate = _rand((count, heads), torch.float32, 425) if "gate" in options else None
+    cap = 1.5 if "cap" in options else 0.0
+    logistic = (_rand((heads,), torch.float32, 426) - 2.0, 7.5) if "logistic" in options else None
+    k_cpu, v_cpu, t_cpu, q_cpu = k_pool.double().cpu(), v_pool.double().cpu(), tables.cpu(), q.double().cpu()
+    context = torch.empty((count, heads * head_dim), dtype=torch.float64)
+    for t, length in enumerate(contexts):
+        first = max(0, length - window) if window > 0 else ((length - 1) // -window * -window if window < 0 else 0)
+        keys = _gather(k_cpu, t_cpu[t], length, page_size)[:, first:].repeat_interleave(group, 0)
+        values = _gather(v_cpu, t_cpu[t], length, page_size)[:, first:].repeat_interleave(group, 0)
+        scores = torch.einsum("hd,hkd->hk", q_cpu[t].reshape(heads, head_dim), keys) * scale
+        if cap:
+            scores = cap * torch.tanh(scores / cap)
+        if logistic is not None:
+            weights = torch.sigmoid(scores + logistic[0].double().cpu()[:, None]) / logistic[1]
+        else:
+            joined = scores if sink is None else torch.cat([scores, sink.double().cpu()[:, None]], 1)
+            weights = torch.softmax(joined, -1)[:, :scores.shape[1]]
+        out = torch.einsum("hk,hkd->hd", weights, values)
+        if gate is not None:
+            out = out * torch.sigmoid(gate[t].double().cpu())[:, None]
+        context[t] = out.reshape(-1)
+    expected = context.to(dtype).cuda().double() @ w.double().t()
+    residual = torch.zeros((count, width), device="cuda")
+    kernels.attention_decode_linear(q, k_pool, v_pool, torch.tensor([c - 1 for c in contexts], dtype=torch.int32, device="cuda"),
+                                    tables, heads, scale, w, kernels.pack_decode_weight(w), None, residual, parts, waves,
+                                    window=window, sink=sink, gate=gate, softcap=cap, logistic=logistic)
+    # (a context value is a bfloat16 on either side, here and there a step apart, and its weights came from a product
+    # of bfloat16 values: 2^-8 of each, of which a third is left in the mean square)
+    assert float((residual.double() - expected).norm() / expected.norm()) < 3e-3
 
 
 @pytest.mark.parametrize("heads,kv_heads,head_dim,page_size", [(12, 12, 64, 16), (4, 2, 128, 12), (2, 1, 256, 16), (3, 3, 192, 8),

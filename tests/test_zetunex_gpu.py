@@ -62,6 +62,47 @@ def test_stream_step_adds_norms_and_clears(width):
     assert torch.allclose(dh.double().cpu(), h - 2 * y, atol=1e-5)
 
 
+# Every number of columns to a thread (1 to 8, rounded up to what is built, and the loop beyond), blocks of four and of
+# sixteen waves, rows that end inside a wave
+@pytest.mark.parametrize("tokens,width", [(257, 60), (300, 600), (257, 768), (300, 1000), (257, 1300), (300, 1600), (257, 2048), (256, 1100),
+                                          (300, 2049), (3, 2050), (2, 3100), (2, 4096), (3, 5001), (2, 6144), (2, 8192), (2, 8200)])
+def test_stream_step_at_every_width(tokens, width):
+    """All operands, and each of them left out."""
+    kernels = _kernels()
+    g = torch.Generator(device="cuda").manual_seed(width)
+    h, y, rows = (torch.randn((tokens, width), generator=g, device="cuda", dtype=torch.float32) for _ in range(3))
+    column, bias, gamma, gamma2 = (1 + 0.3 * torch.randn(width, generator=g, device="cuda") for _ in range(4))
+    for left_out in (None, "add", "column", "rows", "bias", "norm", "norm2", "zero"):
+        for dtype in (torch.float32, torch.bfloat16):
+            has = lambda name: left_out != name
+            stream = torch.cat([h, h[:1]])
+            buffer = torch.cat([y, y[:1]])
+            normed, normed2 = (torch.full((tokens + 1, width), -7.0, dtype=dtype, device="cuda") for _ in range(2))
+            expected = h.double()
+            if has("add"):
+                expected = expected + 0.35 * (column.double() if has("column") else 1.0) * y.double()
+            if has("rows"):
+                expected = expected + rows.double()
+            if has("bias"):
+                expected = expected + bias.double()
+            with_norm = has("norm")
+            kernels.stream_step(stream, tokens, width, add=(buffer, 0.35, column if has("column") else None) if has("add") else None,
+                                bias=bias if has("bias") else None, rows=rows if has("rows") else None,
+                                norm=(gamma, 1e-5, normed) if with_norm else None,
+                                norm2=(gamma2, normed2) if with_norm and has("norm2") else None,
+                                zero=buffer if has("zero") else None)
+            torch.testing.assert_close(stream[:tokens].double(), expected, atol=3e-6, rtol=1e-6)
+            unit = expected * torch.rsqrt((expected * expected).mean(-1, keepdim=True) + 1e-5)
+            tol = 1e-5 if dtype == torch.float32 else 2e-2
+            for out, scale, made in ((normed, gamma, with_norm), (normed2, gamma2, with_norm and has("norm2"))):
+                if made:
+                    torch.testing.assert_close(out[:tokens].double(), unit * scale.double(), atol=tol, rtol=tol)
+                assert bool((out[tokens if made else 0:] == -7.0).all())
+            assert torch.equal(buffer[:tokens], torch.zeros_like(y) if has("zero") else y)
+            # rows behind the tokens stay as they are
+            assert torch.equal(stream[tokens], h[0]) and torch.equal(buffer[tokens], y[0])
+
+
 def test_gate_product_and_pair_of_norms():
     kernels = _kernels()
     g = torch.Generator().manual_seed(3)
