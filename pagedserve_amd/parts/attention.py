@@ -519,8 +519,9 @@ class Attention(Mixer):
           waves take them in one round of loads, if the part's weights are one round too (512 columns: 3 of 25
           heads at width 1,600 over 250 keys in 2 parts 10.2 with eight waves and 9.6 with sixteen, two launches
           10.2); beyond, or without parts, sixteen.
-        * Between one and one and a half pairs per unit, up to 512 keys: four waves, two parts (24
-          requests of 12 heads over 270 keys 15.5 / 12.7; over 1,000 keys 23.6 / 24.5).
+        * Between one and one and a half pairs per unit, up to 512 keys, 256 of wider heads: four waves, two parts (24
+          requests of 12 heads over 270 keys 15.5 / 12.7; over 1,000 keys 23.6 / 24.5; of 12 heads of 128 over one
+          key/value head within 128 and over 250 keys 14.0 / 11.4 and 14.2 / 15.9).
         * Every pair's adds and weights count against it: not beyond 330,000 adds or 500,000 x 64 weights (32 requests of
           8 heads of 128 over 20 keys 9.0 / 10.1; 16 of 16 heads of 64 within 128 9.6 / 9.5).  At widths over 1,024, where the
           projection alone is well spread over the units, only while the pairs' weights come to under 200,000 x 64
@@ -530,7 +531,8 @@ class Attention(Mixer):
           10.7 / 9.6 and 11.3 / 11.8).  Nor where a block would take in more than 128 KB of weights.
         * Heads that share their keys change nothing: a block loads its group's keys again, but out of the cache, and
           the kernel that loads them once per group needs a merge (24 requests of 16 heads over 2 within 128 and over
-          400 keys 13.2 / 9.7 and 16.3 / 14.1; 8 over 4 heads of 64, 8 and 32 heads over one and four: the same order)."""
+          400 keys 13.2 / 9.7 and 16.3 / 14.1, 10 of 16 heads of 128 over one over 20 keys 14.0 / 9.7; of 12 over 2 and 32
+          over 4 likewise, the last up to the lines above)."""
         pairs = count * self.heads
         units = kernels.compute_units()
         visible = self._visible(max_kv_len)
@@ -544,7 +546,7 @@ class Attention(Mixer):
         if keys <= 128:
             parts, waves = max(1, min(12, (5 * units + pairs) // (2 * pairs))), 4
         elif pairs > units:
-            if keys > 512:
+            if keys > (512 if self.head_dim == 64 else 256):
                 return None
             parts, waves = 2, 4
         else:

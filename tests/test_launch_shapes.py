@@ -100,6 +100,8 @@ def test_attention_and_projection_in_one_launch(monkeypatch):
         assert _part(16, 128)._one_launch_decode(3, keys) and _part(16, 128)._one_launch_decode(4, keys) is None
     assert _part(25)._one_launch_decode(3, 256) == (3, 16)      # 34 tiles of columns in a part: two rounds of eight waves
     assert _part(20)._one_launch_decode(3, 256) == (4, 8)
+    assert _part(12)._one_launch_decode(24, 512) and _part(6, 128)._one_launch_decode(48, 128)
+    assert _part(6, 128)._one_launch_decode(48, 256) is None
     assert _part(8, 128)._one_launch_decode(28, 64) and _part(8, 128)._one_launch_decode(32, 64) is None
     for units in (256, 304, 64):
         monkeypatch.setattr(kernels, "compute_units", lambda: units)
