@@ -109,17 +109,21 @@ class Engine:
         capacity = ((7 + 2 * max(1, len(self.query_tiles))) * max_step_tokens + 5 * max_requests + 1
                     + len(groups) * max_requests * self.table_width + 16)
         self._meta_device = torch.empty(capacity, dtype=torch.int32, device=self.device)
-        self._meta_words = [kernels.HostWords(capacity) for _ in range(2)]
+        # chosen tokens: one per wanted row, and a step wants at most one row per token
+        most_tokens = max(max_requests, max_step_tokens)
+        # pinned: two buffers of indices and two of chosen tokens, each in whole pieces of 256 bytes
+        piece, token_piece = -(-capacity // 64) * 64, -(-most_tokens // 64) * 64
+        pinned = kernels.HostWords(2 * (piece + token_piece))
+        self._meta_words = [kernels.HostWords(capacity, pinned, turn * piece) for turn in range(2)]
         self._meta_host = [words.tensor for words in self._meta_words]
         self._meta_events = [torch.cuda.Event(), torch.cuda.Event()]
         self._meta_pending = [False, False]
         self._meta_owner = [None, None]   # replay plan whose constant arrays a buffer holds
         self._meta_turn = 0
         self._logits = None
-        # chosen tokens: one per wanted row, and a step wants at most one row per token
-        self._tokens = torch.zeros(max(max_requests, max_step_tokens), dtype=torch.int32,
-                                   device=self.device)
-        self._tokens_words = [kernels.HostWords(self._tokens.numel()) for _ in range(2)]
+        self._tokens = torch.zeros(most_tokens, dtype=torch.int32, device=self.device)
+        self._tokens_words = [kernels.HostWords(most_tokens, pinned, 2 * piece + turn * token_piece)
+                              for turn in range(2)]
         self._tokens_host = [words.tensor for words in self._tokens_words]
         self._tokens_ready = [torch.cuda.Event(), torch.cuda.Event()]
         self._tokens_turn = 0

@@ -2253,12 +2253,21 @@ class HostWords:
     the trip.
 
     The allocator does not see these accesses.  So one word is copied by the library's own means on every
-    stream that meets the buffer: the allocator then hands its memory out again only behind that stream's work
-    at the time when the buffer goes, and nobody has to wait for the work (a wait, in a finalizer, would break a
+    stream that meets the buffer (to a word behind it): the allocator then hands its memory out again only behind that
+    stream's work at the time when the buffer goes, and nobody has to wait for the work (a wait, in a finalizer, would break a
     capture that is under way in the same thread)."""
 
-    def __init__(self, count: int):
-        self.tensor = torch.empty(count, dtype=torch.int32, pin_memory=True)
+    def __init__(self, count: int, within: "HostWords" = None, begin: int = 0):
+        """``within``: the ``count`` words of another such buffer that start at word ``begin``, instead of memory of
+        its own (which costs the system a call, and every stream its one word)."""
+        if within is not None:
+            if begin < 0 or count < 0 or begin + count > within.tensor.numel():
+                raise KernelError(f"{count} words from {begin} on lie outside a buffer of {within.tensor.numel()}")
+            self.tensor, self._spare, self._streams = within.tensor[begin:begin + count], within._spare, within._streams
+            self.address = within.address + 4 * begin
+            return
+        memory = torch.empty(count + 1, dtype=torch.int32, pin_memory=True)
+        self.tensor, self._spare = memory[:count], memory[count:]
         self._streams = set()
         address = c_void_p()
         _call("ps_host_address", self.tensor.data_ptr(), ctypes.cast(ctypes.pointer(address), c_void_p))
@@ -2270,8 +2279,8 @@ class HostWords:
             raise KernelError(f"{count} words do not fit a host buffer of {self.tensor.numel()} and a contiguous device "
                               f"buffer of {device_words.numel()}")
         stream = _stream()
-        if stream not in self._streams and self.tensor.numel():
-            device_words.new_empty(1).copy_(self.tensor[:1], non_blocking=True)
+        if stream not in self._streams and device_words.numel():
+            self._spare.copy_(device_words[:1], non_blocking=True)
             self._streams.add(stream)
         return stream
 

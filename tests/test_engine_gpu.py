@@ -400,6 +400,16 @@ def test_words_between_host_memory_and_the_device(count, offset):
         words.to_device(device[:3], 4)
     with pytest.raises(kernels.KernelError):
         words.to_device(device.float(), 4)
+    # a part of the buffer, on its own
+    part = kernels.HostWords(8 + offset, words, 64)
+    before = words.tensor.clone()
+    device.fill_(11)
+    part.from_device(device, 5)
+    torch.cuda.synchronize()
+    before[64:69] = 11
+    assert torch.equal(words.tensor, before) and torch.equal(part.tensor, before[64:72 + offset])
+    with pytest.raises(kernels.KernelError):
+        kernels.HostWords(17, words, 70000)
     if count == 1 and offset == 0:
         plain = torch.zeros(64, dtype=torch.int32)
         with pytest.raises(kernels.KernelError):
@@ -430,8 +440,8 @@ def test_an_engine_that_goes_with_work_in_flight_keeps_its_pinned_memory():
     for step in range(4):
         out = engine.step([StepEntry("a", [5 + step], [0])], greedy=True)
     torch.cuda.synchronize()
-    buffers = engine._meta_host + engine._tokens_host
-    mine = {(b.data_ptr(), b.numel()) for b in buffers}
+    blocks = [words.tensor.untyped_storage() for words in engine._meta_words + engine._tokens_words]
+    mine = {(block.data_ptr(), block.nbytes() // 4) for block in blocks}
     stream, gone = engine.stream, weakref.ref(engine)
     # (as many free blocks as are asked for below: memory from the system would wait for the device)
     spare = [torch.empty(count, dtype=torch.int32, pin_memory=True) for _, count in mine]
@@ -441,7 +451,7 @@ def test_an_engine_that_goes_with_work_in_flight_keeps_its_pinned_memory():
         torch.cuda._sleep(400_000_000)      # (a tenth of a second at least)
         for words in engine._meta_words + engine._tokens_words:
             words.from_device(engine._tokens, 1)
-    del engine, out, buffers, words
+    del engine, out, blocks, words
     assert gone() is None
     others = [torch.empty(count, dtype=torch.int32, pin_memory=True) for _, count in mine]
     assert not stream.query(), "the work was over too soon for this test"
