@@ -92,8 +92,8 @@ __global__ __launch_bounds__(256) void gemm_nt_simple_kernel(
   }
 }
 
-// MR: rows held in registers, of which a block has the first, or at 9 to 16 rows the second eight; COLS: output columns per wave.  A lane walks k in
-// steps of 256 values and asks for 4 / COLS such steps of its COLS weight rows at once (four
+// MR: rows held in registers, of which a block has the first, or at 9 to 16 rows the second eight; COLS:
+// output columns per wave.  A lane walks k in steps of 256 values and asks for 4 / COLS such steps of its COLS weight rows at once (four
 // 16-byte loads in flight whatever COLS is); the sums are formed in the order of k either way,
 // so the result does not depend on COLS.
 template <int EPI, int MR, int COLS>

@@ -516,17 +516,17 @@ class Attention(Mixer):
         * Parts until the blocks come to one per unit, but four from 1,024 keys on, which every part reads again (one
           request of 25 heads over 900 keys in 8, 4 and 3 parts 13.2, 10.9 and 10.7, two launches 12.6).  Up to 128
           keys blocks of four waves are over soonest and two or three of them share a unit; up to 512 keys eight
-          waves take them in one round of loads, if the part's weights are one round too (512 columns: 3 of 25
-          heads at width 1,600 over 250 keys in 2 parts 10.2 with eight waves and 9.6 with sixteen, two launches
-          10.2); beyond, or without parts, sixteen.
+          waves take them in one round of loads, if the part's weights are one round too (512 columns: 3 requests of
+          25 heads at width 1,600 over 250 keys, 3 parts of 534, 10.4 with eight waves and 9.6 with sixteen, two
+          launches 10.2); beyond, or without parts, sixteen.
         * Between one and one and a half pairs per unit, up to 512 keys, 256 of wider heads: four waves, two parts (24
           requests of 12 heads over 270 keys 15.5 / 12.7; over 1,000 keys 23.6 / 24.5; of 12 heads of 128 over one
           key/value head within 128 and over 250 keys 14.0 / 11.4 and 14.2 / 15.9).
-        * Every pair's adds and weights count against it: not beyond 330,000 adds or 500,000 x 64 weights (32 requests of
-          8 heads of 128 over 20 keys 9.0 / 10.1; 16 of 16 heads of 64 within 128 9.6 / 9.5).  At widths over 1,024, where the
-          projection alone is well spread over the units, only while the pairs' weights come to under 200,000 x 64
-          values and, with several requests, the pairs fill at most half of the units, since above that the two
-          launches need no ranges (within 128 keys, 4, 6 and 8 requests of 25 heads at width 1,600: 9.4 / 9.1, 8.9 / 11.2
+        * Every pair's adds and weights count against it: not beyond 330,000 adds or 500,000 x 64 weights (32
+          requests of 8 heads of 128 over 20 keys 9.0 / 10.1; 16 of 16 heads of 64 within 128 9.6 / 9.5).  At widths
+          over 1,024, where the projection alone is well spread over the units, several requests take it only while
+          the pairs' weights come to under 200,000 x 64 values and the pairs fill at most half of the units, since
+          above that the two launches need no ranges (within 128 keys, 4, 6 and 8 requests of 25 heads at width 1,600: 9.4 / 9.1, 8.9 / 11.2
           and 9.1 / 12.5, 6 and 8 of 20 heads at 1,280: 9.3 / 8.3 and 8.4 / 9.5; 3 and 4 of 16 heads of 128 at 2,048:
           10.7 / 9.6 and 11.3 / 11.8).  Nor where a block would take in more than 128 KB of weights.
         * Heads that share their keys change nothing: a block loads its group's keys again, but out of the cache, and
