@@ -38,12 +38,14 @@ __device__ inline void mma_step(float, const u32x4_t& a, const u32x4_t& w, f32x1
 typedef const __attribute__((address_space(1))) void* global_ptr_t;
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
-// gelu_tanh(u) = u * sigmoid(2 z), z = sqrt(2/pi) (u + 0.044715 u^3), with the hardware
-// exponential and reciprocal: its error (about 1e-6 relative) is far below the rounding of a
-// bfloat16 result, which is the only place where it is used.
+// gelu_tanh(u) = u * sigmoid(2 z), z = sqrt(2/pi) (u + 0.044715 u^3), as u / (1 + 2^(u (c0 + c1 u^2))) with
+// the hardware exponential and reciprocal: its error (about 1e-6 relative) is far below the rounding of a
+// bfloat16 result, which is the only place where it is used.  Two of its eight instructions take four
+// slots each; with the exactly rounded reciprocal, three times as many instructions, a tile of 256 x 256
+// spent 17 us here, most of it in this function.
 __device__ inline float gelu_tanh_fast(float u) {
-  const float z2 = 1.5957691216057308f * (u + 0.044715f * u * u * u);
-  return u * __frcp_rn(1.0f + __expf(-z2));
+  const float exponent = u * fmaf(u * u, -0.10294324f, -2.3022082f);   // -2 z / ln 2
+  return u * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(exponent));
 }
 
 template <int EPI, typename TOut>
@@ -102,6 +104,41 @@ __device__ inline void store_wave_tile(f32x16 (&acc)[WM][WN], float* region, int
   int64_t pool_offset = 0;
   if (scatters && vec_kv) pool = kv_scatter_col<TOut>(scatter, col0, &pool_offset);
 
+  // What the whole pieces need from memory is asked for before the first of them: the residual rows, and
+  // where each token's keys and values lie (two dependent reads a row).  One trip each, not one per pass.
+  constexpr int PASSES = 32 / EP_ROWS;
+  constexpr bool RESIDUAL = EPI == PS_EPI_RESIDUAL;
+  float4 old[RESIDUAL ? WM : 1][RESIDUAL ? PASSES : 1][2];
+  if (RESIDUAL && !by_column && full) {
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+      for (int pass = 0; pass < PASSES; ++pass) {
+        const int row = row_base + i * 32 + pass * EP_ROWS + row_in_pass;
+        const float* sum = reinterpret_cast<const float*>(c) + (int64_t)(row < m ? row : m - 1) * ldc + col0;
+        old[RESIDUAL ? i : 0][RESIDUAL ? pass : 0][0] = *reinterpret_cast<const float4*>(sum);
+        old[RESIDUAL ? i : 0][RESIDUAL ? pass : 0][1] = *reinterpret_cast<const float4*>(sum + 4);
+      }
+  }
+  constexpr bool PLAIN = EPI == PS_EPI_NONE;
+  int64_t slots[PLAIN ? WM : 1][PLAIN ? PASSES : 1];
+  if (PLAIN && pool != nullptr) {
+    int pos[PLAIN ? WM : 1][PLAIN ? PASSES : 1], item[PLAIN ? WM : 1][PLAIN ? PASSES : 1];
+#pragma unroll
+    for (int i = 0; i < (PLAIN ? WM : 0); ++i)
+#pragma unroll
+      for (int pass = 0; pass < PASSES; ++pass) {
+        const int row = row_base + i * 32 + pass * EP_ROWS + row_in_pass;
+        pos[i][pass] = scatter.tok_pos[row < m ? row : m - 1];
+        item[i][pass] = scatter.tok_item[row < m ? row : m - 1];
+      }
+#pragma unroll
+    for (int i = 0; i < (PLAIN ? WM : 0); ++i)
+#pragma unroll
+      for (int pass = 0; pass < PASSES; ++pass)
+        slots[i][pass] = kv_scatter_slot(scatter, pos[i][pass], item[i][pass]);
+  }
+
 #pragma unroll
   for (int i = 0; i < WM; ++i) {
 #pragma unroll
@@ -139,8 +176,8 @@ __device__ inline void store_wave_tile(f32x16 (&acc)[WM][WN], float* region, int
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       continue;
     }
-#pragma unroll 2
-    for (int pass = 0; pass < 32 / EP_ROWS; ++pass) {
+#pragma unroll
+    for (int pass = 0; pass < PASSES; ++pass) {
       const int r = pass * EP_ROWS + row_in_pass;
       const int row = row_base + i * 32 + r;
       const float4 lo = *reinterpret_cast<const float4*>(region + r * EP_STRIDE + chunk * 8);
@@ -150,11 +187,10 @@ __device__ inline void store_wave_tile(f32x16 (&acc)[WM][WN], float* region, int
 #pragma unroll
       for (int q = 0; q < 8; ++q) v[q] = finish_value<EPI, TOut>(v[q] + b[q]);
       TOut* out = c + (int64_t)row * ldc + col0;
-      if (EPI == PS_EPI_RESIDUAL) {
+      if constexpr (RESIDUAL) {
         float* sum = reinterpret_cast<float*>(out);
         if (full) {
-          float4 o0 = *reinterpret_cast<const float4*>(sum);
-          float4 o1 = *reinterpret_cast<const float4*>(sum + 4);
+          float4 o0 = old[i][pass][0], o1 = old[i][pass][1];
           o0.x += v[0]; o0.y += v[1]; o0.z += v[2]; o0.w += v[3];
           o1.x += v[4]; o1.y += v[5]; o1.z += v[6]; o1.w += v[7];
           *reinterpret_cast<float4*>(sum) = o0;
@@ -163,22 +199,23 @@ __device__ inline void store_wave_tile(f32x16 (&acc)[WM][WN], float* region, int
           for (int q = 0; q < 8; ++q)
             if (col0 + q < n) sum[q] += v[q];
         }
-        continue;
-      }
-      if (full) {
-        // (eight key or value columns that go to their page and that nobody reads from c)
-        if (!(scatters && pool != nullptr && scatter.cache_only)) store8(out, v);
       } else {
-        for (int q = 0; q < 8; ++q)
-          if (col0 + q < n) out[q] = from_float<TOut>(v[q]);
-      }
-      if (scatters) {
-        if (pool != nullptr) {
-          const int64_t slot = kv_scatter_row(scatter, row);
-          if (slot >= 0) store8(pool + slot + pool_offset, v);
-        } else if (!vec_kv) {
+        if (full) {
+          // (eight key or value columns that go to their page and that nobody reads from c)
+          if (!(scatters && pool != nullptr && scatter.cache_only)) store8(out, v);
+        } else {
           for (int q = 0; q < 8; ++q)
-            if (col0 + q < n) kv_scatter_store<TOut>(scatter, row, col0 + q, v[q]);
+            if (col0 + q < n) out[q] = from_float<TOut>(v[q]);
+        }
+        if constexpr (PLAIN) {
+          if (scatters) {
+            if (pool != nullptr) {
+              if (slots[i][pass] >= 0) store8(pool + slots[i][pass] + pool_offset, v);
+            } else if (!vec_kv) {
+              for (int q = 0; q < 8; ++q)
+                if (col0 + q < n) kv_scatter_store<TOut>(scatter, row, col0 + q, v[q]);
+            }
+          }
         }
       }
     }
