@@ -1107,8 +1107,8 @@ _TILED_F32_CHECKED = False
 def attention_tiled_f32(q, k_pool, v_pool, out, tile_item, tile_q0, cu_tokens, kv_lens, tables, heads,
                         scale, window=0, sink=None, gate=None, softcap=0.0, logistic=None):
     """Attention of items with several tokens in true 32-bit, ``PREFILL_TILE`` queries per
-    block: keys and values pass through LDS once per tile of queries instead of once per query
-    (``attention_rowwise``), scores and sums are plain float arithmetic.  The tile list is the
+    listed tile: keys and values are read once per 32 queries instead of once per query
+    (``attention_rowwise``), scores and sums are true 32-bit arithmetic.  The tile list is the
     one of ``attention_prefill`` at that size."""
     global _TILED_F32_CHECKED
     if not _TILED_F32_CHECKED:

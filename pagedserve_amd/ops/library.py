@@ -38,6 +38,7 @@ HIPCC_FLAGS = [
 EXTRA_FLAGS = {
     "attention_prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "attention_mixed.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "attention_tiled_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "gemm_tiled.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 

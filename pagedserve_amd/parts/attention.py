@@ -457,7 +457,7 @@ class Attention(Mixer):
                                       memo=site_memo(self._memo_attention, ctx.workspace),
                                       shared=ctx.shared_calls, sink=sink, gate=gates, softcap=self.score_cap, logistic=self.logistic)
         elif singles < tokens and kernels.tiled_f32_supported(self.dtype, self.head_dim):
-            # 32-bit: tiles of queries too, on plain float arithmetic.  The tiles hold the items
+            # 32-bit: tiles of queries too, in true 32-bit arithmetic.  The tiles hold the items
             # of several tokens; one-token items that the split-KV kernel did not take (a head
             # size that it refuses) go to the kernel that takes all sizes
             tile_item, tile_q0 = ctx.query_tiles[kernels.PREFILL_TILE]
