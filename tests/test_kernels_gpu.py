@@ -1310,6 +1310,68 @@ def test_linear_takes_the_wide_product_for_long_k():
     assert torch.equal(v_pool.view(torch.int16), v_ref.view(torch.int16))
 
 
+@pytest.mark.parametrize("m,n,k", [(256, 640, 256), (300, 1000, 288), (1, 1, 256), (257, 129, 320), (700, 1601, 480), (513, 321, 1600),
+                                   (2300, 385, 352)])
+@pytest.mark.parametrize("width", [2, 3, 4, 5])
+@pytest.mark.parametrize("epilogue", ["none", "gelu_tanh", "residual"])
+def test_gemm_large_tile_shapes(m, n, k, width, epilogue):
+    """The product of thousands of rows at each of its tile widths: as few stages of k as it takes and counts that
+    leave every place of the ring at the end, rows and columns that end inside a tile and a wave's part of it, panels
+    of rows that are not full, output rows that do not allow 16-byte stores, input rows apart from one another."""
+    import ctypes
+
+    from pagedserve_amd.ops import kernels, library
+
+    lib = library.load_library()
+    fn = lib.ps_gemm_nt_large
+    fn.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 8 + [ctypes.c_void_p]
+    a = _rand((m, k + 16), torch.bfloat16, 330, 1.0)[:, :k]
+    w = _rand((n, k), torch.bfloat16, 331, 1.0 / math.sqrt(k))
+    bias = _rand((n,), torch.float32, 332)
+    product = a.double() @ w.double().t() + bias.double()
+    if epilogue == "residual":
+        out = _rand((m, n), torch.float32, 333)
+        expected = out.double() + product
+    else:
+        out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+        expected = F.gelu(product, approximate="tanh") if epilogue == "gelu_tanh" else product
+    status = fn(a.data_ptr(), w.data_ptr(), bias.data_ptr(), out.data_ptr(), m, n, k, a.stride(0), out.stride(0),
+                0 if out.dtype == torch.float32 else 1, kernels.EPILOGUES[epilogue], width,
+                torch.cuda.current_stream().cuda_stream)
+    assert status == 0, lib.ps_last_error().decode()
+    atol, rtol = (1e-4, 1e-5) if epilogue == "residual" else (4e-2, 2e-2)
+    torch.testing.assert_close(out.double(), expected, atol=atol, rtol=rtol)
+    # k in stages of 32, rows in pieces of 16 bytes: the rest is refused
+    for bad_k, bad_lda in ((k - 16, a.stride(0)), (k, a.stride(0) + 4), (224, a.stride(0))):
+        assert fn(a.data_ptr(), w.data_ptr(), bias.data_ptr(), out.data_ptr(), m, n, bad_k, bad_lda, out.stride(0),
+                  0 if out.dtype == torch.float32 else 1, kernels.EPILOGUES[epilogue], width, None) != 0
+
+
+def test_linear_takes_the_large_product_for_thousands_of_rows():
+    """Through ``kernels.linear``: rows and columns that fill the chip with tiles of 256 x 192, with the key/value
+    scatter behind the product, against float64 and a scatter of its own."""
+    from pagedserve_amd.ops import kernels
+
+    heads, kv_heads, head_dim, page_size, k = 24, 12, 64, 16, 768
+    q_cols, kv_cols = heads * head_dim, kv_heads * head_dim
+    n = q_cols + 2 * kv_cols
+    lens = [2000, 2050]
+    k_pool, v_pool, tables = _paged_fixture(torch.bfloat16, lens, kv_heads, head_dim, page_size, 340)
+    tok_item = torch.tensor([0] * 2000 + [1] * 2040, dtype=torch.int32, device="cuda")
+    tok_pos = torch.tensor(list(range(2000)) + list(range(10, 2050)), dtype=torch.int32, device="cuda")
+    x = _rand((4040, k), torch.bfloat16, 341)
+    w = _rand((n, k), torch.bfloat16, 342, 1.0 / math.sqrt(k))
+    bias = _rand((n,), torch.float32, 343)
+    out = torch.empty((4040, n), dtype=torch.bfloat16, device="cuda")
+    pools = k_pool.clone(), v_pool.clone()
+    kernels.linear(x, w, bias, out, packed=kernels.pack_decode_weight(w),
+                   scatter=(k_pool, v_pool, tok_item, tok_pos, tables, q_cols, kv_cols))
+    torch.testing.assert_close(out.double(), x.double() @ w.double().t() + bias.double(), atol=1e-2, rtol=5e-3)
+    kernels.kv_write(out[:, q_cols:q_cols + kv_cols], out[:, q_cols + kv_cols:], *pools, tok_item, tok_pos, tables)
+    assert torch.equal(k_pool.view(torch.int16), pools[0].view(torch.int16))
+    assert torch.equal(v_pool.view(torch.int16), pools[1].view(torch.int16))
+
+
 @pytest.mark.parametrize("heads,kv_heads,head_dim,page_size,width", [(12, 12, 64, 16, 768), (4, 2, 128, 12, 200), (3, 1, 64, 8, 40),
                                                                      (6, 6, 128, 16, 1000)])
 @pytest.mark.parametrize("count", [1, 3, 16, 20])
