@@ -32,33 +32,39 @@ __global__ __launch_bounds__(256) void gla_decay_kernel(
 }
 
 
-// A block (one wave) owns COLS columns of one head's state for one item of the step and walks
-// the item's tokens in order: lane = row group * COLS + column.  The state's rows are dealt to
-// the 64 / COLS row groups, RPL rows per lane, in registers; o needs the sum over the row groups,
-// which is taken through LDS once per chunk.  The walk is one dependent chain per token, so a launch with few
-// blocks takes narrow ones (4 columns, 16 row groups: a quarter of the work per lane and token,
-// four times the blocks), one with many the wide ones (16 columns, 4 row groups).  The
-// tokens' q, k and decays come GLA_CHUNK at a time (32 for key heads up to 64, fewer for larger
-// ones: 32 values per lane and array): a chunk's loads leave together into registers while the
-// chunk before is being worked on from LDS; the work on a chunk has to last as long as a trip
-// to memory for the walk not to wait, hence chunks as long as the registers allow.
-template <int RPL, int COLS, int GLA_CHUNK>
-__global__ __launch_bounds__(64) void gla_scan_kernel(
+// A block owns COLS columns of one head's state for one item of the step and walks the item's tokens in order:
+// thread = row group * COLS + column.  The state's rows are dealt to the row groups, RPL rows per thread, in
+// registers; o needs the sum over the row groups, which is taken through LDS once per chunk.  The tokens' q, k and
+// decays come GLA_CHUNK at a time: a chunk's loads leave together into registers while the chunk before is being
+// worked on from LDS.
+//
+// What bounds it: the walk is one dependent chain per token, so that a prompt waits for what a thread does per
+// token (3 RPL multiply-adds, four LDS reads, one write) and for its part of the staging.  Prompts therefore
+// take four waves to 16 columns, which stage q, k and decays for all of them; blocks of one wave and 4
+// columns staged them four times as often, 57 KB of LDS each, two to a compute unit.  5 prompts of 400 tokens at
+// 12 heads of 64: 151 -> 44 us, 16 of 128: 45 -> 27, one of 2,000: 350 -> 193.  Chunks of 32 let one block into
+// a unit instead of three (16 prompts of 128 45 us, 5 of 400 49).  Steps of single tokens take one wave and 4
+// columns (16 with many blocks), in chunks of 8.
+#define GLA_LONG 16   // tokens of a chunk of a prompt
+
+template <int RPL, int COLS, int GLA_CHUNK, int WAVES, bool HEAD_DECAY>
+__global__ __launch_bounds__(64 * WAVES) void gla_scan_kernel(
     const float* __restrict__ proj, int64_t ld, int q_col, int k_col, int v_col,
     const float* __restrict__ alpha, float* __restrict__ state, float* __restrict__ out,
     const int* __restrict__ cu_tokens, const int* __restrict__ slots, int heads, int key_dim,
     int value_dim, float q_scale, const float* __restrict__ head_decay, int silu_inputs) {
-  constexpr int GROUPS = 64 / COLS;                // row groups
+  constexpr int THREADS = 64 * WAVES;
+  constexpr int GROUPS = THREADS / COLS;                // row groups
   constexpr int ROWS = GROUPS * RPL;               // rows with padding up to the lanes' share
   constexpr int PAD = RPL + 4;                     // row groups start in different banks
-  constexpr int PER = GLA_CHUNK * ROWS / 64;       // values of a chunk per lane and array
-  constexpr int PER_V = (GLA_CHUNK * COLS + 63) / 64;
-  static_assert(GLA_CHUNK * ROWS % 64 == 0 && PER >= 1, "a chunk's rows are dealt evenly to the lanes");
+  constexpr int PER = GLA_CHUNK * ROWS / THREADS;       // values of a chunk per lane and array
+  constexpr int PER_V = (GLA_CHUNK * COLS + THREADS - 1) / THREADS;
+  static_assert(GLA_CHUNK * ROWS % THREADS == 0 && PER >= 1, "a chunk's rows are dealt evenly to the lanes");
   __shared__ __attribute__((aligned(16))) float s_q[GLA_CHUNK][GROUPS * PAD];
   __shared__ __attribute__((aligned(16))) float s_k[GLA_CHUNK][GROUPS * PAD];
   __shared__ __attribute__((aligned(16))) float s_a[GLA_CHUNK][GROUPS * PAD];
   __shared__ float s_v[GLA_CHUNK][COLS];
-  __shared__ float s_o[GLA_CHUNK][65];     // every lane's share of o_t (rows one bank apart)
+  __shared__ float s_o[GLA_CHUNK][THREADS + 1];     // every thread's share of o_t (rows one bank apart)
   const int item = blockIdx.x, head = blockIdx.y;
   const int lane = threadIdx.x;
   const int col = blockIdx.z * COLS + (lane % COLS);
@@ -76,24 +82,24 @@ __global__ __launch_bounds__(64) void gla_scan_kernel(
   const int channels = heads * key_dim;
   float rq[PER], rk[PER], ra[PER], rv[PER_V];
   // one decay per head for all key channels and tokens (then no array of decays is read)
-  const float fixed_decay = head_decay ? head_decay[head] : 0.f;
+  const float fixed_decay = HEAD_DECAY ? head_decay[head] : 0.f;
   // every load is unconditional from a clamped address; what lies outside is masked when stored
   auto fetch = [&](const int base) {
     const int count = (t1 - base) < GLA_CHUNK ? (t1 - base) : GLA_CHUNK;
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
-      const int idx = lane + j * 64;
+      const int idx = lane + j * THREADS;
       const int tt = idx / ROWS;
       const int r = idx - tt * ROWS;
       const int64_t t = base + (tt < count ? tt : 0);
       const int c = head * key_dim + (r < key_dim ? r : 0);
       rq[j] = proj[t * ld + q_col + c];
       rk[j] = proj[t * ld + k_col + c];
-      ra[j] = head_decay ? fixed_decay : alpha[t * channels + c];
+      ra[j] = HEAD_DECAY ? fixed_decay : alpha[t * channels + c];
     }
 #pragma unroll
     for (int j = 0; j < PER_V; ++j) {
-      const int idx = (lane + j * 64) % (GLA_CHUNK * COLS);
+      const int idx = (lane + j * THREADS) % (GLA_CHUNK * COLS);
       const int tt = idx / COLS;
       const int c = blockIdx.z * COLS + (idx - tt * COLS);
       const int64_t t = base + (tt < count ? tt : 0);
@@ -102,28 +108,32 @@ __global__ __launch_bounds__(64) void gla_scan_kernel(
   };
   auto stash = [&](const int base) {
     const int count = (t1 - base) < GLA_CHUNK ? (t1 - base) : GLA_CHUNK;
+    if (silu_inputs) {
+#pragma unroll
+      for (int j = 0; j < PER; ++j) {
+        rq[j] = rq[j] / (1.0f + expf(-rq[j]));
+        rk[j] = rk[j] / (1.0f + expf(-rk[j]));
+      }
+#pragma unroll
+      for (int j = 0; j < PER_V; ++j) rv[j] = rv[j] / (1.0f + expf(-rv[j]));
+    }
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
-      const int idx = lane + j * 64;
+      const int idx = lane + j * THREADS;
       const int tt = idx / ROWS;
       const int r = idx - tt * ROWS;
       const bool valid = tt < count && r < key_dim;
       const int at = (r / RPL) * PAD + (r % RPL);
-      if (silu_inputs) {
-        rq[j] = rq[j] / (1.0f + expf(-rq[j]));
-        rk[j] = rk[j] / (1.0f + expf(-rk[j]));
-      }
       s_q[tt][at] = valid ? rq[j] * q_scale : 0.f;
       s_k[tt][at] = valid ? rk[j] : 0.f;
       s_a[tt][at] = valid ? ra[j] : 0.f;
     }
 #pragma unroll
     for (int j = 0; j < PER_V; ++j) {
-      const int idx = lane + j * 64;
+      const int idx = lane + j * THREADS;
       if (idx < GLA_CHUNK * COLS) {
         const int tt = idx / COLS;
         const int c = blockIdx.z * COLS + (idx - tt * COLS);
-        if (silu_inputs) rv[j] = rv[j] / (1.0f + expf(-rv[j]));
         s_v[tt][idx - tt * COLS] = (tt < count && c < value_dim) ? rv[j] : 0.f;
       }
     }
@@ -157,7 +167,7 @@ __global__ __launch_bounds__(64) void gla_scan_kernel(
       for (int tt = 0; tt < count; ++tt) s_o[tt][lane] = token(tt);
     }
     __syncthreads();
-    for (int idx = lane; idx < count * COLS; idx += 64) {
+    for (int idx = lane; idx < count * COLS; idx += THREADS) {
       const int tt = idx / COLS;
       const int c = idx - tt * COLS;
       float sum = 0.f;
@@ -325,37 +335,39 @@ extern "C" int ps_gla_scan(const float* proj, int64_t ld, int q_col, int k_col, 
   PS_REQUIRE(heads <= 65535 && (value_dim + 3) / 4 <= 65535, "ps_gla_scan: grid too large");
   if (items == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
-  // narrow blocks while wide ones would leave the chip's SIMDs (four to a compute unit) idle
+  // items of a few tokens at most (decode steps): chunks of 8, which cost less to stage, and blocks of one wave,
+  // narrow ones while wide ones would leave the chip's SIMDs (four to a compute unit) idle
   const int64_t wide_blocks = (int64_t)items * heads * ((value_dim + 15) / 16);
   const bool narrow = wide_blocks < 2 * (int64_t)ps_compute_units();
-  // items of a few tokens at most (decode steps): chunks of 8, which cost less to stage
   const bool brief = longest > 0 && longest <= 8;
-#define PS_LAUNCH_GLA_C(RPL, COLS, CHUNK)                                                         \
-  hipLaunchKernelGGL((gla_scan_kernel<RPL, COLS, CHUNK>),                                         \
+#define PS_LAUNCH_GLA_H(RPL, COLS, CHUNK, WAVES, HEAD)                                            \
+  hipLaunchKernelGGL((gla_scan_kernel<RPL, COLS, CHUNK, WAVES, HEAD>),                            \
                      dim3(items, heads, (value_dim + COLS - 1) / COLS),                           \
-                     dim3(64), 0, s, proj, ld, q_col, k_col, v_col, alpha, state, out, cu_tokens, \
-                     slots, heads, key_dim, value_dim, q_scale, head_decay, silu_inputs)
-#define PS_LAUNCH_GLA(RPL, COLS)                                                                  \
+                     dim3(64 * WAVES), 0, s, proj, ld, q_col, k_col, v_col, alpha, state, out,    \
+                     cu_tokens, slots, heads, key_dim, value_dim, q_scale, head_decay, silu_inputs)
+#define PS_LAUNCH_GLA(RPL, COLS, CHUNK, WAVES)                                                    \
   do {                                                                                            \
-    if (brief) {                                                                                  \
-      PS_LAUNCH_GLA_C(RPL, COLS, 8);                                                              \
-    } else {                                                                                      \
-      PS_LAUNCH_GLA_C(RPL, COLS, (2048 / (64 / COLS * RPL) < 32 ? 2048 / (64 / COLS * RPL) : 32)); \
-    }                                                                                             \
+    if (head_decay != nullptr) PS_LAUNCH_GLA_H(RPL, COLS, CHUNK, WAVES, true);                    \
+    else PS_LAUNCH_GLA_H(RPL, COLS, CHUNK, WAVES, false);                                         \
   } while (0)
-  if (narrow) {
-    if (key_dim <= 32) PS_LAUNCH_GLA(2, 4);
-    else if (key_dim <= 64) PS_LAUNCH_GLA(4, 4);
-    else if (key_dim <= 128) PS_LAUNCH_GLA(8, 4);
-    else PS_LAUNCH_GLA(16, 4);
+  if (!brief) {
+    if (key_dim <= 32) PS_LAUNCH_GLA(2, 16, GLA_LONG, 4);
+    else if (key_dim <= 64) PS_LAUNCH_GLA(4, 16, GLA_LONG, 4);
+    else if (key_dim <= 128) PS_LAUNCH_GLA(8, 16, GLA_LONG, 4);
+    else PS_LAUNCH_GLA(16, 16, GLA_LONG / 2, 4);
+  } else if (narrow) {
+    if (key_dim <= 32) PS_LAUNCH_GLA(2, 4, 8, 1);
+    else if (key_dim <= 64) PS_LAUNCH_GLA(4, 4, 8, 1);
+    else if (key_dim <= 128) PS_LAUNCH_GLA(8, 4, 8, 1);
+    else PS_LAUNCH_GLA(16, 4, 8, 1);
   } else {
-    if (key_dim <= 32) PS_LAUNCH_GLA(8, 16);
-    else if (key_dim <= 64) PS_LAUNCH_GLA(16, 16);
-    else if (key_dim <= 128) PS_LAUNCH_GLA(32, 16);
-    else PS_LAUNCH_GLA(64, 16);
+    if (key_dim <= 32) PS_LAUNCH_GLA(8, 16, 8, 1);
+    else if (key_dim <= 64) PS_LAUNCH_GLA(16, 16, 8, 1);
+    else if (key_dim <= 128) PS_LAUNCH_GLA(32, 16, 8, 1);
+    else PS_LAUNCH_GLA(64, 16, 8, 1);
   }
 #undef PS_LAUNCH_GLA
-#undef PS_LAUNCH_GLA_C
+#undef PS_LAUNCH_GLA_H
   PS_CHECK_LAUNCH("ps_gla_scan");
   return 0;
 }
