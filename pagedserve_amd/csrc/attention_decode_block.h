@@ -4,6 +4,8 @@
 #pragma once
 #include <math.h>
 
+#include <type_traits>
+
 #include "common.h"
 
 // 2^x (the arguments here are never positive).  Scores are kept in units of log 2, so that no
@@ -44,11 +46,18 @@ struct DecodeLds {
   float ml[AD_WAVES][2];
 };
 
+struct NothingAhead {
+  __device__ void operator()() const {}
+};
+
 // The work of one block: token n of the list, one head, one range of its keys.  The caller
 // provides the block's LDS (the kernel below its own; a kernel that runs blocks of several
 // kinds in one launch a share of what all of them need).  `context` (one split only): the head's
 // finished values go there, into LDS, for the caller to go on with, instead of to `out`.
-template <typename T, int LPK, int AD_WAVES, int AD_UNROLL, bool NT>
+// `ahead` runs once in every wave, behind the first loads of keys and values: loads that the caller
+// wants to travel beside them and needs later.  (A wave's loads come back in the order of issue; asked
+// for earlier they would hold back the block table and with it the keys.)
+template <typename T, int LPK, int AD_WAVES, int AD_UNROLL, bool NT, typename Ahead = NothingAhead>
 __device__ __forceinline__ void attention_decode_block(
     DecodeLds<AD_WAVES>& lds, const int n, const int head, const int split,
     const T* __restrict__ q, int64_t q_stride, const T* __restrict__ k_pool,
@@ -57,7 +66,7 @@ __device__ __forceinline__ void attention_decode_block(
     const int* __restrict__ tok_item, const int* __restrict__ tok_pos,
     const int* __restrict__ tables, int table_width, int heads, int kv_heads, int head_dim,
     int page_size, int page_shift, int num_pages, float scale_log2, int window, int splits,
-    const AttnExtras extra, T* context = nullptr) {
+    const AttnExtras extra, T* context = nullptr, Ahead ahead = Ahead()) {
   constexpr int GROUPS = 64 / LPK;               // keys per wave load
   constexpr int KEYS_PER_WAVE = GROUPS * AD_UNROLL;
   float (&s_acc)[AD_WAVES][256] = lds.acc;
@@ -112,8 +121,7 @@ __device__ __forceinline__ void attention_decode_block(
   }
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 
-  for (int base = range_begin + wave * KEYS_PER_WAVE; base < range_end;
-       base += AD_WAVES * KEYS_PER_WAVE) {
+  auto turn = [&](const int base, auto first) {
     Raw8<T> kr[AD_UNROLL], vr[AD_UNROLL];
     bool valid[AD_UNROLL];
     // Every load is unconditional from a clamped address and masked afterwards, so that the
@@ -147,6 +155,11 @@ __device__ __forceinline__ void attention_decode_block(
           (has_dims ? dim0 : 0);
       kr[u].template load<NT>(k_pool + offset);
       vr[u].template load<NT>(v_pool + offset);
+    }
+    if constexpr (decltype(first)::value) {
+      __builtin_amdgcn_sched_barrier(0);
+      ahead();
+      __builtin_amdgcn_sched_barrier(0);
     }
     float s[AD_UNROLL];
     float m_new = m;
@@ -196,7 +209,15 @@ __device__ __forceinline__ void attention_decode_block(
       }
       m = m_new;
     }
+  };
+  int base = range_begin + wave * KEYS_PER_WAVE;
+  if constexpr (!std::is_same<Ahead, NothingAhead>::value) {
+    // the first turn on its own, so that its waits know which loads are behind its own
+    if (base < range_end) turn(base, std::true_type{});
+    else ahead();
+    base += AD_WAVES * KEYS_PER_WAVE;
   }
+  for (; base < range_end; base += AD_WAVES * KEYS_PER_WAVE) turn(base, std::false_type{});
   if (!has_dims) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc[i] = 0.f;

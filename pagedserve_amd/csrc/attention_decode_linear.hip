@@ -7,8 +7,8 @@
 // the exchange between the waves; then the rows of the context, the weights, the exchange, the add.  The
 // second chain mostly repeats waits of the first.  Here block (t, h, p) computes head h of token t over all
 // its keys (attention_decode_block.h) and multiplies it with the piece of W that belongs to head h
-// and to the p-th part of the columns, out of the packed copy of W (pagedserve_hip.h).  The piece is asked for before
-// the keys and travels beside them.  Blocks that differ in p repeat the attention: while the keys are few that costs
+// and to the p-th part of the columns, out of the packed copy of W (pagedserve_hip.h).  The piece is asked for right
+// behind the keys and travels beside them.  Blocks that differ in p repeat the attention: while the keys are few that costs
 // less than leaving compute units idle, since a unit takes in some 55 KB/us and what it has to take in (its
 // keys and its piece of W) is what the launch waits for beside the chain.  The sum over heads is made
 // by float atomic adds into the residual rows, in an order that differs from run to run within float
@@ -68,12 +68,11 @@ __global__ __launch_bounds__(64 * AD_WAVES) void attention_decode_linear_kernel(
           w_raw[c][st][h] = *reinterpret_cast<const uint4*>(w_tile + (st * 2 + h) * 512);
     }
   };
-  load_weights(0);
 
   attention_decode_block<bf16_t, 8 * STEPS, AD_WAVES, AD_UNROLL, false>(
       lds, token, head, 0, q, q_stride, k_pool, v_pool, (bf16_t*)nullptr, 0, nullptr, nullptr, nullptr,
       tok_pos, tables, table_width, heads, kv_heads, HEAD_DIM, page_size, page_shift, num_pages,
-      scale_log2, window, 1, extra, context);
+      scale_log2, window, 1, extra, context, [&] { load_weights(0); });
   __syncthreads();
 
   // row operand: row 0 is the head's context, the other fifteen are zero; lane l holds row l % 16,
