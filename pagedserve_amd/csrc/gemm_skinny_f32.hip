@@ -185,37 +185,49 @@ __global__ __launch_bounds__(512) void gemm_nt_skinny_norm_f32_kernel(
   const int sub = lane & 15;
   const int group = lane >> 4;
   const float* w_row = w + (int64_t)(n0 + sub < n ? n0 + sub : n - 1) * k;
-  f32x4 wf[UNROLL][2];
-#pragma unroll
-  for (int u = 0; u < UNROLL; ++u)
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int kk = (u * WAVES + wave) * SF_STEP + h * 16 + group * 4;
-      wf[u][h] = *reinterpret_cast<const f32x4*>(w_row + (kk < k ? kk : 0));
-      if (kk >= k) wf[u][h] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-#pragma unroll
-  for (int half = 0; half < 2; ++half) {
-    const int r = wave + half * WAVES;
-    if (r >= m) continue;
+  // The rows and the norm's scale and shift are asked for in front of the weights: a wave's loads come back in
+  // the order of issue, and the norm works while the weights travel.
+  const bool shifts = !norm.rms && norm.beta != nullptr;
+  const float* shift = shifts ? norm.beta : norm.gamma;
+  const bool two = m > WAVES;                        // a second row per wave
+  float v[2][PIECES][4], g[PIECES][4], b[PIECES][4];
+  auto load_row = [&](int half) {
+    const int r = wave + half * WAVES < m ? wave + half * WAVES : m - 1;
     const float* src = norm.h + (int64_t)(norm.rows ? norm.rows[r] : r) * norm.ldh;
-    const bool shifts = !norm.rms && norm.beta != nullptr;
-    const float* shift = shifts ? norm.beta : norm.gamma;
-    float v[PIECES][4], g[PIECES][4], b[PIECES][4];
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+      const int col = (lane + i * 64) * 4;
+      *reinterpret_cast<float4*>(v[half][i]) = *reinterpret_cast<const float4*>(src + (col < k ? col : k - 4));
+    }
+  };
+  f32x4 wf[UNROLL][2];
+  auto load_rest = [&] {
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) {
       const int col = (lane + i * 64) * 4;
       const int safe = col < k ? col : k - 4;
-      *reinterpret_cast<float4*>(v[i]) = *reinterpret_cast<const float4*>(src + safe);
       *reinterpret_cast<float4*>(g[i]) = *reinterpret_cast<const float4*>(norm.gamma + safe);
       *reinterpret_cast<float4*>(b[i]) = *reinterpret_cast<const float4*>(shift + safe);
     }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int kk = (u * WAVES + wave) * SF_STEP + h * 16 + group * 4;
+        wf[u][h] = *reinterpret_cast<const f32x4*>(w_row + (kk < k ? kk : 0));
+      }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto finish_row = [&](int half) {
+    const int r = wave + half * WAVES;
+    if (r >= m) return;
     float mean = 0.f;
     if (!norm.rms) {
       float sum = 0.f;
 #pragma unroll
       for (int i = 0; i < PIECES; ++i)
-        if ((lane + i * 64) * 4 < k) sum += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
+        if ((lane + i * 64) * 4 < k) sum += (v[half][i][0] + v[half][i][1]) + (v[half][i][2] + v[half][i][3]);
       mean = wave_sum(sum) / (float)k;
     }
     float sq = 0.f;
@@ -223,8 +235,8 @@ __global__ __launch_bounds__(512) void gemm_nt_skinny_norm_f32_kernel(
     for (int i = 0; i < PIECES; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        v[i][j] = (lane + i * 64) * 4 < k ? v[i][j] - mean : 0.f;
-        sq = fmaf(v[i][j], v[i][j], sq);
+        v[half][i][j] = (lane + i * 64) * 4 < k ? v[half][i][j] - mean : 0.f;
+        sq = fmaf(v[half][i][j], v[half][i][j], sq);
       }
     const float inv_std = 1.0f / sqrtf(wave_sum(sq) / (float)k + norm.eps);
 #pragma unroll
@@ -234,10 +246,27 @@ __global__ __launch_bounds__(512) void gemm_nt_skinny_norm_f32_kernel(
       f32x4 y;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        y[j] = shifts ? fmaf(v[i][j] * inv_std, g[i][j], b[i][j]) : v[i][j] * inv_std * g[i][j];
+        y[j] = shifts ? fmaf(v[half][i][j] * inv_std, g[i][j], b[i][j]) : v[half][i][j] * inv_std * g[i][j];
       *reinterpret_cast<f32x4*>(rows + r * STRIDE + col) = y;
     }
+  };
+  // (two paths, so that the waits of each know how many loads are behind the ones they wait for)
+  if (two) {
+    load_row(0);
+    load_row(1);
+    load_rest();
+    finish_row(0);
+    finish_row(1);
+  } else {
+    load_row(0);
+    load_rest();
+    finish_row(0);
   }
+#pragma unroll
+  for (int u = 0; u < UNROLL; ++u)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      if ((u * WAVES + wave) * SF_STEP + h * 16 + group * 4 >= k) wf[u][h] = f32x4{0.f, 0.f, 0.f, 0.f};
   __syncthreads();
   // (rows of LDS beyond m stay as they are: they only feed outputs that are never stored)
   constexpr int SETS = 3;     // (as above; the normed rows carry a rounding of their own)
