@@ -1,27 +1,36 @@
-// bfloat16 matrix product of thousands of rows in tiles of 256 x 128 to 256 x 320:
+// bfloat16 matrix product of hundreds to thousands of rows in tiles of 128 x 64 to 256 x 320:
 //   C[m, n] = epi(sum_k A[m, k] W[n, k] + b[n]),   k a multiple of 32.
 //
-// Eight waves, four along m and two along n, one block per compute unit; a wave owns 64 rows x 32 FN columns,
-// FN being 2 to 5.  Both operands go from global memory straight into LDS in stages of 32 values of k,
-// four to six of them in a ring.  What such a block can do is bounded by LDS: loads fill it at 64 bytes per
-// cycle and reads take 128, one after the other (a lone block of 64 x 64 takes 500 cycles for a k tile of 64,
-// 250 of each, however many stages or operands are fetched ahead).  A block of BM x BN therefore needs
-// 2 (BM + BN) + 2 BM + 4 BN cycles per 64 values of k where its products take BM BN / 32: the tiles are as
-// large as registers and LDS allow.
+// Eight waves, four along m and two along n, one block per compute unit; a wave owns 32 FM rows x 32 FN columns,
+// FM being 1 or 2 and FN 1 to 5.  Both operands go from global memory straight into LDS in stages of ROW bytes of
+// every row, two to six of them in a ring.  Two things bound such a block.
+//
+// What it takes in: a compute unit gets 45 KB/us of stages of 64-byte rows and 60 to 75 of 128-byte rows, which are
+// whole lines of the L2 (2048 x 2304 x 3072 in tiles of 128 x 192: 48 us with 64 bytes, 38 with 128; 256 x 128 at
+// 4096 x 1600 x 6400: 115 and 98).  Tiles up to 256 x 128 therefore have rows of 128 bytes.
+//
+// LDS, at the larger tiles: loads fill it at 64 bytes per cycle and reads take 128, one after the other (a lone block
+// of 64 x 64 takes 500 cycles for a k tile of 64, 250 of each, however many stages or operands are fetched ahead).
+// A block of 256 x BN therefore needs 2 (256 + BN) + 512 + 4 BN cycles per 64 values of k where its products take
+// 8 BN: the tiles are as large as registers and LDS allow.  There the number of stages counts for more than the
+// lines (256 x 320 at 4096 x 4800 x 1600: four of 64 bytes 65 us, two of 128 bytes 70; 256 x 256 at 4096 x 6400 x
+// 1600 104 and 109; 256 x 192 at 4096 x 2304 x 768 23.6 and 25.4).
 //
 // A load instruction blocks its wave until the address unit takes it.  Eight in a row kept the matrix cores idle at
 // the head of every stage (8,192 cubed: 1.21 PFLOP/s with the loads in a row, 1.98 with none, which is the
 // clock's limit), so each step issues its share of loads and its reads of the next step's operands between its
-// products.  A step is 16 values of k, two steps to a stage.  Step 1 of stage s meets the other waves in front of
-// its products: stage s has then been read by all of them, and stage s + 1 has landed.  It asks for the first half
-// of stage s + RING, step 0 of stage s + 1 for the second half.
+// products.  A step is 16 values of k, SUB = 2 or 4 steps to a stage.  The last step of stage s meets the other waves
+// in front of its products: stage s has then been read by all of them, and stage s + 1 has landed.  It asks for the
+// first part of stage s + RING, the steps of stage s + 1 but the last for the other parts.
 //
-// A stage holds 64 bytes of every row; piece c (16 bytes) of row r lies in slot c ^ ((r >> 2) & 3), so that the 16
-// lanes that read one piece of 16 consecutive rows touch every bank once.
+// A stage holds 64 or 128 bytes of every row; piece c (16 bytes) of row r lies in slot c ^ ((r >> 2) & 3) or
+// c ^ ((r >> 1) & 7), so that the 16 lanes that read one piece of 16 consecutive rows touch every bank once.
 //
 // Measured with weights from memory, in us, against the kernels that these products went to before (64 x 256 with
 // the weights past LDS, and the ring of 128 x 128): 4096 x 4800 x 1600 75 / 88, 4096 x 6400 x 1600 107 / 118,
-// 8192 x 2304 x 768 45 / 51, 8192 x 3072 x 768 58 / 67, 4096 x 4096 x 1024 44 / 55, 2048 x 6400 x 1600 57 / 73.  In a
+// 8192 x 2304 x 768 45 / 51, 8192 x 3072 x 768 58 / 67, 4096 x 4096 x 1024 44 / 55, 2048 x 6400 x 1600 57 / 73.  In tiles
+// of up to 256 x 128, against the same: 4096 x 1600 x 6400 98 / 131, 2048 x 3072 x 768 18.0 / 19.9, 2048 x 2304 x 768
+// 13.9 / 16.7, 2048 x 3072 x 1024 20 / 24, 544 x 4096 x 1024 13.6 / 14.9, 544 x 3072 x 1024 9.9 / 11.7.  In a
 // prefill that lasts 0.2 s the card's power sets the clock and 4096 x 6400 x 1600 is level (104 / 102).  What is
 // left beside the products is the ends of the tiles, 10 us a round, in which a unit that holds one block
 // multiplies nothing.
@@ -29,11 +38,8 @@
 
 #include "gemm_tile.h"
 
-#define GL_ROW 64          // bytes of a row and stage
 #define GL_WAVES_M 4
 #define GL_WAVES_N 2
-#define GL_BM 256
-#define GL_FM 2            // 32-row fragments of a wave
 
 template <int I, int N, typename F>
 __device__ __forceinline__ void gl_for(F&& f) {
@@ -56,36 +62,40 @@ __device__ __forceinline__ void gl_wait_and_sync() {
 }
 
 // The columns of a wave in slices of SLICE fragments: the region of LDS that a slice is turned through is smaller.
-template <int FN, int SLICE, int FIRST, typename TOut, int EPI>
-__device__ __forceinline__ void gl_store(f32x16 (&acc)[GL_FM][FN], float* region, int lane, int row, int col,
+template <int FM, int FN, int SLICE, int FIRST, typename TOut, int EPI>
+__device__ __forceinline__ void gl_store(f32x16 (&acc)[FM][FN], float* region, int lane, int row, int col,
                                          int m, int n, int ldc, TOut* c, const float* bias,
                                          const KvScatter& scatter) {
   if constexpr (FIRST < FN) {
     constexpr int COUNT = FIRST + SLICE <= FN ? SLICE : FN - FIRST;
-    f32x16 slice[GL_FM][COUNT];
+    f32x16 slice[FM][COUNT];
 #pragma unroll
-    for (int i = 0; i < GL_FM; ++i)
+    for (int i = 0; i < FM; ++i)
 #pragma unroll
       for (int j = 0; j < COUNT; ++j) slice[i][j] = acc[i][FIRST + j];
-    store_wave_tile<GL_FM, COUNT, TOut, EPI>(slice, region, lane, row, col + FIRST * 32, m, n, ldc, c, bias, 0, 1,
+    store_wave_tile<FM, COUNT, TOut, EPI>(slice, region, lane, row, col + FIRST * 32, m, n, ldc, c, bias, 0, 1,
                                              scatter);
-    gl_store<FN, SLICE, FIRST + COUNT, TOut, EPI>(acc, region, lane, row, col, m, n, ldc, c, bias, scatter);
+    gl_store<FM, FN, SLICE, FIRST + COUNT, TOut, EPI>(acc, region, lane, row, col, m, n, ldc, c, bias, scatter);
   }
 }
 
-template <int FN, int RING, typename TOut, int EPI>
+template <int FM, int FN, int ROW, int RING, typename TOut, int EPI>
 __global__ __launch_bounds__(512) void gemm_nt_bf16_large_kernel(
     const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, const float* __restrict__ bias,
     TOut* __restrict__ c, int m, int n, int k, int lda, int ldc, int tiles_m, int tiles_n, int panel,
     KvScatter scatter) {
   constexpr int WAVES = GL_WAVES_M * GL_WAVES_N;
-  constexpr int BN = 32 * FN * GL_WAVES_N;
-  constexpr int STAGE_BYTES = (GL_BM + BN) * GL_ROW;
-  constexpr int GROUPS = (GL_BM + BN) / 16;              // a load instruction fills 16 rows of a stage
+  constexpr int BM = 32 * FM * GL_WAVES_M, BN = 32 * FN * GL_WAVES_N;
+  static_assert(ROW == 64 || ROW == 128, "rows of half a line or of a whole one");
+  constexpr int SUB = ROW / 32;                          // steps of a stage
+  constexpr int PIECES = ROW / 16, SHIFT = ROW == 64 ? 2 : 1;
+  constexpr int GROUP = 1024 / ROW;                      // rows of a stage that a load instruction fills
+  constexpr int STAGE_BYTES = (BM + BN) * ROW;
+  constexpr int GROUPS = (BM + BN) / GROUP;
   constexpr int LOADS = (GROUPS + WAVES - 1) / WAVES;
-  constexpr int FIRST_HALF = (LOADS + 1) / 2;
-  constexpr int READS = GL_FM + FN, PRODUCTS = GL_FM * FN;
-  static_assert((RING - 1) * LOADS + FIRST_HALF < 64, "the load counter has six bits");
+  constexpr int FIRST_PART = (LOADS + SUB - 1) / SUB;    // part p: the loads from p LOADS / SUB on, rounded up
+  constexpr int READS = FM + FN, PRODUCTS = FM * FN;
+  static_assert((RING - 1) * LOADS + FIRST_PART < 64, "the load counter has six bits");
   __shared__ __attribute__((aligned(1024))) unsigned char lds[RING * STAGE_BYTES];
 
   const int tid = threadIdx.x;
@@ -100,11 +110,11 @@ __global__ __launch_bounds__(512) void gemm_nt_bf16_large_kernel(
   const int first_row = tile / (panel * tiles_n) * panel;
   const int within = tile - first_row * tiles_n;
   const int panel_rows = min(panel, tiles_m - first_row);
-  const int m0 = (first_row + within % panel_rows) * GL_BM;
+  const int m0 = (first_row + within % panel_rows) * BM;
   const int n0 = within / panel_rows * BN;
-  const int stages = k / 32;
+  const int stages = k / (ROW / 2);
 
-  // ---- loads: lane l of an instruction fills slot l % 4 of row l / 4 of its 16 rows.  Rows beyond m or n are
+  // ---- loads: lane l of an instruction fills slot l % PIECES of row l / PIECES of its rows.  Rows beyond m or n are
   // fetched from the last valid one (they feed outputs that are never stored).  Where the groups do not go
   // round, the last waves fetch the last group once more.
   const char* base_a = reinterpret_cast<const char*>(a + (int64_t)m0 * lda);
@@ -115,133 +125,171 @@ __global__ __launch_bounds__(512) void gemm_nt_bf16_large_kernel(
 #pragma unroll
   for (int j = 0; j < LOADS; ++j) {
     const int group = j * WAVES + wave < GROUPS ? j * WAVES + wave : GROUPS - 1;
-    const int row = group * 16 + (lane >> 2);
-    const int piece = (lane & 3) ^ ((row >> 2) & 3);
-    of_a[j] = group * 16 < GL_BM;
+    const int row = group * GROUP + lane / PIECES;
+    const int piece = (lane & (PIECES - 1)) ^ ((row >> SHIFT) & (PIECES - 1));
+    of_a[j] = group * GROUP < BM;
     offset[j] = of_a[j] ? (uint32_t)min(row, m - 1 - m0) * (uint32_t)lda * 2u + piece * 16
-                        : (uint32_t)min(row - GL_BM, n - 1 - n0) * (uint32_t)k * 2u + piece * 16;
-    target[j] = group * 16 * GL_ROW;
+                        : (uint32_t)min(row - BM, n - 1 - n0) * (uint32_t)k * 2u + piece * 16;
+    target[j] = group * GROUP * ROW;
   }
   auto load = [&](int stage, int j) {
-    const char* base = (of_a[j] ? base_a : base_w) + (int64_t)stage * GL_ROW;
+    const char* base = (of_a[j] ? base_a : base_w) + (int64_t)stage * ROW;
     __builtin_amdgcn_global_load_lds((global_ptr_t)(base + offset[j]),
                                      (lds_ptr_t)(lds + (stage % RING) * STAGE_BYTES + target[j]), 16, 0, 0);
   };
 
-  f32x16 acc[GL_FM][FN];
+  f32x16 acc[FM][FN];
 #pragma unroll
-  for (int i = 0; i < GL_FM; ++i)
+  for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
   // ---- operands: lane l reads the 16 bytes of k piece 2 s + l / 32 of row l % 32
-  const int key = (lane >> 2) & 3;
+  const int key = (lane >> SHIFT) & (PIECES - 1);
   const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_ptr_t)lds;
-  const uint32_t a_row = lds_base + (wave_m * GL_FM * 32 + (lane & 31)) * GL_ROW;
-  const uint32_t w_row = lds_base + (GL_BM + wave_n * FN * 32 + (lane & 31)) * GL_ROW;
-  const uint32_t slot[2] = {(uint32_t)(((lane >> 5) ^ key) << 4), (uint32_t)(((2 + (lane >> 5)) ^ key) << 4)};
+  const uint32_t a_row = lds_base + (wave_m * FM * 32 + (lane & 31)) * ROW;
+  const uint32_t w_row = lds_base + (BM + wave_n * FN * 32 + (lane & 31)) * ROW;
+  uint32_t slot[SUB];
+#pragma unroll
+  for (int q = 0; q < SUB; ++q) slot[q] = (uint32_t)(((2 * q + (lane >> 5)) ^ key) << 4);
   u32x4_t operands[2][READS];
   auto read = [&](uint32_t stage_offset, auto step, auto index, u32x4_t* to) {
     constexpr int R = decltype(index)::value;
-    const uint32_t at = stage_offset + slot[decltype(step)::value] + (R < GL_FM ? a_row : w_row);
-    gl_read<(R < GL_FM ? R : R - GL_FM) * 32 * GL_ROW>(to[R], at);
+    const uint32_t at = stage_offset + slot[decltype(step)::value] + (R < FM ? a_row : w_row);
+    gl_read<(R < FM ? R : R - FM) * 32 * ROW>(to[R], at);
   };
-  // Step S of a stage: the products of operands[S], the reads of the next step's operands and half of a stage's
+  // Step S of a stage: the products of operands[S % 2], the reads of the next step's operands and a part of a stage's
   // loads between them.  LOAD: the stage that is asked for exists; AHEAD: how many stages behind the next one may
   // be on their way when that one has to be there, -1: there is no next step.
   auto step = [&](int stage, auto which, auto loads, auto ahead) {
     constexpr int S = decltype(which)::value, AHEAD = decltype(ahead)::value;
     constexpr bool LOAD = decltype(loads)::value, NEXT = AHEAD >= 0;
-    constexpr int FROM = S == 1 ? 0 : FIRST_HALF, COUNT = S == 1 ? FIRST_HALF : LOADS - FIRST_HALF;
-    const uint32_t next_stage = (uint32_t)(((S == 1 ? stage + 1 : stage) % RING) * STAGE_BYTES);
+    constexpr bool LAST = S == SUB - 1;
+    constexpr int PART = (S + 1) % SUB;
+    constexpr int FROM = (PART * LOADS + SUB - 1) / SUB, COUNT = ((PART + 1) * LOADS + SUB - 1) / SUB - FROM;
+    const uint32_t next_stage = (uint32_t)(((LAST ? stage + 1 : stage) % RING) * STAGE_BYTES);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    if constexpr (S == 1 && NEXT) gl_wait_and_sync<(AHEAD > 0 ? AHEAD : 0) * LOADS>();
+    if constexpr (LAST && NEXT) gl_wait_and_sync<(AHEAD > 0 ? AHEAD : 0) * LOADS>();
 #pragma unroll
-    for (int r = 0; r < READS; ++r) asm volatile("" : "+v"(operands[S][r]));   // used only behind the wait
+    for (int r = 0; r < READS; ++r) asm volatile("" : "+v"(operands[S & 1][r]));   // used only behind the wait
     gl_for<0, PRODUCTS>([&](auto product) {
       constexpr int Q = decltype(product)::value;
       constexpr int I = Q / FN, J = Q % FN;
-      acc[I][J] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, operands[S][I]),
-                                                          __builtin_bit_cast(bf16x8, operands[S][GL_FM + J]),
+      acc[I][J] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, operands[S & 1][I]),
+                                                          __builtin_bit_cast(bf16x8, operands[S & 1][FM + J]),
                                                           acc[I][J], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (NEXT)
         gl_for<Q * READS / PRODUCTS, (Q + 1) * READS / PRODUCTS>([&](auto index) {
-          read(next_stage, std::integral_constant<int, S ^ 1>{}, index, operands[S ^ 1]);
+          read(next_stage, std::integral_constant<int, PART>{}, index, operands[(S + 1) & 1]);
         });
       if constexpr (LOAD)
         gl_for<0, COUNT>([&](auto index) {
           constexpr int L = decltype(index)::value;
           if constexpr (Q == (2 * L + 1) * PRODUCTS / (2 * COUNT))
-            load(S == 1 ? stage + RING : stage + RING - 1, FROM + L);
+            load(LAST ? stage + RING : stage + RING - 1, FROM + L);
         });
       __builtin_amdgcn_sched_barrier(0);
     });
   };
   using Zero = std::integral_constant<int, 0>;
-  using One = std::integral_constant<int, 1>;
+  using Last = std::integral_constant<int, SUB - 1>;
   using Yes = std::true_type;
   using No = std::false_type;
 
-  // stages 0 .. RING - 2, and the first half of stage RING - 1 (the host sends no product of fewer than RING stages)
+  // stages 0 .. RING - 2, and the first part of stage RING - 1 (the host sends no product of fewer than RING stages)
 #pragma unroll
   for (int d = 0; d < RING - 1; ++d)
 #pragma unroll
     for (int j = 0; j < LOADS; ++j) load(d, j);
 #pragma unroll
-  for (int j = 0; j < FIRST_HALF; ++j) load(RING - 1, j);
-  gl_wait_and_sync<(RING - 2) * LOADS + FIRST_HALF>();
+  for (int j = 0; j < FIRST_PART; ++j) load(RING - 1, j);
+  gl_wait_and_sync<(RING - 2) * LOADS + FIRST_PART>();
   gl_for<0, READS>([&](auto index) { read(0, Zero{}, index, operands[0]); });
   using Full = std::integral_constant<int, RING - 2>;
   int stage = 0;
   for (; stage + RING < stages; ++stage) {
-    step(stage, Zero{}, Yes{}, Full{});
-    step(stage, One{}, Yes{}, Full{});
+    gl_for<0, SUB>([&](auto which) { step(stage, which, Yes{}, Full{}); });
   }
-  // the last RING stages; the first of them still asks for the second half of the last one
+  // the last RING stages; the first of them still asks for the other parts of the last one
   gl_for<0, RING>([&](auto index) {
     constexpr int T = decltype(index)::value;
-    step(stage + T, Zero{}, std::integral_constant<bool, T == 0>{}, Full{});
-    step(stage + T, One{}, No{},
+    gl_for<0, SUB - 1>([&](auto which) { step(stage + T, which, std::integral_constant<bool, T == 0>{}, Full{}); });
+    step(stage + T, Last{}, No{},
          std::integral_constant<int, T == RING - 1 ? -1 : (RING - 2 - T > 0 ? RING - 2 - T : 0)>{});
   });
 
   // ---- epilogue: no load or read is on its way, and every wave is past its last operand
-  constexpr int SLICE = FN < 5 ? 2 : 1;      // (FN = 5 has registers for one fragment's residual rows)
+  constexpr int SLICE = FN > 1 && FN < 5 ? 2 : 1;      // (FN = 5 has registers for one fragment's residual rows)
   static_assert(WAVES * 32 * (SLICE * 32 + 8) * 4 <= RING * STAGE_BYTES, "the epilogue reuses the stages");
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  gl_store<FN, SLICE, 0, TOut, EPI>(acc, reinterpret_cast<float*>(lds) + wave * 32 * (SLICE * 32 + 8), lane,
-                                    m0 + wave_m * GL_FM * 32, n0 + wave_n * FN * 32, m, n, ldc, c, bias, scatter);
+  gl_store<FM, FN, SLICE, 0, TOut, EPI>(acc, reinterpret_cast<float*>(lds) + wave * 32 * (SLICE * 32 + 8), lane,
+                                    m0 + wave_m * FM * 32, n0 + wave_n * FN * 32, m, n, ldc, c, bias, scatter);
 }
 
 // --------------------------------------------------------------------------------- host
-// Which width (FN) a product takes, 0: not this kernel.  A block has its compute unit to itself, so that time goes
-// in rounds: `share` is the part of the rounds' outputs that the product needs.  At a full chip a tile's outputs per
-// time stand as 0.70, 0.87, 0.95 and 1 for FN of 2 to 5 (256 x 128 44 us for 1600 values of k where 256 x 320
-// takes 78).  Against the other kernels the line lies at 0.6 of a full chip of the widest tiles: 2048 x 4800 x 1600
-// (0.68) 44 us where they take 50, 4096 x 3072 x 768 (0.87) 31 and 39; 4096 x 1600 x 1600 (0.55) 38 and 36,
-// 8192 x 768 x 3072 (0.52) 57 and 58, 4096 x 1024 x 4096 (0.35) 57 and 50.  Short products are left to them: with k
+// The tiles by number: 10 x the fragments of a wave along m + those along n (12: 128 x 128); 2 to 5 are 256 x 128 to
+// 256 x 320 in rows of 64 bytes.
+static int tile_rows(int shape) { return 32 * GL_WAVES_M * (shape < 20 && shape > 9 ? 1 : 2); }
+static int tile_columns(int shape) { return 32 * GL_WAVES_N * (shape % 10); }
+
+// Tiles of up to 256 x 128, for a product that they cover in one round of blocks: the smallest of them that does, as a
+// unit without a block does nothing and a second round takes as long as the first.  What 64 x 64 tiles cover in one
+// round is left to them (1000 x 1024 x 1024 9.0 us, in 128 x 64 9.6; 300 x 3072 x 768 7.2 and 8.1).  In us, former kernel
+// and this one: in 128 x 64 tiles 544 x 3072 x 1024 11.7 and 9.9, 300 x 4096 x 1024 11.5 and 10.0, 2048 x 1024 x 4096 33.5
+// and 29.2; 128 x 128 1000 x 3072 x 768 13.3 and 11.9, 640 x 4096 x 1024 15.5 and 14.5, 2048 x 1600 x 6400 68 and 63, 2800
+// x 768 x 3072 46 and 31; 128 x 192 2048 x 3072 x 1024 22.8 and 20.0, 2048 x 2304 x 768 16.7 and 14.5; 256 x 128 2048 x 4096
+// x 1024 27.7 and 24.7, 8192 x 768 x 3072 53 and 46, 4096 x 1600 x 6400 116 and 95.
+// 128 x 64 on few of the units are behind two blocks of 64 x 64 on each: on 132 of them 1400 x 768 x 3072 takes 18.6 us
+// there and 20.5 here, on 144 330 x 3072 x 768 is level, on 180 544 x 2304 x 768 takes 8.3 and 7.9.  A residual product
+// reads the rows that it adds to behind its last product, which two blocks hide from each other: on 192 units 2048 x 768 x
+// 3072 takes 21.8 there and 22.7 here.  With k under 768 the ends of a tile take longer than its products (600 x 4096 x 512
+// 8.9 there, 9.3 here).
+static int medium_shape(int m, int n, int k, int epilogue) {
+  if (m <= 128 || k < 768 || k % 64 != 0) return 0;
+  const int units = ps_compute_units();
+  if ((int64_t)((m + 63) / 64) * ((n + 63) / 64) <= units) return 0;
+  static const int shapes[] = {11, 12, 13, 22};
+  for (int shape : shapes) {
+    const int rows = tile_rows(shape), columns = tile_columns(shape);
+    const int64_t tiles = (int64_t)((m + rows - 1) / rows) * ((n + columns - 1) / columns);
+    if (tiles > units) continue;
+    return shape == 11 && 8 * tiles <= (epilogue == PS_EPI_RESIDUAL ? 6 : 5) * units ? 0 : shape;
+  }
+  return 0;
+}
+
+// Which width (FN) a product of several rounds or of wider tiles takes, 0: not this kernel.  A block has its compute
+// unit to itself, so that time goes in rounds: `share` is the part of the rounds' outputs that the product needs.  At a
+// full chip a tile's outputs per time stand as 0.85, 0.87, 0.95 and 1 for FN of 2 to 5 (0.70 for FN = 2 in rows of 64
+// bytes).  Against the other kernels the line lies at 0.6 of a full chip of the widest tiles: 2048 x 4800 x 1600
+// (0.68) 44 us where they take 50, 4096 x 3072 x 768 (0.87) 31 and 39.  Short products are left to them: with k
 // under 768 the ends of a tile take longer than its products.
 static int large_width(int m, int n, int k) {
-  static const float rate[] = {0.f, 0.f, 0.70f, 0.87f, 0.95f, 1.f};
+  const float rate[] = {0.f, 0.f, k % 64 == 0 ? 0.85f : 0.70f, 0.87f, 0.95f, 1.f};
   if (m < 1024 || n < 256 || k < 768) return 0;
   const int units = ps_compute_units();
-  const int64_t tiles_m = (m + GL_BM - 1) / GL_BM;
+  const int64_t tiles_m = (m + 255) / 256;
   int best = 0;
   float best_value = 0.6f;
   for (int width = 2; width <= 5; ++width) {
-    const int bn = 32 * width * GL_WAVES_N;
+    const int bn = tile_columns(width);
     const int64_t tiles = tiles_m * ((n + bn - 1) / bn);
     const int64_t rounds = (tiles + units - 1) / units;
-    const float share = (float)m * (float)n / ((float)(rounds * units) * GL_BM * bn);
+    const float share = (float)m * (float)n / ((float)(rounds * units) * 256 * bn);
     if (share * rate[width] > best_value) {
       best_value = share * rate[width];
       best = width;
     }
   }
-  return best;
+  return best == 2 && k % 64 == 0 ? 22 : best;
+}
+
+static int shape_for(int m, int n, int k, int epilogue) {
+  const int medium = medium_shape(m, n, k, epilogue);
+  return medium != 0 ? medium : large_width(m, n, k);
 }
 
 // (k a multiple of 32 for whole stages; a tile's rows lie within 32-bit offsets)
@@ -250,21 +298,24 @@ static bool large_takes(const void* a, const void* w, int m, int n, int k, int l
          (reinterpret_cast<uintptr_t>(a) & 15u) == 0 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
 }
 
-bool ps_gemm_nt_bf16_large_supported(const void* a, const void* w, int m, int n, int k, int lda) {
-  return large_takes(a, w, m, n, k, lda) && large_width(m, n, k) != 0;
+bool ps_gemm_nt_bf16_large_supported(const void* a, const void* w, int m, int n, int k, int lda, int epilogue) {
+  return large_takes(a, w, m, n, k, lda) && shape_for(m, n, k, epilogue) != 0;
 }
 
-template <int FN, int RING, typename TOut>
+// `most_rows`: rows of tiles to a panel.
+template <int FM, int FN, int ROW, int RING, typename TOut>
 static int launch_large(const void* a, const void* w, const float* bias, void* c, int m, int n, int k, int lda,
-                        int ldc, int epilogue, const KvScatter& scatter, hipStream_t s) {
-  constexpr int BN = 32 * FN * GL_WAVES_N;
-  const int tiles_m = (m + GL_BM - 1) / GL_BM, tiles_n = (n + BN - 1) / BN;
-  const int panel = tiles_m < 8 ? tiles_m : 8;
+                        int ldc, int epilogue, int most_rows, const KvScatter& scatter, hipStream_t s) {
+  constexpr int BM = 32 * FM * GL_WAVES_M, BN = 32 * FN * GL_WAVES_N;
+  PS_REQUIRE(k % (ROW / 2) == 0 && k / (ROW / 2) >= RING, "ps_linear: k of %d is not whole stages of these tiles", k);
+  const int tiles_m = (m + BM - 1) / BM, tiles_n = (n + BN - 1) / BN;
+  const int panel = tiles_m < most_rows ? tiles_m : most_rows;
   PS_REQUIRE((int64_t)tiles_m * tiles_n < ((int64_t)1 << 31), "ps_linear: too many tiles");
   dim3 grid(tiles_m * tiles_n);
-#define PS_LAUNCH_GL(EPI)                                                                                      \
-  hipLaunchKernelGGL((gemm_nt_bf16_large_kernel<FN, RING, TOut, EPI>), grid, dim3(512), 0, s, (const bf16_t*)a, \
-                     (const bf16_t*)w, bias, (TOut*)c, m, n, k, lda, ldc, tiles_m, tiles_n, panel, scatter)
+#define PS_LAUNCH_GL(EPI)                                                                                       \
+  hipLaunchKernelGGL((gemm_nt_bf16_large_kernel<FM, FN, ROW, RING, TOut, EPI>), grid, dim3(512), 0, s,          \
+                     (const bf16_t*)a, (const bf16_t*)w, bias, (TOut*)c, m, n, k, lda, ldc, tiles_m, tiles_n,   \
+                     panel, scatter)
   switch (epilogue) {
     case PS_EPI_NONE: PS_LAUNCH_GL(PS_EPI_NONE); break;
     case PS_EPI_GELU_TANH: PS_LAUNCH_GL(PS_EPI_GELU_TANH); break;
@@ -278,19 +329,27 @@ static int launch_large(const void* a, const void* w, const float* bias, void* c
   return 0;
 }
 
-// width: FN, 0: by the rule.  Stages as many as LDS holds (160 KB).
+// shape: a tile's number, 0: by the rule.  Stages as many as LDS holds (160 KB); of 128 x 64 and 128 x 128 four, which
+// measured no slower than five or six.
 int ps_gemm_nt_bf16_large(const void* a, const void* w, const float* bias, void* c, int m, int n, int k, int lda,
-                          int ldc, int c_dtype, int epilogue, const KvScatter& scatter, int width, hipStream_t s) {
-  if (width == 0) width = large_width(m, n, k);
-#define PS_LARGE(FN, RING)                                                                                      \
-  (c_dtype == PS_F32 ? launch_large<FN, RING, float>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s)    \
-                     : launch_large<FN, RING, bf16_t>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s))
-  if (width == 2) return PS_LARGE(2, 6);
-  if (width == 3) return PS_LARGE(3, 5);
-  if (width == 4) return PS_LARGE(4, 4);
-  if (width == 5) return PS_LARGE(5, 4);
+                          int ldc, int c_dtype, int epilogue, const KvScatter& scatter, int shape, hipStream_t s) {
+  if (shape == 0) shape = shape_for(m, n, k, epilogue);
+#define PS_LARGE(FM, FN, ROW, RING, PANEL)                                                                          \
+  (c_dtype == PS_F32                                                                                                \
+       ? launch_large<FM, FN, ROW, RING, float>(a, w, bias, c, m, n, k, lda, ldc, epilogue, PANEL, scatter, s)      \
+       : launch_large<FM, FN, ROW, RING, bf16_t>(a, w, bias, c, m, n, k, lda, ldc, epilogue, PANEL, scatter, s))
+  switch (shape) {
+    case 11: return PS_LARGE(1, 1, 128, 4, 4);
+    case 12: return PS_LARGE(1, 2, 128, 4, 4);
+    case 13: return PS_LARGE(1, 3, 128, 4, 4);
+    case 22: return PS_LARGE(2, 2, 128, 3, 4);
+    case 2: return PS_LARGE(2, 2, 64, 6, 8);
+    case 3: return PS_LARGE(2, 3, 64, 5, 8);
+    case 4: return PS_LARGE(2, 4, 64, 4, 8);
+    case 5: return PS_LARGE(2, 5, 64, 4, 8);
+  }
 #undef PS_LARGE
-  ps_set_error("ps_linear: the large product has tiles of 2 to 5 fragments, not %d", width);
+  ps_set_error("ps_linear: the large product has no tiles of number %d", shape);
   return 1;
 }
 

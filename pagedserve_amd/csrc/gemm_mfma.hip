@@ -437,7 +437,7 @@ int ps_gemm_nt_bf16_wide(const void* a, const void* w_packed, const float* bias,
 int ps_gemm_nt_bf16_tiled(const void* a, const void* w, const float* bias, void* c, int m, int n,
                           int k, int lda, int ldc, int c_dtype, int epilogue,
                           const KvScatter& scatter, hipStream_t s);
-bool ps_gemm_nt_bf16_large_supported(const void* a, const void* w, int m, int n, int k, int lda);
+bool ps_gemm_nt_bf16_large_supported(const void* a, const void* w, int m, int n, int k, int lda, int epilogue);
 int ps_gemm_nt_bf16_large(const void* a, const void* w, const float* bias, void* c, int m, int n, int k, int lda,
                           int ldc, int c_dtype, int epilogue, const KvScatter& scatter, int width, hipStream_t s);
 
@@ -646,7 +646,7 @@ int ps_gemm_nt_mfma(const void* a, const void* w, const float* bias, void* c, in
                  m, n, k);
     return 1;
   }
-  if (dtype == PS_BF16 && ps_gemm_nt_bf16_large_supported(a, w, m, n, k, lda))
+  if (dtype == PS_BF16 && ps_gemm_nt_bf16_large_supported(a, w, m, n, k, lda, epilogue))
     return ps_gemm_nt_bf16_large(a, w, bias, c, m, n, k, lda, ldc, c_dtype, epilogue, scatter, 0, s);
   if (dtype == PS_BF16 && ps_gemm_nt_bf16_wide_supported(a, wp, m, n, k, lda))
     return ps_gemm_nt_bf16_wide(a, wp, bias, c, m, n, k, lda, ldc, c_dtype, epilogue, scatter, 0, s);

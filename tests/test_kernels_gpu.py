@@ -1347,6 +1347,67 @@ def test_gemm_large_tile_shapes(m, n, k, width, epilogue):
                   0 if out.dtype == torch.float32 else 1, kernels.EPILOGUES[epilogue], width, None) != 0
 
 
+@pytest.mark.parametrize("m,n,k", [(256, 640, 256), (300, 1000, 320), (1, 1, 256), (129, 65, 384), (700, 1601, 448), (513, 321, 1600)])
+@pytest.mark.parametrize("tile", [11, 12, 13, 22])
+@pytest.mark.parametrize("epilogue", ["none", "gelu_tanh", "residual"])
+def test_gemm_large_tiles_in_rows_of_whole_lines(m, n, k, tile, epilogue):
+    """The tiles of 128 x 64 to 256 x 128, whose stages are 64 values of k: as few stages as the ring holds and every
+    remainder at its end, rows and columns that end inside a tile and a wave's part of it, panels that are not full,
+    rows that do not allow 16-byte stores."""
+    import ctypes
+
+    from pagedserve_amd.ops import kernels, library
+
+    lib = library.load_library()
+    fn = lib.ps_gemm_nt_large
+    fn.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 8 + [ctypes.c_void_p]
+    a = _rand((m, k + 16), torch.bfloat16, 350, 1.0)[:, :k]
+    w = _rand((n, k), torch.bfloat16, 351, 1.0 / math.sqrt(k))
+    bias = _rand((n,), torch.float32, 352)
+    product = a.double() @ w.double().t() + bias.double()
+    if epilogue == "residual":
+        out = _rand((m, n), torch.float32, 353)
+        expected = out.double() + product
+    else:
+        out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+        expected = F.gelu(product, approximate="tanh") if epilogue == "gelu_tanh" else product
+    status = fn(a.data_ptr(), w.data_ptr(), bias.data_ptr(), out.data_ptr(), m, n, k, a.stride(0), out.stride(0),
+                0 if out.dtype == torch.float32 else 1, kernels.EPILOGUES[epilogue], tile,
+                torch.cuda.current_stream().cuda_stream)
+    assert status == 0, lib.ps_last_error().decode()
+    # (sums of k products of about 1 / sqrt(k) in 32 bits; a bfloat16 result is half a unit of its last place off, 2^-9)
+    atol, rtol = (1e-4, 1e-5) if epilogue == "residual" else (1e-4, 4e-3)
+    torch.testing.assert_close(out.double(), expected, atol=atol, rtol=rtol)
+    # half a stage of k is refused
+    assert fn(a.data_ptr(), w.data_ptr(), bias.data_ptr(), out.data_ptr(), m, n, k - 32, a.stride(0), out.stride(0),
+              0 if out.dtype == torch.float32 else 1, kernels.EPILOGUES[epilogue], tile, None) != 0
+
+
+@pytest.mark.parametrize("m", [261, 545, 1030, 2050])
+def test_linear_of_hundreds_of_rows_with_scatter(m):
+    """Through ``kernels.linear``: rows and columns that tiles of 128 x 64, 128 x 128, 128 x 192 and 256 x 128 cover in one
+    round, with the key/value scatter behind the product, against float64 and a scatter of its own."""
+    from pagedserve_amd.ops import kernels
+
+    heads, kv_heads, head_dim, page_size, k = 32, 16, 64, 16, 832
+    q_cols, kv_cols = heads * head_dim, kv_heads * head_dim
+    n = q_cols + 2 * kv_cols
+    k_pool, v_pool, tables = _paged_fixture(torch.bfloat16, [m + 40, 60], kv_heads, head_dim, page_size, 360)
+    tok_item = torch.tensor([1] * 50 + [0] * (m - 50), dtype=torch.int32, device="cuda")
+    tok_pos = torch.tensor(list(range(10, 60)) + list(range(90, m + 40)), dtype=torch.int32, device="cuda")
+    x = _rand((m, k), torch.bfloat16, 361)
+    w = _rand((n, k), torch.bfloat16, 362, 1.0 / math.sqrt(k))
+    bias = _rand((n,), torch.float32, 363)
+    out = torch.empty((m, n), dtype=torch.bfloat16, device="cuda")
+    pools = k_pool.clone(), v_pool.clone()
+    kernels.linear(x, w, bias, out, packed=kernels.pack_decode_weight(w),
+                   scatter=(k_pool, v_pool, tok_item, tok_pos, tables, q_cols, kv_cols))
+    torch.testing.assert_close(out.double(), x.double() @ w.double().t() + bias.double(), atol=1e-4, rtol=4e-3)
+    kernels.kv_write(out[:, q_cols:q_cols + kv_cols], out[:, q_cols + kv_cols:], *pools, tok_item, tok_pos, tables)
+    assert torch.equal(k_pool.view(torch.int16), pools[0].view(torch.int16))
+    assert torch.equal(v_pool.view(torch.int16), pools[1].view(torch.int16))
+
+
 def test_linear_takes_the_large_product_for_thousands_of_rows():
     """Through ``kernels.linear``: rows and columns that fill the chip with tiles of 256 x 192, with the key/value
     scatter behind the product, against float64 and a scatter of its own."""
