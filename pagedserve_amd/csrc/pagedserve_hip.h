@@ -434,6 +434,10 @@ int ps_stream_step(float* h, const float* y, float factor, const float* column_s
 int ps_silu_gate(const float* gu, int64_t ld, void* out, int64_t out_ld, int tokens, int inner,
                  int activation, float limit, float slope, float shift, const float* row_scale,
                  int dtype, void* stream);
+// The same result straight from the rows [gate | up] of a bfloat16 matrix in its packed copy and up to 64 rows of a:
+// c[t * ldc + i] = unit((a W^T)[t, i], (a W^T)[t, inner + i]) (* row_scale[t]).  inner in whole tiles of 16, k of 64.
+int ps_linear_gated(const void* a, const void* w_packed, void* c, int m, int inner, int k, int lda, int64_t ldc,
+                    int activation, float limit, float slope, float shift, const float* row_scale, void* stream);
 // p[t * ld + first + c] = silu(...) in place for c < count.
 int ps_silu_columns(float* p, int64_t ld, int first, int count, int tokens, void* stream);
 // y += share * (rms_norm(a) * wa + rms_norm(b) * wb) over rows of width floats; a and b are cleared.

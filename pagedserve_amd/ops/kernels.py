@@ -81,6 +81,8 @@ _SIGNATURES = {
     "ps_silu_columns": [c_void_p, c_int64, c_int, c_int, c_int, c_void_p],
     "ps_silu_gate": [c_void_p, c_int64, c_void_p, c_int64, c_int, c_int, c_int, c_float, c_float,
                      c_float, c_void_p, c_int, c_void_p],
+    "ps_linear_gated": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int64, c_int, c_float, c_float,
+                        c_float, c_void_p, c_void_p],
     "ps_pair_norm_mix": [c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_float, c_void_p, c_int,
                          c_int, c_void_p],
     "ps_moe_route": [c_void_p, c_int64, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float,
@@ -1866,6 +1868,39 @@ def silu_gate(gu, out, activation="silu", form=PLAIN_GATE, row_scale=None):
     _call("ps_silu_gate", gu.data_ptr(), _rows(gu, "gu"), out.data_ptr(), _rows(out, "out"), tokens,
           inner, GATE_ACTIVATIONS[activation], *_gate_form(form), _ptr(row_scale), dtype_code(out.dtype),
           _stream())
+
+
+# Up to so many rows the gate runs inside its product (csrc/gemm_skinny_gated.hip), up to the second number over a k of
+# at most 1,024 and fewer than 16,384 columns.  Every block of 16 rows reads the weights anew: 64 x (2 x 4096) x 1024
+# 9.9 us, the two launches 14.6, but 48 x (2 x 6400) x 1600, where the product is the tiled one, 20.7 and 15.2.
+GATED_PRODUCT_ROWS = (16, 64)
+
+
+def linear_gated(x, w, out, packed, activation="silu", form=PLAIN_GATE, row_scale=None) -> bool:
+    """``out = act(x W_gate^T) * (x W_up^T)`` in one launch, for ``w`` the rows ``[gate | up]`` and ``packed`` its
+    ``pack_decode_weight``; the options are those of ``silu_gate``, whose result after ``linear`` this is, bit for
+    bit.  False, and nothing done, for what the kernel does not take: more than ``GATED_PRODUCT_ROWS`` rows, a pending
+    norm, other types than bfloat16, columns not in whole tiles of 16, rows not aligned to 16 bytes, operands that do
+    not fit each other (``linear`` says what is wrong with them)."""
+    if (packed is None or isinstance(x, PendingNorm) or activation not in GATE_ACTIVATIONS
+            or x.ndim != 2 or out.ndim != 2):
+        return False
+    rows, k = x.shape
+    inner = out.shape[1]
+    most = GATED_PRODUCT_ROWS[1 if k <= 1024 and 2 * inner < 16384 else 0]
+    if not (0 < rows <= most and w.shape == (2 * inner, k) and inner % 16 == 0 and out.shape[0] == rows
+            and x.dtype == w.dtype == out.dtype == torch.bfloat16 and packed.numel() == w.numel()
+            and packed.is_contiguous() and x.is_cuda and out.is_cuda and packed.is_cuda
+            and x.stride(1) == 1 and out.stride(1) == 1):
+        return False
+    lda, ldc = _rows(x, "x"), _rows(out, "out")
+    if lda < k or lda % 8 != 0 or ldc < inner or x.data_ptr() % 16 != 0 or packed.data_ptr() % 16 != 0:
+        return False
+    if row_scale is not None:
+        _float_vector(row_scale, "row_scale", rows)
+    _call("ps_linear_gated", x.data_ptr(), packed.data_ptr(), out.data_ptr(), rows, inner, k, lda, ldc,
+          GATE_ACTIVATIONS[activation], *_gate_form(form), _ptr(row_scale), _stream())
+    return True
 
 
 def silu_columns(rows, first, count):

@@ -106,12 +106,15 @@ class GatedFeedForward(FeedForward):
 
     def forward(self, x, residual, ctx, row_scale=None):
         tokens = ctx.tokens
-        whole, both, ridden = ctx.workspace.column_views("ffn_gate_up", 2 * self.inner + self.ride, torch.float32,
-                                                         tokens, (2 * self.inner, self.ride))
-        kernels.linear(x, self.gate_up_weight, None, whole, packed=self.gate_up_packed,
-                       memo=site_memo(self._memo_up, ctx.workspace), shared=ctx.shared_calls)
         hidden = ctx.workspace.first_rows("ffn", self.inner, self.dtype, tokens)
-        kernels.silu_gate(both, hidden, self.activation, form=self.form, row_scale=row_scale)
+        # (few rows: the gate in the product's epilogue)
+        if self.ride or not kernels.linear_gated(x, self.gate_up_weight, hidden, self.gate_up_packed, self.activation,
+                                                 form=self.form, row_scale=row_scale):
+            whole, both, ridden = ctx.workspace.column_views("ffn_gate_up", 2 * self.inner + self.ride, torch.float32,
+                                                             tokens, (2 * self.inner, self.ride))
+            kernels.linear(x, self.gate_up_weight, None, whole, packed=self.gate_up_packed,
+                           memo=site_memo(self._memo_up, ctx.workspace), shared=ctx.shared_calls)
+            kernels.silu_gate(both, hidden, self.activation, form=self.form, row_scale=row_scale)
         kernels.linear(hidden, self.down_weight, None, residual, epilogue="residual",
                        packed=self.down_packed, memo=site_memo(self._memo_down, ctx.workspace),
                        shared=ctx.shared_calls)

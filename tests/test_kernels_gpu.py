@@ -1347,6 +1347,37 @@ def test_gemm_large_tile_shapes(m, n, k, width, epilogue):
                   0 if out.dtype == torch.float32 else 1, kernels.EPILOGUES[epilogue], width, None) != 0
 
 
+@pytest.mark.parametrize("m,inner,k", [(1, 16, 64), (8, 3072, 768), (3, 48, 832), (16, 320, 1024), (5, 80, 1600), (15, 16, 192), (40, 48, 832),
+                                       (64, 320, 1024)])
+@pytest.mark.parametrize("activation,form", [("silu", None), ("silu", (0.7, 1.702, 1.0)), ("gelu_tanh", None), ("relu", None)])
+def test_gate_in_the_product_of_few_rows(m, inner, k, activation, form):
+    """The bits of the product and the gate as two launches: one step of k and counts that the waves do not share
+    evenly, columns and rows down to one tile and one row, rows apart from one another; and what is left to them."""
+    from pagedserve_amd.ops import kernels
+
+    x = _rand((m, k + 8), torch.bfloat16, 370, 1.0)[:, :k]
+    w = _rand((2 * inner, k), torch.bfloat16, 371, 2.0 / math.sqrt(k))
+    scale = _rand((m,), torch.float32, 372) if form else None
+    form = form or kernels.PLAIN_GATE
+    packed = kernels.pack_decode_weight(w)
+    both = torch.empty((m, 2 * inner), dtype=torch.float32, device="cuda")
+    expected = torch.empty((m, inner), dtype=torch.bfloat16, device="cuda")
+    kernels.linear(x, w, None, both, packed=packed)
+    kernels.silu_gate(both, expected, activation, form=form, row_scale=scale)
+    whole = torch.full((m + 1, inner + 8), -7.0, dtype=torch.bfloat16, device="cuda")
+    assert kernels.linear_gated(x, w, whole[:m, :inner], packed, activation, form=form, row_scale=scale)
+    assert torch.equal(whole[:m, :inner].view(torch.int16), expected.view(torch.int16))
+    assert bool((whole[m] == -7.0).all()) and bool((whole[:, inner:] == -7.0).all())
+    out = torch.full((m, inner), -7.0, dtype=torch.bfloat16, device="cuda")
+    many = torch.cat([x] * (kernels.GATED_PRODUCT_ROWS[k <= 1024] // m + 1))
+    assert not kernels.linear_gated(many, w, out.new_empty((many.shape[0], inner)), packed, activation)
+    assert not kernels.linear_gated(x, w, out, None, activation)
+    assert not kernels.linear_gated(_rand((m, k + 1), torch.bfloat16, 373, 1.0)[:, 1:], w, out, packed, activation)
+    assert not kernels.linear_gated(x, w, out[:, 1:], packed, activation)
+    assert not kernels.linear_gated(x.float(), w, out, packed, activation)
+    assert bool((out == -7.0).all())
+
+
 @pytest.mark.parametrize("m,n,k", [(256, 640, 256), (300, 1000, 320), (1, 1, 256), (129, 65, 384), (700, 1601, 448), (513, 321, 1600)])
 @pytest.mark.parametrize("tile", [11, 12, 13, 22])
 @pytest.mark.parametrize("epilogue", ["none", "gelu_tanh", "residual"])
