@@ -366,7 +366,8 @@ static int launch_variant(const void* a, const void* w, const float* bias, void*
 
 // Tile shapes by the number of blocks they give against the chip's compute units: a product
 // of this size is over in a few microseconds, so filling them counts for more than the reuse
-// inside a large tile.
+// inside a large tile.  (More than 128 rows with a k of 768 and more come here where 64 x 64 tiles or two rounds of
+// larger ones suit them better than gemm_large_bf16.hip, which takes many of the shapes that drew the lines below.)
 template <typename TOut>
 static int launch_tiled_bf16(const void* a, const void* w, const float* bias, void* c, int m,
                              int n, int k, int lda, int ldc, int epilogue,
