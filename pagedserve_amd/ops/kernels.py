@@ -1876,6 +1876,15 @@ def silu_gate(gu, out, activation="silu", form=PLAIN_GATE, row_scale=None):
 GATED_PRODUCT_ROWS = (16, 64)
 
 
+def gated_product_rows(w, packed) -> int:
+    """Up to how many rows ``linear_gated`` takes for these matrices ``[gate | up]`` (0: none).  A part asks once, when
+    weights are bound: the checks of a call that is turned away cost a step that is not replayed 3 us a layer."""
+    n, k = w.shape
+    if packed is None or n % 32 != 0 or w.dtype != torch.bfloat16:
+        return 0
+    return GATED_PRODUCT_ROWS[1 if k <= 1024 and n < 16384 else 0]
+
+
 def linear_gated(x, w, out, packed, activation="silu", form=PLAIN_GATE, row_scale=None) -> bool:
     """``out = act(x W_gate^T) * (x W_up^T)`` in one launch, for ``w`` the rows ``[gate | up]`` and ``packed`` its
     ``pack_decode_weight``; the options are those of ``silu_gate``, whose result after ``linear`` this is, bit for
@@ -1887,9 +1896,8 @@ def linear_gated(x, w, out, packed, activation="silu", form=PLAIN_GATE, row_scal
         return False
     rows, k = x.shape
     inner = out.shape[1]
-    most = GATED_PRODUCT_ROWS[1 if k <= 1024 and 2 * inner < 16384 else 0]
-    if not (0 < rows <= most and w.shape == (2 * inner, k) and inner % 16 == 0 and out.shape[0] == rows
-            and x.dtype == w.dtype == out.dtype == torch.bfloat16 and packed.numel() == w.numel()
+    if not (0 < rows <= gated_product_rows(w, packed) and w.shape == (2 * inner, k) and out.shape[0] == rows
+            and x.dtype == out.dtype == torch.bfloat16 and packed.numel() == w.numel()
             and packed.is_contiguous() and x.is_cuda and out.is_cuda and packed.is_cuda
             and x.stride(1) == 1 and out.stride(1) == 1):
         return False

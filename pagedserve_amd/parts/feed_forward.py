@@ -101,6 +101,8 @@ class GatedFeedForward(FeedForward):
         self.down_weight = tensors["down.weight"]
         self.gate_up_packed = kernels.pack_decode_weight(self.gate_up_weight)
         self.down_packed = kernels.pack_decode_weight(self.down_weight)
+        # (rows that ride along are float columns of the product, which the fused gate does not leave)
+        self.fused_rows = 0 if self.ride else kernels.gated_product_rows(self.gate_up_weight, self.gate_up_packed)
         self._memo_up.clear()
         self._memo_down.clear()
 
@@ -108,8 +110,8 @@ class GatedFeedForward(FeedForward):
         tokens = ctx.tokens
         hidden = ctx.workspace.first_rows("ffn", self.inner, self.dtype, tokens)
         # (few rows: the gate in the product's epilogue)
-        if self.ride or not kernels.linear_gated(x, self.gate_up_weight, hidden, self.gate_up_packed, self.activation,
-                                                 form=self.form, row_scale=row_scale):
+        if tokens > self.fused_rows or not kernels.linear_gated(x, self.gate_up_weight, hidden, self.gate_up_packed,
+                                                                self.activation, form=self.form, row_scale=row_scale):
             whole, both, ridden = ctx.workspace.column_views("ffn_gate_up", 2 * self.inner + self.ride, torch.float32,
                                                              tokens, (2 * self.inner, self.ride))
             kernels.linear(x, self.gate_up_weight, None, whole, packed=self.gate_up_packed,
