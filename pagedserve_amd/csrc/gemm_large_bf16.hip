@@ -246,7 +246,8 @@ static int tile_columns(int shape) { return 32 * GL_WAVES_N * (shape % 10); }
 // there and 20.5 here, on 144 330 x 3072 x 768 is level, on 180 544 x 2304 x 768 takes 8.3 and 7.9.  A residual product
 // reads the rows that it adds to behind its last product, which two blocks hide from each other: on 192 units 2048 x 768 x
 // 3072 takes 21.8 there and 22.7 here.  With k under 768 the ends of a tile take longer than its products (600 x 4096 x 512
-// 8.9 there, 9.3 here).
+// 8.9 there, 9.3 here).  Nor do larger tiles pay that lie half behind the product's ends: 259 x 6144 x 768 is 0.38 of what
+// 256 tiles of 128 x 128 hold and takes 12.1 us in them, 11.0 in 64 x 64 (544 x 4096 x 1024, 0.53, 13.6 and 14.9).
 static int medium_shape(int m, int n, int k, int epilogue) {
   if (m <= 128 || k < 768 || k % 64 != 0) return 0;
   const int units = ps_compute_units();
@@ -256,6 +257,7 @@ static int medium_shape(int m, int n, int k, int epilogue) {
     const int rows = tile_rows(shape), columns = tile_columns(shape);
     const int64_t tiles = (int64_t)((m + rows - 1) / rows) * ((n + columns - 1) / columns);
     if (tiles > units) continue;
+    if (shape != 11 && 100 * (int64_t)m * n < 45 * (int64_t)units * rows * columns) return 0;
     return shape == 11 && 8 * tiles <= (epilogue == PS_EPI_RESIDUAL ? 6 : 5) * units ? 0 : shape;
   }
   return 0;
