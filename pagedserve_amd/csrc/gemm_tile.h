@@ -38,14 +38,18 @@ __device__ inline void mma_step(float, const u32x4_t& a, const u32x4_t& w, f32x1
 typedef const __attribute__((address_space(1))) void* global_ptr_t;
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
-// gelu_tanh(u) = u * sigmoid(2 z), z = sqrt(2/pi) (u + 0.044715 u^3), as u / (1 + 2^(u (c0 + c1 u^2))) with
-// the hardware exponential and reciprocal: its error (about 1e-6 relative) is far below the rounding of a
-// bfloat16 result, which is the only place where it is used.  Two of its eight instructions take four
-// slots each; with the exactly rounded reciprocal, three times as many instructions, a tile of 256 x 256
-// spent 17 us here, most of it in this function.
+// gelu_tanh(u) = u * sigmoid(2 z), z = sqrt(2/pi) (u + 0.044715 u^3), with the hardware
+// exponential: its error (about 1e-6 relative) is far below the rounding of a bfloat16 result, which is the
+// only place where it is used.  The reciprocal is the hardware's and one step of Newton's method, four instructions
+// where a division takes ten (a tile of 256 x 256 spent 17 us in this function with that); the two agree for every d up to
+// 2^126, beyond it this one is 0 where the division's is subnormal.  Where d is infinite, the step is no number
+// without the maximum, with it the reciprocal stays 0.
 __device__ inline float gelu_tanh_fast(float u) {
-  const float exponent = u * fmaf(u * u, -0.10294324f, -2.3022082f);   // -2 z / ln 2
-  return u * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(exponent));
+  const float z2 = 1.5957691216057308f * (u + 0.044715f * u * u * u);
+  const float d = 1.0f + __expf(-z2);
+  const float r = __builtin_amdgcn_rcpf(d);
+  const float e = fmaxf(fmaf(-d, r, 1.0f), -1.0f);
+  return u * fmaf(r, e, r);
 }
 
 template <int EPI, typename TOut>

@@ -1414,6 +1414,46 @@ def test_gemm_large_tiles_in_rows_of_whole_lines(m, n, k, tile, epilogue):
               0 if out.dtype == torch.float32 else 1, kernels.EPILOGUES[epilogue], tile, None) != 0
 
 
+def _gelu_tanh_bits(u):
+    """``u / (1 + exp(-2 z))``, ``2 z = 2 sqrt(2 / pi) (u + 0.044715 u^3)``, in float as the tiled products round it:
+    every product and the division once, the cube's last product and sum together, ``exp`` as a power of two.  (A product
+    of two floats is exact in float64.)"""
+    def f(value):
+        return value.to(torch.float32).double()
+
+    u = u.double()
+    inner = f(f(f(u * f(torch.tensor(0.044715, device=u.device))) * u) * u + u)
+    z2 = f(inner * f(torch.tensor(1.5957691216057308, device=u.device)))
+    power = torch.exp2(f(-z2 * f(torch.tensor(1.4426950408889634, device=u.device))).float()).double()
+    return f(u * f(1.0 / f(1.0 + power))).float().to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("m,k", [(129, 64), (300, 256), (2048, 768), (2050, 1024)])
+def test_gelu_of_the_tiled_products_keeps_its_bits(m, k):
+    """GELU behind a bfloat16 product of many rows rounds as it always has, in each of the kernels: values whose result
+    lies within a few float roundings of the middle between two bfloat16 numbers, and the ends of the range."""
+    from pagedserve_amd.ops import kernels
+
+    g = torch.Generator(device="cuda").manual_seed(380)
+    u = torch.rand(1 << 24, generator=g, device="cuda") * 12 - 6
+    exact = F.gelu(u.double(), approximate="tanh")
+    spacing = torch.exp2(torch.floor(torch.log2(exact.abs())) - 7)
+    off = ((exact / spacing).abs() % 1.0 - 0.5).abs() * spacing / exact.abs()
+    u = u[off < 2e-7][:4000]
+    assert u.numel() > 1000
+    ends = torch.tensor([0.0, -0.0, 1e-30, -1e-30, 9.0, -9.0, 30.0, -30.0, 1e4, -1e4, 1e19, -1e19, 3e38, -3e38, math.inf,
+                         math.nan], device="cuda")
+    bias = torch.cat([u, ends, torch.zeros(4096 - u.numel() - ends.numel(), device="cuda")])
+    x = torch.zeros((m, k), dtype=torch.bfloat16, device="cuda")
+    w = _rand((4096, k), torch.bfloat16, 381, 1.0)
+    out = torch.empty((m, 4096), dtype=torch.bfloat16, device="cuda")
+    kernels.linear(x, w, bias, out, epilogue="gelu_tanh", packed=kernels.pack_decode_weight(w))
+    expected = _gelu_tanh_bits(bias)
+    number = ~torch.isnan(expected)
+    assert torch.equal(torch.isnan(out), ~number.expand(m, -1))
+    assert torch.equal(out[:, number], expected[number].expand(m, -1))
+
+
 @pytest.mark.parametrize("m", [261, 545, 1030, 2050])
 def test_linear_of_hundreds_of_rows_with_scatter(m):
     """Through ``kernels.linear``: rows and columns that tiles of 128 x 64, 128 x 128, 128 x 192 and 256 x 128 cover in one
