@@ -7,8 +7,8 @@
 // the exchange between the waves; then the rows of the context, the weights, the exchange, the add.  The
 // second chain mostly repeats waits of the first.  Here block (t, h, p) computes head h of token t over all
 // its keys (attention_decode_block.h) and multiplies it with the piece of W that belongs to head h
-// and to the p-th part of the columns, out of the packed copy of W (pagedserve_hip.h).  The piece is asked for right
-// behind the keys and travels beside them.  Blocks that differ in p repeat the attention: while the keys are few that costs
+// and to the p-th part of the columns, out of the packed copy of W (pagedserve_hip.h).  The piece is asked for
+// beside the keys and travels with them.  Blocks that differ in p repeat the attention: while the keys are few that costs
 // less than leaving compute units idle, since a unit takes in some 55 KB/us and what it has to take in (its
 // keys and its piece of W) is what the launch waits for beside the chain.  The sum over heads is made
 // by float atomic adds into the residual rows, in an order that differs from run to run within float
@@ -30,8 +30,11 @@
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 
-// STEPS: head_dim / 64; AHEAD: tiles of 16 columns per wave whose weights are asked for before the
-// attention (further ones follow behind it).
+// STEPS: head_dim / 64; AHEAD: tiles of 16 columns per wave whose weights are asked for beside the keys
+// (further ones follow behind the attention): heads of 64 right behind the first keys and values, heads of 128 in front
+// of the attention.  Those hold twice the weights, which the first turn over the keys has no registers left for (16
+// waves spill 16 of them; 8 requests of 8 heads of 128 over 250 keys 9.5 us with the weights in front, 11.7 behind; one of 16
+// heads over 400 keys 10.6 and 12.1; heads of 64, 8 requests of 12 over 540 keys 9.5 and 9.2).
 template <int STEPS, int AD_WAVES, int AD_UNROLL, int AHEAD>
 __global__ __launch_bounds__(64 * AD_WAVES) void attention_decode_linear_kernel(
     const bf16_t* __restrict__ q, int64_t q_stride, const bf16_t* __restrict__ k_pool,
@@ -69,10 +72,18 @@ __global__ __launch_bounds__(64 * AD_WAVES) void attention_decode_linear_kernel(
     }
   };
 
-  attention_decode_block<bf16_t, 8 * STEPS, AD_WAVES, AD_UNROLL, false>(
-      lds, token, head, 0, q, q_stride, k_pool, v_pool, (bf16_t*)nullptr, 0, nullptr, nullptr, nullptr,
-      tok_pos, tables, table_width, heads, kv_heads, HEAD_DIM, page_size, page_shift, num_pages,
-      scale_log2, window, 1, extra, context, [&] { load_weights(0); });
+  auto attend = [&](auto ahead) {
+    attention_decode_block<bf16_t, 8 * STEPS, AD_WAVES, AD_UNROLL, false>(
+        lds, token, head, 0, q, q_stride, k_pool, v_pool, (bf16_t*)nullptr, 0, nullptr, nullptr, nullptr,
+        tok_pos, tables, table_width, heads, kv_heads, HEAD_DIM, page_size, page_shift, num_pages,
+        scale_log2, window, 1, extra, context, ahead);
+  };
+  if constexpr (STEPS == 1) {
+    attend([&] { load_weights(0); });
+  } else {
+    load_weights(0);
+    attend(NothingAhead());
+  }
   __syncthreads();
 
   // row operand: row 0 is the head's context, the other fifteen are zero; lane l holds row l % 16,
