@@ -140,7 +140,7 @@ __device__ inline void store_wave_tile(f32x16 (&acc)[WM][WN], float* region, int
     for (int i = 0; i < (PLAIN ? WM : 0); ++i)
 #pragma unroll
       for (int pass = 0; pass < PASSES; ++pass)
-        slots[i][pass] = kv_scatter_slot(scatter, pos[i][pass], item[i][pass]);
+        slots[i][pass] = kv_scatter_slot(scatter, pos[i][pass], &item[i][pass]);
   }
 
 #pragma unroll

@@ -69,15 +69,16 @@ struct NormPrologue {
 // column: kv_scatter_row gives the element offset of (page, slot) of a token, or -1;
 // kv_scatter_col gives the pool and the offset of (head, dim) inside a page, or null for a
 // query column.
-__device__ inline int64_t kv_scatter_slot(const KvScatter& s, int pos, int item) {
+// (the item by its address: where it lies in memory it is read behind the first check)
+__device__ inline int64_t kv_scatter_slot(const KvScatter& s, int pos, const int* item) {
   const int logical = s.page_shift >= 0 ? (pos >> s.page_shift) : pos / s.page_size;
   if (logical >= s.table_width) return -1;
-  const int page = s.tables[(int64_t)item * s.table_width + logical];
+  const int page = s.tables[(int64_t)*item * s.table_width + logical];
   if (page < 0 || page >= s.num_pages) return -1;
   return ((int64_t)page * s.kv_heads * s.page_size + (pos - logical * s.page_size)) * s.head_dim;
 }
 __device__ inline int64_t kv_scatter_row(const KvScatter& s, int row) {
-  return kv_scatter_slot(s, s.tok_pos[row], s.tok_item[row]);
+  return kv_scatter_slot(s, s.tok_pos[row], s.tok_item + row);
 }
 
 template <typename T>
