@@ -39,8 +39,9 @@
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float af_f32x4;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float af_f32x16;
 
-// DF: 32 head dimensions each; RAGGED: the head size is not 32 DF
-template <int DF, bool RAGGED>
+// DF: 32 head dimensions each; RAGGED: the head size is not 32 DF; PAIRS: one block takes the 64 queries of a tile
+// whose keys are at most 64
+template <int DF, bool RAGGED, bool PAIRS>
 __global__ __launch_bounds__(64 * AF_WAVES) void attention_tiled_f32_kernel(
     const float* __restrict__ q, int64_t q_stride, const float* __restrict__ k_pool,
     const float* __restrict__ v_pool, float* __restrict__ out, int64_t out_stride,
@@ -66,15 +67,23 @@ __global__ __launch_bounds__(64 * AF_WAVES) void attention_tiled_f32_kernel(
   const int kv_head = head / (heads / kv_heads);
 
   const int item = tile_item[tile_index];
-  const int q0 = tile_q0[tile_index] + part * AF_ROWS;
+  const int tile_q = tile_q0[tile_index];
   const int tok0 = cu_tokens[item];
   const int count = cu_tokens[item + 1] - tok0;
-  if (q0 >= count) return;                      // (the whole block)
   const int start = kv_lens[item] - count;      // position of the portion's first token
   const int* table = tables + (int64_t)item * table_width;
+  const int tile_last = tile_q + AF_TILE - 1 < count ? tile_q + AF_TILE - 1 : count - 1;
+  // two waves to 32 queries where the keys are no more than two turns: four would leave two of them without any
+  const bool paired =
+      PAIRS && start + tile_last + 1 - first_visible_key(start + tile_q, window) <= 2 * AF_ROWS;
+  const int turns = paired ? 2 : AF_WAVES;      // waves that share the keys of 32 queries
+  const int turn = paired ? wave & 1 : wave;    // which of them this one is
+  const int first_q = tile_q + part * AF_ROWS;  // of the block
+  if (first_q >= count || (paired && part != 0)) return;      // (the whole block)
+  const int q0 = paired ? first_q + (wave >> 1) * AF_ROWS : first_q;
   const int last_q = q0 + AF_ROWS - 1 < count ? q0 + AF_ROWS - 1 : count - 1;
-  const int key_end = start + last_q + 1;
   const int key_begin = first_visible_key(start + q0, window);
+  const int key_end = q0 < count ? start + last_q + 1 : key_begin;
 
   const int q_pos = q0 + column < count ? start + q0 + column : -1;
   const int q_first = q_pos < 0 ? 0 : first_visible_key(q_pos, window);
@@ -133,7 +142,7 @@ __global__ __launch_bounds__(64 * AF_WAVES) void attention_tiled_f32_kernel(
   };
 
   // (a sink is a score without key or value: it starts the denominator, in one lane half of one wave)
-  const bool starts = wave == 0 && extra.sink != nullptr;
+  const bool starts = turn == 0 && extra.sink != nullptr;
   float run_max = starts ? extra.sink[head] : -INFINITY;
   float run_sum = starts && half == 0 ? 1.f : 0.f;     // of the lane's own keys
   af_f32x16 acc[DF];
@@ -142,9 +151,9 @@ __global__ __launch_bounds__(64 * AF_WAVES) void attention_tiled_f32_kernel(
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[f][e] = 0.f;
 
-  int k0 = key_begin + wave * AF_ROWS;
+  int k0 = key_begin + turn * AF_ROWS;
   if (k0 < key_end) {
-    constexpr int TURN = AF_WAVES * AF_ROWS;
+    const int TURN = turns * AF_ROWS;
     int64_t row = row_of(k0, page_of(k0));
     load_keys(row);
     int next_page = page_of(k0 + TURN);
@@ -242,34 +251,40 @@ __global__ __launch_bounds__(64 * AF_WAVES) void attention_tiled_f32_kernel(
     s_sum[wave * AF_ROWS + column] = run_sum;
   }
   __syncthreads();
-  // eight threads to a query
-  const int row = tid >> 3;
-  if (q0 + row >= count) return;
+  // eight threads to a query, four where the block has 64 of them
+  const int shift = paired ? 2 : 3;
+  const int row = tid >> shift;
+  const int part_of_query = tid - (row << shift);
+  const int first = paired ? (row >> 5) * 2 * AF_ROWS + (row & 31) : row;   // the query in its first wave's results
+  if (first_q + row >= count) return;
   float total_max = -INFINITY;
 #pragma unroll
-  for (int w = 0; w < AF_WAVES; ++w) total_max = fmaxf(total_max, s_max[w * AF_ROWS + row]);
+  for (int w = 0; w < AF_WAVES; ++w)
+    if (w < turns) total_max = fmaxf(total_max, s_max[w * AF_ROWS + first]);
   float factor[AF_WAVES], total = 0.f;
 #pragma unroll
   for (int w = 0; w < AF_WAVES; ++w) {
-    const float wave_max = s_max[w * AF_ROWS + row];
+    if (w >= turns) continue;
+    const float wave_max = s_max[w * AF_ROWS + first];
     factor[w] = wave_max == -INFINITY ? 0.f : expf(wave_max - total_max);
-    total += s_sum[w * AF_ROWS + row] * factor[w];
+    total += s_sum[w * AF_ROWS + first] * factor[w];
   }
   if (extra.logistic != nullptr) {
 #pragma unroll
     for (int w = 0; w < AF_WAVES; ++w) factor[w] = 1.f;
     total = extra.logistic_norm;
   }
-  const float inverse = (total != 0.f ? 1.f / total : 0.f) * gate_factor(extra, tok0 + q0 + row, head);
-  float* to = out + (int64_t)(tok0 + q0 + row) * out_stride + (int64_t)head * head_dim;
+  const float inverse = (total != 0.f ? 1.f / total : 0.f) * gate_factor(extra, tok0 + first_q + row, head);
+  float* to = out + (int64_t)(tok0 + first_q + row) * out_stride + (int64_t)head * head_dim;
 #pragma unroll
-  for (int v = 0; v < DF; ++v) {
-    const int dim = 4 * (tid & 7) + 32 * v;
-    if (RAGGED && dim >= head_dim) continue;
+  for (int v = 0; v < 2 * DF; ++v) {
+    const int dim = 4 * part_of_query + ((4 * v) << shift);
+    if (dim >= head_dim) continue;
     float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
     for (int w = 0; w < AF_WAVES; ++w) {
-      const float4 value = *reinterpret_cast<const float4*>(s_out + (w * AF_ROWS + row) * STRIDE + dim);
+      if (w >= turns) continue;
+      const float4 value = *reinterpret_cast<const float4*>(s_out + (w * AF_ROWS + first) * STRIDE + dim);
       sum.x = fmaf(factor[w], value.x, sum.x);
       sum.y = fmaf(factor[w], value.y, sum.y);
       sum.z = fmaf(factor[w], value.z, sum.z);
@@ -313,22 +328,33 @@ extern "C" int ps_attention_tiled_f32(const void* q, int64_t q_stride, const voi
   if (blocks == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
   const AttnExtras extra = {sink, gate, gate_ld, softcap, logistic, logistic_norm};
+  // Short portions.  Of the two blocks of a tile of 33 to 64 keys one has a wave with keys, the other two; that the
+  // others are idle costs nothing while the blocks are on the chip at once, two to a unit with heads of 33 to 64.
+  // Beyond that one block takes both halves, two waves each (us; before these tiles, two blocks, one: 128 portions of
+  // 40 tokens at 12 heads of 64 49, 57 and 50, of 64 tokens 53, 61 and 53, 24 of 40 16.3, 16.5 and 13.5; but 8 of 40 8.9 and 9.4).
+  // Narrower heads fit three blocks into a unit and lose by it (128 of 64 tokens at 4 heads of 32 14.3 and 16.7), wider
+  // ones, one block to a unit, too (at 16 heads of 128 182 and 198; 192 before).
+  const bool pairs = head_dim > 32 && head_dim <= 64 && blocks > 2 * (int64_t)ps_compute_units();
 #define PS_LAUNCH_AF(DF)                                                                          \
   do {                                                                                            \
     if (head_dim == 32 * DF)                                                                      \
-      PS_LAUNCH_AF_FORM(DF, false);                                                               \
+      PS_LAUNCH_AF_FORM(DF, false, false);                                                        \
     else                                                                                          \
-      PS_LAUNCH_AF_FORM(DF, true);                                                                \
+      PS_LAUNCH_AF_FORM(DF, true, false);                                                         \
   } while (0)
-#define PS_LAUNCH_AF_FORM(DF, RAGGED)                                                             \
-  hipLaunchKernelGGL((attention_tiled_f32_kernel<DF, RAGGED>), dim3((unsigned)blocks),            \
+#define PS_LAUNCH_AF_FORM(DF, RAGGED, PAIRS)                                                      \
+  hipLaunchKernelGGL((attention_tiled_f32_kernel<DF, RAGGED, PAIRS>), dim3((unsigned)blocks),     \
                      dim3(64 * AF_WAVES), 0, s,                                                   \
                      (const float*)q, q_stride, (const float*)k_pool, (const float*)v_pool,       \
                      (float*)out, out_stride, tile_item, tile_q0, cu_tokens, kv_lens, tables,     \
                      table_width, heads, kv_heads, head_dim, page_size, num_pages, scale, window, extra)
   switch ((head_dim + 31) / 32) {
     case 1: PS_LAUNCH_AF(1); break;
-    case 2: PS_LAUNCH_AF(2); break;
+    case 2:
+      if (!pairs) PS_LAUNCH_AF(2);
+      else if (head_dim == 64) PS_LAUNCH_AF_FORM(2, false, true);
+      else PS_LAUNCH_AF_FORM(2, true, true);
+      break;
     case 3: PS_LAUNCH_AF(3); break;
     default: PS_LAUNCH_AF(4); break;
   }
