@@ -289,9 +289,44 @@ static int large_width(int m, int n, int k) {
   return best == 2 && k % 64 == 0 ? 22 : best;
 }
 
-static int shape_for(int m, int n, int k, int epilogue) {
+// Outputs that the unit with the most tiles makes where the other kernels take the product (gemm_mfma.hip asks this one
+// first): the wide one's blocks of 64 x 256, or tiles of 128 x 64 or 64 x 64.
+static int64_t fullest_elsewhere(int m, int n, int k, bool wide) {
+  const int units = ps_compute_units();
+  const int64_t tiles_128 = (int64_t)((m + 127) / 128) * ((n + 63) / 64);
+  const int rows = !wide && 2 * tiles_128 >= (k >= 2048 ? 2 : 3) * units ? 128 : 64;
+  const int columns = wide ? 256 : 64;
+  const int64_t tiles = (int64_t)((m + rows - 1) / rows) * ((n + columns - 1) / columns);
+  return (tiles + units - 1) / units * rows * columns;
+}
+
+// Which tiles a product takes, 0: not this kernel.  `wide`: the wide kernel would take it otherwise.
+//
+// Not where the fullest unit makes one and a half times the outputs that it would make elsewhere.  Of 350 products of 113
+// to 4,116 rows those with a ratio of up to 1.33 take 0.51 to 0.998 of the other kernel's time with bfloat16 outputs or
+// as residual (one with 1.2 1.02), the four beyond 1.07 to 1.10 (1293 x 1536 x 768, 504 tiles of 64 x 64 or 132 of
+// 128 x 128, 8.9 us there and 9.7 here; 1300 x 3072 x 1024, 252 blocks of 64 x 256, 14.5 and 15.7).
+//
+// Float outputs that are not added to what is there are twice the bytes at the end of a tile, which blocks that
+// share a unit hide from each other.  With k up to 1,024 they leave nothing to gain at 128 x 64 (515 x 3072 x 1024
+// 10.5 there and 11.2 here, 26 products 0.98 to 1.07; k = 1280 0.90 to 0.93), at a ratio of 1.33 (0.97 to 1.02; k =
+// 1280 0.87 to 0.93) and, against the wide kernel, at 256 x 128 and 256 x 192 where more than 6 % of the tiles lie behind the
+// product's ends (785 x 8192 x 1024 24.0 and 27.0, 2596 x 4096 x 1024 35.8 and 38.2; with less 3292 x 3072 x 1024 37.7 and
+// 34.4, 2048 x 4096 x 1024 28.5 and 27.0).
+static int shape_for(int m, int n, int k, int c_dtype, int epilogue, bool wide) {
   const int medium = medium_shape(m, n, k, epilogue);
-  return medium != 0 ? medium : large_width(m, n, k);
+  const int shape = medium != 0 ? medium : large_width(m, n, k);
+  if (shape == 0) return 0;
+  const int rows = tile_rows(shape), columns = tile_columns(shape);
+  const int units = ps_compute_units();
+  const int64_t tiles = (int64_t)((m + rows - 1) / rows) * ((n + columns - 1) / columns);
+  const int64_t here = (tiles + units - 1) / units * rows * columns, there = fullest_elsewhere(m, n, k, wide);
+  if (2 * here >= 3 * there) return 0;
+  if (c_dtype == PS_F32 && epilogue != PS_EPI_RESIDUAL && k <= 1024) {
+    const bool padded = 100 * (int64_t)m * n < 94 * tiles * rows * columns;
+    if (shape == 11 || 10 * here > 13 * there || (wide && padded && (shape == 22 || shape == 3))) return 0;
+  }
+  return shape;
 }
 
 // (k a multiple of 32 for whole stages; a tile's rows lie within 32-bit offsets)
@@ -300,8 +335,9 @@ static bool large_takes(const void* a, const void* w, int m, int n, int k, int l
          (reinterpret_cast<uintptr_t>(a) & 15u) == 0 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
 }
 
-bool ps_gemm_nt_bf16_large_supported(const void* a, const void* w, int m, int n, int k, int lda, int epilogue) {
-  return large_takes(a, w, m, n, k, lda) && shape_for(m, n, k, epilogue) != 0;
+int ps_gemm_nt_bf16_large_shape(const void* a, const void* w, int m, int n, int k, int lda, int c_dtype, int epilogue,
+                                bool wide) {
+  return large_takes(a, w, m, n, k, lda) ? shape_for(m, n, k, c_dtype, epilogue, wide) : 0;
 }
 
 // `most_rows`: rows of tiles to a panel.
@@ -331,11 +367,10 @@ static int launch_large(const void* a, const void* w, const float* bias, void* c
   return 0;
 }
 
-// shape: a tile's number, 0: by the rule.  Stages as many as LDS holds (160 KB); of 128 x 64 and 128 x 128 four, which
+// shape: a tile's number.  Stages as many as LDS holds (160 KB); of 128 x 64 and 128 x 128 four, which
 // measured no slower than five or six.
 int ps_gemm_nt_bf16_large(const void* a, const void* w, const float* bias, void* c, int m, int n, int k, int lda,
                           int ldc, int c_dtype, int epilogue, const KvScatter& scatter, int shape, hipStream_t s) {
-  if (shape == 0) shape = shape_for(m, n, k, epilogue);
 #define PS_LARGE(FM, FN, ROW, RING, PANEL)                                                                          \
   (c_dtype == PS_F32                                                                                                \
        ? launch_large<FM, FN, ROW, RING, float>(a, w, bias, c, m, n, k, lda, ldc, epilogue, PANEL, scatter, s)      \
@@ -357,12 +392,12 @@ int ps_gemm_nt_bf16_large(const void* a, const void* w, const float* bias, void*
 
 // The large product on its own, for tests and measurements of its tile shapes.
 extern "C" int ps_gemm_nt_large(const void* a, const void* w, const float* bias, void* c, int m, int n, int k,
-                                int lda, int ldc, int c_dtype, int epilogue, int width, void* stream) {
+                                int lda, int ldc, int c_dtype, int epilogue, int tile, void* stream) {
   PS_REQUIRE(a && w && c && large_takes(a, w, m, n, k, lda) && ldc >= n,
              "ps_gemm_nt_large: bad sizes or unaligned operand (m %d, n %d, k %d, lda %d, ldc %d)", m, n, k, lda, ldc);
   PS_REQUIRE(c_dtype == PS_F32 || c_dtype == PS_BF16, "ps_gemm_nt_large: unknown output dtype");
   PS_REQUIRE(epilogue != PS_EPI_RESIDUAL || c_dtype == PS_F32,
              "ps_gemm_nt_large: the residual epilogue needs a float output");
   KvScatter none = {};
-  return ps_gemm_nt_bf16_large(a, w, bias, c, m, n, k, lda, ldc, c_dtype, epilogue, none, width, (hipStream_t)stream);
+  return ps_gemm_nt_bf16_large(a, w, bias, c, m, n, k, lda, ldc, c_dtype, epilogue, none, tile, (hipStream_t)stream);
 }

@@ -437,9 +437,10 @@ int ps_gemm_nt_bf16_wide(const void* a, const void* w_packed, const float* bias,
 int ps_gemm_nt_bf16_tiled(const void* a, const void* w, const float* bias, void* c, int m, int n,
                           int k, int lda, int ldc, int c_dtype, int epilogue,
                           const KvScatter& scatter, hipStream_t s);
-bool ps_gemm_nt_bf16_large_supported(const void* a, const void* w, int m, int n, int k, int lda, int epilogue);
+int ps_gemm_nt_bf16_large_shape(const void* a, const void* w, int m, int n, int k, int lda, int c_dtype, int epilogue,
+                                bool wide);
 int ps_gemm_nt_bf16_large(const void* a, const void* w, const float* bias, void* c, int m, int n, int k, int lda,
-                          int ldc, int c_dtype, int epilogue, const KvScatter& scatter, int width, hipStream_t s);
+                          int ldc, int c_dtype, int epilogue, const KvScatter& scatter, int shape, hipStream_t s);
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
@@ -629,6 +630,22 @@ bool ps_gemm_nt_mfma_skinny(const void* a, const void* w, int m, int n, int k, i
   return skinny_k || !ps_gemm_nt_bf16_tiled_supported(a, w, m, k, lda);
 }
 
+// What takes a bfloat16 product that the skinny kernel does not: a tile's number of the large one, the wide one, or
+// 0: the ring kernel or, where its operands do not suit that, the plain tiles.
+#define WIDE_PRODUCT 1
+static int choice_of_many_rows(const void* a, const void* w, const void* wp, int m, int n, int k, int lda,
+                               int c_dtype, int epilogue) {
+  const bool wide = ps_gemm_nt_bf16_wide_supported(a, wp, m, n, k, lda);
+  const int shape = ps_gemm_nt_bf16_large_shape(a, w, m, n, k, lda, c_dtype, epilogue, wide);
+  return shape != 0 ? shape : (wide ? WIDE_PRODUCT : 0);
+}
+
+extern "C" int ps_linear_choice(int m, int n, int k, int c_dtype, int epilogue, int packed) {
+  const void* aligned = reinterpret_cast<const void*>((uintptr_t)256);
+  if (ps_gemm_nt_mfma_skinny(aligned, aligned, m, n, k, k, PS_BF16, epilogue)) return 0;
+  return choice_of_many_rows(aligned, aligned, packed ? aligned : nullptr, m, n, k, k, c_dtype, epilogue);
+}
+
 int ps_gemm_nt_mfma(const void* a, const void* w, const float* bias, void* c, int m, int n, int k,
                     int lda, int ldc, int dtype, int c_dtype, int epilogue,
                     const KvScatter& scatter, const void* w_packed, int layouts,
@@ -646,9 +663,10 @@ int ps_gemm_nt_mfma(const void* a, const void* w, const float* bias, void* c, in
                  m, n, k);
     return 1;
   }
-  if (dtype == PS_BF16 && ps_gemm_nt_bf16_large_supported(a, w, m, n, k, lda, epilogue))
-    return ps_gemm_nt_bf16_large(a, w, bias, c, m, n, k, lda, ldc, c_dtype, epilogue, scatter, 0, s);
-  if (dtype == PS_BF16 && ps_gemm_nt_bf16_wide_supported(a, wp, m, n, k, lda))
+  const int choice = dtype == PS_BF16 ? choice_of_many_rows(a, w, wp, m, n, k, lda, c_dtype, epilogue) : 0;
+  if (choice > WIDE_PRODUCT)
+    return ps_gemm_nt_bf16_large(a, w, bias, c, m, n, k, lda, ldc, c_dtype, epilogue, scatter, choice, s);
+  if (choice == WIDE_PRODUCT)
     return ps_gemm_nt_bf16_wide(a, wp, bias, c, m, n, k, lda, ldc, c_dtype, epilogue, scatter, 0, s);
   if (dtype == PS_BF16 && ps_gemm_nt_bf16_tiled_supported(a, w, m, k, lda))
     return ps_gemm_nt_bf16_tiled(a, w, bias, c, m, n, k, lda, ldc, c_dtype, epilogue, scatter, s);

@@ -108,6 +108,9 @@ typedef struct PsLinearArgs {
 
 int ps_linear(const PsLinearArgs* args, void* stream);
 int ps_linear_args_size(void);   // sizeof(PsLinearArgs) as this library was built
+// Which kernel takes a bfloat16 product of aligned operands in dense rows, for tests of the dispatch: 1 the wide one
+// (packed: the packed copy is there), a tile's number of the large one (gemm_large_bf16.hip), 0 another.
+int ps_linear_choice(int m, int n, int k, int c_dtype, int epilogue, int packed);
 
 // Store keys and values of the step's tokens into their pages.
 //   k, v: [tokens, kv_heads * head_dim] with row stride `stride`;

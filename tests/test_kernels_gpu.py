@@ -1310,6 +1310,37 @@ def test_linear_takes_the_wide_product_for_long_k():
     assert torch.equal(v_pool.view(torch.int16), v_ref.view(torch.int16))
 
 
+def _linear_choice(m, n, k, dtype, epilogue="none", packed=True):
+    """Which kernel takes a bfloat16 product: 0, 1 (the wide one) or a tile of the large one."""
+    from pagedserve_amd.ops import kernels, library
+
+    return library.load_library().ps_linear_choice(m, n, k, 0 if dtype == torch.float32 else 1, kernels.EPILOGUES[epilogue],
+                                                   1 if packed else 0)
+
+
+@pytest.mark.parametrize("m,n,k,plain,floats", [
+    (1293, 1536, 768, 0, 0), (1300, 3072, 1024, 1, 1), (1540, 2560, 1024, 1, 1), (320, 12800, 1600, 1, 1),     # twice, 1.5
+    (515, 3072, 1024, 11, 0), (544, 2304, 768, 11, 0), (284, 4800, 1600, 11, 11),                              # 128 x 64
+    (544, 4096, 1024, 12, 0), (626, 3840, 1280, 12, 12), (1295, 2560, 1024, 12, 12),                           # 1.33 and 1
+    (785, 8192, 1024, 22, 1), (2596, 4096, 1024, 3, 1), (2048, 3840, 1280, 22, 22), (2048, 3904, 768, 22, 22),
+    (3292, 3072, 1024, 3, 3), (2048, 4096, 1024, 22, 22), (1568, 1280, 5120, 12, 12),
+    (2048, 3072, 1024, 13, 13), (4090, 4096, 1024, 4, 4), (4089, 4800, 1600, 5, 5), (2048, 4000, 800, 2, 2)])
+def test_who_takes_a_product_of_many_rows(m, n, k, plain, floats):
+    """Products on both sides of each line between the large kernel and the others, with bfloat16 and with float
+    outputs; without the packed copy the wide kernel takes none, and float rows that are added to what is there stay with
+    the large one's tiles."""
+    from pagedserve_amd.ops import kernels
+
+    if kernels.compute_units() != 256:
+        pytest.skip("the lines are drawn for 256 compute units")
+    assert _linear_choice(m, n, k, torch.bfloat16) == plain
+    assert _linear_choice(m, n, k, torch.bfloat16, "gelu_tanh") == plain
+    assert _linear_choice(m, n, k, torch.float32) == floats
+    assert _linear_choice(m, n, k, torch.bfloat16, packed=False) != 1
+    assert _linear_choice(m, n, k, torch.float32, "residual") in (plain, 0)
+    assert k < 2048 or _linear_choice(m, n, k, torch.float32, "residual") == plain
+
+
 @pytest.mark.parametrize("m,n,k", [(256, 640, 256), (300, 1000, 288), (1, 1, 256), (257, 129, 320), (700, 1601, 480), (513, 321, 1600),
                                    (2300, 385, 352)])
 @pytest.mark.parametrize("width", [2, 3, 4, 5])
