@@ -810,6 +810,44 @@ def test_attention_tiled_f32(heads, kv_heads, head_dim, page_size, window):
     torch.testing.assert_close(out, rowwise, atol=2e-5, rtol=2e-5)
 
 
+@pytest.mark.parametrize("heads,kv_heads,head_dim,page_size", [(12, 12, 64, 16), (12, 4, 48, 8), (13, 13, 36, 16), (20, 20, 128, 16),
+                                                                (16, 2, 32, 16)])
+@pytest.mark.parametrize("window", [0, 20])
+def test_attention_tiled_f32_of_many_short_portions(heads, kv_heads, head_dim, page_size, window):
+    """So many portions of 1 to 65 tokens, fresh and behind some keys, that heads of 33 to 64 take tiles of up to 64 keys
+    in one block, beside tiles of more keys in the same launch; other heads take two."""
+    from pagedserve_amd.ops import kernels
+
+    items = [(0, 64), (0, 33), (0, 32), (31, 33), (32, 33), (0, 65), (200, 64), (3, 1), (0, 2), (62, 2), (20, 40), (0, 63)] * 4
+    totals = [past + new for past, new in items]
+    k_pool, v_pool, tables = _paged_fixture(torch.float32, totals, kv_heads, head_dim, page_size, 56)
+    q = _rand((sum(new for _, new in items), heads * head_dim), torch.float32, 57)
+    tok_item, tok_pos, tile_item, tile_q0, cu = [], [], [], [], [0]
+    for index, (past, new) in enumerate(items):
+        tok_item += [index] * new
+        tok_pos += list(range(past, past + new))
+        cu.append(cu[-1] + new)
+        tile_item += [index] * -(-new // 64)
+        tile_q0 += range(0, new, 64)
+    assert 2 * len(tile_item) * heads > 2 * kernels.compute_units()
+
+    def dev(values):
+        return torch.tensor(values, dtype=torch.int32, device="cuda")
+
+    scale = head_dim ** -0.5
+    sink = _rand((heads,), torch.float32, 58)
+    for with_sink in (None, sink):
+        out, rowwise = torch.full_like(q, float("nan")), torch.full_like(q, float("nan"))
+        kernels.attention_tiled_f32(q, k_pool, v_pool, out, dev(tile_item), dev(tile_q0), dev(cu), dev(totals), tables,
+                                    heads, scale, window=window, sink=with_sink)
+        kernels.attention_rowwise(q, k_pool, v_pool, rowwise, dev(tok_item), dev(tok_pos), tables, heads, scale,
+                                  window=window, sink=with_sink)
+        torch.testing.assert_close(out, rowwise, atol=2e-5, rtol=2e-5)
+        if with_sink is None:
+            expected = _attention_expected(q, k_pool, v_pool, tables, tok_item, tok_pos, heads, scale, window)
+            torch.testing.assert_close(out.double(), expected, atol=3e-5, rtol=3e-5)
+
+
 def test_attention_tiled_f32_refuses_what_it_cannot_take():
     from pagedserve_amd.ops import kernels
 
