@@ -93,27 +93,28 @@ __device__ inline void store_wave_tile(f32x16 (&acc)[WM][WN], float* region, int
   const int chunk = lane % EP_CHUNKS;
   const int row_in_pass = lane / EP_CHUNKS;
   const int col0 = col_base + chunk * 8;
-  const bool full = col0 + 8 <= n;
   const bool vec_c = ldc % (16 / (int)sizeof(TOut)) == 0 && (reinterpret_cast<uintptr_t>(c) & 15u) == 0;
-  const bool by_column = !vec_c || k_splits > 1;
+  constexpr bool PLAIN = EPI == PS_EPI_NONE;
+  // eight key or value columns lie in one head, and no piece ends behind n
+  const bool whole_kv = !PLAIN || scatter.k_pool == nullptr ||
+                        ((scatter.head_dim | scatter.q_cols | scatter.kv_cols) & 7) == 0;
+  const bool whole = (n & 7) == 0 || col_base + WN * 32 <= n;
+  const bool by_column = !vec_c || !whole || !whole_kv || k_splits > 1;
   float b[8];
 #pragma unroll
   for (int q = 0; q < 8; ++q) b[q] = (bias && split == 0 && col0 + q < n) ? bias[col0 + q] : 0.f;
-  // key and value columns also go into cache pages: eight consecutive columns lie in one head
-  const bool scatters = EPI == PS_EPI_NONE && scatter.k_pool != nullptr && col0 < n &&
-                        col0 + 8 > scatter.q_cols;
-  const bool vec_kv = full && col0 >= scatter.q_cols && scatter.head_dim % 8 == 0 &&
-                      scatter.q_cols % 8 == 0 && scatter.kv_cols % 8 == 0;
+  // key and value columns also go into cache pages
   TOut* pool = nullptr;
   int64_t pool_offset = 0;
-  if (scatters && vec_kv) pool = kv_scatter_col<TOut>(scatter, col0, &pool_offset);
+  if (PLAIN && !by_column && scatter.k_pool != nullptr && col0 < n && col0 >= scatter.q_cols)
+    pool = kv_scatter_col<TOut>(scatter, col0, &pool_offset);
 
   // What the whole pieces need from memory is asked for before the first of them: the residual rows, and
   // where each token's keys and values lie (two dependent reads a row).  One trip each, not one per pass.
   constexpr int PASSES = 32 / EP_ROWS;
   constexpr bool RESIDUAL = EPI == PS_EPI_RESIDUAL;
   float4 old[RESIDUAL ? WM : 1][RESIDUAL ? PASSES : 1][2];
-  if (RESIDUAL && !by_column && full) {
+  if (RESIDUAL && !by_column && col0 < n) {
 #pragma unroll
     for (int i = 0; i < WM; ++i)
 #pragma unroll
@@ -124,7 +125,6 @@ __device__ inline void store_wave_tile(f32x16 (&acc)[WM][WN], float* region, int
         old[RESIDUAL ? i : 0][RESIDUAL ? pass : 0][1] = *reinterpret_cast<const float4*>(sum + 4);
       }
   }
-  constexpr bool PLAIN = EPI == PS_EPI_NONE;
   int64_t slots[PLAIN ? WM : 1][PLAIN ? PASSES : 1];
   if (PLAIN && pool != nullptr) {
     int pos[PLAIN ? WM : 1][PLAIN ? PASSES : 1], item[PLAIN ? WM : 1][PLAIN ? PASSES : 1];
@@ -153,8 +153,8 @@ __device__ inline void store_wave_tile(f32x16 (&acc)[WM][WN], float* region, int
             acc[i][j][e];
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     if (by_column) {
-      // rows that cannot leave in aligned pieces, and partial sums of a split k: a wave's
-      // lanes take consecutive columns of one row
+      // rows that cannot leave in whole aligned pieces, heads that are no whole pieces, and partial sums of a
+      // split k: a wave's lanes take consecutive columns of one row
 #pragma unroll 8
       for (int r = 0; r < 32; ++r) {
         const int row = row_base + i * 32 + r;
@@ -193,34 +193,16 @@ __device__ inline void store_wave_tile(f32x16 (&acc)[WM][WN], float* region, int
       TOut* out = c + (int64_t)row * ldc + col0;
       if constexpr (RESIDUAL) {
         float* sum = reinterpret_cast<float*>(out);
-        if (full) {
-          float4 o0 = old[i][pass][0], o1 = old[i][pass][1];
-          o0.x += v[0]; o0.y += v[1]; o0.z += v[2]; o0.w += v[3];
-          o1.x += v[4]; o1.y += v[5]; o1.z += v[6]; o1.w += v[7];
-          *reinterpret_cast<float4*>(sum) = o0;
-          *reinterpret_cast<float4*>(sum + 4) = o1;
-        } else {
-          for (int q = 0; q < 8; ++q)
-            if (col0 + q < n) sum[q] += v[q];
-        }
+        float4 o0 = old[i][pass][0], o1 = old[i][pass][1];
+        o0.x += v[0]; o0.y += v[1]; o0.z += v[2]; o0.w += v[3];
+        o1.x += v[4]; o1.y += v[5]; o1.z += v[6]; o1.w += v[7];
+        *reinterpret_cast<float4*>(sum) = o0;
+        *reinterpret_cast<float4*>(sum + 4) = o1;
       } else {
-        if (full) {
-          // (eight key or value columns that go to their page and that nobody reads from c)
-          if (!(scatters && pool != nullptr && scatter.cache_only)) store8(out, v);
-        } else {
-          for (int q = 0; q < 8; ++q)
-            if (col0 + q < n) out[q] = from_float<TOut>(v[q]);
-        }
-        if constexpr (PLAIN) {
-          if (scatters) {
-            if (pool != nullptr) {
-              if (slots[i][pass] >= 0) store8(pool + slots[i][pass] + pool_offset, v);
-            } else if (!vec_kv) {
-              for (int q = 0; q < 8; ++q)
-                if (col0 + q < n) kv_scatter_store<TOut>(scatter, row, col0 + q, v[q]);
-            }
-          }
-        }
+        // (eight key or value columns that go to their page and that nobody reads from c)
+        if (!(PLAIN && pool != nullptr && scatter.cache_only)) store8(out, v);
+        if constexpr (PLAIN)
+          if (pool != nullptr && slots[i][pass] >= 0) store8(pool + slots[i][pass] + pool_offset, v);
       }
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");

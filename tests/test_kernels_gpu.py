@@ -1523,6 +1523,52 @@ def test_gelu_of_the_tiled_products_keeps_its_bits(m, k):
     assert torch.equal(out[:, number], expected[number].expand(m, -1))
 
 
+@pytest.mark.parametrize("m,n,k", [(100, 321, 128), (300, 996, 64), (700, 3081, 768), (2048, 3084, 768), (1300, 3068, 1024)])
+@pytest.mark.parametrize("epilogue,dtype", [("none", torch.float32), ("none", torch.bfloat16), ("gelu_tanh", torch.bfloat16),
+                                            ("residual", torch.float32)])
+def test_rows_that_end_inside_a_piece(m, n, k, epilogue, dtype):
+    """Outputs in rows that allow pieces of 16 bytes but end inside one, in each of the kernels for many rows: every
+    column is there and what lies behind the last one stays."""
+    from pagedserve_amd.ops import kernels
+
+    x, w = _rand((m, k), torch.bfloat16, 390, 1.0), _rand((n, k), torch.bfloat16, 391, 1.0 / math.sqrt(k))
+    bias = _rand((n,), torch.float32, 392)
+    whole = _rand((m, (n + 15) // 8 * 8), torch.float32, 393).to(dtype)
+    before, out = whole.clone(), whole[:, :n]
+    kernels.linear(x, w, bias, out, epilogue=epilogue, packed=kernels.pack_decode_weight(w))
+    expected = x.double() @ w.double().t() + bias.double()
+    if epilogue == "residual":
+        expected = before[:, :n].double() + expected
+    elif epilogue == "gelu_tanh":
+        expected = F.gelu(expected, approximate="tanh")
+    # (sums of k products of about 1 / sqrt(k) in 32 bits; a bfloat16 result is half a unit of its last place off, 2^-9)
+    torch.testing.assert_close(out.double(), expected, atol=1e-4, rtol=4e-3 if dtype == torch.bfloat16 else 1e-5)
+    assert torch.equal(whole[:, n:], before[:, n:])
+
+
+@pytest.mark.parametrize("heads,kv_heads,head_dim", [(5, 3, 12), (3, 3, 20), (7, 1, 64), (5, 2, 28)])
+@pytest.mark.parametrize("m,k", [(70, 128), (300, 64), (1100, 768)])
+def test_scatter_of_heads_that_are_no_whole_pieces(heads, kv_heads, head_dim, m, k):
+    """The key/value scatter behind products of many rows where heads, or the queries' columns, are no whole pieces
+    of eight, against a scatter of its own; one width that is."""
+    from pagedserve_amd.ops import kernels
+
+    q_cols, kv_cols = heads * head_dim, kv_heads * head_dim
+    n = q_cols + 2 * kv_cols
+    k_pool, v_pool, tables = _paged_fixture(torch.bfloat16, [m, 40], kv_heads, head_dim, 16, 400)
+    tok_item = torch.tensor([1] * 30 + [0] * (m - 30), dtype=torch.int32, device="cuda")
+    tok_pos = torch.tensor(list(range(10, 40)) + list(range(30, m)), dtype=torch.int32, device="cuda")
+    x, w = _rand((m, k), torch.bfloat16, 401), _rand((n, k), torch.bfloat16, 402, 1.0 / math.sqrt(k))
+    whole = torch.empty((m, (n + 7) // 8 * 8), dtype=torch.bfloat16, device="cuda")
+    out, pools = whole[:, :n], (k_pool.clone(), v_pool.clone())
+    kernels.linear(x, w, None, out, packed=kernels.pack_decode_weight(w),
+                   scatter=(k_pool, v_pool, tok_item, tok_pos, tables, q_cols, kv_cols))
+    torch.testing.assert_close(out.double(), x.double() @ w.double().t(), atol=1e-4, rtol=4e-3)
+    kernels.kv_write(out[:, q_cols:q_cols + kv_cols], out[:, q_cols + kv_cols:], *pools, tok_item, tok_pos, tables)
+    assert torch.equal(k_pool.view(torch.int16), pools[0].view(torch.int16))
+    assert torch.equal(v_pool.view(torch.int16), pools[1].view(torch.int16))
+
+
 @pytest.mark.parametrize("m", [261, 545, 1030, 2050])
 def test_linear_of_hundreds_of_rows_with_scatter(m):
     """Through ``kernels.linear``: rows and columns that tiles of 128 x 64, 128 x 128, 128 x 192 and 256 x 128 cover in one
