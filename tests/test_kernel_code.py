@@ -1,0 +1,57 @@
+"""The machine code of the kernels whose loads are written in assembly: no register is used before its load is there."""
+
+import os
+
+import pytest
+
+import kernel_code
+from pagedserve_amd.ops import library
+
+LISTING = """
+0000000000001000 <waits>:
+\tds_read_b128 v[4:7], v0                                     // 000000001000: D9FE0000 04000000
+\tds_read_b128 v[8:11], v0 offset:16                          // 000000001008: D9FE0010 08000000
+\ts_waitcnt lgkmcnt(1)                                        // 000000001010: BF8CC17F
+\t{first}                            // 000000001014: 7E000304
+\ts_cbranch_scc1 65530                                        // 000000001018: BF85FFFA <waits>
+\ts_waitcnt lgkmcnt(0)                                        // 00000000101C: BF8CC07F
+\tglobal_load_dwordx4 v[4:7], v[8:9], off                     // 000000001020: DC5C8000 047F0008
+\tglobal_store_dword v[8:9], v10, off                         // 000000001028: DC708000 007F0A08
+\ts_waitcnt vmcnt({left})                                        // 000000001030: BF8C0F70
+\tv_mov_b32_e32 v1, v5                                        // 000000001034: 7E020305
+\ts_endpgm                                                    // 000000001038: BF810000
+"""
+
+
+@pytest.mark.parametrize("first,left,registers", [
+    ("v_mov_b32_e32 v0, v4", 1, set()),
+    ("v_mov_b32_e32 v0, v4", 2, {("v", 5)}),             # the store is behind the load: two may be left
+    ("v_mov_b32_e32 v0, v9", 0, {("v", 9)}),             # the second read, one may be left
+    ("v_mov_b32_e32 v9, v4", 0, {("v", 9)}),             # what is on its way overwrites it
+    ("global_store_dword v[0:1], v11, off", 1, {("v", 11)}),
+])
+def test_the_scan_finds_uses_before_the_wait(first, left, registers):
+    (name, code), = kernel_code.kernels(LISTING.format(first=first, left=left))
+    assert name == "waits" and len(code) == 11
+    assert {register for _, _, register in kernel_code.early_uses(code)} == registers
+
+
+@pytest.mark.skipif(kernel_code.disassembler() is None, reason="no disassembler")
+@pytest.mark.parametrize("kernel", ["gemm_nt_bf16_large_kernel", "gemm_nt_ring_kernel", "attention_prefill_kernel",
+                                    "attention_mixed_kernel"])
+def test_no_register_is_used_before_its_load(kernel, tmp_path):
+    """Every instance of the kernels that read their operands from LDS by assembly, as built.  (The wide product's
+    last tiles wait by counts known at run time, which the scan cannot follow.)"""
+    path = os.path.join(library.in_tree_dir(), library.LIB_NAME)
+    if not os.path.isfile(path):
+        pytest.skip("the library is not built in the tree")
+    images = [image for image in kernel_code.code_objects(path, library.ARCH) if kernel.encode() in image]
+    assert images, "no source file holds this kernel"
+    seen = 0
+    for image in images:
+        for name, code in kernel_code.kernels(kernel_code.disassemble(image, library.ARCH, tmp_path)):
+            if kernel in name:
+                seen += 1
+                assert any(operation.startswith("ds_read") for _, operation, _, _ in code), name
+                assert not kernel_code.early_uses(code), (name, kernel_code.early_uses(code)[:4])
+    assert seen
