@@ -236,7 +236,8 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_wide_kernel(
 // 1600 x 6400 68.0 against 92.5; but 768 x 3072 (three blocks side by side) 29.9 against 27.1,
 // and at k = 768 the two are level.  (With the same weights at every launch, out of the L2,
 // this kernel looks better than it is.)  gemm_large_bf16.hip is asked first and takes most of these: what stays are
-// products whose larger tiles would leave the last round half empty.
+// products whose larger tiles would leave the last round half empty, make the fullest unit work half as long again, or leave
+// much of the tiles behind the ends of a float output.
 bool ps_gemm_nt_bf16_wide_supported(const void* a, const void* w_packed, int m, int n, int k,
                                     int lda) {
   const int64_t blocks = (int64_t)((n + GW_BN - 1) / GW_BN) * ((m + 63) / 64);
