@@ -64,10 +64,10 @@ static int large_width(int m, int n, int k) {
 
 // Outputs that the unit with the most tiles makes where the other kernels take the product (gemm_mfma.hip asks this one
 // first): the wide one's blocks of 64 x 256, or tiles of 128 x 64 or 64 x 64.
-static int64_t fullest_elsewhere(int m, int n, int k, bool wide) {
+static int64_t fullest_elsewhere(int m, int n, bool wide) {
   const int units = ps_compute_units();
   const int64_t tiles_128 = (int64_t)((m + 127) / 128) * ((n + 63) / 64);
-  const int rows = !wide && 2 * tiles_128 >= (k >= 2048 ? 2 : 3) * units ? 128 : 64;
+  const int rows = !wide && 2 * tiles_128 >= 3 * units ? 128 : 64;
   const int columns = wide ? 256 : 64;
   const int64_t tiles = (int64_t)((m + rows - 1) / rows) * ((n + columns - 1) / columns);
   return (tiles + units - 1) / units * rows * columns;
@@ -76,9 +76,11 @@ static int64_t fullest_elsewhere(int m, int n, int k, bool wide) {
 // Which tiles a product takes, 0: not this kernel.  `wide`: the wide kernel would take it otherwise.
 //
 // Not where the fullest unit makes one and a half times the outputs that it would make elsewhere.  Of 350 products of 113
-// to 4,116 rows those with a ratio of up to 1.33 take 0.51 to 0.998 of the other kernel's time with bfloat16 outputs or
-// as residual (one with 1.2 1.02), the four beyond 1.07 to 1.10 (1293 x 1536 x 768, 504 tiles of 64 x 64 or 132 of
-// 128 x 128, 8.9 us there and 9.7 here; 1300 x 3072 x 1024, 252 blocks of 64 x 256, 14.5 and 15.7).
+// to 4,116 rows those with a ratio of up to 1.33 take 0.57 to 0.998 of the other kernel's time with bfloat16 outputs or
+// as residual (one with 1.2 1.02).  Beyond, one block of 64 x 256 per unit is ahead at any k (1300 x 3072 x 1024 14.5 us
+// there and 15.7 here, x 2048 22.9 and 24.0, x 4096 level), two blocks of 64 x 64 up to a k of 1,600 (1294 x 1536 x 768 9.2
+// and 9.8, as residual 9.7 and 11.2, x 1600 14.4 and 14.1, 15.0 and 16.0; x 2048 18.2 and 16.8, 18.3 and 18.7; 1568 x 1280 x
+// 5120 40.5 and 35.9, 41.5 and 38.0).
 //
 // Float outputs that are not added to what is there are twice the bytes at the end of a tile, which blocks that
 // share a unit hide from each other.  With k up to 1,024 they leave nothing to gain at 128 x 64 (515 x 3072 x 1024
@@ -93,8 +95,8 @@ static int shape_for(int m, int n, int k, int c_dtype, int epilogue, bool wide) 
   const int rows = tile_rows(shape), columns = tile_columns(shape);
   const int units = ps_compute_units();
   const int64_t tiles = (int64_t)((m + rows - 1) / rows) * ((n + columns - 1) / columns);
-  const int64_t here = (tiles + units - 1) / units * rows * columns, there = fullest_elsewhere(m, n, k, wide);
-  if (2 * here >= 3 * there) return 0;
+  const int64_t here = (tiles + units - 1) / units * rows * columns, there = fullest_elsewhere(m, n, wide);
+  if (2 * here >= 3 * there && (wide || k < 2048)) return 0;
   if (c_dtype == PS_F32 && epilogue != PS_EPI_RESIDUAL && k <= 1024) {
     const bool padded = 100 * (int64_t)m * n < 94 * tiles * rows * columns;
     if (shape == 11 || 10 * here > 13 * there || (wide && padded && (shape == 22 || shape == 3))) return 0;

@@ -377,16 +377,12 @@ static int launch_tiled_bf16(const void* a, const void* w, const float* bias, vo
   const int units = ps_compute_units();
   if (m > 64 && tiles_128 >= 3 * units)
     return launch_variant<bf16_t, 2, 2, 2, TOut>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
-  // 128 x 64: three stages while two blocks per unit hold them all (1100 x 3072 x 1024 with
-  // weights from memory: 16.1 against 17.7 us), two stages, which let a third block in, beyond
+  // 128 x 64: three stages while two blocks per unit hold them all (2000 x 1600 x 640 added to rows, with weights from
+  // memory: 13.2 against 13.9 us; 4100 x 768 x 512 12.0 and 12.6), two stages, which let a third block in, beyond
   if (m > 64 && tiles_128_64 >= units + units / 2 && tiles_128_64 <= 2 * units)
     return launch_variant<bf16_t, 2, 1, 3, TOut>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
   if (m > 64 && tiles_128_64 >= units + units / 2)
     return launch_variant<bf16_t, 2, 1, 2, TOut>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
-  // a long k with a block per compute unit: four stages of 128 x 64 (2048 x 1024 x 4096 with
-  // weights from memory: 34.7 us against 37.8 for 64 x 64 tiles)
-  if (m > 64 && k >= 2048 && tiles_128_64 >= units)
-    return launch_variant<bf16_t, 2, 1, 4, TOut>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
   // 64 x 64 tiles.  What a compute unit has in flight decides how long a k tile takes to
   // arrive from memory.  Many blocks fill a unit by their number and keep two stages, which
   // lets five of them in; up to two blocks per unit get four stages each.  That also holds for
@@ -413,7 +409,7 @@ static int launch_tiled_bf16(const void* a, const void* w, const float* bias, vo
     return launch_variant<bf16_t, 1, 1, 6, TOut, 2>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
   if ((tiles_64 <= 2 * units && k_tiles > 2) || k >= 2048)
     return launch_variant<bf16_t, 1, 1, 4, TOut>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
-  // up to three blocks per unit: three stages each (544 x 4096 x 1024: 15.9 against 18.2 us)
+  // up to three blocks per unit: three stages each (544 x 4096 x 1024 to float: 13.1 against 13.5 us)
   if (tiles_64 <= 3 * units && k_tiles > 2)
     return launch_variant<bf16_t, 1, 1, 3, TOut>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
   return launch_variant<bf16_t, 1, 1, 2, TOut>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);

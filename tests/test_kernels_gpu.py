@@ -1361,7 +1361,7 @@ def _linear_choice(m, n, k, dtype, epilogue="none", packed=True):
     (515, 3072, 1024, 11, 0), (544, 2304, 768, 11, 0), (284, 4800, 1600, 11, 11),                              # 128 x 64
     (544, 4096, 1024, 12, 0), (626, 3840, 1280, 12, 12), (1295, 2560, 1024, 12, 12),                           # 1.33 and 1
     (785, 8192, 1024, 22, 1), (2596, 4096, 1024, 3, 1), (2048, 3840, 1280, 22, 22), (2048, 3904, 768, 22, 22),
-    (3292, 3072, 1024, 3, 3), (2048, 4096, 1024, 22, 22), (1568, 1280, 5120, 12, 12),
+    (3292, 3072, 1024, 3, 3), (2048, 4096, 1024, 22, 22), (1568, 1280, 5120, 12, 12), (1294, 1536, 2048, 12, 12), (1300, 3072, 4096, 1, 1),
     (2048, 3072, 1024, 13, 13), (4090, 4096, 1024, 4, 4), (4089, 4800, 1600, 5, 5), (2048, 4000, 800, 2, 2)])
 def test_who_takes_a_product_of_many_rows(m, n, k, plain, floats):
     """Products on both sides of each line between the large kernel and the others, with bfloat16 and with float
