@@ -1321,14 +1321,17 @@ def test_linear_takes_the_wide_product_for_long_k():
     LDS), also with the key/value scatter behind it."""
     from pagedserve_amd.ops import kernels
 
-    m, k = 1300, 1024
+    m, k = 2050, 1024
     heads, kv_heads, head_dim, page_size = 32, 16, 64, 16
     q_cols, kv_cols = heads * head_dim, kv_heads * head_dim
-    n = q_cols + 2 * kv_cols          # 4,096 columns: 16 x 21 blocks of 64 rows x 256 columns
-    lens = [700, 650]
+    n = q_cols + 2 * kv_cols          # 4,096 columns: 16 x 33 blocks of 64 rows x 256 columns
+    if kernels.compute_units() == 256:
+        assert _linear_choice(m, n, k, torch.bfloat16) == 1
+        assert _linear_choice(m, n, k, torch.bfloat16, packed=False) == 0
+    lens = [1100, 1000]
     k_pool, v_pool, tables = _paged_fixture(torch.bfloat16, lens, kv_heads, head_dim, page_size, 320)
-    tok_item = torch.tensor([0] * 680 + [1] * 620, dtype=torch.int32, device="cuda")
-    tok_pos = torch.tensor(list(range(20, 700)) + list(range(30, 650)), dtype=torch.int32, device="cuda")
+    tok_item = torch.tensor([0] * 1080 + [1] * 970, dtype=torch.int32, device="cuda")
+    tok_pos = torch.tensor(list(range(20, 1100)) + list(range(30, 1000)), dtype=torch.int32, device="cuda")
     x = _rand((m, k), torch.bfloat16, 321)
     w = _rand((n, k), torch.bfloat16, 322, 1.0 / math.sqrt(k))
     bias = _rand((n,), torch.float32, 323)
@@ -1379,11 +1382,29 @@ def test_who_takes_a_product_of_many_rows(m, n, k, plain, floats):
     assert k < 2048 or _linear_choice(m, n, k, torch.float32, "residual") == plain
 
 
+LARGE_EPILOGUES = [("none", torch.bfloat16), ("gelu_tanh", torch.bfloat16), ("gelu_erf", torch.bfloat16),
+                   ("relu2", torch.bfloat16), ("none", torch.float32), ("gelu_tanh", torch.float32),
+                   ("gelu_erf", torch.float32), ("relu2", torch.float32), ("residual", torch.float32)]
+
+
+def _activated(product, epilogue):
+    if epilogue == "relu2":
+        return torch.relu(product) ** 2
+    return F.gelu(product, approximate="tanh" if epilogue == "gelu_tanh" else "none") if "gelu" in epilogue else product
+
+
+def _assert_product(out, expected, epilogue):
+    """Sums of k products of about 1 / sqrt(k) in 32 bits, values of a few units (squared: some tens, whose error grows
+    with them); a bfloat16 result is half a unit of its last place off, 2^-9."""
+    rtol = 4e-3 if out.dtype == torch.bfloat16 else (1e-4 if epilogue == "relu2" else 1e-5)
+    torch.testing.assert_close(out.double(), expected, atol=1e-4, rtol=rtol)
+
+
 @pytest.mark.parametrize("m,n,k", [(256, 640, 256), (300, 1000, 288), (1, 1, 256), (257, 129, 320), (700, 1601, 480), (513, 321, 1600),
                                    (2300, 385, 352)])
 @pytest.mark.parametrize("width", [2, 3, 4, 5])
-@pytest.mark.parametrize("epilogue", ["none", "gelu_tanh", "residual"])
-def test_gemm_large_tile_shapes(m, n, k, width, epilogue):
+@pytest.mark.parametrize("epilogue,dtype", LARGE_EPILOGUES)
+def test_gemm_large_tile_shapes(m, n, k, width, epilogue, dtype):
     """The product of thousands of rows at each of its tile widths: as few stages of k as it takes and counts that
     leave every place of the ring at the end, rows and columns that end inside a tile and a wave's part of it, panels
     of rows that are not full, output rows that do not allow 16-byte stores, input rows apart from one another."""
@@ -1402,14 +1423,13 @@ def test_gemm_large_tile_shapes(m, n, k, width, epilogue):
         out = _rand((m, n), torch.float32, 333)
         expected = out.double() + product
     else:
-        out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
-        expected = F.gelu(product, approximate="tanh") if epilogue == "gelu_tanh" else product
+        out = torch.full((m, n), float("nan"), dtype=dtype, device="cuda")
+        expected = _activated(product, epilogue)
     status = fn(a.data_ptr(), w.data_ptr(), bias.data_ptr(), out.data_ptr(), m, n, k, a.stride(0), out.stride(0),
                 0 if out.dtype == torch.float32 else 1, kernels.EPILOGUES[epilogue], width,
                 torch.cuda.current_stream().cuda_stream)
     assert status == 0, lib.ps_last_error().decode()
-    atol, rtol = (1e-4, 1e-5) if epilogue == "residual" else (4e-2, 2e-2)
-    torch.testing.assert_close(out.double(), expected, atol=atol, rtol=rtol)
+    _assert_product(out, expected, epilogue)
     # k in stages of 32, rows in pieces of 16 bytes: the rest is refused
     for bad_k, bad_lda in ((k - 16, a.stride(0)), (k, a.stride(0) + 4), (224, a.stride(0))):
         assert fn(a.data_ptr(), w.data_ptr(), bias.data_ptr(), out.data_ptr(), m, n, bad_k, bad_lda, out.stride(0),
@@ -1417,7 +1437,7 @@ def test_gemm_large_tile_shapes(m, n, k, width, epilogue):
 
 
 @pytest.mark.parametrize("m,inner,k", [(1, 16, 64), (8, 3072, 768), (3, 48, 832), (16, 320, 1024), (5, 80, 1600), (15, 16, 192), (40, 48, 832),
-                                       (64, 320, 1024)])
+                                       (64, 320, 1024), (8, 8192, 64), (16, 8192, 128), (1, 8208, 1088)])
 @pytest.mark.parametrize("activation,form", [("silu", None), ("silu", (0.7, 1.702, 1.0)), ("gelu_tanh", None), ("relu", None)])
 def test_gate_in_the_product_of_few_rows(m, inner, k, activation, form):
     """The bits of the product and the gate as two launches: one step of k and counts that the waves do not share
@@ -1449,8 +1469,8 @@ def test_gate_in_the_product_of_few_rows(m, inner, k, activation, form):
 
 @pytest.mark.parametrize("m,n,k", [(256, 640, 256), (300, 1000, 320), (1, 1, 256), (129, 65, 384), (700, 1601, 448), (513, 321, 1600)])
 @pytest.mark.parametrize("tile", [11, 12, 13, 22])
-@pytest.mark.parametrize("epilogue", ["none", "gelu_tanh", "residual"])
-def test_gemm_large_tiles_in_rows_of_whole_lines(m, n, k, tile, epilogue):
+@pytest.mark.parametrize("epilogue,dtype", LARGE_EPILOGUES)
+def test_gemm_large_tiles_in_rows_of_whole_lines(m, n, k, tile, epilogue, dtype):
     """The tiles of 128 x 64 to 256 x 128, whose stages are 64 values of k: as few stages as the ring holds and every
     remainder at its end, rows and columns that end inside a tile and a wave's part of it, panels that are not full,
     rows that do not allow 16-byte stores."""
@@ -1469,15 +1489,13 @@ def test_gemm_large_tiles_in_rows_of_whole_lines(m, n, k, tile, epilogue):
         out = _rand((m, n), torch.float32, 353)
         expected = out.double() + product
     else:
-        out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
-        expected = F.gelu(product, approximate="tanh") if epilogue == "gelu_tanh" else product
+        out = torch.full((m, n), float("nan"), dtype=dtype, device="cuda")
+        expected = _activated(product, epilogue)
     status = fn(a.data_ptr(), w.data_ptr(), bias.data_ptr(), out.data_ptr(), m, n, k, a.stride(0), out.stride(0),
                 0 if out.dtype == torch.float32 else 1, kernels.EPILOGUES[epilogue], tile,
                 torch.cuda.current_stream().cuda_stream)
     assert status == 0, lib.ps_last_error().decode()
-    # (sums of k products of about 1 / sqrt(k) in 32 bits; a bfloat16 result is half a unit of its last place off, 2^-9)
-    atol, rtol = (1e-4, 1e-5) if epilogue == "residual" else (1e-4, 4e-3)
-    torch.testing.assert_close(out.double(), expected, atol=atol, rtol=rtol)
+    _assert_product(out, expected, epilogue)
     # half a stage of k is refused
     assert fn(a.data_ptr(), w.data_ptr(), bias.data_ptr(), out.data_ptr(), m, n, k - 32, a.stride(0), out.stride(0),
               0 if out.dtype == torch.float32 else 1, kernels.EPILOGUES[epilogue], tile, None) != 0
@@ -1569,15 +1587,19 @@ def test_scatter_of_heads_that_are_no_whole_pieces(heads, kv_heads, head_dim, m,
     assert torch.equal(v_pool.view(torch.int16), pools[1].view(torch.int16))
 
 
-@pytest.mark.parametrize("m", [261, 545, 1030, 2050])
-def test_linear_of_hundreds_of_rows_with_scatter(m):
-    """Through ``kernels.linear``: rows and columns that tiles of 128 x 64, 128 x 128, 128 x 192 and 256 x 128 cover in one
-    round, with the key/value scatter behind the product, against float64 and a scatter of its own."""
+@pytest.mark.parametrize("m,heads,kv_heads,k,tile", [
+    (261, 32, 16, 832, 11), (545, 32, 16, 832, 12), (1030, 32, 16, 832, 13), (2040, 32, 16, 832, 22), (2040, 32, 16, 800, 2),
+    (2050, 25, 25, 832, 3), (3000, 32, 16, 832, 4), (3500, 25, 25, 832, 5), (2050, 32, 16, 832, 0)])
+def test_linear_of_many_rows_with_scatter(m, heads, kv_heads, k, tile):
+    """Through ``kernels.linear``: products that go to each of the large kernel's tiles, and one that goes past it, with
+    the key/value scatter behind the product, against float64 and a scatter of its own."""
     from pagedserve_amd.ops import kernels
 
-    heads, kv_heads, head_dim, page_size, k = 32, 16, 64, 16, 832
+    head_dim, page_size = 64, 16
     q_cols, kv_cols = heads * head_dim, kv_heads * head_dim
     n = q_cols + 2 * kv_cols
+    if kernels.compute_units() == 256:
+        assert _linear_choice(m, n, k, torch.bfloat16) == tile
     k_pool, v_pool, tables = _paged_fixture(torch.bfloat16, [m + 40, 60], kv_heads, head_dim, page_size, 360)
     tok_item = torch.tensor([1] * 50 + [0] * (m - 50), dtype=torch.int32, device="cuda")
     tok_pos = torch.tensor(list(range(10, 60)) + list(range(90, m + 40)), dtype=torch.int32, device="cuda")
