@@ -31,11 +31,12 @@ typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 
 // STEPS: head_dim / 64; AHEAD: tiles of 16 columns per wave whose weights are asked for beside the keys
-// (further ones follow behind the attention): heads of 64 right behind the first keys and values, heads of 128 in front
-// of the attention.  Those hold twice the weights, which the first turn over the keys has no registers left for (16
-// waves spill 16 of them; 8 requests of 8 heads of 128 over 250 keys 9.5 us with the weights in front, 11.7 behind; one of 16
-// heads over 400 keys 10.6 and 12.1; heads of 64, 8 requests of 12 over 540 keys 9.5 and 9.2).
-template <int STEPS, int AD_WAVES, int AD_UNROLL, int AHEAD>
+// (further ones follow behind the attention): right behind the first keys and values, or FIRST, in front of the
+// attention, where they hold back the block table and with it the keys, but nothing of a wave's later turns
+// (parts/attention.py says where the line lies).  Heads of 128 hold twice the weights, which the first turn over the keys has
+// no registers left for (16 waves spill 16 of them; 8 requests of 8 heads over 250 keys 9.5 us with the weights in front,
+// 11.7 behind; one of 16 heads over 400 keys 10.6 and 12.1): always in front.
+template <int STEPS, int AD_WAVES, int AD_UNROLL, int AHEAD, bool FIRST>
 __global__ __launch_bounds__(64 * AD_WAVES) void attention_decode_linear_kernel(
     const bf16_t* __restrict__ q, int64_t q_stride, const bf16_t* __restrict__ k_pool,
     const bf16_t* __restrict__ v_pool, const int* __restrict__ tok_pos,
@@ -78,11 +79,11 @@ __global__ __launch_bounds__(64 * AD_WAVES) void attention_decode_linear_kernel(
         tok_pos, tables, table_width, heads, kv_heads, HEAD_DIM, page_size, page_shift, num_pages,
         scale_log2, window, 1, extra, context, ahead);
   };
-  if constexpr (STEPS == 1) {
-    attend([&] { load_weights(0); });
-  } else {
+  if constexpr (FIRST) {
     load_weights(0);
     attend(NothingAhead());
+  } else {
+    attend([&] { load_weights(0); });
   }
   __syncthreads();
 
@@ -129,7 +130,7 @@ extern "C" int ps_attention_decode_linear(const void* q, int64_t q_stride, const
                                           int64_t gate_ld, float softcap, const float* logistic,
                                           float logistic_norm, const void* w_packed,
                                           const float* bias, float* residual, int64_t ld_res, int n,
-                                          int parts, int waves, void* stream) {
+                                          int parts, int waves, int weights_first, void* stream) {
   PS_REQUIRE(count >= 0 && count <= 64 && heads > 0 && heads <= 65535 && kv_heads > 0 &&
                  heads % kv_heads == 0 && page_size > 0 && num_pages > 0 && table_width > 0,
              "ps_attention_decode_linear: bad sizes (count %d, heads %d, kv_heads %d)", count, heads,
@@ -155,20 +156,23 @@ extern "C" int ps_attention_decode_linear(const void* q, int64_t q_stride, const
   const AttnExtras extra{sink, gate, gate_ld, softcap, logistic, logistic_norm};
   dim3 grid(count, heads, (tiles_n + tiles_per_block - 1) / tiles_per_block);
   hipStream_t s = (hipStream_t)stream;
-#define PS_LAUNCH_ADL(STEPS, WAVES, UNROLL, AHEAD)                                                 \
-  hipLaunchKernelGGL((attention_decode_linear_kernel<STEPS, WAVES, UNROLL, AHEAD>), grid,          \
+#define PS_LAUNCH_ADL(STEPS, WAVES, UNROLL, AHEAD, FIRST)                                          \
+  hipLaunchKernelGGL((attention_decode_linear_kernel<STEPS, WAVES, UNROLL, AHEAD, FIRST>), grid,   \
                      dim3(64 * WAVES), 0, s, (const bf16_t*)q, q_stride, (const bf16_t*)k_pool,    \
                      (const bf16_t*)v_pool, tok_pos, tables, table_width, heads, kv_heads,         \
                      page_size, page_shift, num_pages, scale * 1.4426950408889634f, window, extra, \
                      (const bf16_t*)w_packed, bias, residual, ld_res, n, tiles_per_block)
   if (head_dim == 64) {
-    if (waves == 4) PS_LAUNCH_ADL(1, 4, 4, 4);
-    else if (waves == 8) PS_LAUNCH_ADL(1, 8, 8, 4);
-    else PS_LAUNCH_ADL(1, 16, 8, 3);
+    // (eight waves are behind with the weights in front everywhere)
+    if (waves == 4 && weights_first) PS_LAUNCH_ADL(1, 4, 4, 4, true);
+    else if (waves == 4) PS_LAUNCH_ADL(1, 4, 4, 4, false);
+    else if (waves == 8) PS_LAUNCH_ADL(1, 8, 8, 4, false);
+    else if (weights_first) PS_LAUNCH_ADL(1, 16, 8, 3, true);
+    else PS_LAUNCH_ADL(1, 16, 8, 3, false);
   } else {
-    if (waves == 4) PS_LAUNCH_ADL(2, 4, 4, 4);
-    else if (waves == 8) PS_LAUNCH_ADL(2, 8, 8, 4);
-    else PS_LAUNCH_ADL(2, 16, 8, 2);
+    if (waves == 4) PS_LAUNCH_ADL(2, 4, 4, 4, true);
+    else if (waves == 8) PS_LAUNCH_ADL(2, 8, 8, 4, true);
+    else PS_LAUNCH_ADL(2, 16, 8, 2, true);
   }
 #undef PS_LAUNCH_ADL
   PS_CHECK_LAUNCH("ps_attention_decode_linear");

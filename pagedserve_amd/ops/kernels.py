@@ -114,7 +114,7 @@ _SIGNATURES = {
     "ps_attention_decode_linear": [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int,
                                    c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_void_p, c_void_p,
                                    c_int64, c_float, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_int64,
-                                   c_int, c_int, c_int, c_void_p],
+                                   c_int, c_int, c_int, c_int, c_void_p],
     "ps_attention_merge_linear": [c_void_p, c_int64, c_void_p, c_int, c_int, c_int, c_int, c_void_p,
                                   c_void_p, c_void_p, c_int64, c_int, c_int, c_void_p],
     "ps_attention_tiled_f32": [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_void_p,
@@ -915,10 +915,11 @@ def decode_linear_supported(dtype, tokens, head_dim, packed) -> bool:
 
 
 def attention_decode_linear(q, k_pool, v_pool, tok_pos, tables, heads, scale, w, packed, bias, residual, parts, waves,
-                            window=0, sink=None, gate=None, softcap=0.0, logistic=None):
+                            window=0, sink=None, gate=None, softcap=0.0, logistic=None, weights_first=False):
     """residual[t] += (decode attention of token t, which is item t) w^T + bias, in one launch; ``packed`` is
     ``pack_decode_weight(w)``.  ``parts``: into how many parts the columns are dealt, one block per (token,
-    head, part); ``waves``: 4, 8 or 16 to a block."""
+    head, part); ``waves``: 4, 8 or 16 to a block.  ``weights_first``: heads of 64 in blocks of 4 or 16 waves ask for the
+    weights in front of the keys; it steers the order of loads only."""
     _check(q, "q", torch.bfloat16, 2)
     pages, kv_heads, page_size, head_dim = _check_pools(k_pool, v_pool, q.dtype)
     q_stride = _rows(q, "q")
@@ -944,7 +945,7 @@ def attention_decode_linear(q, k_pool, v_pool, tok_pos, tables, heads, scale, w,
           tok_pos.data_ptr(), tables.data_ptr(), tables.shape[1], tokens, heads, kv_heads, head_dim, page_size, pages,
           float(scale), int(window), _check_sink(sink, heads), gate_ptr, gate_ld, _check_cap(softcap),
           *_check_logistic(logistic, heads), packed.data_ptr(), _ptr(bias), residual.data_ptr(),
-          _rows(residual, "residual"), n, int(parts), int(waves), _stream())
+          _rows(residual, "residual"), n, int(parts), int(waves), int(weights_first), _stream())
     return residual
 
 

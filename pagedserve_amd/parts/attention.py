@@ -381,7 +381,8 @@ class Attention(Mixer):
                 kernels.attention_decode_linear(q, cache.k_pool, cache.v_pool, ctx.positions, tables, self.heads,
                                                 self.scale, self.out_weight, self.out_packed, self.out_bias, residual,
                                                 *shape, window=self.span, sink=sink, gate=gates,
-                                                softcap=self.score_cap, logistic=self.logistic)
+                                                softcap=self.score_cap, logistic=self.logistic,
+                                                weights_first=self._weights_first(*shape, ctx.max_kv_len))
                 return
         merged_splits = 0
         if residual is not None and gates is None and singles == tokens and kernels.merge_linear_supported(
@@ -558,6 +559,18 @@ class Attention(Mixer):
         if self.width * self.head_dim * 2 > 131072 * parts:
             return None
         return parts, waves
+
+    def _weights_first(self, parts: int, waves: int, max_kv_len: int) -> bool:
+        """Whether the blocks of that kernel ask for their weights in front of the keys, not behind the first of them.  A
+        wave's loads come back in the order of issue: in front, the weights hold back the block table and the
+        first keys; behind, the keys of a wave's second turn, and with sixteen waves there is more to hold
+        back.  (Keys and weights from memory, behind and in front, heads of 64: four waves within 128 keys 0.98 on
+        average, 1 of 12 heads over 60 keys 4.37 / 4.40; beyond, where a wave takes several turns, 1.02 to 1.13, 24 requests of
+        12 heads over 270 keys 13.3 / 11.85.  Eight waves, one turn, 0.88 to 1.02.  Sixteen waves in one part 0.99 up to
+        400 keys, 1.01 to 1.06 from 500 on, 16 of 12 heads over 1,000 16.4 / 15.6; in several parts 0.97 to 1.04, where the
+        weights are more than one round 1.02 to 1.04.)"""
+        visible = self._visible(max_kv_len)
+        return (waves == 4 and visible > 128) or (waves == 16 and (parts > 1 or visible > 512))
 
     def _range_records(self, ctx):
         """Scratch for one record per (token, head, key range): always asked for at its largest

@@ -91,6 +91,11 @@ def test_attention_and_projection_in_one_launch(monkeypatch):
     assert _part(12)._one_launch_decode(8, 512) == (2, 8) and _part(12)._one_launch_decode(16, 1024) == (1, 16)
     assert _part(12)._one_launch_decode(1, 1024) == (4, 16) and _part(12)._one_launch_decode(1, 2048) is None
     assert _part(12)._one_launch_decode(24, 512) == (2, 4) and _part(12)._one_launch_decode(24, 1024) is None
+    # the weights in front of the keys where a wave takes several turns over them
+    assert not _part(12)._weights_first(3, 4, 128) and _part(12)._weights_first(2, 4, 256)
+    assert not _part(12, window=64)._weights_first(7, 4, 1024) and not _part(12)._weights_first(2, 8, 512)
+    assert not _part(12)._weights_first(1, 16, 512) and _part(12)._weights_first(1, 16, 1024)
+    assert _part(25)._weights_first(3, 16, 256)
     # wide models
     for keys in (128, 256, 512):
         for count in (5, 6, 7, 8):
