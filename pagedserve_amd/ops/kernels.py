@@ -1873,7 +1873,8 @@ def silu_gate(gu, out, activation="silu", form=PLAIN_GATE, row_scale=None):
 
 # Up to so many rows the gate runs inside its product (csrc/gemm_skinny_gated.hip), up to the second number over a k of
 # at most 1,024 and fewer than 16,384 columns.  Every block of 16 rows reads the weights anew: 64 x (2 x 4096) x 1024
-# 9.9 us, the two launches 14.6, but 48 x (2 x 6400) x 1600, where the product is the tiled one, 20.7 and 15.2.
+# 9.9 us, the two launches 14.6, but 48 x (2 x 6400) x 1600, where the product is the tiled one, 20.7 and 15.2.  Up to
+# 16 rows one launch is ahead at every width: 8 x (2 x 8192) x 1024 8.5 and 10.6, 16 x (2 x 11008) x 4096 37.8 and 39.6.
 GATED_PRODUCT_ROWS = (16, 64)
 
 
