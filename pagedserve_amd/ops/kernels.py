@@ -1874,7 +1874,10 @@ def silu_gate(gu, out, activation="silu", form=PLAIN_GATE, row_scale=None):
 # Up to so many rows the gate runs inside its product (csrc/gemm_skinny_gated.hip), up to the second number over a k of
 # at most 1,024 and fewer than 16,384 columns.  Every block of 16 rows reads the weights anew: 64 x (2 x 4096) x 1024
 # 9.9 us, the two launches 14.6, but 48 x (2 x 6400) x 1600, where the product is the tiled one, 20.7 and 15.2.  Up to
-# 16 rows one launch is ahead at every width: 8 x (2 x 8192) x 1024 8.5 and 10.6, 16 x (2 x 11008) x 4096 37.8 and 39.6.
+# 16 rows over a k of at most 3,072 one launch is ahead at every width (8 x (2 x 8192) x 1024 8.5 and 10.6).  Over a longer
+# one its blocks walk k in more rounds than those of the two launches, which are twice as many: ahead only where its
+# blocks, 16 columns each, fill one round of the units to five eighths or come to seven quarters of it (8 x (2 x 3072) x
+# 4096 0.77 of the two, 16 x (2 x 11008) x 4096 0.95; but 8 x (2 x 2048) x 4096 1.09, 8 x (2 x 1024) x 8192 1.2 to 1.3).
 GATED_PRODUCT_ROWS = (16, 64)
 
 
@@ -1884,6 +1887,10 @@ def gated_product_rows(w, packed) -> int:
     n, k = w.shape
     if packed is None or n % 32 != 0 or w.dtype != torch.bfloat16:
         return 0
+    if k > 3072:
+        blocks, units = n // 32, compute_units()
+        if not (5 * units <= 8 * blocks <= 8 * units or 4 * blocks >= 7 * units):
+            return 0
     return GATED_PRODUCT_ROWS[1 if k <= 1024 and n < 16384 else 0]
 
 

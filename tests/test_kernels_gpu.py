@@ -1467,6 +1467,21 @@ def test_gate_in_the_product_of_few_rows(m, inner, k, activation, form):
     assert bool((out == -7.0).all())
 
 
+@pytest.mark.parametrize("inner,k,rows", [(2048, 3072, 16), (2048, 4096, 0), (1024, 8192, 0), (2560, 4096, 16), (4096, 6144, 16),
+                                          (4608, 4096, 0), (7168, 4096, 16), (512, 1024, 64), (512, 1088, 16)])
+def test_where_the_gate_stays_out_of_its_product(inner, k, rows):
+    """Over a long k the two launches are ahead unless the blocks of the one fill the units."""
+    from pagedserve_amd.ops import kernels
+
+    if kernels.compute_units() != 256:
+        pytest.skip("the lines are drawn for 256 compute units")
+    w = torch.zeros((2 * inner, k), dtype=torch.bfloat16, device="cuda")
+    packed = kernels.pack_decode_weight(w)
+    assert kernels.gated_product_rows(w, packed) == rows
+    x, out = w.new_zeros((8, k)), w.new_empty((8, inner))
+    assert kernels.linear_gated(x, w, out, packed) == (rows > 0)
+
+
 @pytest.mark.parametrize("m,n,k", [(256, 640, 256), (300, 1000, 320), (1, 1, 256), (129, 65, 384), (700, 1601, 448), (513, 321, 1600)])
 @pytest.mark.parametrize("tile", [11, 12, 13, 22])
 @pytest.mark.parametrize("epilogue,dtype", LARGE_EPILOGUES)
