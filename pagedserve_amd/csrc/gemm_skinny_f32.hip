@@ -201,7 +201,7 @@ __global__ __launch_bounds__(512) void gemm_nt_skinny_norm_f32_kernel(
     }
   };
   f32x4 wf[UNROLL][2];
-  auto load_rest = [&] {
+  auto load_scale = [&] {
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) {
       const int col = (lane + i * 64) * 4;
@@ -210,6 +210,8 @@ __global__ __launch_bounds__(512) void gemm_nt_skinny_norm_f32_kernel(
       *reinterpret_cast<float4*>(b[i]) = *reinterpret_cast<const float4*>(shift + safe);
     }
     __builtin_amdgcn_sched_barrier(0);
+  };
+  auto load_weights = [&] {
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u)
 #pragma unroll
@@ -250,17 +252,22 @@ __global__ __launch_bounds__(512) void gemm_nt_skinny_norm_f32_kernel(
       *reinterpret_cast<f32x4*>(rows + r * STRIDE + col) = y;
     }
   };
-  // (two paths, so that the waits of each know how many loads are behind the ones they wait for)
+  // (paths of their own, so that the waits of each know how many loads are behind the ones they wait for; a wave
+  // without a row asks for weights alone: 4 x 6144 x 1000, where units have more than one block, 10.3 and 9.7 us)
   if (two) {
     load_row(0);
     load_row(1);
-    load_rest();
+    load_scale();
+    load_weights();
     finish_row(0);
     finish_row(1);
-  } else {
+  } else if (wave < m) {
     load_row(0);
-    load_rest();
+    load_scale();
+    load_weights();
     finish_row(0);
+  } else {
+    load_weights();
   }
 #pragma unroll
   for (int u = 0; u < UNROLL; ++u)
