@@ -19,8 +19,9 @@
 // keys per block a portion of 300 tokens at 12 heads of 64 took 55 us, now 17; 512 tokens 86 and 21, 2 x 1,024
 // tokens 179 and 64 (a third of the time the matrix cores are busy).
 //
-// The tiles are those of the bfloat16 kernel (`tile_item`, `tile_q0`: the item of each tile of 64 queries and
-// its first query within the item's tokens of this step), two blocks each, and so are the rules: query i of an
+// The tiles are those of the bfloat16 kernel (`tile_item`, `tile_q0`: the item of each tile and its first query within
+// the item's tokens of this step), of 32 queries or of 64, which are two blocks or one (ops/kernels.py says where), and so
+// are the rules: query i of an
 // item whose cached length after the step is L and which brings n tokens stands at position
 // L - n + i and sees keys first_visible_key(position, window) .. position.
 //
@@ -39,8 +40,8 @@
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float af_f32x4;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float af_f32x16;
 
-// DF: 32 head dimensions each; RAGGED: the head size is not 32 DF; PAIRS: one block takes the 64 queries of a tile
-// whose keys are at most 64
+// DF: 32 head dimensions each; RAGGED: the head size is not 32 DF; PAIRS: one block takes the 64 queries of a tile,
+// two waves to 32 of them; `parts`: else, blocks to a listed tile (of 32 queries each)
 template <int DF, bool RAGGED, bool PAIRS>
 __global__ __launch_bounds__(64 * AF_WAVES) void attention_tiled_f32_kernel(
     const float* __restrict__ q, int64_t q_stride, const float* __restrict__ k_pool,
@@ -48,7 +49,7 @@ __global__ __launch_bounds__(64 * AF_WAVES) void attention_tiled_f32_kernel(
     const int* __restrict__ tile_item, const int* __restrict__ tile_q0,
     const int* __restrict__ cu_tokens, const int* __restrict__ kv_lens,
     const int* __restrict__ tables, int table_width, int heads, int kv_heads, int head_dim,
-    int page_size, int num_pages, float scale, int window, const AttnExtras extra) {
+    int page_size, int num_pages, float scale, int window, int parts, const AttnExtras extra) {
   constexpr int STEPS = 4 * DF;                 // pieces of 2 x 4 dimensions of a score
   constexpr int STRIDE = 32 * DF + 4;           // floats from query to query of a wave's result
   __shared__ __attribute__((aligned(16))) float s_out[AF_WAVES * AF_ROWS * STRIDE];
@@ -59,10 +60,11 @@ __global__ __launch_bounds__(64 * AF_WAVES) void attention_tiled_f32_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int column = lane & 31;                 // the lane's query, and its key when keys are read
   const int half = lane >> 5;
-  // An item's later queries see more keys: its last tiles go first, so that no long block is left for the end.
-  const int index = gridDim.x - 1 - blockIdx.x;
-  const int tile_index = index / (2 * heads);
-  const int part = (index - tile_index * 2 * heads) / heads;   // which 32 queries of the listed tile
+  // (the lists begin with the tiles that see the most keys, and so do the blocks, the later half of a tile first: with the
+  // longest at the end prompts of 500, 20, 35, 800 and 64 tokens at 16 heads of 64 take 56 us, this way 40)
+  const int index = blockIdx.x;
+  const int tile_index = index / (parts * heads);
+  const int part = parts - 1 - (index - tile_index * parts * heads) / heads;   // which 32 queries of the listed tile
   const int head = index % heads;
   const int kv_head = head / (heads / kv_heads);
 
@@ -72,15 +74,11 @@ __global__ __launch_bounds__(64 * AF_WAVES) void attention_tiled_f32_kernel(
   const int count = cu_tokens[item + 1] - tok0;
   const int start = kv_lens[item] - count;      // position of the portion's first token
   const int* table = tables + (int64_t)item * table_width;
-  const int tile_last = tile_q + AF_TILE - 1 < count ? tile_q + AF_TILE - 1 : count - 1;
-  // two waves to 32 queries where the keys are no more than two turns: four would leave two of them without any
-  const bool paired =
-      PAIRS && start + tile_last + 1 - first_visible_key(start + tile_q, window) <= 2 * AF_ROWS;
-  const int turns = paired ? 2 : AF_WAVES;      // waves that share the keys of 32 queries
-  const int turn = paired ? wave & 1 : wave;    // which of them this one is
+  constexpr int TURNS = PAIRS ? 2 : AF_WAVES;   // waves that share the keys of 32 queries
+  const int turn = PAIRS ? wave & 1 : wave;     // which of them this one is
   const int first_q = tile_q + part * AF_ROWS;  // of the block
-  if (first_q >= count || (paired && part != 0)) return;      // (the whole block)
-  const int q0 = paired ? first_q + (wave >> 1) * AF_ROWS : first_q;
+  if (first_q >= count) return;                 // (the whole block)
+  const int q0 = PAIRS ? first_q + (wave >> 1) * AF_ROWS : first_q;
   const int last_q = q0 + AF_ROWS - 1 < count ? q0 + AF_ROWS - 1 : count - 1;
   const int key_begin = first_visible_key(start + q0, window);
   const int key_end = q0 < count ? start + last_q + 1 : key_begin;
@@ -153,7 +151,7 @@ __global__ __launch_bounds__(64 * AF_WAVES) void attention_tiled_f32_kernel(
 
   int k0 = key_begin + turn * AF_ROWS;
   if (k0 < key_end) {
-    const int TURN = turns * AF_ROWS;
+    constexpr int TURN = TURNS * AF_ROWS;
     int64_t row = row_of(k0, page_of(k0));
     load_keys(row);
     int next_page = page_of(k0 + TURN);
@@ -252,38 +250,34 @@ __global__ __launch_bounds__(64 * AF_WAVES) void attention_tiled_f32_kernel(
   }
   __syncthreads();
   // eight threads to a query, four where the block has 64 of them
-  const int shift = paired ? 2 : 3;
-  const int row = tid >> shift;
-  const int part_of_query = tid - (row << shift);
-  const int first = paired ? (row >> 5) * 2 * AF_ROWS + (row & 31) : row;   // the query in its first wave's results
+  constexpr int SHARE = PAIRS ? 4 : 8;
+  const int row = tid / SHARE;
+  const int first = PAIRS ? (row >> 5) * 2 * AF_ROWS + (row & 31) : row;   // the query in its first wave's results
   if (first_q + row >= count) return;
   float total_max = -INFINITY;
 #pragma unroll
-  for (int w = 0; w < AF_WAVES; ++w)
-    if (w < turns) total_max = fmaxf(total_max, s_max[w * AF_ROWS + first]);
-  float factor[AF_WAVES], total = 0.f;
+  for (int w = 0; w < TURNS; ++w) total_max = fmaxf(total_max, s_max[w * AF_ROWS + first]);
+  float factor[TURNS], total = 0.f;
 #pragma unroll
-  for (int w = 0; w < AF_WAVES; ++w) {
-    if (w >= turns) continue;
+  for (int w = 0; w < TURNS; ++w) {
     const float wave_max = s_max[w * AF_ROWS + first];
     factor[w] = wave_max == -INFINITY ? 0.f : expf(wave_max - total_max);
     total += s_sum[w * AF_ROWS + first] * factor[w];
   }
   if (extra.logistic != nullptr) {
 #pragma unroll
-    for (int w = 0; w < AF_WAVES; ++w) factor[w] = 1.f;
+    for (int w = 0; w < TURNS; ++w) factor[w] = 1.f;
     total = extra.logistic_norm;
   }
   const float inverse = (total != 0.f ? 1.f / total : 0.f) * gate_factor(extra, tok0 + first_q + row, head);
   float* to = out + (int64_t)(tok0 + first_q + row) * out_stride + (int64_t)head * head_dim;
 #pragma unroll
-  for (int v = 0; v < 2 * DF; ++v) {
-    const int dim = 4 * part_of_query + ((4 * v) << shift);
-    if (dim >= head_dim) continue;
+  for (int v = 0; v < 8 * DF / SHARE; ++v) {
+    const int dim = 4 * (tid % SHARE) + 4 * SHARE * v;
+    if (RAGGED && dim >= head_dim) continue;
     float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-    for (int w = 0; w < AF_WAVES; ++w) {
-      if (w >= turns) continue;
+    for (int w = 0; w < TURNS; ++w) {
       const float4 value = *reinterpret_cast<const float4*>(s_out + (w * AF_ROWS + first) * STRIDE + dim);
       sum.x = fmaf(factor[w], value.x, sum.x);
       sum.y = fmaf(factor[w], value.y, sum.y);
@@ -309,7 +303,7 @@ extern "C" int ps_attention_tiled_f32(const void* q, int64_t q_stride, const voi
                                       int page_size, int num_pages, float scale, int window,
                                       const float* sink, const float* gate, int64_t gate_ld,
                                       float softcap, const float* logistic, float logistic_norm,
-                                      void* stream) {
+                                      int query_tile, int paired, void* stream) {
   PS_REQUIRE(tiles >= 0 && heads > 0 && kv_heads > 0 && page_size > 0 && num_pages > 0 &&
                  table_width > 0,
              "ps_attention_tiled_f32: bad sizes");
@@ -323,18 +317,16 @@ extern "C" int ps_attention_tiled_f32(const void* q, int64_t q_stride, const voi
                  ((uintptr_t)out % 16) == 0 && ((uintptr_t)k_pool % 16) == 0 &&
                  ((uintptr_t)v_pool % 16) == 0,
              "ps_attention_tiled_f32: rows of q, out and the pools must allow 16-byte accesses");
-  const int64_t blocks = (int64_t)tiles * heads * (AF_TILE / AF_ROWS);
+  PS_REQUIRE(query_tile == AF_TILE || query_tile == AF_ROWS,
+             "ps_attention_tiled_f32: tiles of %d or %d queries, not %d", AF_TILE, AF_ROWS, query_tile);
+  PS_REQUIRE(!paired || (query_tile == AF_TILE && head_dim > 32 && head_dim <= 64),
+             "ps_attention_tiled_f32: one block takes a tile of %d queries with heads of 33 to 64 only", AF_TILE);
+  const int parts = paired ? 1 : query_tile / AF_ROWS;
+  const int64_t blocks = (int64_t)tiles * heads * parts;
   PS_REQUIRE(blocks < ((int64_t)1 << 31), "ps_attention_tiled_f32: too many blocks");
   if (blocks == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
   const AttnExtras extra = {sink, gate, gate_ld, softcap, logistic, logistic_norm};
-  // Short portions.  Of the two blocks of a tile of 33 to 64 keys one has a wave with keys, the other two; that the
-  // others are idle costs nothing while the blocks are on the chip at once, two to a unit with heads of 33 to 64.
-  // Beyond that one block takes both halves, two waves each (us; before these tiles, two blocks, one: 128 portions of
-  // 40 tokens at 12 heads of 64 49, 57 and 50, of 64 tokens 53, 61 and 53, 24 of 40 16.3, 16.5 and 13.5; but 8 of 40 8.9 and 9.4).
-  // Narrower heads fit three blocks into a unit and lose by it (128 of 64 tokens at 4 heads of 32 14.3 and 16.7), wider
-  // ones, one block to a unit, too (at 16 heads of 128 182 and 198; 192 before).
-  const bool pairs = head_dim > 32 && head_dim <= 64 && blocks > 2 * (int64_t)ps_compute_units();
 #define PS_LAUNCH_AF(DF)                                                                          \
   do {                                                                                            \
     if (head_dim == 32 * DF)                                                                      \
@@ -347,11 +339,11 @@ extern "C" int ps_attention_tiled_f32(const void* q, int64_t q_stride, const voi
                      dim3(64 * AF_WAVES), 0, s,                                                   \
                      (const float*)q, q_stride, (const float*)k_pool, (const float*)v_pool,       \
                      (float*)out, out_stride, tile_item, tile_q0, cu_tokens, kv_lens, tables,     \
-                     table_width, heads, kv_heads, head_dim, page_size, num_pages, scale, window, extra)
+                     table_width, heads, kv_heads, head_dim, page_size, num_pages, scale, window, parts, extra)
   switch ((head_dim + 31) / 32) {
     case 1: PS_LAUNCH_AF(1); break;
     case 2:
-      if (!pairs) PS_LAUNCH_AF(2);
+      if (!paired) PS_LAUNCH_AF(2);
       else if (head_dim == 64) PS_LAUNCH_AF_FORM(2, false, true);
       else PS_LAUNCH_AF_FORM(2, true, true);
       break;

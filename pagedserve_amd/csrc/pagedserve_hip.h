@@ -140,9 +140,10 @@ int ps_attention_rowwise(const void* q, int64_t q_stride, const void* k_pool, co
                          float logistic_norm, int dtype, void* stream);
 
 // The same result in true 32-bit for the items of several tokens (prompt portions), a block
-// of four waves per (tile of ps_attention_tiled_f32_tile() queries, head): float pools, float
-// q and out, keys and values through LDS, scores by plain fused multiply-adds.  The tiles are
-// listed as for ps_attention_prefill (item and first query of each, cut at the tile size).
+// of four waves per (32 queries, head): float pools, float q and out, true 32-bit products on the
+// matrix cores.  The tiles are listed as for ps_attention_prefill (item and first query of each, cut at
+// query_tile = 32, or 64 = ps_attention_tiled_f32_tile() queries, which are two blocks or, `paired` and
+// with heads of 33 to 64, one).
 // head_dim a multiple of 4 up to 128 (ps_attention_tiled_f32_supported); 16-byte aligned rows.
 int ps_attention_tiled_f32_supported(int head_dim);
 int ps_attention_tiled_f32_tile();
@@ -152,7 +153,7 @@ int ps_attention_tiled_f32(const void* q, int64_t q_stride, const void* k_pool, 
                            int table_width, int heads, int kv_heads, int head_dim, int page_size,
                            int num_pages, float scale, int window, const float* sink, const float* gate,
                            int64_t gate_ld, float softcap, const float* logistic,
-                         float logistic_norm, void* stream);
+                         float logistic_norm, int query_tile, int paired, void* stream);
 
 // The same result for single queries, with each token's keys cut into `splits` ranges that
 // run as separate blocks of `waves` (4 or 16) waves; `partial` is scratch of

@@ -461,11 +461,14 @@ class Attention(Mixer):
             # 32-bit: tiles of queries too, in true 32-bit arithmetic.  The tiles hold the items
             # of several tokens; one-token items that the split-KV kernel did not take (a head
             # size that it refuses) go to the kernel that takes all sizes
-            tile_item, tile_q0 = ctx.query_tiles[kernels.PREFILL_TILE]
-            if tile_item.numel():
-                kernels.attention_tiled_f32(q, cache.k_pool, cache.v_pool, context, tile_item, tile_q0,
+            tiles = ctx.query_tiles[kernels.PREFILL_TILE][0].numel()
+            if tiles:
+                size, paired = kernels.tiled_f32_shape(self.heads, self.head_dim, tiles,
+                                                       ctx.query_tiles[kernels.PREFILL_SMALL_TILE][0].numel(), ctx.max_kv_len)
+                kernels.attention_tiled_f32(q, cache.k_pool, cache.v_pool, context, *ctx.query_tiles[size],
                                             ctx.cu_tokens, ctx.kv_lens, tables, self.heads, self.scale,
-                                            self.span, sink=sink, gate=gates, softcap=self.score_cap, logistic=self.logistic)
+                                            self.span, sink=sink, gate=gates, softcap=self.score_cap, logistic=self.logistic,
+                                            query_tile=size, paired=paired)
             if not singles and ctx.single_tokens is not None and ctx.single_tokens.numel():
                 kernels.attention_rowwise(q, cache.k_pool, cache.v_pool, context, ctx.tok_item,
                                           ctx.positions, tables, self.heads, self.scale, self.span,

@@ -1,6 +1,7 @@
 """Each HIP kernel alone against a plain float64 torch formula, at sizes that differ
 from the engine's tiny models (ragged widths, odd row counts, head sizes 16..128)."""
 
+import itertools
 import math
 
 import pytest
@@ -814,32 +815,34 @@ def test_attention_tiled_f32(heads, kv_heads, head_dim, page_size, window):
                                                                 (16, 2, 32, 16)])
 @pytest.mark.parametrize("window", [0, 20])
 def test_attention_tiled_f32_of_many_short_portions(heads, kv_heads, head_dim, page_size, window):
-    """So many portions of 1 to 65 tokens, fresh and behind some keys, that heads of 33 to 64 take tiles of up to 64 keys
-    in one block, beside tiles of more keys in the same launch; other heads take two."""
+    """So many portions of 1 to 65 tokens, fresh and behind some keys, that the blocks are not on the chip at once: tiles of
+    64 queries in two blocks, of 32, and, heads of 33 to 64, of 64 in one, whose keys may be more than its waves take
+    in a turn."""
     from pagedserve_amd.ops import kernels
 
     items = [(0, 64), (0, 33), (0, 32), (31, 33), (32, 33), (0, 65), (200, 64), (3, 1), (0, 2), (62, 2), (20, 40), (0, 63)] * 4
+    forms = [(64, False), (32, False)] + ([(64, True)] if 32 < head_dim <= 64 else [])
     totals = [past + new for past, new in items]
     k_pool, v_pool, tables = _paged_fixture(torch.float32, totals, kv_heads, head_dim, page_size, 56)
     q = _rand((sum(new for _, new in items), heads * head_dim), torch.float32, 57)
-    tok_item, tok_pos, tile_item, tile_q0, cu = [], [], [], [], [0]
+    tok_item, tok_pos, cu = [], [], [0]
     for index, (past, new) in enumerate(items):
         tok_item += [index] * new
         tok_pos += list(range(past, past + new))
         cu.append(cu[-1] + new)
-        tile_item += [index] * -(-new // 64)
-        tile_q0 += range(0, new, 64)
-    assert 2 * len(tile_item) * heads > 2 * kernels.compute_units()
 
     def dev(values):
         return torch.tensor(values, dtype=torch.int32, device="cuda")
 
     scale = head_dim ** -0.5
     sink = _rand((heads,), torch.float32, 58)
-    for with_sink in (None, sink):
+    for (size, paired), with_sink in itertools.product(forms, (None, sink)):
+        tiles = [(index, at) for index, (_, new) in enumerate(items) for at in range(0, new, size)]
+        assert len(tiles) * heads > 2 * kernels.compute_units()
         out, rowwise = torch.full_like(q, float("nan")), torch.full_like(q, float("nan"))
-        kernels.attention_tiled_f32(q, k_pool, v_pool, out, dev(tile_item), dev(tile_q0), dev(cu), dev(totals), tables,
-                                    heads, scale, window=window, sink=with_sink)
+        kernels.attention_tiled_f32(q, k_pool, v_pool, out, dev([index for index, _ in tiles]), dev([at for _, at in tiles]),
+                                    dev(cu), dev(totals), tables, heads, scale, window=window, sink=with_sink,
+                                    query_tile=size, paired=paired)
         kernels.attention_rowwise(q, k_pool, v_pool, rowwise, dev(tok_item), dev(tok_pos), tables, heads, scale,
                                   window=window, sink=with_sink)
         torch.testing.assert_close(out, rowwise, atol=2e-5, rtol=2e-5)
@@ -863,6 +866,12 @@ def test_attention_tiled_f32_refuses_what_it_cannot_take():
         with pytest.raises(kernels.KernelError, match="multiple of 4 up to 128"):
             kernels.attention_tiled_f32(q, pool, pool.clone(), torch.zeros_like(q), index, index, cu, lens, tables,
                                         1, 1.0)
+    for head_dim, size, paired in ((64, 48, False), (64, 128, False), (64, 32, True), (32, 64, True), (68, 64, True)):
+        q = torch.zeros((2, head_dim), device="cuda")
+        pool = torch.zeros((4, 1, 8, head_dim), device="cuda")
+        with pytest.raises(kernels.KernelError, match="tile"):
+            kernels.attention_tiled_f32(q, pool, pool.clone(), torch.zeros_like(q), index, index, cu, lens, tables,
+                                        1, 1.0, query_tile=size, paired=paired)
     q = torch.zeros((2, 64), device="cuda", dtype=torch.bfloat16)
     pool = torch.zeros((4, 1, 8, 64), device="cuda", dtype=torch.bfloat16)
     with pytest.raises(kernels.KernelError):
