@@ -319,8 +319,8 @@ extern "C" int ps_attention_tiled_f32(const void* q, int64_t q_stride, const voi
              "ps_attention_tiled_f32: rows of q, out and the pools must allow 16-byte accesses");
   PS_REQUIRE(query_tile == AF_TILE || query_tile == AF_ROWS,
              "ps_attention_tiled_f32: tiles of %d or %d queries, not %d", AF_TILE, AF_ROWS, query_tile);
-  PS_REQUIRE(!paired || (query_tile == AF_TILE && head_dim > 32 && head_dim <= 64),
-             "ps_attention_tiled_f32: one block takes a tile of %d queries with heads of 33 to 64 only", AF_TILE);
+  PS_REQUIRE(!paired || query_tile == AF_TILE, "ps_attention_tiled_f32: one block takes a tile of %d queries, not of %d",
+             AF_TILE, query_tile);
   const int parts = paired ? 1 : query_tile / AF_ROWS;
   const int64_t blocks = (int64_t)tiles * heads * parts;
   PS_REQUIRE(blocks < ((int64_t)1 << 31), "ps_attention_tiled_f32: too many blocks");
@@ -329,10 +329,10 @@ extern "C" int ps_attention_tiled_f32(const void* q, int64_t q_stride, const voi
   const AttnExtras extra = {sink, gate, gate_ld, softcap, logistic, logistic_norm};
 #define PS_LAUNCH_AF(DF)                                                                          \
   do {                                                                                            \
-    if (head_dim == 32 * DF)                                                                      \
-      PS_LAUNCH_AF_FORM(DF, false, false);                                                        \
-    else                                                                                          \
-      PS_LAUNCH_AF_FORM(DF, true, false);                                                         \
+    if (head_dim == 32 * DF && paired) PS_LAUNCH_AF_FORM(DF, false, true);                        \
+    else if (head_dim == 32 * DF) PS_LAUNCH_AF_FORM(DF, false, false);                            \
+    else if (paired) PS_LAUNCH_AF_FORM(DF, true, true);                                           \
+    else PS_LAUNCH_AF_FORM(DF, true, false);                                                      \
   } while (0)
 #define PS_LAUNCH_AF_FORM(DF, RAGGED, PAIRS)                                                      \
   hipLaunchKernelGGL((attention_tiled_f32_kernel<DF, RAGGED, PAIRS>), dim3((unsigned)blocks),     \
@@ -342,11 +342,7 @@ extern "C" int ps_attention_tiled_f32(const void* q, int64_t q_stride, const voi
                      table_width, heads, kv_heads, head_dim, page_size, num_pages, scale, window, parts, extra)
   switch ((head_dim + 31) / 32) {
     case 1: PS_LAUNCH_AF(1); break;
-    case 2:
-      if (!paired) PS_LAUNCH_AF(2);
-      else if (head_dim == 64) PS_LAUNCH_AF_FORM(2, false, true);
-      else PS_LAUNCH_AF_FORM(2, true, true);
-      break;
+    case 2: PS_LAUNCH_AF(2); break;
     case 3: PS_LAUNCH_AF(3); break;
     default: PS_LAUNCH_AF(4); break;
   }

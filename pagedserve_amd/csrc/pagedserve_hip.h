@@ -142,8 +142,7 @@ int ps_attention_rowwise(const void* q, int64_t q_stride, const void* k_pool, co
 // The same result in true 32-bit for the items of several tokens (prompt portions), a block
 // of four waves per (32 queries, head): float pools, float q and out, true 32-bit products on the
 // matrix cores.  The tiles are listed as for ps_attention_prefill (item and first query of each, cut at
-// query_tile = 32, or 64 = ps_attention_tiled_f32_tile() queries, which are two blocks or, `paired` and
-// with heads of 33 to 64, one).
+// query_tile = 32, or 64 = ps_attention_tiled_f32_tile() queries, which are two blocks or, `paired`, one).
 // head_dim a multiple of 4 up to 128 (ps_attention_tiled_f32_supported); 16-byte aligned rows.
 int ps_attention_tiled_f32_supported(int head_dim);
 int ps_attention_tiled_f32_tile();

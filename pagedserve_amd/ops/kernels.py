@@ -1111,18 +1111,16 @@ def tiled_f32_shape(heads, head_dim, tiles, small_tiles, max_kv_len):
     """(``query_tile``, ``paired``) with which ``attention_tiled_f32`` takes a step whose portions are ``tiles`` tiles of 64
     queries or ``small_tiles`` of 32.  A tile of 64 is two blocks, which read the same keys side by side (32 portions of
     64 tokens behind 64 at 16 heads of 128 55 us, as tiles of 32 59); where most tiles end in their first half, every
-    other block would start for nothing, and the tiles of 32 are taken (64 portions of 2 tokens at 3 heads of 100 22 us, 17).
+    other block would start for nothing, and the tiles of 32 are taken (64 portions of 2 tokens at 3 heads of 100 22 us, 12).
 
     Paired: the keys of 32 queries are shared out to the four waves of a block, 32 to a turn; where no request has more
-    than 64, two of them have none.  That costs nothing while the blocks are on the chip at once, two to a unit with heads of
-    33 to 64; beyond, one block takes both halves of a tile, two waves each (us; one block for 64 queries, plain
-    multiply-adds, before these tiles; two blocks; one: 128 portions of 40 tokens at 12 heads of 64 49, 57 and 50, of 64 tokens
-    53, 61 and 53, 24 of 40 16.3, 16.5 and 13.5; but 8 of 40 8.9 and 9.4).  Narrower heads fit three blocks into a unit
-    and lose by it (128 of 64 tokens at 4 heads of 32 14.3 and 16.7), wider ones, one block to a unit, too (at 16 heads
-    of 128 182 and 198; 192 before)."""
-    if 32 < head_dim <= 64 and max_kv_len <= 64 and small_tiles * heads > 2 * compute_units():
-        return PREFILL_TILE, True
-    return (PREFILL_SMALL_TILE if 4 * small_tiles <= 5 * tiles else PREFILL_TILE), False
+    than 64, two of them have none.  That costs nothing while every block has a compute unit to itself; beyond, one block takes
+    both halves of a tile, two waves each (us, two blocks and one: 128 portions of 40 tokens at 12 heads of 64 57 and 37, 16
+    of 64 13.1 and 10.4, but 8 of 64 9.4 and 10.0; 12 of 64 at 16 heads of 128 23.7 and 15.4, 8 of 64 13.0 and 14.8; 64 of 64 at
+    4 heads of 32 10.0 and 7.8, 32 7.3 and 7.6)."""
+    if 4 * small_tiles <= 5 * tiles:
+        return PREFILL_SMALL_TILE, False
+    return PREFILL_TILE, max_kv_len <= 64 and small_tiles * heads > compute_units()
 
 
 def attention_tiled_f32(q, k_pool, v_pool, out, tile_item, tile_q0, cu_tokens, kv_lens, tables, heads,
@@ -1132,7 +1130,7 @@ def attention_tiled_f32(q, k_pool, v_pool, out, tile_item, tile_q0, cu_tokens, k
     ``PREFILL_SMALL_TILE``) per listed tile: keys and values are read once per 32 queries instead of once per query
     (``attention_rowwise``), scores and sums are true 32-bit arithmetic.  The tile list is the
     one of ``attention_prefill`` at that size; tiles of 64 are two blocks (one of which has nothing to do where
-    a tile ends in its first half), or one (``paired``, heads of 33 to 64; see ``tiled_f32_shape``)."""
+    a tile ends in its first half), or one (``paired``; see ``tiled_f32_shape``)."""
     global _TILED_F32_CHECKED
     if not _TILED_F32_CHECKED:
         lib = load_library()

@@ -82,13 +82,14 @@ def test_documented_cases(monkeypatch):
 
 
 def test_tiles_of_short_portions_in_32_bit(monkeypatch):
-    """One block to a tile of 64 queries: heads of 33 to 64, at most 64 keys, more blocks than two per unit.  Tiles of
-    32 where most of those of 64 would be half empty."""
+    """One block to a tile of 64 queries: at most 64 keys, more halves of tiles than units.  Tiles of 32 where most of
+    those of 64 would be half empty."""
     monkeypatch.setattr(kernels, "compute_units", lambda: 256)
-    assert kernels.tiled_f32_shape(12, 64, 22, 43, 64) == (64, True) and kernels.tiled_f32_shape(12, 64, 21, 42, 64) == (64, False)
-    assert kernels.tiled_f32_shape(12, 64, 50, 100, 65) == (64, False)
-    for head_dim in (32, 68):
-        assert kernels.tiled_f32_shape(12, head_dim, 50, 100, 64) == (64, False)
+    for head_dim in (16, 64, 128):
+        assert kernels.tiled_f32_shape(12, head_dim, 11, 22, 64) == (64, True)
+        assert kernels.tiled_f32_shape(12, head_dim, 11, 21, 64) == (64, False)
+        assert kernels.tiled_f32_shape(12, head_dim, 50, 100, 65) == (64, False)
+        assert kernels.tiled_f32_shape(12, head_dim, 50, 50, 20) == (32, False)
     assert kernels.tiled_f32_shape(12, 64, 4, 5, 300) == (32, False) and kernels.tiled_f32_shape(12, 64, 4, 6, 300) == (64, False)
 
 
