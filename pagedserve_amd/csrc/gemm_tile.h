@@ -92,21 +92,30 @@ __device__ inline void store_wave_tile(f32x16 (&acc)[WM][WN], float* region, int
   constexpr int EP_ROWS = 64 / EP_CHUNKS;         // rows per pass of the wave
   const int chunk = lane % EP_CHUNKS;
   const int row_in_pass = lane / EP_CHUNKS;
-  const int col0 = col_base + chunk * 8;
+  // The piece that the end of the rows lies in begins further left where that is aligned and within the wave's columns
+  // (float rows of whole fours): both pieces then write the same values to the columns that they share.
+  const bool reaches_back = sizeof(TOut) == 4 && (n & 3) == 0 && n - col_base >= 8;
+  const int first = col_base + chunk * 8;
+  const int col0 = reaches_back && first < n && first + 8 > n ? n - 8 : first;
   const bool vec_c = ldc % (16 / (int)sizeof(TOut)) == 0 && (reinterpret_cast<uintptr_t>(c) & 15u) == 0;
   constexpr bool PLAIN = EPI == PS_EPI_NONE;
-  // eight key or value columns lie in one head, and no piece ends behind n
+  const bool full = col0 + 8 <= n;
+  // eight key or value columns lie in one head (then n is whole pieces too)
   const bool whole_kv = !PLAIN || scatter.k_pool == nullptr ||
                         ((scatter.head_dim | scatter.q_cols | scatter.kv_cols) & 7) == 0;
-  const bool whole = (n & 7) == 0 || col_base + WN * 32 <= n;
-  const bool by_column = !vec_c || !whole || !whole_kv || k_splits > 1;
+  const bool by_column = !vec_c || !whole_kv || k_splits > 1;
   float b[8];
 #pragma unroll
   for (int q = 0; q < 8; ++q) b[q] = (bias && split == 0 && col0 + q < n) ? bias[col0 + q] : 0.f;
+  // otherwise the columns behind the last whole piece go eight rows at a time
+  const bool ends_inside =
+      !reaches_back && (n & 7) != 0 && (n & ~7) >= col_base && (n & ~7) < col_base + WN * 32;
+  const int last_col = (n & ~7) + (lane & 7);
+  const float last_bias = bias && split == 0 && ends_inside && last_col < n ? bias[last_col] : 0.f;
   // key and value columns also go into cache pages
   TOut* pool = nullptr;
   int64_t pool_offset = 0;
-  if (PLAIN && !by_column && scatter.k_pool != nullptr && col0 < n && col0 >= scatter.q_cols)
+  if (PLAIN && !by_column && scatter.k_pool != nullptr && full && col0 >= scatter.q_cols)
     pool = kv_scatter_col<TOut>(scatter, col0, &pool_offset);
 
   // What the whole pieces need from memory is asked for before the first of them: the residual rows, and
@@ -114,7 +123,7 @@ __device__ inline void store_wave_tile(f32x16 (&acc)[WM][WN], float* region, int
   constexpr int PASSES = 32 / EP_ROWS;
   constexpr bool RESIDUAL = EPI == PS_EPI_RESIDUAL;
   float4 old[RESIDUAL ? WM : 1][RESIDUAL ? PASSES : 1][2];
-  if (RESIDUAL && !by_column && col0 < n) {
+  if (RESIDUAL && !by_column && full) {
 #pragma unroll
     for (int i = 0; i < WM; ++i)
 #pragma unroll
@@ -153,8 +162,8 @@ __device__ inline void store_wave_tile(f32x16 (&acc)[WM][WN], float* region, int
             acc[i][j][e];
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     if (by_column) {
-      // rows that cannot leave in whole aligned pieces, heads that are no whole pieces, and partial sums of a
-      // split k: a wave's lanes take consecutive columns of one row
+      // rows that cannot leave in aligned pieces, heads that are no whole pieces, and partial sums of a split k: a
+      // wave's lanes take consecutive columns of one row
 #pragma unroll 8
       for (int r = 0; r < 32; ++r) {
         const int row = row_base + i * 32 + r;
@@ -184,9 +193,9 @@ __device__ inline void store_wave_tile(f32x16 (&acc)[WM][WN], float* region, int
     for (int pass = 0; pass < PASSES; ++pass) {
       const int r = pass * EP_ROWS + row_in_pass;
       const int row = row_base + i * 32 + r;
-      const float4 lo = *reinterpret_cast<const float4*>(region + r * EP_STRIDE + chunk * 8);
-      const float4 hi = *reinterpret_cast<const float4*>(region + r * EP_STRIDE + chunk * 8 + 4);
-      if (row >= m || col0 >= n) continue;
+      const float4 lo = *reinterpret_cast<const float4*>(region + r * EP_STRIDE + col0 - col_base);
+      const float4 hi = *reinterpret_cast<const float4*>(region + r * EP_STRIDE + col0 - col_base + 4);
+      if (row >= m || !full) continue;
       float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
 #pragma unroll
       for (int q = 0; q < 8; ++q) v[q] = finish_value<EPI, TOut>(v[q] + b[q]);
@@ -203,6 +212,19 @@ __device__ inline void store_wave_tile(f32x16 (&acc)[WM][WN], float* region, int
         if (!(PLAIN && pool != nullptr && scatter.cache_only)) store8(out, v);
         if constexpr (PLAIN)
           if (pool != nullptr && slots[i][pass] >= 0) store8(pool + slots[i][pass] + pool_offset, v);
+      }
+    }
+    if (ends_inside) {
+      // (in the passes this code would stand in every one)
+#pragma unroll 1
+      for (int t = 0; t < 4; ++t) {
+        const int r = t * 8 + (lane >> 3);
+        const int row = row_base + i * 32 + r;
+        if (row >= m || last_col >= n) continue;
+        const float v = finish_value<EPI, TOut>(region[r * EP_STRIDE + last_col - col_base] + last_bias);
+        TOut* out = c + (int64_t)row * ldc + last_col;
+        if constexpr (RESIDUAL) *reinterpret_cast<float*>(out) += v;
+        else *out = from_float<TOut>(v);
       }
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
