@@ -124,17 +124,19 @@ __device__ __forceinline__ void attention_decode_block(
   int base = range_begin + wave * KEYS_PER_WAVE;
   if constexpr (!std::is_same<Ahead, NothingAhead>::value) {
     // the first turn on its own, so that its waits know which loads are behind its own
-    if (base < range_end) {
-      constexpr bool FIRST = true;
+    auto turn = [&](const int base, auto first) {
+      constexpr bool FIRST = decltype(first)::value;
 #include "attention_decode_turn.h"
-    } else {
-      ahead();
-    }
+    };
+    if (base < range_end) turn(base, std::true_type{});
+    else ahead();
     base += AD_WAVES * KEYS_PER_WAVE;
-  }
-  for (; base < range_end; base += AD_WAVES * KEYS_PER_WAVE) {
-    constexpr bool FIRST = false;
+    for (; base < range_end; base += AD_WAVES * KEYS_PER_WAVE) turn(base, std::false_type{});
+  } else {
+    for (; base < range_end; base += AD_WAVES * KEYS_PER_WAVE) {
+      constexpr bool FIRST = false;
 #include "attention_decode_turn.h"
+    }
   }
   if (!has_dims) {
 #pragma unroll

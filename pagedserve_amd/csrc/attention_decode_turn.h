@@ -1,7 +1,8 @@
 // The body of the loop over keys in attention_decode_block.h: the keys base .. base + KEYS_PER_WAVE of a wave into its
-// running maximum, sum and values.  FIRST: `ahead` runs behind the loads.  It is text that stands inside the function, and not a
+// running maximum, sum and values.  FIRST: `ahead` runs behind the loads.  It is text that stands inside the loop and not a
 // lambda or a function of its own: as one of those, inlined, its addresses took twice as many multiplications and decode
-// attention 1 to 3 % longer (one request of 12 heads of 64 over 144 keys 5.76 us, this way 5.61).
+// attention 1 to 3 % longer (one request of 12 heads of 64 over 144 keys 5.76 us, this way 5.61).  Only the loop whose first
+// turn stands apart has it as a lambda, which is the faster there (with the projection, over 60 keys 4.22 us, as text 4.37).
     Raw8<T> kr[AD_UNROLL], vr[AD_UNROLL];
     bool valid[AD_UNROLL];
     // Every load is unconditional from a clamped address and masked afterwards, so that the

@@ -570,10 +570,13 @@ class Attention(Mixer):
         back.  (Keys and weights from memory, behind and in front, heads of 64: four waves within 128 keys 0.98 on
         average, 1 of 12 heads over 60 keys 4.37 / 4.40; beyond, where a wave takes several turns, 1.02 to 1.13, 24 requests of
         12 heads over 270 keys 13.3 / 11.85.  Eight waves, one turn, 0.88 to 1.02.  Sixteen waves in one part 0.99 up to
-        400 keys, 1.01 to 1.06 from 500 on, 16 of 12 heads over 1,000 16.4 / 15.6; in several parts 0.97 to 1.04, where the
-        weights are more than one round 1.02 to 1.04.)"""
+        400 keys, 1.01 to 1.06 from 500 on, 16 of 12 heads over 1,000 16.4 / 15.6.  Sixteen in several parts: up to 512 keys
+        0.98 to 1.04; beyond, 0.97 at 540 keys, 0.99 at 700, 1.01 at 1,000, but with more than one round of weights
+        (48 tiles of columns) 1.02 to 1.05.)"""
         visible = self._visible(max_kv_len)
-        return (waves == 4 and visible > 128) or (waves == 16 and (parts > 1 or visible > 512))
+        if waves == 16 and parts > 1:
+            return visible <= 512 or self.width > 768 * parts
+        return (waves == 4 and visible > 128) or (waves == 16 and visible > 512)
 
     def _range_records(self, ctx):
         """Scratch for one record per (token, head, key range): always asked for at its largest

@@ -107,7 +107,8 @@ def test_attention_and_projection_in_one_launch(monkeypatch):
     assert not _part(12)._weights_first(3, 4, 128) and _part(12)._weights_first(2, 4, 256)
     assert not _part(12, window=64)._weights_first(7, 4, 1024) and not _part(12)._weights_first(2, 8, 512)
     assert not _part(12)._weights_first(1, 16, 512) and _part(12)._weights_first(1, 16, 1024)
-    assert _part(25)._weights_first(3, 16, 256)
+    assert _part(25)._weights_first(3, 16, 256) and not _part(12)._weights_first(2, 16, 1024)
+    assert _part(25)._weights_first(2, 16, 1024) and not _part(25)._weights_first(4, 16, 1024)
     # wide models
     for keys in (128, 256, 512):
         for count in (5, 6, 7, 8):
