@@ -90,6 +90,9 @@ __device__ inline void store_wave_tile(f32x16 (&acc)[WM][WN], float* region, int
   constexpr int EP_STRIDE = WN * 32 + 8;          // floats; 4 rows further is 32 banks further
   constexpr int EP_CHUNKS = WN * 4;               // pieces of eight columns per row
   constexpr int EP_ROWS = 64 / EP_CHUNKS;         // rows per pass of the wave
+  // The callers read operands by assembly and wait for them just in front of this.  What is worked out of the lane here
+  // must not be moved in front of that wait, into a register that such a read may still be filling.
+  asm volatile("" : "+v"(lane));
   const int chunk = lane % EP_CHUNKS;
   const int row_in_pass = lane / EP_CHUNKS;
   // The piece that the end of the rows lies in begins further left where that is aligned and within the wave's columns
