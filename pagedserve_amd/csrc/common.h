@@ -330,6 +330,15 @@ __device__ inline float gate_factor(const AttnExtras& extra, long long token, in
   return 1.0f / (1.0f + expf(-extra.gate[token * extra.gate_ld + head]));
 }
 
+// Arguments that a kernel needs later are read here, while its first loads travel: left to itself the compiler reads
+// each where it is used, a trip of its own for every 64 bytes of arguments.
+__device__ inline void read_arguments() {}
+template <typename First, typename... Others>
+__device__ inline void read_arguments(First first, Others... others) {
+  asm volatile("" ::"s"(first));
+  read_arguments(others...);
+}
+
 // ---- error channel -------------------------------------------------------
 void ps_set_error(const char* fmt, ...);
 

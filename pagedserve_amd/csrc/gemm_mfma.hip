@@ -311,13 +311,26 @@ __device__ inline void skinny_top_choice(float (*partial)[SK_WAVES][MB][4][64], 
     __hip_atomic_store(top_choice_ticket(top, threadIdx.x), 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// What bounds a launch of few rows is the chain from its start to its last store, so nothing in it is waited for that
+// could have been asked for before.  The arguments in front of the bias are the ones that the first loads need: the
+// launch brings them along in registers (14 words), where every further one is a read of its own.  A wave whose steps are all
+// there asks for the packed weights by one address and constant distances; the general form, with a clamped
+// address per load, needed 200 instructions in front of its last load.  Before and now, in a step of GPT-2 small, launch included: 1 x 768 x
+// 3072 3.34 and 2.99 us, 64 x 2304 x 768 with its scatter 5.24 and 4.83, 64 x 3072 x 768 4.64 and 4.26, 64 x 768 x 3072
+// 5.05 and 4.42.
+#define SK_A_PACKED 1   // the rows of A lie in the packed order (packed_offset)
+#define SK_C_PACKED 2   // C is to be written in it
+#define SK_W_PACKED 4   // w is the packed copy
+#define SK_K_SPLIT 8    // k is split over blocks: C is added to with atomics
+#define SK_ROW_BITS 16  // in front of these flags stands the number of rows
 template <typename TOut, int EPI, int MB, int NT, int UNROLL>
 __global__ __launch_bounds__(64 * SK_WAVES) void gemm_nt_skinny_kernel(
-    const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, const float* __restrict__ bias,
-    TOut* __restrict__ c, int m, int n, int k, int lda, int ldc, int k_chunk, int k_splits,
-    KvScatter scatter, const bf16_t* __restrict__ wp, int layouts, TopChoice top) {
-  // layouts: bit 0, the rows of A lie in the packed order (packed_offset); bit 1, C is to be
-  // written in it.
+    const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, const int* __restrict__ tok_pos,
+    const int* __restrict__ tok_item, int rows_and_flags, int n, int k, int lda, int k_chunk,
+    const float* __restrict__ bias, TOut* __restrict__ c, int ldc, KvScatter scatter, TopChoice top) {
+  const int m = rows_and_flags & ((1 << SK_ROW_BITS) - 1);
+  const int layouts = rows_and_flags >> SK_ROW_BITS;
+  const int k_splits = layouts & SK_K_SPLIT ? 2 : 1;    // one range or several
   // NT tiles of 16 columns per block share the loads of the rows of A: with very many
   // columns (the output head) those loads, though they come from the L2, are as many bytes
   // as the weights themselves.
@@ -331,25 +344,13 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_nt_skinny_kernel(
   const int k_end = k_begin + k_chunk < k ? k_begin + k_chunk : k;
   const int sub = lane & 15;
   const int group = lane >> 4;
-  const bf16_t* w_ptr[NT];
-#pragma unroll
-  for (int j = 0; j < NT; ++j) {
-    const int w_row = n0 + j * 16 + sub < n ? n0 + j * 16 + sub : n - 1;
-    w_ptr[j] = w + (int64_t)w_row * k + group * 16;
-    if (wp != nullptr) {
-      // packed copy: the 16 x 64 tile of step s lies in the order in which the lanes hold it,
-      // first the halves of the first product, then those of the second (1 KB each)
-      const int tiles = (n + 15) / 16;
-      const int tile = n0 / 16 + j < tiles ? n0 / 16 + j : tiles - 1;
-      w_ptr[j] = wp + (int64_t)tile * (k / 64) * 1024 + lane * 8;
-    }
-  }
+  const bool a_packed = layouts & SK_A_PACKED;
+  const bool w_packed = layouts & SK_W_PACKED;
   const bf16_t* a_ptr[MB];
 #pragma unroll
   for (int b = 0; b < MB; ++b) {
     const int row = row0 + b * 16 + sub < m ? row0 + b * 16 + sub : m - 1;
-    a_ptr[b] = a + (int64_t)row * lda + group * 16;
-    if (layouts & 1) a_ptr[b] = a + (int64_t)(row >> 4) * (k / 64) * 1024 + lane * 8;
+    a_ptr[b] = a_packed ? a + (int64_t)(row >> 4) * (k / 64) * 1024 + lane * 8 : a + (int64_t)row * lda + group * 16;
   }
   f32x4 acc[NT][MB];
 #pragma unroll
@@ -357,10 +358,52 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_nt_skinny_kernel(
 #pragma unroll
     for (int b = 0; b < MB; ++b) acc[j][b] = f32x4{0.f, 0.f, 0.f, 0.f};
 
+  SkinnyEnds<TOut, EPI, MB> ends[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) ends[j].ask_rows(tok_pos, tok_item, m, row0);
+
   const uint4 zero = {0u, 0u, 0u, 0u};
-  // wave `wave` takes the 64-k steps wave, wave + 4, ... of the block's range
-  for (int k0 = k_begin + wave * 64; k0 < k_end; k0 += SK_WAVES * UNROLL * 64) {
-    uint4 wf[UNROLL][NT][2], xf[UNROLL][MB][2];
+  uint4 wf[UNROLL][NT][2], xf[UNROLL][MB][2];
+  // the steps k0, k0 + 4 x 64, ... of a wave
+  auto load = [&](int k0) {
+    if (w_packed && k0 + (UNROLL - 1) * SK_WAVES * 64 + 64 <= k_end) {
+      // packed copy: the 16 x 64 tile of step s lies in the order in which the lanes hold it,
+      // first the halves of the first product, then those of the second (1 KB each)
+      const int tiles = (n + 15) / 16;
+      const bf16_t* w_tile[NT];
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const int tile = n0 / 16 + j < tiles ? n0 / 16 + j : tiles - 1;
+        w_tile[j] = w + ((int64_t)tile * (k / 64) + k0 / 64) * 1024;
+      }
+      const int a_step = a_packed ? SK_WAVES * 1024 : SK_WAVES * 64, a_half = a_packed ? 512 : 8;
+      const int a_first = a_packed ? k0 * 16 : k0;
+#pragma unroll
+      for (int u = 0; u < UNROLL; ++u) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            wf[u][j][h] = *reinterpret_cast<const uint4*>(w_tile[j] + u * SK_WAVES * 1024 + h * 512 + lane * 8);
+#pragma unroll
+        for (int b = 0; b < MB; ++b)
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            xf[u][b][h] = *reinterpret_cast<const uint4*>(a_ptr[b] + a_first + u * a_step + h * a_half);
+      }
+      return;
+    }
+    const bf16_t* w_ptr[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const int w_row = n0 + j * 16 + sub < n ? n0 + j * 16 + sub : n - 1;
+      w_ptr[j] = w + (int64_t)w_row * k + group * 16;
+      if (w_packed) {
+        const int tiles = (n + 15) / 16;
+        const int tile = n0 / 16 + j < tiles ? n0 / 16 + j : tiles - 1;
+        w_ptr[j] = w + (int64_t)tile * (k / 64) * 1024 + lane * 8;
+      }
+    }
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
       const int ku = k0 + u * SK_WAVES * 64;
@@ -372,15 +415,15 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_nt_skinny_kernel(
       const int o0 = first ? ku : k_begin - group * 16;
       const int o1 = second ? ku + 8 : k_begin - group * 16;
       // (packed: k is a multiple of 64, so a step is whole or absent)
-      const int p0 = wp != nullptr ? (first ? (ku / 64) * 1024 : 0) : o0;
-      const int p1 = wp != nullptr ? p0 + 512 : o1;
+      const int p0 = w_packed ? (first ? (ku / 64) * 1024 : 0) : o0;
+      const int p1 = w_packed ? p0 + 512 : o1;
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
         wf[u][j][0] = *reinterpret_cast<const uint4*>(w_ptr[j] + p0);
         wf[u][j][1] = *reinterpret_cast<const uint4*>(w_ptr[j] + p1);
       }
-      const int q0 = (layouts & 1) ? (first ? (ku / 64) * 1024 : 0) : o0;
-      const int q1 = (layouts & 1) ? q0 + 512 : o1;
+      const int q0 = a_packed ? (first ? (ku / 64) * 1024 : 0) : o0;
+      const int q1 = a_packed ? q0 + 512 : o1;
 #pragma unroll
       for (int b = 0; b < MB; ++b) {
         xf[u][b][0] = *reinterpret_cast<const uint4*>(a_ptr[b] + q0);
@@ -399,6 +442,18 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_nt_skinny_kernel(
         for (int b = 0; b < MB; ++b) xf[u][b][1] = zero;
       }
     }
+  };
+  // wave `wave` takes the 64-k steps wave, wave + 4, ... of the block's range
+  int k0 = k_begin + wave * 64;
+  if (k0 < k_end) load(k0);
+  read_arguments(bias, c, ldc);
+  if (EPI == PS_EPI_NONE && tok_pos != nullptr) read_scatter(scatter);
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    ends[j].ask(bias, c, m, n, ldc, n0 + j * 16, row0, split, k_splits, scatter, tok_pos, layouts & SK_C_PACKED);
+    ends[j].ask_pages(scatter, tok_pos, n0 + j * 16);
+  }
+  while (k0 < k_end) {
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u)
 #pragma unroll
@@ -410,6 +465,8 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_nt_skinny_kernel(
             acc[j][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                 *reinterpret_cast<const bf16x8*>(&wf[u][j][h]),
                 *reinterpret_cast<const bf16x8*>(&xf[u][b][h]), acc[j][b], 0, 0, 0);
+    k0 += SK_WAVES * UNROLL * 64;
+    if (k0 < k_end) load(k0);
   }
 
 #pragma unroll
@@ -422,8 +479,8 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_nt_skinny_kernel(
   // element i of a 16 x 16 accumulator: weight row (lane / 16) * 4 + i, activation row lane % 16
 #pragma unroll
   for (int j = 0; j < NT; ++j)
-    skinny_epilogue<TOut, EPI, MB>(partial[j], bias, c, m, n, ldc, n0 + j * 16, row0, split,
-                                   k_splits, scatter, layouts & 2);
+    skinny_epilogue<TOut, EPI, MB>(partial[j], ends[j], c, m, n, ldc, n0 + j * 16, row0, k_splits, scatter,
+                                   layouts & SK_C_PACKED);
   if (EPI == PS_EPI_NONE && sizeof(TOut) == 4 && top.keys != nullptr)
     skinny_top_choice<MB, NT>(partial, bias, m, n, n0, row0, top);
 }
@@ -494,6 +551,9 @@ static void launch_skinny_mb(const void* a, const void* w, const float* bias, vo
   // the k ranges give few blocks, the rows are spread over more of them (every one reads the
   // same weights, which the L2 absorbs; blocks that differ only in z run on one XCD when the
   // number of column blocks is a multiple of 8).
+  const int rows_and_flags =
+      m | (((layouts & (SK_A_PACKED | SK_C_PACKED)) | (wp != nullptr ? SK_W_PACKED : 0) |
+            (k_splits > 1 ? SK_K_SPLIT : 0)) << SK_ROW_BITS);
   const int row_blocks = (m + 15) / 16;
   const int grid_xy = ((n + 15) / 16) * k_splits;
   // (up to three blocks per compute unit: 64 x 2304 x 768 with weights from memory takes 5.0 us
@@ -509,8 +569,9 @@ static void launch_skinny_mb(const void* a, const void* w, const float* bias, vo
   const bool three = k_chunk <= SK_WAVES * 3 * 64;
 #define PS_LAUNCH_SKU(MB, NT, UNROLL)                                                          \
   hipLaunchKernelGGL((gemm_nt_skinny_kernel<TOut, EPI, MB, NT, UNROLL>), grid, block, 0, s,    \
-                     (const bf16_t*)a, (const bf16_t*)w, bias, (TOut*)c, m, n, k, lda, ldc,    \
-                     k_chunk, k_splits, scatter, wp, layouts, top)
+                     (const bf16_t*)a, wp ? wp : (const bf16_t*)w,                             \
+                     scatter.k_pool ? scatter.tok_pos : nullptr, scatter.tok_item,             \
+                     rows_and_flags, n, k, lda, k_chunk, bias, (TOut*)c, ldc, scatter, top)
 #define PS_LAUNCH_SK(MB)                                                                       \
   do {                                                                                         \
     if (three) PS_LAUNCH_SKU(MB, 1, 3);                                                        \
@@ -548,9 +609,7 @@ static void launch_skinny_mb(const void* a, const void* w, const float* bias, vo
     }
   } else if (per <= 1 && k_chunk > SK_WAVES * SK_UNROLL * 64) {
     // up to 16 rows leave registers for twice the loads: a k of up to 2048 in one round
-    hipLaunchKernelGGL((gemm_nt_skinny_kernel<TOut, EPI, 1, 1, 2 * SK_UNROLL>), grid, block, 0, s,
-                       (const bf16_t*)a, (const bf16_t*)w, bias, (TOut*)c, m, n, k, lda, ldc,
-                       k_chunk, k_splits, scatter, wp, layouts, top);
+    PS_LAUNCH_SKU(1, 1, 2 * SK_UNROLL);
   } else if (per <= 1) PS_LAUNCH_SK(1);
   else if (per == 2) PS_LAUNCH_SK(2);
   else if (per == 3) PS_LAUNCH_SK(3);

@@ -14,6 +14,11 @@ struct KvScatter {
   int cache_only;        // the key and value columns need not be written to the output as well
 };
 
+__device__ inline void read_scatter(const KvScatter& s) {
+  read_arguments(s.k_pool, s.v_pool, s.tables, s.table_width, s.q_cols, s.kv_cols, s.head_dim, s.kv_heads, s.page_size,
+                 s.page_shift, s.num_pages);
+}
+
 // The product of the output head may also choose each row's token (the column of its largest
 // value, the lowest one on ties) instead of leaving that to a kernel of its own.  Blocks
 // raise 64-bit keys (value in an order that integers keep, then the column counted from
@@ -69,13 +74,17 @@ struct NormPrologue {
 // column: kv_scatter_row gives the element offset of (page, slot) of a token, or -1;
 // kv_scatter_col gives the pool and the offset of (head, dim) inside a page, or null for a
 // query column.
+__device__ inline int64_t kv_page_slot(const KvScatter& s, int pos, int page) {
+  const int logical = s.page_shift >= 0 ? (pos >> s.page_shift) : pos / s.page_size;
+  return ((int64_t)page * s.kv_heads * s.page_size + (pos - logical * s.page_size)) * s.head_dim;
+}
 // (the item by its address: where it lies in memory it is read behind the first check)
 __device__ inline int64_t kv_scatter_slot(const KvScatter& s, int pos, const int* item) {
   const int logical = s.page_shift >= 0 ? (pos >> s.page_shift) : pos / s.page_size;
   if (logical >= s.table_width) return -1;
   const int page = s.tables[(int64_t)*item * s.table_width + logical];
   if (page < 0 || page >= s.num_pages) return -1;
-  return ((int64_t)page * s.kv_heads * s.page_size + (pos - logical * s.page_size)) * s.head_dim;
+  return kv_page_slot(s, pos, page);
 }
 __device__ inline int64_t kv_scatter_row(const KvScatter& s, int row) {
   return kv_scatter_slot(s, s.tok_pos[row], s.tok_item + row);
@@ -100,20 +109,9 @@ __device__ inline T* kv_scatter_col(const KvScatter& s, int col, int64_t* offset
 // (reference: src/model/kv_manager.py:303-308,403-404).
 template <typename T>
 __device__ inline void kv_scatter_store(const KvScatter& s, int row, int col, float v) {
-  if (s.k_pool == nullptr || col < s.q_cols) return;
-  int within = col - s.q_cols;
-  T* pool = reinterpret_cast<T*>(s.k_pool);
-  if (within >= s.kv_cols) {
-    within -= s.kv_cols;
-    pool = reinterpret_cast<T*>(s.v_pool);
-  }
-  const int head = within / s.head_dim;
-  const int dim = within - head * s.head_dim;
-  const int pos = s.tok_pos[row];
-  const int logical = s.page_shift >= 0 ? (pos >> s.page_shift) : pos / s.page_size;
-  if (logical >= s.table_width) return;
-  const int page = s.tables[(int64_t)s.tok_item[row] * s.table_width + logical];
-  if (page < 0 || page >= s.num_pages) return;
-  pool[(((int64_t)page * s.kv_heads + head) * s.page_size + (pos - logical * s.page_size)) *
-           s.head_dim + dim] = from_float<T>(v);
+  int64_t offset;
+  T* pool = kv_scatter_col<T>(s, col, &offset);
+  if (pool == nullptr) return;
+  const int64_t slot = kv_scatter_row(s, row);
+  if (slot >= 0) pool[slot + offset] = from_float<T>(v);
 }
