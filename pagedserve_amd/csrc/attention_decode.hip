@@ -79,19 +79,16 @@ static int launch_decode(const void* q, int64_t q_stride, const void* k_pool, co
                          int table_width, int count, int heads, int kv_heads, int head_dim,
                          int page_size, int num_pages, float scale, int window, int splits,
                          int waves, const AttnExtras extra, hipStream_t s) {
-  int page_shift = -1;
-  if ((page_size & (page_size - 1)) == 0) {
-    page_shift = 0;
-    while ((1 << page_shift) < page_size) ++page_shift;
-  }
+  const int form = decode_form(head_dim, page_size, kv_heads, tok_list == nullptr && tok_item == nullptr &&
+                                                                  window == 0 && splits == 1);
   dim3 grid(count, heads, splits);
 #define PS_LAUNCH_ADN(LPK, WAVES, NT)                                                            \
   hipLaunchKernelGGL((attention_decode_kernel<T, LPK, WAVES, (WAVES == 16 && sizeof(T) == 2 ? 8 : 4), NT>), grid, \
                      dim3(64 * WAVES), 0, s,                                                     \
-                     (const T*)q, q_stride, (const T*)k_pool, (const T*)v_pool, (T*)out,         \
-                     out_stride, partial, tok_list, tok_item, tok_pos, tables, table_width,      \
-                     heads, kv_heads, head_dim, page_size, page_shift, num_pages,                \
-                     scale * 1.4426950408889634f, window, splits, extra)
+                     tables, tok_pos, tok_list, tok_item, (const T*)q, q_stride, table_width,    \
+                     form, page_size, heads, kv_heads, heads / kv_heads,                         \
+                     num_pages, (const T*)k_pool, (const T*)v_pool, (T*)out, out_stride,         \
+                     partial, scale * 1.4426950408889634f, window, splits, extra)
   // more blocks than compute units: the step is bound by memory bandwidth, not by one round trip
   const bool streaming = sizeof(T) == 2 && (int64_t)count * heads * splits > ps_compute_units();
 #define PS_LAUNCH_ADW(LPK, WAVES)          \

@@ -18,9 +18,10 @@
 // instructions are few and free beside the loads, and with the context as row operand the sixteen
 // results of a tile lie in sixteen consecutive lanes, whose adds fall into one 64-byte piece.
 //
-// Measured (us, keys and weights from memory, attention + projection in two launches before): one request of
-// 12 heads over 144 keys 8.6 -> 5.9, 8 over 540 keys 13.6 -> 10.5, 16 over 540 keys 16.4 -> 12.3; 8 of 16
-// heads over 270 keys 11.8 -> 9.8.  parts/attention.py says where the lines lie.
+// Measured (us, keys and weights from memory; while every load had an address and a block-table exchange of its own, now):
+// one request of 12 heads over 100, 250 and 540 keys 4.36 -> 3.63, 5.75 -> 4.71 and 8.31 -> 6.78, 8 requests 6.30 -> 5.10,
+// 6.81 -> 6.15 and 10.06 -> 8.49, 16 over 540 keys 11.5 -> 10.7; 8 of 8 heads of 128 over 400 keys 11.8 -> 11.2.
+// parts/attention.py says where the lines lie.
 #include <math.h>
 
 #include "attention_decode_block.h"
@@ -33,17 +34,14 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 // STEPS: head_dim / 64; AHEAD: tiles of 16 columns per wave whose weights are asked for beside the keys
 // (further ones follow behind the attention): right behind the first keys and values, or FIRST, in front of the
 // attention, where they hold back the block table and with it the keys, but nothing of a wave's later turns
-// (parts/attention.py says where the line lies).  Heads of 128 hold twice the weights, which the first turn over the keys has
-// no registers left for (16 waves spill 16 of them; 8 requests of 8 heads over 250 keys 9.5 us with the weights in front,
-// 11.7 behind; one of 16 heads over 400 keys 10.6 and 12.1): always in front.
+// (parts/attention.py says where the line lies).
 template <int STEPS, int AD_WAVES, int AD_UNROLL, int AHEAD, bool FIRST>
 __global__ __launch_bounds__(64 * AD_WAVES) void attention_decode_linear_kernel(
-    const bf16_t* __restrict__ q, int64_t q_stride, const bf16_t* __restrict__ k_pool,
-    const bf16_t* __restrict__ v_pool, const int* __restrict__ tok_pos,
-    const int* __restrict__ tables, int table_width, int heads, int kv_heads, int page_size,
-    int page_shift, int num_pages, float scale_log2, int window, const AttnExtras extra,
-    const bf16_t* __restrict__ wp, const float* __restrict__ bias, float* __restrict__ residual,
-    int64_t ld_res, int n, int tiles_per_block) {
+    const int* __restrict__ tables, const int* __restrict__ tok_pos, const bf16_t* __restrict__ q, int64_t q_stride,
+    const bf16_t* __restrict__ wp, int table_width, int form, int heads, int n, int tiles_per_block, int kv_group,
+    int page_size, int kv_heads, int num_pages, const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool,
+    float scale_log2, int window, const float* __restrict__ bias, float* __restrict__ residual, int64_t ld_res,
+    const AttnExtras extra) {
   constexpr int HEAD_DIM = STEPS * 64;
   __shared__ DecodeLds<AD_WAVES> lds;
   __shared__ __attribute__((aligned(16))) bf16_t context[HEAD_DIM];
@@ -59,6 +57,7 @@ __global__ __launch_bounds__(64 * AD_WAVES) void attention_decode_linear_kernel(
   const int k_steps = heads * STEPS;
   const bf16_t* w_head = wp + (int64_t)head * STEPS * 1024 + lane * 8;
   uint4 w_raw[AHEAD][STEPS][2];
+  float b[AHEAD];       // lane l < 16: the bias of column l of the tile (added by the blocks of head 0)
   auto load_weights = [&](int round) {
 #pragma unroll
     for (int c = 0; c < AHEAD; ++c) {
@@ -71,12 +70,23 @@ __global__ __launch_bounds__(64 * AD_WAVES) void attention_decode_linear_kernel(
         for (int h = 0; h < 2; ++h)
           w_raw[c][st][h] = *reinterpret_cast<const uint4*>(w_tile + (st * 2 + h) * 512);
     }
+    if (bias != nullptr && head == 0) {
+#pragma unroll
+      for (int c = 0; c < AHEAD; ++c) {
+        const int col = (first_tile + (round * AHEAD + c) * AD_WAVES + wave) * 16 + (lane & 15);
+        b[c] = bias[col < n ? col : n - 1];
+      }
+    } else {
+#pragma unroll
+      for (int c = 0; c < AHEAD; ++c) b[c] = 0.f;
+    }
   };
 
   auto attend = [&](auto ahead) {
     attention_decode_block<bf16_t, 8 * STEPS, AD_WAVES, AD_UNROLL, false>(
         lds, token, head, 0, q, q_stride, k_pool, v_pool, (bf16_t*)nullptr, 0, nullptr, nullptr, nullptr,
-        tok_pos, tables, table_width, heads, kv_heads, HEAD_DIM, page_size, page_shift, num_pages,
+        tok_pos, tables, table_width, heads, kv_heads, kv_group,
+        (form & 0xffff) | (HEAD_DIM << 16), page_size, num_pages,
         scale_log2, window, 1, extra, context, ahead);
   };
   if constexpr (FIRST) {
@@ -114,9 +124,7 @@ __global__ __launch_bounds__(64 * AD_WAVES) void attention_decode_linear_kernel(
       // row 0 of the tile lies in the first element of lanes 0 to 15, a column each
       const int col = tile * 16 + lane;
       if (tile < end_tile && lane < 16 && col < n) {
-        float v = acc[0];
-        if (head == 0 && bias != nullptr) v += bias[col];
-        unsafeAtomicAdd(residual + (int64_t)token * ld_res + col, v);
+        unsafeAtomicAdd(residual + (int64_t)token * ld_res + col, acc[0] + b[c]);
       }
     }
   }
@@ -147,32 +155,27 @@ extern "C" int ps_attention_decode_linear(const void* q, int64_t q_stride, const
                  (reinterpret_cast<uintptr_t>(w_packed) & 15u) == 0,
              "ps_attention_decode_linear: null or unaligned operand");
   if (count == 0) return 0;
-  int page_shift = -1;
-  if ((page_size & (page_size - 1)) == 0) {
-    page_shift = 0;
-    while ((1 << page_shift) < page_size) ++page_shift;
-  }
   const int tiles_per_block = (tiles_n + parts - 1) / parts;
+  const int form = decode_form(head_dim, page_size, kv_heads, window == 0);
   const AttnExtras extra{sink, gate, gate_ld, softcap, logistic, logistic_norm};
   dim3 grid(count, heads, (tiles_n + tiles_per_block - 1) / tiles_per_block);
   hipStream_t s = (hipStream_t)stream;
 #define PS_LAUNCH_ADL(STEPS, WAVES, UNROLL, AHEAD, FIRST)                                          \
   hipLaunchKernelGGL((attention_decode_linear_kernel<STEPS, WAVES, UNROLL, AHEAD, FIRST>), grid,   \
-                     dim3(64 * WAVES), 0, s, (const bf16_t*)q, q_stride, (const bf16_t*)k_pool,    \
-                     (const bf16_t*)v_pool, tok_pos, tables, table_width, heads, kv_heads,         \
-                     page_size, page_shift, num_pages, scale * 1.4426950408889634f, window, extra, \
-                     (const bf16_t*)w_packed, bias, residual, ld_res, n, tiles_per_block)
+                     dim3(64 * WAVES), 0, s, tables, tok_pos, (const bf16_t*)q, q_stride,          \
+                     (const bf16_t*)w_packed, table_width, form, heads, n, tiles_per_block,        \
+                     heads / kv_heads, page_size, kv_heads, num_pages, (const bf16_t*)k_pool,      \
+                     (const bf16_t*)v_pool, scale * 1.4426950408889634f, window, bias, residual,   \
+                     ld_res, extra)
+  // (sixteen waves leave a wave 128 registers, too few for the keys and the weights of a turn: over 800 keys 8 requests of
+  // 12 heads 12.3 us, with eight waves and two turns 10.8.  Who asks for them gets eight.)
   if (head_dim == 64) {
-    // (eight waves are behind with the weights in front everywhere)
     if (waves == 4 && weights_first) PS_LAUNCH_ADL(1, 4, 4, 4, true);
     else if (waves == 4) PS_LAUNCH_ADL(1, 4, 4, 4, false);
-    else if (waves == 8) PS_LAUNCH_ADL(1, 8, 8, 4, false);
-    else if (weights_first) PS_LAUNCH_ADL(1, 16, 8, 3, true);
-    else PS_LAUNCH_ADL(1, 16, 8, 3, false);
+    else PS_LAUNCH_ADL(1, 8, 8, 4, false);
   } else {
-    if (waves == 4) PS_LAUNCH_ADL(2, 4, 4, 4, true);
-    else if (waves == 8) PS_LAUNCH_ADL(2, 8, 8, 4, true);
-    else PS_LAUNCH_ADL(2, 16, 8, 2, true);
+    if (waves == 4) PS_LAUNCH_ADL(2, 4, 4, 4, false);
+    else PS_LAUNCH_ADL(2, 8, 8, 4, false);
   }
 #undef PS_LAUNCH_ADL
   PS_CHECK_LAUNCH("ps_attention_decode_linear");

@@ -24,17 +24,16 @@
 
 template <int NDB, int LPK, bool NT>
 __global__ __launch_bounds__(64 * AM_WAVES) void attention_mixed_kernel(
-    const bf16_t* __restrict__ q, int64_t q_stride, const bf16_t* __restrict__ k_pool,
-    const bf16_t* __restrict__ v_pool, bf16_t* __restrict__ out, int64_t out_stride,
-    // the items of one token
-    int decode_blocks, const int* __restrict__ tok_list, const int* __restrict__ tok_item,
-    const int* __restrict__ tok_pos,
+    // the items of one token (`singles` of them)
+    const int* __restrict__ tok_list, const int* __restrict__ tok_item, const int* __restrict__ tok_pos,
+    // both
+    const int* __restrict__ tables, const bf16_t* __restrict__ q, int64_t q_stride, int decode_blocks, int singles,
+    int table_width, int form, int heads, int kv_heads, int kv_group, int page_size, int num_pages,
+    const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool, bf16_t* __restrict__ out,
+    int64_t out_stride, float scale, int window,
     // the items of several
     const int* __restrict__ tile_item, const int* __restrict__ tile_q0,
-    const int* __restrict__ cu_tokens, const int* __restrict__ kv_lens,
-    // both
-    const int* __restrict__ tables, int table_width, int heads, int kv_heads, int page_size,
-    int page_shift, int num_pages, float scale, int window, const AttnExtras extra) {
+    const int* __restrict__ cu_tokens, const int* __restrict__ kv_lens, const AttnExtras extra) {
   typedef PrefillLds<NDB, 2, 2, 1> TileLds;
   union Lds {
     TileLds tiles;
@@ -44,13 +43,12 @@ __global__ __launch_bounds__(64 * AM_WAVES) void attention_mixed_kernel(
   const int block = blockIdx.x;
   if (block < decode_blocks) {
     // tokens fastest, as in the decode kernel's own grid
-    const int count = decode_blocks / heads;
-    const int head = block / count;
-    const int n = block - head * count;
+    const int head = block / singles;
+    const int n = block - head * singles;
     attention_decode_block<bf16_t, LPK, AM_WAVES, AM_UNROLL, NT>(
         lds.decode, n, head, 0, q, q_stride, k_pool, v_pool, out, out_stride, nullptr, tok_list,
-        tok_item, tok_pos, tables, table_width, heads, kv_heads, NDB * 16, page_size, page_shift,
-        num_pages, scale * 1.4426950408889634f, window, 1, extra);
+        tok_item, tok_pos, tables, table_width, heads, kv_heads, kv_group,
+        (form & 0xffff) | (NDB << 20), page_size, num_pages, scale * 1.4426950408889634f, window, 1, extra);
   } else {
     // heads fastest, as in the tiled kernel's own grid: the tiles that see the most keys first
     const int rest = block - decode_blocks;
@@ -58,7 +56,7 @@ __global__ __launch_bounds__(64 * AM_WAVES) void attention_mixed_kernel(
     const int head = rest - tile_index * heads;
     attention_prefill_block<NDB, 2, 2, 1>(lds.tiles, head, tile_index, q, q_stride, k_pool, v_pool, out,
                                           out_stride, tile_item, tile_q0, cu_tokens, kv_lens, tables,
-                                          table_width, heads, kv_heads, page_size, page_shift,
+                                          table_width, heads, kv_heads, page_size, AD_SHIFT(form),
                                           num_pages, scale, window, extra);
   }
 }
@@ -98,12 +96,8 @@ extern "C" int ps_attention_mixed(const void* q, int64_t q_stride, const void* k
   const int64_t blocks = (int64_t)singles * heads + (int64_t)tiles * heads;
   PS_REQUIRE(blocks < ((int64_t)1 << 31), "ps_attention_mixed: too many blocks");
   if (blocks == 0) return 0;
-  int page_shift = -1;
-  if ((page_size & (page_size - 1)) == 0) {
-    page_shift = 0;
-    while ((1 << page_shift) < page_size) ++page_shift;
-  }
   hipStream_t s = (hipStream_t)stream;
+  const int form = decode_form(head_dim, page_size, kv_heads, false);
   const AttnExtras extra = {sink, gate, gate_ld, softcap, logistic, logistic_norm};
   const int decode_blocks = singles * heads;
   // as the decode kernel chooses: more blocks of its kind than compute units read their keys
@@ -111,11 +105,11 @@ extern "C" int ps_attention_mixed(const void* q, int64_t q_stride, const void* k
   const bool streaming = decode_blocks > ps_compute_units();
 #define PS_LAUNCH_AM(NDB, LPK, NT)                                                              \
   hipLaunchKernelGGL((attention_mixed_kernel<NDB, LPK, NT>), dim3((unsigned)blocks),            \
-                     dim3(64 * AM_WAVES), 0, s, (const bf16_t*)q, q_stride,                     \
+                     dim3(64 * AM_WAVES), 0, s, tok_list, tok_item, tok_pos, tables,            \
+                     (const bf16_t*)q, q_stride, decode_blocks, singles, table_width, form,     \
+                     heads, kv_heads, heads / kv_heads, page_size, num_pages,                   \
                      (const bf16_t*)k_pool, (const bf16_t*)v_pool, (bf16_t*)out, out_stride,    \
-                     decode_blocks, tok_list, tok_item, tok_pos, tile_item, tile_q0, cu_tokens, \
-                     kv_lens, tables, table_width, heads, kv_heads, page_size, page_shift,      \
-                     num_pages, scale, window, extra)
+                     scale, window, tile_item, tile_q0, cu_tokens, kv_lens, extra)
 #define PS_LAUNCH_AM_NT(NDB, LPK)     \
   do {                                \
     if (streaming) {                  \

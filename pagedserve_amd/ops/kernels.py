@@ -918,8 +918,8 @@ def attention_decode_linear(q, k_pool, v_pool, tok_pos, tables, heads, scale, w,
                             window=0, sink=None, gate=None, softcap=0.0, logistic=None, weights_first=False):
     """residual[t] += (decode attention of token t, which is item t) w^T + bias, in one launch; ``packed`` is
     ``pack_decode_weight(w)``.  ``parts``: into how many parts the columns are dealt, one block per (token,
-    head, part); ``waves``: 4, 8 or 16 to a block.  ``weights_first``: heads of 64 in blocks of 4 or 16 waves ask for the
-    weights in front of the keys; it steers the order of loads only."""
+    head, part); ``waves``: 4 or 8 to a block (16 are run as 8).  ``weights_first``: heads of 64 in blocks of 4 waves ask for
+    the weights in front of the keys; it steers the order of loads only."""
     _check(q, "q", torch.bfloat16, 2)
     pages, kv_heads, page_size, head_dim = _check_pools(k_pool, v_pool, q.dtype)
     q_stride = _rows(q, "q")

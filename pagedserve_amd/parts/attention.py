@@ -393,9 +393,9 @@ class Attention(Mixer):
             # the output projection, which is split over the heads: no launch for the merge
             splits = merged_splits
             partial = self._range_records(ctx)
-            kernels.attention_decode_partial(q, cache.k_pool, cache.v_pool, partial, ctx.tok_item,
-                                             ctx.positions, tables, self.heads, self.scale, splits,
-                                             window=self.span, waves=4, sink=sink, softcap=self.score_cap, logistic=self.logistic)
+            kernels.attention_decode_partial(q, cache.k_pool, cache.v_pool, partial, None, ctx.positions,
+                                             tables, self.heads, self.scale, splits, window=self.span, waves=4,
+                                             sink=sink, softcap=self.score_cap, logistic=self.logistic)
             kernels.attention_merge_linear(partial, singles, self.heads, self.head_dim, splits,
                                            self.out_weight, self.out_packed, self.out_bias, residual)
             return
@@ -421,18 +421,16 @@ class Attention(Mixer):
         elif singles:
             # one-token items: keys of a request are cut into ranges so that few requests
             # still fill the chip
-            splits, waves = self._splits(singles, ctx.max_kv_len)
+            splits, waves = self._splits(singles, ctx.max_kv_len,
+                                         self.heads == self.kv_heads and self.dtype == torch.bfloat16)
             partial = None
             if splits > 1:
                 partial = self._range_records(ctx)
             # in a step of single tokens only, token t is item t: without the index the kernel
-            # asks for its block table a trip to memory earlier (64 requests of 12 heads: 1.6 %
-            # of the step).  The path above, of few blocks with one or two pages each, measured
-            # 0.6 % slower with it, and so did a grid of more than four blocks per compute unit,
-            # which waits for bytes and not for a trip (64 requests of 25 heads: 1 us a launch):
-            # both keep the index.
-            direct = (singles == tokens
-                      and singles * self.heads * splits <= 4 * kernels.compute_units())
+            # asks for its block table a trip to memory earlier (us, with the index and without:
+            # 48 requests of 12 heads over 20 and 200 keys 4.65 / 4.42 and 9.92 / 9.53, 64 of 25 heads
+            # over 100, 400 and 800 keys 12.5 / 12.0, 31.4 / 31.6 and 59.1 / 58.8).
+            direct = singles == tokens
             kernels.attention_decode(q, cache.k_pool, cache.v_pool, context,
                                      None if direct else ctx.tok_item,
                                      ctx.positions, tables, self.heads, self.scale, splits,
@@ -517,12 +515,14 @@ class Attention(Mixer):
           400 keys 9.0 / 7.1, 11.9 / 9.3 and 14.9 / 11.0; one over 20 keys 7.8 / 4.3); beyond, ranges are ahead (1 and 8
           over 2,000 keys 10.2 / 13.8 and 18.3 / 18.9) unless the pairs fill half of the units, where the two-launch
           path has few ranges or none either (23.9 / 20.5 with 12 requests).
-        * Parts until the blocks come to one per unit, but four from 1,024 keys on, which every part reads again (one
-          request of 25 heads over 900 keys in 8, 4 and 3 parts 13.2, 10.9 and 10.7, two launches 12.6).  Up to 128
-          keys blocks of four waves are over soonest and two or three of them share a unit; up to 512 keys eight
-          waves take them in one round of loads, if the part's weights are one round too (512 columns: 3 requests of
-          25 heads at width 1,600 over 250 keys, 3 parts of 534, 10.4 with eight waves and 9.6 with sixteen, two
-          launches 10.2); beyond, or without parts, sixteen.
+        * Up to 128 keys blocks of four waves are over soonest.  Parts until the blocks come to one per unit while that is
+          four or more (4 requests of 12 heads over 100 keys in 5 and 12 parts 3.9 and 5.6), else until two or three of them
+          share a unit (16 over 60 keys in 1, 2 and 3 parts 5.9, 5.9 and 5.6).
+        * Beyond, eight waves take up to 512 keys in one round of loads (8 of 12 heads over 250 and 540 keys in two parts
+          6.2 and 8.5, with four waves 6.5 and 10.0).  Parts until the blocks come to one per unit, but four from 1,024
+          keys on, which every part reads again (one request of 25 heads over 900 keys in 8, 4 and 3 parts 13.2, 10.9
+          and 10.7, two launches 12.6).  What asks for sixteen waves (longer contexts, blocks without parts, more
+          columns than eight waves hold) is run as eight as well, see attention_decode_linear.hip.
         * Between one and one and a half pairs per unit, up to 512 keys, 256 of wider heads: four waves, two parts (24
           requests of 12 heads over 270 keys 15.5 / 12.7; over 1,000 keys 23.6 / 24.5; of 12 heads of 128 over one
           key/value head within 128 and over 250 keys 14.0 / 11.4 and 14.2 / 15.9).
@@ -548,7 +548,8 @@ class Attention(Mixer):
             return None
         tiles = -(-self.width // 16)
         if keys <= 128:
-            parts, waves = max(1, min(12, (5 * units + pairs) // (2 * pairs))), 4
+            parts = units // pairs if units >= 4 * pairs else (5 * units + pairs) // (2 * pairs)
+            parts, waves = max(1, min(12, parts)), 4
         elif pairs > units:
             if keys > (512 if self.head_dim == 64 else 256):
                 return None
@@ -566,13 +567,10 @@ class Attention(Mixer):
     def _weights_first(self, parts: int, waves: int, max_kv_len: int) -> bool:
         """Whether the blocks of that kernel ask for their weights in front of the keys, not behind the first of them.  A
         wave's loads come back in the order of issue: in front, the weights hold back the block table and the
-        first keys; behind, the keys of a wave's second turn, and with sixteen waves there is more to hold
-        back.  (Keys and weights from memory, behind and in front, heads of 64: four waves within 128 keys 0.98 on
-        average, 1 of 12 heads over 60 keys 4.37 / 4.40; beyond, where a wave takes several turns, 1.02 to 1.13, 24 requests of
-        12 heads over 270 keys 13.3 / 11.85.  Eight waves, one turn, 0.88 to 1.02.  Sixteen waves in one part 0.99 up to
-        400 keys, 1.01 to 1.06 from 500 on, 16 of 12 heads over 1,000 16.4 / 15.6.  Sixteen in several parts: up to 512 keys
-        0.98 to 1.04; beyond, 0.97 at 540 keys, 0.99 at 700, 1.01 at 1,000, but with more than one round of weights
-        (48 tiles of columns) 1.02 to 1.05.)"""
+        first keys; behind, the keys of a wave's second turn.  (Keys and weights from memory, behind and in front,
+        heads of 64, four waves: one request of 12 heads over 60 keys 3.55 / 3.85; where a wave takes several turns and
+        the blocks come to more than one per unit, 24 over 250 and 400 keys 10.4 / 10.1 and 13.5 / 12.7.)  Blocks of
+        more waves, which hold more of a block's keys in one turn, ask for them behind whatever is said here."""
         visible = self._visible(max_kv_len)
         if waves == 16 and parts > 1:
             return visible <= 512 or self.width > 768 * parts
@@ -631,23 +629,32 @@ class Attention(Mixer):
         room = 1 + 6 * units // (count * self.heads)
         return max(1, min(wanted, most, room, 64))
 
-    def _splits(self, count: int, max_kv_len: int):
+    def _splits(self, count: int, max_kv_len: int, own_keys: bool = False):
         """(ranges per request, waves per block) of the decode kernel, by the number of (token,
-        head) pairs per compute unit and the keys that a query sees:
+        head) pairs per compute unit and the keys that a query sees (us in brackets: bfloat16, keys from memory):
 
-        * from three and a half pairs per unit: one block of 4 waves per pair fills the chip;
+        * up to 128 keys (a turn of 4 waves, if that is more), and from three and a half pairs per unit:
+          one block of 4 waves per pair (8 requests of 8 heads of 128 over 20 keys: 3.7, in blocks of 16
+          waves 4.4, in two ranges 5.9);
         * from one and a half: the same at short contexts; from 2,048 keys on a handful of long
           blocks per unit would leave units idle towards the end, so the keys are cut into
           ranges until six blocks come to a unit;
-        * between one and one and a half: blocks of 16 waves would come two to some units and
-          one to the others, and the kernel would last as long as the units with two (24
-          requests of 12 heads at 1,000 keys: 22.3 us): ranges of 4-wave blocks, four blocks to a
-          unit (19.0 us with the launch that merges them), six over thousands of keys;
-        * up to one pair per unit: one block of 16 waves takes a whole request's keys and no
-          second launch is needed (two or three such blocks per request while each still has
-          a unit of its own); just under a pair per unit and from 4,096 keys on, ranges of
-          4-wave blocks are ahead again;
-        * few pairs: ranges of 4-wave blocks until four blocks come to a unit.
+        * between one and one and a half: up to 512 keys the same (24 requests of 12 heads at 400
+          keys 10.6, in two ranges 12.2); beyond, blocks of 16 waves would come two to some units and
+          one to the others, and one block of 4 waves is long (24 over 1,500 and 2,000 keys 27.0 and 33.6):
+          ranges of 4-wave blocks, four blocks to a unit (24.6 and 31.3 with the launch that merges them),
+          six over thousands of keys;
+        * between half a pair and one: one block of 16 waves takes a whole request's keys and no
+          second launch is needed; from 16 turns of four waves on (2,048 keys of 64 values) that is behind
+          ranges of 4-wave blocks, four blocks to a unit, where every head has bfloat16 keys of its own
+          (``own_keys``; 16 over 2,000 keys 25.3 and 22.6, 12 over 4,000 38.6 and 31.0; heads that share keys find them in the cache: 20 of 12 heads over 4
+          18.1 and 22.0; in float 39.6 and 42.3, so there from 4,096 on, just under a pair per unit, as before);
+        * fewer pairs: up to 512 keys that a block of 16 waves takes in one turn that block (one request of 12
+          heads over 200 and 400 keys 4.3 and 5.8, in ranges 6.0 and 6.5), beyond ranges of a turn of 4-wave blocks or
+          more until three blocks come to a unit, up to 16 ranges, 32 over 64 turns (8 of 12 heads over 800 and 2,000
+          keys 9.4 and 14.5, in one and two blocks of 16 waves 10.5 and 16.7; one over 4,000 keys in 16 and 32 ranges
+          10.1 and 10.5).  That holds to 8,192 keys and, from a quarter of a pair per unit on, to 2,048; beyond,
+          ranges until four blocks come to a unit, or two or three blocks of 16 waves.
 
         Never more ranges than the keys of the longest request can feed, and never more than
         six blocks per unit beside one per pair (the scratch for the records is sized for
@@ -655,27 +662,31 @@ class Attention(Mixer):
         visible = self._visible(max_kv_len)
         pairs = count * self.heads
         units = kernels.compute_units()
-        if 2 * pairs >= 7 * units:
+        turn = kernels.decode_keys_per_block(self.head_dim, 4)      # keys that 4 waves take at once: 128 of 64 values
+        if visible <= max(128, turn) or 2 * pairs >= 7 * units:
             return 1, 4
         if pairs >= units + units // 2:
-            # One block of 4 waves per pair fills the chip at short contexts.  At long ones a
-            # handful of blocks per unit, each walking thousands of keys, leaves units idle
-            # towards the end: ranges until six blocks come to a unit (32 requests of 12 heads
-            # at 8,192 keys: 126 instead of 172 us), none under 2,048 keys.
+            # (32 requests of 12 heads at 8,192 keys: 126 instead of 172 us; none under 2,048 keys)
             return max(1, min(-(-6 * units // pairs), visible // 1024)), 4
         if pairs > units:
             # (four blocks to a unit, six over thousands of keys)
             blocks = (6 if visible >= 4096 else 4) * units
-            return max(1, min(-(-blocks // pairs), visible // 256)), 4
+            return (max(1, min(-(-blocks // pairs), visible // 256)) if visible > 512 else 1), 4
         if 4 * pairs >= 3 * units and visible >= 4096:
             # nearly a pair per unit over thousands of keys: six blocks of 4 waves to a unit are
             # ahead of one block of 16 waves per pair (17 requests of 12 heads at 4,096 keys:
             # 41.4 against 44.2 us, at 16,384 keys 141 against 155)
             return min(-(-6 * units // pairs), 64), 4
-        if pairs >= units // 4 and visible > kernels.decode_keys_per_block(self.head_dim, 4):
-            # contexts of several thousand keys: two or three such blocks per request, as
+        if 2 * pairs > units:
+            return (4 * units // pairs, 4) if visible >= 16 * turn and own_keys else (1, 16)
+        if visible <= (2048 if 4 * pairs >= units else 8192):
+            if visible <= min(4 * turn, 512):
+                return 1, 16
+            return max(1, min(3 * units // pairs, visible // turn, 32 if visible >= 64 * turn else 16)), 4
+        if pairs >= units // 4:
+            # contexts of many thousand keys: two or three such blocks per request, as
             # long as every block still has a compute unit of its own
             return max(1, min(units // pairs, visible // 1024)), 16
-        most = max(1, -(-visible // kernels.decode_keys_per_block(self.head_dim, 4)))
+        most = max(1, -(-visible // turn))
         wanted = max(1, -(-4 * units // pairs))
         return min(most, wanted, 64), 4

@@ -1149,6 +1149,39 @@ def test_norm_product_scatters_keys_and_values(m, geometry):
     assert torch.equal(k_pool.view(view), k_ref.view(view)) and torch.equal(v_pool.view(view), v_ref.view(view))
 
 
+@pytest.mark.parametrize("head_dim,page_size", [(64, 8), (64, 16), (128, 16), (32, 64), (48, 16), (256, 2), (64, 4), (64, 12)])
+@pytest.mark.parametrize("window", [0, 5])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_attention_decode_pages_of_a_load(dtype, window, head_dim, page_size):
+    """Pages that hold the keys of one load and pages that do not: contexts that end at the edges of loads, turns and
+    pages, windows that begin inside a load, entries behind a context that name no page, a context longer than its
+    block table, with and without an index, in one range and in three."""
+    from pagedserve_amd.ops import kernels
+
+    heads = 3
+    contexts = [1, 7, 8, 9, 16, 17, 32, 33, 64, 65, 127, 129, 257, 300]
+    k_pool, v_pool, tables = _paged_fixture(dtype, contexts, heads, head_dim, page_size, 521)
+    for row, context in enumerate(contexts):
+        used = -(-context // page_size)
+        tables[row, used::2], tables[row, used + 1::2] = -1, k_pool.shape[0] + 7
+    tables = tables[:, :280 // page_size].contiguous()       # (the last context's keys from 280 on have no page)
+    q = _rand((len(contexts), heads * head_dim), dtype, 522)
+    item = torch.arange(len(contexts), dtype=torch.int32, device="cuda")
+    pos = torch.tensor([c - 1 for c in contexts], dtype=torch.int32, device="cuda")
+    scale = head_dim ** -0.5
+    seen = pos.clone() if window else pos.clamp(max=tables.shape[1] * page_size - 1)
+    rows = len(contexts) - 1 if window else len(contexts)    # (a window behind the table sees nothing)
+    expected = _attention_expected(q[:rows], k_pool, v_pool, tables, item[:rows], seen[:rows], heads, scale, window)
+    atol, rtol = (3e-5, 3e-5) if dtype == torch.float32 else (2e-2, 2e-2)     # as for the other tests of this kernel
+    for index in (None, item):
+        for splits, waves in ((1, 4), (1, 16), (3, 4)):
+            partial = torch.full((len(contexts) * heads * splits * (head_dim + 2),), float("nan"), device="cuda")
+            out = torch.full_like(q, float("nan"))
+            kernels.attention_decode(q, k_pool, v_pool, out, index, pos, tables, heads, scale, splits, partial=partial,
+                                     window=window, waves=waves)
+            torch.testing.assert_close(out[:rows].double(), expected, atol=atol, rtol=rtol)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_attention_decode_sixteen_waves(dtype):
     from pagedserve_amd.ops import kernels
