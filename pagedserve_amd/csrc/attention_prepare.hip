@@ -25,26 +25,35 @@
 #include "common.h"
 #include "pagedserve_hip.h"
 
+// A launch of few tokens is a chain of trips to memory: the arguments that do not come with it, position, item and
+// frequencies in one; block table, columns, weights and earlier values in the next; nothing else waits.  (8 tokens of 12
+// heads of 64 over 4, in a decode step, trip by trip and now: 5.3 and 4.5 us.)
 template <typename T>
 __global__ __launch_bounds__(1024) void attention_prepare_kernel(
-    const float* __restrict__ proj, int64_t ld, int q_col, int k_col, int v_col,
+    const float* __restrict__ proj, int64_t ld, const int* __restrict__ tok_pos, const int* __restrict__ tok_item,
+    const float* __restrict__ freqs, int rot_dims, int threads, int q_col, int k_col, int v_col,
     T* __restrict__ q_out, int64_t q_stride, T* __restrict__ k_pool, T* __restrict__ v_pool,
-    const float* __restrict__ q_gamma, const float* __restrict__ k_gamma, float eps,
-    const float* __restrict__ freqs, int rot_dims, T* __restrict__ v_first,
-    const float* __restrict__ v_lambda, int v_mode, const int* __restrict__ tok_item,
-    const int* __restrict__ tok_pos, const int* __restrict__ tables, int table_width, int heads,
+    const float* __restrict__ q_gamma, const float* __restrict__ k_gamma, float eps, T* __restrict__ v_first,
+    const float* __restrict__ v_lambda, int v_mode, const int* __restrict__ tables, int table_width, int heads,
     int kv_heads, int key_dim, int value_dim, int cache_dim, int page_size, int num_pages,
     int v_heads, int store, int q_dim, int q_maps) {
   __shared__ float red[2][16];
   __shared__ float s_cos[128], s_sin[128];   // the token's angles, one per rotated pair of a head
   const int t = blockIdx.x;
   const float* row = proj + (int64_t)t * ld;
-  const int pos = tok_pos[t];
+  const int pos = tok_pos[t], item = tok_item[t];
+  const int angles = rot_dims / 2;
+  float freq = 0.f;
+  if (angles > 0) freq = freqs[(int)threadIdx.x < angles ? (int)threadIdx.x : angles - 1];
+  read_arguments(pos, item, q_col, k_col, v_col, q_out, q_stride, k_pool, v_pool, q_gamma, k_gamma, eps, v_first, v_lambda,
+                 v_mode, tables, table_width, heads, kv_heads, key_dim, value_dim, cache_dim, page_size, num_pages, v_heads,
+                 store, q_dim, q_maps);
   const int q_cols = heads * q_dim, k_cols = kv_heads * key_dim;
-  const int logical = pos / page_size;
-  int page = -1;
-  if (logical < table_width) page = tables[(int64_t)tok_item[t] * table_width + logical];
-  const bool stored = page >= 0 && page < num_pages;
+  // (the same in every lane, and asked for without a branch: a position behind the table reads its first entry)
+  const int logical = __builtin_amdgcn_readfirstlane(pos / page_size);
+  const int page = scalar_load(tables + (logical < table_width ? (int64_t)item * table_width + logical : 0));
+  float lambda = 0.f;
+  if (v_mode == 2) lambda = scalar_load(v_lambda);
   const int offset = pos - logical * page_size;
   const int half = cache_dim / 2;   // cache_dim is even
   // Queries and keys, a pair of neighbouring dimensions per thread and turn.  A pair's values
@@ -53,9 +62,15 @@ __global__ __launch_bounds__(1024) void attention_prepare_kernel(
   // step of few tokens makes one trip to memory; further pairs of a thread are read again.
   const int q_pairs = heads * half, k_pairs = store ? kv_heads * half : 0;
   struct Pair {
-    float a, b, wa, wb;
+    float a, b, wa, wb;      // (as loaded: a place that is not the head's holds what stands at another)
     int head, d0;
-    bool is_q;
+    bool is_q, has_a, has_b, weighted;
+    __device__ void settle() {
+      asm volatile("" : "+v"(a), "+v"(b));      // (waited for here, not where they are asked for)
+      if (!has_a) a = 0.f;
+      if (!has_b) b = 0.f;
+      if (!weighted) wa = wb = 1.f;
+    }
   };
   auto load_pair = [&](const int i) -> Pair {
     Pair p;
@@ -65,23 +80,47 @@ __global__ __launch_bounds__(1024) void attention_prepare_kernel(
     p.d0 = (j - p.head * half) * 2;
     // the head's own dimensions: `own` of them, from place `begin` of its row on
     const int own = p.is_q ? q_dim : key_dim;
-    const int begin = p.is_q ? (p.head % q_maps) * q_dim : 0;
+    const int begin = p.is_q && q_maps > 1 ? (p.head % q_maps) * q_dim : 0;
     const int at = p.d0 - begin;
-    const int src = (p.is_q ? q_col : k_col) + p.head * own + at;
     const float* gamma = p.is_q ? q_gamma : k_gamma;
-    const bool has_a = at >= 0 && at < own, has_b = at + 1 >= 0 && at + 1 < own;
-    p.a = has_a ? row[src] : 0.f;
-    p.b = has_b ? row[src + 1] : 0.f;
-    p.wa = (gamma && has_a) ? gamma[p.head * own + at] : 1.f;
-    p.wb = (gamma && has_b) ? gamma[p.head * own + at + 1] : 1.f;
+    p.has_a = at >= 0 && at < own;
+    p.has_b = at + 1 >= 0 && at + 1 < own;
+    p.weighted = gamma != nullptr;
+    const float* weights = p.weighted ? gamma : row + (p.is_q ? q_col : k_col);
+    const float* src = row + (p.is_q ? q_col : k_col) + p.head * own;
+    const int place_a = p.has_a ? at : 0, place_b = p.has_b ? at + 1 : 0;
+    p.a = src[place_a];
+    p.b = src[place_b];
+    p.wa = weights[p.head * own + place_a];
+    p.wb = weights[p.head * own + place_b];
     return p;
   };
   const int pairs = q_pairs + k_pairs;
-  // every head turns by the same angles: they are worked out once per token, not once per head
-  for (int i = threadIdx.x; i < rot_dims / 2; i += blockDim.x) sincosf((float)pos * freqs[i], &s_sin[i], &s_cos[i]);
   const bool has_first = (int)threadIdx.x < pairs;
   Pair first = {};
   if (has_first) first = load_pair(threadIdx.x);
+  // a place of the cached values: what is projected, and what an earlier layer left
+  const int values = store ? kv_heads * cache_dim : 0;
+  struct Value {
+    float v;
+    T before;
+    int head, d;
+  };
+  auto load_value = [&](const int i) -> Value {
+    Value p = {};
+    p.head = i / cache_dim;
+    p.d = i - p.head * cache_dim;
+    const int d = p.d < value_dim ? p.d : 0;
+    p.v = row[v_col + (v_heads < kv_heads ? p.head % v_heads : p.head) * value_dim + d];
+    if (v_mode == 2) p.before = v_first[((int64_t)t * kv_heads + p.head) * value_dim + d];
+    return p;
+  };
+  Value first_value = {};
+  if ((int)threadIdx.x < values) first_value = load_value(threadIdx.x);
+  // every head turns by the same angles: they are worked out once per token, not once per head
+  if ((int)threadIdx.x < angles) sincosf((float)pos * freq, &s_sin[threadIdx.x], &s_cos[threadIdx.x]);
+  for (int i = threadIdx.x + threads; i < angles; i += threads) sincosf((float)pos * freqs[i], &s_sin[i], &s_cos[i]);
+  first.settle();
   float q_inv = 1.f, k_inv = 1.f;
   if (q_gamma != nullptr || k_gamma != nullptr) {
     float q_sum = 0.f, k_sum = 0.f;
@@ -89,33 +128,34 @@ __global__ __launch_bounds__(1024) void attention_prepare_kernel(
       const float sq = first.a * first.a + first.b * first.b;
       if (first.is_q) q_sum = sq; else k_sum = sq;
     }
-    for (int i = threadIdx.x + blockDim.x; i < pairs; i += blockDim.x) {
-      const Pair p = load_pair(i);
+    for (int i = threadIdx.x + threads; i < pairs; i += threads) {
+      Pair p = load_pair(i);
+      p.settle();
       const float sq = p.a * p.a + p.b * p.b;
       if (p.is_q) q_sum += sq; else k_sum += sq;
     }
     q_sum = wave_sum(q_sum);
     k_sum = wave_sum(k_sum);
-    const int wave = threadIdx.x >> 6;
-    const int waves = (blockDim.x + 63) >> 6;
-    if ((threadIdx.x & 63) == 0) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = (threads + 63) >> 6;
+    if (lane == 0) {
       red[0][wave] = q_sum;
       red[1][wave] = k_sum;
     }
     __syncthreads();
-    q_sum = 0.f;
-    k_sum = 0.f;
-    for (int w = 0; w < waves; ++w) {
-      q_sum += red[0][w];
-      k_sum += red[1][w];
-    }
+    q_sum = read_lane(lanes_sum<16>(lane < waves ? red[0][lane] : 0.f), 0);
+    k_sum = read_lane(lanes_sum<16>(lane < waves ? red[1][lane] : 0.f), 0);
     if (q_gamma != nullptr) q_inv = 1.0f / sqrtf(q_sum / (float)q_cols + eps);
     if (k_gamma != nullptr) k_inv = 1.0f / sqrtf(k_sum / (float)k_cols + eps);
   } else {
     __syncthreads();      // the angles
   }
-  for (int i = threadIdx.x; i < pairs; i += blockDim.x) {
-    const Pair p = i == (int)threadIdx.x ? first : load_pair(i);
+  const bool stored = logical < table_width && page >= 0 && page < num_pages;
+  for (int i = threadIdx.x; i < pairs; i += threads) {
+    Pair p = first;
+    if (i != (int)threadIdx.x) {
+      p = load_pair(i);
+      p.settle();
+    }
     const float inv = p.is_q ? q_inv : k_inv;
     const float a = p.a * inv * p.wa, b = p.b * inv * p.wb;
     const bool turned = p.d0 + 1 < rot_dims;
@@ -132,19 +172,15 @@ __global__ __launch_bounds__(1024) void attention_prepare_kernel(
       dst[1] = from_float<T>(rb);
     }
   }
-  const float lambda = v_mode == 2 ? v_lambda[0] : 0.f;
-  for (int i = threadIdx.x; i < (store ? kv_heads * cache_dim : 0); i += blockDim.x) {
-    const int head = i / cache_dim;
-    const int d = i - head * cache_dim;
-    float v = 0.f;
-    if (d < value_dim) {
-      v = row[v_col + (head % v_heads) * value_dim + d];
-      const int64_t at = ((int64_t)t * kv_heads + head) * value_dim + d;
-      if (v_mode == 1) v_first[at] = from_float<T>(v);
-      if (v_mode == 2) v = (1.f - lambda) * v + lambda * to_float<T>(v_first[at]);
+  for (int i = threadIdx.x; i < values; i += threads) {
+    const Value p = i == (int)threadIdx.x ? first_value : load_value(i);
+    float v = p.d < value_dim ? p.v : 0.f;
+    if (p.d < value_dim) {
+      if (v_mode == 1) v_first[((int64_t)t * kv_heads + p.head) * value_dim + p.d] = from_float<T>(v);
+      if (v_mode == 2) v = (1.f - lambda) * v + lambda * to_float<T>(p.before);
     }
     if (stored)
-      v_pool[(((int64_t)page * kv_heads + head) * page_size + offset) * cache_dim + d] = from_float<T>(v);
+      v_pool[(((int64_t)page * kv_heads + p.head) * page_size + offset) * cache_dim + p.d] = from_float<T>(v);
   }
 }
 
@@ -190,16 +226,16 @@ extern "C" int ps_attention_prepare(const float* proj, int64_t ld, int q_col, in
   int threads = widest >= 1024 ? 1024 : (widest + 63) / 64 * 64;
   if (tokens > 256 && threads > 256) threads = 256;   // (many rows fill the chip anyway)
   if (dtype == PS_F32)
-    hipLaunchKernelGGL(attention_prepare_kernel<float>, dim3(tokens), dim3(threads), 0, s, proj, ld, q_col,
-                       k_col, v_col, (float*)q_out, q_stride, (float*)k_pool, (float*)v_pool, q_gamma,
-                       k_gamma, eps, freqs, rot_dims, (float*)v_first, v_lambda, v_mode, tok_item,
-                       tok_pos, tables, table_width, heads, kv_heads, key_dim, value_dim, cache_dim,
+    hipLaunchKernelGGL(attention_prepare_kernel<float>, dim3(tokens), dim3(threads), 0, s, proj, ld, tok_pos,
+                       tok_item, freqs, rot_dims, threads, q_col, k_col, v_col, (float*)q_out, q_stride,
+                       (float*)k_pool, (float*)v_pool, q_gamma, k_gamma, eps, (float*)v_first, v_lambda, v_mode,
+                       tables, table_width, heads, kv_heads, key_dim, value_dim, cache_dim,
                        page_size, num_pages, v_heads, store, q_dim, q_maps);
   else
-    hipLaunchKernelGGL(attention_prepare_kernel<bf16_t>, dim3(tokens), dim3(threads), 0, s, proj, ld, q_col,
-                       k_col, v_col, (bf16_t*)q_out, q_stride, (bf16_t*)k_pool, (bf16_t*)v_pool,
-                       q_gamma, k_gamma, eps, freqs, rot_dims, (bf16_t*)v_first, v_lambda, v_mode,
-                       tok_item, tok_pos, tables, table_width, heads, kv_heads, key_dim, value_dim,
+    hipLaunchKernelGGL(attention_prepare_kernel<bf16_t>, dim3(tokens), dim3(threads), 0, s, proj, ld, tok_pos,
+                       tok_item, freqs, rot_dims, threads, q_col, k_col, v_col, (bf16_t*)q_out, q_stride,
+                       (bf16_t*)k_pool, (bf16_t*)v_pool, q_gamma, k_gamma, eps, (bf16_t*)v_first, v_lambda, v_mode,
+                       tables, table_width, heads, kv_heads, key_dim, value_dim,
                        cache_dim, page_size, num_pages, v_heads, store, q_dim, q_maps);
   PS_CHECK_LAUNCH("ps_attention_prepare");
   return 0;
@@ -273,18 +309,25 @@ __device__ inline RotationPlace rotation_place(int d, int rot_dims, bool halves)
 // at a time, all of whose loads are on their way together, a lane NR dimensions of each.
 template <typename T, int NR, int HB>
 __global__ __launch_bounds__(1024) void attention_prepare_heads_kernel(
-    const float* __restrict__ proj, int64_t ld, int q_col, int k_col, int v_col,
+    const float* __restrict__ proj, int64_t ld, const int* __restrict__ tok_pos, const int* __restrict__ tok_item,
+    const float* __restrict__ freqs, int rot_dims, int threads, int q_col, int k_col, int v_col,
     T* __restrict__ q_out, int64_t q_stride, T* __restrict__ k_pool, T* __restrict__ v_pool,
-    const float* __restrict__ freqs, int rot_dims, int halves, float magnitude, int head_norm,
+    int halves, float magnitude, int head_norm,
     const float* __restrict__ q_gamma, const float* __restrict__ k_gamma, float eps,
-    const int* __restrict__ tok_item, const int* __restrict__ tok_pos,
     const int* __restrict__ tables, int table_width, int heads, int kv_heads, int key_dim,
     int value_dim, int cache_dim, int page_size, int num_pages) {
   __shared__ float s_cos[128], s_sin[128];
   const int t = blockIdx.x;
   const float* row = proj + (int64_t)t * ld;
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = threads >> 6;
+  // (the trips as in attention_prepare_kernel)
+  const int pos = tok_pos[t], item = tok_item[t];
+  const int angles = rot_dims / 2;
+  float freq = 0.f;
+  if (angles > 0) freq = freqs[(int)threadIdx.x < angles ? (int)threadIdx.x : angles - 1];
+  read_arguments(pos, item, q_col, k_col, v_col, q_out, q_stride, k_pool, v_pool, halves, magnitude, head_norm, q_gamma,
+                 k_gamma, eps, tables, table_width, heads, kv_heads, key_dim, value_dim, cache_dim, page_size, num_pages);
   const int total = heads + 2 * kv_heads;      // query heads, key heads, value heads
   float value[HB][NR], other[HB][NR];          // a lane's dimensions, and the other ones of their pairs
   int partner[NR];
@@ -309,13 +352,11 @@ __global__ __launch_bounds__(1024) void attention_prepare_heads_kernel(
       }
     }
   };
-  load(wave);
-  const int pos = tok_pos[t];
-  const int logical = pos / page_size;
-  int page = -1;
-  if (logical < table_width) page = tables[(int64_t)tok_item[t] * table_width + logical];
-  const bool stored = page >= 0 && page < num_pages;
+  // (the same in every lane, and asked for without a branch: a position behind the table reads its first entry)
+  const int logical = __builtin_amdgcn_readfirstlane(pos / page_size);
+  const int page = scalar_load(tables + (logical < table_width ? (int64_t)item * table_width + logical : 0));
   const int offset = pos - logical * page_size;
+  load(wave);
   // weights of a lane's dimensions: of the queries' norm, of the keys', and of the pairs' other ones
   float q_weight[NR], k_weight[NR], q_other[NR], k_other[NR];
 #pragma unroll
@@ -326,13 +367,14 @@ __global__ __launch_bounds__(1024) void attention_prepare_heads_kernel(
     q_other[r] = q_gamma != nullptr && partner[r] >= 0 ? q_gamma[partner[r]] : 1.f;
     k_other[r] = k_gamma != nullptr && partner[r] >= 0 ? k_gamma[partner[r]] : 1.f;
   }
-  for (int i = threadIdx.x; i < rot_dims / 2; i += blockDim.x) {
+  for (int i = threadIdx.x; i < angles; i += threads) {
     float sn, cs;
-    sincosf((float)pos * freqs[i], &sn, &cs);
+    sincosf((float)pos * (i == (int)threadIdx.x ? freq : freqs[i]), &sn, &cs);
     s_cos[i] = cs * magnitude;
     s_sin[i] = sn * magnitude;
   }
   __syncthreads();
+  const bool stored = logical < table_width && page >= 0 && page < num_pages;
   float turn_cos[NR], turn_sin[NR];      // (the sine with its sign)
 #pragma unroll
   for (int r = 0; r < NR; ++r) {
@@ -429,10 +471,10 @@ extern "C" int ps_attention_prepare_heads(const float* proj, int64_t ld, int q_c
   const int threads = tokens <= 256 ? 64 * (total < 16 ? total : 16) : 256;
 #define PS_PREPARE_HEADS(T, NR, HB)                                                                \
   hipLaunchKernelGGL((attention_prepare_heads_kernel<T, NR, HB>), dim3(tokens), dim3(threads), 0, s, proj, \
-                     ld, q_col, k_col, v_col, (T*)q_out, q_stride, (T*)k_pool, (T*)v_pool, freqs,   \
-                     rot_dims, halves, magnitude, head_norm, q_gamma, k_gamma, eps, tok_item,       \
-                     tok_pos, tables, table_width, heads, kv_heads, key_dim, value_dim, cache_dim,  \
-                     page_size, num_pages)
+                     ld, tok_pos, tok_item, freqs, rot_dims, threads, q_col, k_col, v_col,          \
+                     (T*)q_out, q_stride, (T*)k_pool, (T*)v_pool, halves, magnitude, head_norm,     \
+                     q_gamma, k_gamma, eps, tables, table_width, heads, kv_heads, key_dim,          \
+                     value_dim, cache_dim, page_size, num_pages)
 #define PS_PREPARE_HEADS_OF(T)                       \
   do {                                               \
     if (cache_dim <= 64) PS_PREPARE_HEADS(T, 1, 5);  \
@@ -459,55 +501,80 @@ extern "C" int ps_attention_prepare_heads(const float* proj, int64_t ld, int q_c
 // so that a query's product with a key row is the score, and the weighted sum of the key rows
 // holds the weighted latent in its first `rank` places.  A block per token.
 template <typename T>
-__global__ __launch_bounds__(256) void latent_prepare_kernel(
-    const float* __restrict__ proj, int64_t ld, const float* __restrict__ queries, int64_t queries_ld,
-    int q_col, int kv_col, T* __restrict__ q_out,
-    int64_t q_stride, T* __restrict__ k_pool, const float* __restrict__ gamma, float eps,
-    const float* __restrict__ freqs, int rot_dims, int halves, float magnitude,
-    const int* __restrict__ tok_item, const int* __restrict__ tok_pos,
+__global__ __launch_bounds__(1024) void latent_prepare_kernel(
+    const float* __restrict__ proj, int64_t ld, const int* __restrict__ tok_pos, const int* __restrict__ tok_item,
+    const float* __restrict__ freqs, int rot_dims, int threads, int q_col, int kv_col,
+    const float* __restrict__ queries, int64_t queries_ld, T* __restrict__ q_out,
+    int64_t q_stride, T* __restrict__ k_pool, const float* __restrict__ gamma, float eps, int halves, float magnitude,
     const int* __restrict__ tables, int table_width, int heads, int dim, int rank, int cache_dim,
     int page_size, int num_pages) {
   __shared__ float s_cos[128], s_sin[128];
-  __shared__ float scratch[16];
+  __shared__ __attribute__((aligned(16))) float scratch[16];
   const int t = blockIdx.x;
   const float* row = proj + (int64_t)t * ld;
+  // (the trips as in attention_prepare_kernel)
+  const int pos = tok_pos[t], item = tok_item[t];
+  const int angles = rot_dims / 2;
+  float freq = 0.f;
+  if (angles > 0) freq = freqs[(int)threadIdx.x < angles ? (int)threadIdx.x : angles - 1];
+  read_arguments(pos, item, q_col, kv_col, queries, queries_ld, q_out, q_stride, k_pool, gamma, eps, halves, magnitude,
+                 tables, table_width, heads, dim, rank, cache_dim, page_size, num_pages);
   const float* q_row = queries + (int64_t)t * queries_ld;
-  const int pos = tok_pos[t];
-  const int logical = pos / page_size;
-  int page = -1;
-  if (logical < table_width) page = tables[(int64_t)tok_item[t] * table_width + logical];
-  const bool stored = page >= 0 && page < num_pages;
+  // (the same in every lane, and asked for without a branch: a position behind the table reads its first entry)
+  const int logical = __builtin_amdgcn_readfirstlane(pos / page_size);
+  const int page = scalar_load(tables + (logical < table_width ? (int64_t)item * table_width + logical : 0));
   const int offset = pos - logical * page_size;
-  for (int i = threadIdx.x; i < rot_dims / 2; i += blockDim.x) {
+  // a thread's first value of the latent, and its first place of the rotated parts: vector 0 is the key's, vector 1 + h
+  // the query's of head h
+  const int first = (int)threadIdx.x < rank ? (int)threadIdx.x : rank - 1;
+  const float latent = row[kv_col + first], weight = gamma[first];
+  struct Turned {
+    float v, other;
+    int vec, d;
+    RotationPlace place;
+  };
+  auto load_turned = [&](const int i) -> Turned {
+    Turned p;
+    p.vec = i / rot_dims;
+    p.d = i - p.vec * rot_dims;
+    const float* src = p.vec == 0 ? row + kv_col + rank : q_row + q_col + (p.vec - 1) * (dim + rot_dims) + dim;
+    p.place = rotation_place(p.d, rot_dims, halves != 0);
+    p.v = src[p.d];
+    p.other = src[p.place.partner];
+    return p;
+  };
+  const int turned = (heads + 1) * rot_dims;
+  Turned first_turned = {};
+  if ((int)threadIdx.x < turned) first_turned = load_turned(threadIdx.x);
+  for (int i = threadIdx.x; i < angles; i += threads) {
     float sn, cs;
-    sincosf((float)pos * freqs[i], &sn, &cs);
+    sincosf((float)pos * (i == (int)threadIdx.x ? freq : freqs[i]), &sn, &cs);
     s_cos[i] = cs * magnitude;
     s_sin[i] = sn * magnitude;
   }
-  float squares = 0.f;
-  for (int i = threadIdx.x; i < rank; i += blockDim.x) squares = fmaf(row[kv_col + i], row[kv_col + i], squares);
-  const float inv = 1.0f / sqrtf(block_sum(squares, scratch) / (float)rank + eps);   // (also the barrier for the angles)
+  float squares = (int)threadIdx.x < rank ? latent * latent : 0.f;
+  for (int i = threadIdx.x + threads; i < rank; i += threads) squares = fmaf(row[kv_col + i], row[kv_col + i], squares);
+  // (also the barrier for the angles)
+  const float inv = 1.0f / sqrtf(block_total(squares, scratch, threads >> 6) / (float)rank + eps);
+  const bool stored = logical < table_width && page >= 0 && page < num_pages;
   T* key = stored ? k_pool + ((int64_t)page * page_size + offset) * cache_dim : nullptr;
   if (key != nullptr) {
-    for (int i = threadIdx.x; i < rank; i += blockDim.x)
+    if ((int)threadIdx.x < rank) key[threadIdx.x] = from_float<T>(latent * inv * weight);
+    for (int i = threadIdx.x + threads; i < rank; i += threads)
       key[i] = from_float<T>(row[kv_col + i] * inv * gamma[i]);
-    for (int i = rank + rot_dims + threadIdx.x; i < cache_dim; i += blockDim.x) key[i] = from_float<T>(0.f);
+    for (int i = rank + rot_dims + threadIdx.x; i < cache_dim; i += threads) key[i] = from_float<T>(0.f);
   }
-  // the rotated parts: vector 0 is the key's, vector 1 + h the query's of head h
   const int behind = cache_dim - rank - rot_dims;
-  for (int i = threadIdx.x; i < (heads + 1) * rot_dims; i += blockDim.x) {
-    const int vec = i / rot_dims;
-    const int d = i - vec * rot_dims;
-    const float* src = vec == 0 ? row + kv_col + rank : q_row + q_col + (vec - 1) * (dim + rot_dims) + dim;
-    const RotationPlace place = rotation_place(d, rot_dims, halves != 0);
-    const float v = src[d] * s_cos[place.angle] + place.sign * src[place.partner] * s_sin[place.angle];
-    if (vec == 0) {
-      if (key != nullptr) key[rank + d] = from_float<T>(v);
+  for (int i = threadIdx.x; i < turned; i += threads) {
+    const Turned p = i == (int)threadIdx.x ? first_turned : load_turned(i);
+    const float v = p.v * s_cos[p.place.angle] + p.place.sign * p.other * s_sin[p.place.angle];
+    if (p.vec == 0) {
+      if (key != nullptr) key[rank + p.d] = from_float<T>(v);
     } else {
-      q_out[(int64_t)t * q_stride + (int64_t)(vec - 1) * cache_dim + rank + d] = from_float<T>(v);
+      q_out[(int64_t)t * q_stride + (int64_t)(p.vec - 1) * cache_dim + rank + p.d] = from_float<T>(v);
     }
   }
-  for (int i = threadIdx.x; i < heads * behind; i += blockDim.x) {
+  for (int i = threadIdx.x; i < heads * behind; i += threads) {
     const int head = i / behind;
     q_out[(int64_t)t * q_stride + (int64_t)head * cache_dim + rank + rot_dims + (i - head * behind)] =
         from_float<T>(0.f);
@@ -537,16 +604,16 @@ extern "C" int ps_latent_prepare(const float* proj, int64_t ld, const float* que
   PS_REQUIRE(dtype == PS_F32 || dtype == PS_BF16, "ps_latent_prepare: unknown dtype %d", dtype);
   if (tokens == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
-  if (dtype == PS_F32)
-    hipLaunchKernelGGL(latent_prepare_kernel<float>, dim3(tokens), dim3(256), 0, s, proj, ld, queries, queries_ld, q_col,
-                       kv_col, (float*)q_out, q_stride, (float*)k_pool, gamma, eps, freqs, rot_dims,
-                       halves, magnitude, tok_item, tok_pos, tables, table_width, heads, dim, rank,
-                       cache_dim, page_size, num_pages);
-  else
-    hipLaunchKernelGGL(latent_prepare_kernel<bf16_t>, dim3(tokens), dim3(256), 0, s, proj, ld, queries, queries_ld, q_col,
-                       kv_col, (bf16_t*)q_out, q_stride, (bf16_t*)k_pool, gamma, eps, freqs, rot_dims,
-                       halves, magnitude, tok_item, tok_pos, tables, table_width, heads, dim, rank,
-                       cache_dim, page_size, num_pages);
+  // few tokens: a thread per rotated place as far as a block has them; many fill the chip with four waves each
+  const int places = (heads + 1) * rot_dims > rank ? (heads + 1) * rot_dims : rank;
+  const int threads = tokens > 256 ? 256 : (places >= 1024 ? 1024 : (places + 63) / 64 * 64);
+#define PS_LAUNCH_LP(T)                                                                                            \
+  hipLaunchKernelGGL(latent_prepare_kernel<T>, dim3(tokens), dim3(threads), 0, s, proj, ld, tok_pos, tok_item, freqs, \
+                     rot_dims, threads, q_col, kv_col, queries, queries_ld, (T*)q_out, q_stride, (T*)k_pool, gamma,   \
+                     eps, halves, magnitude, tables, table_width, heads, dim, rank, cache_dim, page_size, num_pages)
+  if (dtype == PS_F32) PS_LAUNCH_LP(float);
+  else PS_LAUNCH_LP(bf16_t);
+#undef PS_LAUNCH_LP
   PS_CHECK_LAUNCH("ps_latent_prepare");
   return 0;
 }

@@ -221,19 +221,25 @@ __device__ inline float wave_max(float v) {
   return fmaxf(fmaxf(read_lane(v, 0), read_lane(v, 16)), fmaxf(read_lane(v, 32), read_lane(v, 48)));
 }
 
-// Sum over a block of up to 1024 threads; every thread receives the total.
-// `scratch` holds at least 16 floats of shared memory.
-__device__ inline float block_sum(float v, float* scratch) {
+// Sum over a block of `waves` whole waves, up to 16; every thread receives the total.  `scratch`: as many floats of
+// shared memory, aligned to 16 bytes, which nobody else reads or writes between the barriers around this call (a
+// second sum takes a place of its own, or block_sum).  One barrier; the waves' sums meet in a row of lanes.
+__device__ inline float block_total(float v, float* scratch, int waves) {
   const int lane = threadIdx.x & (PS_WAVE - 1);
-  const int wave = threadIdx.x / PS_WAVE;
-  const int waves = (blockDim.x + PS_WAVE - 1) / PS_WAVE;
   v = wave_sum(v);
+  if (lane == 0) scratch[threadIdx.x / PS_WAVE] = v;
   __syncthreads();
-  if (lane == 0) scratch[wave] = v;
+  if (waves == 4) {
+    const float4 sums = *reinterpret_cast<const float4*>(scratch);
+    return (sums.x + sums.y) + (sums.z + sums.w);
+  }
+  return read_lane(lanes_sum<16>(lane < waves ? scratch[lane] : 0.f), 0);
+}
+
+// The same for blocks of any number of threads up to 1024, with scratch (at least 16 floats) that has been used before.
+__device__ inline float block_sum(float v, float* scratch) {
   __syncthreads();
-  float total = 0.f;
-  for (int i = 0; i < waves; ++i) total += scratch[i];
-  return total;
+  return block_total(v, scratch, (blockDim.x + PS_WAVE - 1) / PS_WAVE);
 }
 
 __device__ inline float gelu_tanh_f(float u) {
@@ -330,13 +336,25 @@ __device__ inline float gate_factor(const AttnExtras& extra, long long token, in
   return 1.0f / (1.0f + expf(-extra.gate[token * extra.gate_ld + head]));
 }
 
+// A value at an address that is the same in every lane, of memory that nobody writes while the kernel runs, by the
+// scalar unit (which the compiler takes by itself only where it sees that nothing before can have written there).
+template <typename T>
+__device__ inline T scalar_load(const T* p) {
+  return *reinterpret_cast<const __attribute__((address_space(4))) T*>(reinterpret_cast<uintptr_t>(p));
+}
+
 // Arguments that a kernel needs later are read here, while its first loads travel: left to itself the compiler reads
 // each where it is used, a trip of its own for every 64 bytes of arguments.
-__device__ inline void read_arguments() {}
+__device__ inline void argument_is_read() {}
 template <typename First, typename... Others>
-__device__ inline void read_arguments(First first, Others... others) {
+__device__ inline void argument_is_read(First first, Others... others) {
   asm volatile("" ::"s"(first));
-  read_arguments(others...);
+  argument_is_read(others...);
+}
+template <typename... T>
+__device__ inline void read_arguments(T... values) {
+  __builtin_amdgcn_sched_barrier(0);     // (not in front of the loads that stand in front)
+  argument_is_read(values...);
 }
 
 // ---- error channel -------------------------------------------------------

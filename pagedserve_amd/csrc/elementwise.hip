@@ -55,38 +55,59 @@ int ps_compute_units() {
 // launch: h0 <- h0 / sqrt(mean(h0^2) + eps) * norm_gamma.  `copy`: the rows are written there too.
 // The id of token t is ids[t], or carried[src[t]] where src[t] >= 0: a token that an earlier
 // step chose on the device and that the host has not seen yet.
+// (The chain: ids, sources and positions at once -> a carried token -> rows of both tables.  The arguments in front of
+// `out` come with the launch.)
 template <typename T>
-__global__ void embed_kernel(const T* __restrict__ table, const T* __restrict__ pos_table,
-                             const int* __restrict__ ids, const int* __restrict__ src,
+__global__ void embed_kernel(const int* __restrict__ ids, const int* __restrict__ src,
                              const int* __restrict__ carried, const int* __restrict__ positions,
-                             float* __restrict__ out, float* __restrict__ copy, int width, int vocab,
-                             float scale, const float* __restrict__ norm_gamma, float norm_eps) {
-  __shared__ float scratch[16];
+                             const T* __restrict__ table, const T* __restrict__ pos_table, int width, int vocab,
+                             float* __restrict__ out, float* __restrict__ copy, float scale,
+                             const float* __restrict__ norm_gamma, float norm_eps) {
+  constexpr int AT_ONCE = 4;       // columns of a thread whose loads leave together
+  __shared__ __attribute__((aligned(16))) float scratch[16];
   const int t = blockIdx.x;
   int id = ids[t];
-  if (src != nullptr) {
-    const int from = src[t];
-    if (from >= 0) id = carried[from];
-  }
+  const int from = src != nullptr ? src[t] : -1;
+  const int position = pos_table != nullptr ? positions[t] : 0;
+  read_arguments(out, copy, scale, norm_gamma);
+  if (from >= 0) id = carried[from];
   id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);   // never a read outside the table
   const T* row = table + (int64_t)id * width;
+  const T* prow = pos_table != nullptr ? pos_table + (int64_t)position * width : row;
   float* dst = out + (int64_t)t * width;
-  if (pos_table != nullptr) {
-    const T* prow = pos_table + (int64_t)positions[t] * width;
-    for (int i = threadIdx.x; i < width; i += blockDim.x)
-      dst[i] = to_float<T>(row[i]) * scale + to_float<T>(prow[i]);
-  } else {
-    for (int i = threadIdx.x; i < width; i += blockDim.x) dst[i] = to_float<T>(row[i]) * scale;
+  const int threads = blockDim.x;
+  float sum = 0.f;
+  for (int first = threadIdx.x; first < width; first += AT_ONCE * threads) {
+    T value[AT_ONCE], place[AT_ONCE];
+#pragma unroll
+    for (int j = 0; j < AT_ONCE; ++j) {
+      const int i = first + j * threads < width ? first + j * threads : width - 1;
+      value[j] = row[i];
+      place[j] = prow[i];
+    }
+#pragma unroll
+    for (int j = 0; j < AT_ONCE; ++j) {
+      const int i = first + j * threads;
+      float v = to_float<T>(value[j]) * scale;
+      if (pos_table != nullptr) v += to_float<T>(place[j]);
+      if (i >= width) continue;
+      dst[i] = v;
+      if (norm_gamma == nullptr && copy != nullptr) copy[(int64_t)t * width + i] = v;
+      sum = fmaf(v, v, sum);
+    }
   }
+  if (norm_gamma == nullptr) return;
   // (each thread reads back what it wrote itself)
-  if (norm_gamma != nullptr) {
-    float sum = 0.f;
-    for (int i = threadIdx.x; i < width; i += blockDim.x) sum = fmaf(dst[i], dst[i], sum);
-    const float inv = 1.0f / sqrtf(block_sum(sum, scratch) / (float)width + norm_eps);
-    for (int i = threadIdx.x; i < width; i += blockDim.x) dst[i] = dst[i] * inv * norm_gamma[i];
-  }
-  if (copy != nullptr)
-    for (int i = threadIdx.x; i < width; i += blockDim.x) copy[(int64_t)t * width + i] = dst[i];
+  const float inv = 1.0f / sqrtf(block_sum(sum, scratch) / (float)width + norm_eps);
+  for (int first = threadIdx.x; first < width; first += AT_ONCE * threads)
+#pragma unroll
+    for (int j = 0; j < AT_ONCE; ++j) {
+      const int i = first + j * threads;
+      if (i >= width) continue;
+      const float v = dst[i] * inv * norm_gamma[i];
+      dst[i] = v;
+      if (copy != nullptr) copy[(int64_t)t * width + i] = v;
+    }
 }
 
 extern "C" int ps_embed(const void* table, const void* pos_table, const int* ids, const int* src,
@@ -103,13 +124,13 @@ extern "C" int ps_embed(const void* table, const void* pos_table, const int* ids
   const int threads = width >= 256 ? 256 : 64;
   hipStream_t s = (hipStream_t)stream;
   if (dtype == PS_F32)
-    hipLaunchKernelGGL(embed_kernel<float>, dim3(tokens), dim3(threads), 0, s, (const float*)table,
-                       (const float*)pos_table, ids, src, carried, positions, out, copy, width, vocab,
-                       scale, norm_gamma, norm_eps);
+    hipLaunchKernelGGL(embed_kernel<float>, dim3(tokens), dim3(threads), 0, s, ids, src, carried, positions,
+                       (const float*)table, (const float*)pos_table, width, vocab, out, copy, scale, norm_gamma,
+                       norm_eps);
   else
-    hipLaunchKernelGGL(embed_kernel<bf16_t>, dim3(tokens), dim3(threads), 0, s,
-                       (const bf16_t*)table, (const bf16_t*)pos_table, ids, src, carried,
-                       positions, out, copy, width, vocab, scale, norm_gamma, norm_eps);
+    hipLaunchKernelGGL(embed_kernel<bf16_t>, dim3(tokens), dim3(threads), 0, s, ids, src, carried, positions,
+                       (const bf16_t*)table, (const bf16_t*)pos_table, width, vocab, out, copy, scale, norm_gamma,
+                       norm_eps);
   PS_CHECK_LAUNCH("ps_embed");
   return 0;
 }
@@ -174,7 +195,7 @@ __global__ __launch_bounds__(256) void norm_wave_kernel(
 // waves share a row and meet through LDS: one where rows are many, four where they are few and what
 // counts is the one trip to memory (then a thread holds one or two pieces).  Measured, in us, single
 // values per lane before and now: 64 x 768 3.3 / 2.85, 544 x 1024 3.7 / 3.1, 2048 x 768 4.5 / 4.2, 4096 x
-// 1600 11.9 / 10.6.  Short rows, a handful of values per lane either way, stay with norm_wave_kernel (launch_norm
+// 1600 11.9 / 10.6; with one barrier to a sum 64 x 768 in a decode step 3.0 -> 2.4.  Short rows, a handful of values per lane either way, stay with norm_wave_kernel (launch_norm
 // says up to where).
 template <typename T>
 __device__ inline void store4(T* out, const float* v);
@@ -192,7 +213,7 @@ __global__ __launch_bounds__(256) void norm_vec_kernel(
     const float* __restrict__ x, const int* __restrict__ rows, const float* __restrict__ gamma,
     const float* __restrict__ beta, T* __restrict__ out, int n_rows, int width, float eps,
     int packed) {
-  __shared__ float scratch[16];
+  __shared__ __attribute__((aligned(16))) float scratch[2][WAVES];    // a place for each of the two sums
   const int at = WAVES == 1 ? threadIdx.x & 63 : threadIdx.x;
   const int r = WAVES == 1 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
   if (WAVES == 1 && r >= n_rows) return;
@@ -214,7 +235,7 @@ __global__ __launch_bounds__(256) void norm_vec_kernel(
 #pragma unroll
     for (int i = 0; i < PIECES; ++i)
       if ((at + i * 64 * WAVES) * 4 < width) sum += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
-    mean = (WAVES == 1 ? wave_sum(sum) : block_sum(sum, scratch)) / (float)width;
+    mean = (WAVES == 1 ? wave_sum(sum) : block_total(sum, scratch[0], WAVES)) / (float)width;
   }
   float sq = 0.f;
 #pragma unroll
@@ -226,7 +247,7 @@ __global__ __launch_bounds__(256) void norm_vec_kernel(
       sq = fmaf(v[i][j], v[i][j], sq);
     }
   }
-  const float total = WAVES == 1 ? wave_sum(sq) : block_sum(sq, scratch);
+  const float total = WAVES == 1 ? wave_sum(sq) : block_total(sq, scratch[1], WAVES);
   const float inv_std = 1.0f / sqrtf(total / (float)width + eps);
 #pragma unroll
   for (int i = 0; i < PIECES; ++i) {
@@ -251,7 +272,7 @@ template <typename T, bool RMS, int VPT>
 __global__ __launch_bounds__(256) void norm_row_kernel(
     const float* __restrict__ x, const int* __restrict__ rows, const float* __restrict__ gamma,
     const float* __restrict__ beta, T* __restrict__ out, int width, float eps, int packed) {
-  __shared__ float scratch[16];
+  __shared__ __attribute__((aligned(16))) float scratch[16];
   const int r = blockIdx.x;
   const float* src = x + (int64_t)(rows ? rows[r] : r) * width;
   float v[VPT], g[VPT], b[VPT];
@@ -295,7 +316,7 @@ template <typename T, bool RMS>
 __global__ void norm_block_kernel(const float* __restrict__ x, const int* __restrict__ rows,
                                   const float* __restrict__ gamma, const float* __restrict__ beta,
                                   T* __restrict__ out, int width, float eps) {
-  __shared__ float scratch[16];
+  __shared__ __attribute__((aligned(16))) float scratch[16];
   const int r = blockIdx.x;
   const float* src = x + (int64_t)(rows ? rows[r] : r) * width;
   T* dst = out + (int64_t)r * width;

@@ -209,7 +209,7 @@ __global__ __launch_bounds__(256) void row_norm_gate_kernel(
     const float* __restrict__ o, const float* __restrict__ w, float eps,
     const float* __restrict__ gate, int64_t gate_ld, T* __restrict__ out, int64_t out_stride,
     int columns) {
-  __shared__ float scratch[16];
+  __shared__ __attribute__((aligned(16))) float scratch[16];
   const int t = blockIdx.x;
   const float* row = o + (int64_t)t * columns;
   float sum = 0.f;

@@ -630,7 +630,7 @@ struct OutputArgs {
 // group's last column where a thread has none).
 template <typename T, int LANES, int HELD>
 __global__ __launch_bounds__(256) void state_output_kernel(const OutputArgs p, T* __restrict__ out) {
-  __shared__ float scratch[16];
+  __shared__ __attribute__((aligned(16))) float scratch[16];
   const int groups = p.heads * p.value_dim / p.group;
   const int64_t index = LANES == 64 ? (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6) : (int64_t)blockIdx.x;
   const int lane = threadIdx.x % LANES;

@@ -16,62 +16,79 @@
 // one column.  A product's sum added, normed and cleared, with 256 threads to a row and a trip per operand before and
 // now, in us: 8 x 768 4.0 / 3.2, 8 x 4096 10.5 / 4.3, 2048 x 768 8.3 / 7.0, 2048 x 1600 17.4 / 15.0.  HELD = 0:
 // rows longer than a block holds.
+// The arguments in front of `column_scale` come with the launch; the rarer operands, whose addresses have to be read
+// first, are asked for behind the others (8 x 768 in a decode step 4.3 -> 2.9 us).
+#define SS_PIECES 1         // column_scale, rows, bias or gamma2 is there
+#define SS_WAVES(form) ((form) >> 1)
 template <typename T, int HELD>
 __global__ __launch_bounds__(1024) void stream_step_kernel(
-    float* __restrict__ h, const float* y, float factor, const float* __restrict__ column_scale,
-    const float* __restrict__ rows, const float* __restrict__ bias, const float* __restrict__ gamma, float eps,
-    T* __restrict__ normed, const float* __restrict__ gamma2, T* __restrict__ normed2, float* zero, int width) {
-  __shared__ float scratch[16];
+    float* __restrict__ h, const float* y, float* zero, const float* __restrict__ gamma, T* __restrict__ normed,
+    float factor, float eps, int width, int form, const float* __restrict__ column_scale,
+    const float* __restrict__ rows, const float* __restrict__ bias, const float* __restrict__ gamma2,
+    T* __restrict__ normed2) {
+  __shared__ __attribute__((aligned(16))) float scratch[16];
   const int64_t t = blockIdx.x;
+  const int waves = SS_WAVES(form), threads = waves * 64;
   float* row = h + t * width;
   float sum = 0.f;
   if constexpr (HELD > 0) {
     const float* y_row = y != nullptr ? y + t * width : row;
-    const float* rows_row = rows != nullptr ? rows + t * width : row;
-    const float* column = column_scale != nullptr ? column_scale : row;
-    const float* bias_row = bias != nullptr ? bias : row;
     const float* scale_row = gamma != nullptr ? gamma : row;
-    const float* scale2_row = gamma2 != nullptr ? gamma2 : row;
     float held[HELD], vy[HELD], vc[HELD], vr[HELD], vb[HELD], scale[HELD], scale2[HELD];
 #pragma unroll
     for (int i = 0; i < HELD; ++i) {
-      const int at = threadIdx.x + blockDim.x * i;
+      const int at = threadIdx.x + threads * i;
       const int d = at < width ? at : width - 1;
       held[i] = row[d];
       vy[i] = y_row[d];
-      vc[i] = column[d];
-      vr[i] = rows_row[d];
-      vb[i] = bias_row[d];
       scale[i] = scale_row[d];
-      scale2[i] = scale2_row[d];
     }
+    if (form & SS_PIECES) {
+      const float* rows_row = rows != nullptr ? rows + t * width : row;
+      const float* column = column_scale != nullptr ? column_scale : row;
+      const float* bias_row = bias != nullptr ? bias : row;
+      const float* scale2_row = gamma2 != nullptr ? gamma2 : row;
+#pragma unroll
+      for (int i = 0; i < HELD; ++i) {
+        const int at = threadIdx.x + threads * i;
+        const int d = at < width ? at : width - 1;
+        vc[i] = column[d];
+        vr[i] = rows_row[d];
+        vb[i] = bias_row[d];
+        scale2[i] = scale2_row[d];
+      }
+    }
+    const bool changed = y != nullptr || ((form & SS_PIECES) && (rows != nullptr || bias != nullptr));
 #pragma unroll
     for (int i = 0; i < HELD; ++i) {
-      const int d = threadIdx.x + blockDim.x * i;
-      float v = held[i];
-      if (y != nullptr) v = fmaf(column_scale != nullptr ? factor * vc[i] : factor, vy[i], v);
-      if (rows != nullptr) v += vr[i];
-      if (bias != nullptr) v += vb[i];
+      const int d = threadIdx.x + threads * i;
+      float v = held[i], by = factor;
+      if ((form & SS_PIECES) && column_scale != nullptr) by *= vc[i];
+      if (y != nullptr) v = fmaf(by, vy[i], v);
+      if (form & SS_PIECES) {
+        if (rows != nullptr) v += vr[i];
+        if (bias != nullptr) v += vb[i];
+      }
       if (d < width) {
-        if (y != nullptr || rows != nullptr || bias != nullptr) row[d] = v;
+        if (changed) row[d] = v;
         if (zero != nullptr) zero[t * width + d] = 0.f;
         sum = fmaf(v, v, sum);
       }
       held[i] = v;
     }
     if (gamma == nullptr) return;
-    const float inv = 1.0f / sqrtf(block_sum(sum, scratch) / (float)width + eps);
+    const float inv = 1.0f / sqrtf(block_total(sum, scratch, waves) / (float)width + eps);
 #pragma unroll
     for (int i = 0; i < HELD; ++i) {
-      const int d = threadIdx.x + blockDim.x * i;
+      const int d = threadIdx.x + threads * i;
       if (d < width) {
         normed[t * width + d] = from_float<T>(held[i] * inv * scale[i]);
-        if (gamma2 != nullptr) normed2[t * width + d] = from_float<T>(held[i] * inv * scale2[i]);
+        if ((form & SS_PIECES) && gamma2 != nullptr) normed2[t * width + d] = from_float<T>(held[i] * inv * scale2[i]);
       }
     }
     return;
   }
-  for (int d = threadIdx.x; d < width; d += blockDim.x) {
+  for (int d = threadIdx.x; d < width; d += threads) {
     float v = row[d];
     if (y != nullptr) v = fmaf(column_scale ? factor * column_scale[d] : factor, y[t * width + d], v);
     if (rows != nullptr) v += rows[t * width + d];
@@ -81,9 +98,9 @@ __global__ __launch_bounds__(1024) void stream_step_kernel(
     sum = fmaf(v, v, sum);
   }
   if (gamma == nullptr) return;
-  const float inv = 1.0f / sqrtf(block_sum(sum, scratch) / (float)width + eps);
+  const float inv = 1.0f / sqrtf(block_total(sum, scratch, waves) / (float)width + eps);
   // (each thread reads back what it wrote itself)
-  for (int d = threadIdx.x; d < width; d += blockDim.x) {
+  for (int d = threadIdx.x; d < width; d += threads) {
     const float v = row[d] * inv;
     normed[t * width + d] = from_float<T>(v * gamma[d]);
     if (gamma2 != nullptr) normed2[t * width + d] = from_float<T>(v * gamma2[d]);
@@ -121,7 +138,7 @@ __global__ __launch_bounds__(256) void silu_columns_kernel(float* __restrict__ p
 __global__ __launch_bounds__(256) void pair_norm_mix_kernel(
     float* __restrict__ a, float* __restrict__ b, const float* __restrict__ wa,
     const float* __restrict__ wb, float eps, float share, float* __restrict__ y, int width) {
-  __shared__ float scratch_a[16], scratch_b[16];
+  __shared__ __attribute__((aligned(16))) float scratch_a[16], scratch_b[16];
   const int64_t t = blockIdx.x;
   float* ra = a + t * width;
   float* rb = b + t * width;
@@ -158,9 +175,10 @@ extern "C" int ps_stream_step(float* h, const float* y, float factor, const floa
   int threads = width >= 1024 ? 1024 : (width + 63) / 64 * 64;
   if (tokens > 256 && width <= 256 * 8) threads = 256;
   const int held = (width + threads - 1) / threads;
+  const int form = (threads / 64) << 1 | (column_scale || rows || bias || gamma2 ? SS_PIECES : 0);
 #define PS_LAUNCH_SS(T, HELD)                                                                          \
-  hipLaunchKernelGGL((stream_step_kernel<T, HELD>), dim3(tokens), dim3(threads), 0, s, h, y, factor, \
-                     column_scale, rows, bias, gamma, eps, (T*)normed, gamma2, (T*)normed2, zero, width)
+  hipLaunchKernelGGL((stream_step_kernel<T, HELD>), dim3(tokens), dim3(threads), 0, s, h, y, zero, gamma, \
+                     (T*)normed, factor, eps, width, form, column_scale, rows, bias, gamma2, (T*)normed2)
 #define PS_LAUNCH_SS_T(T)                   \
   do {                                      \
     if (held <= 1) PS_LAUNCH_SS(T, 1);      \
@@ -237,7 +255,7 @@ __global__ __launch_bounds__(1024) void gated_norm_step_kernel(
     const float* __restrict__ gate_bias, const float* __restrict__ gamma, const float* __restrict__ beta,
     const float* __restrict__ gamma2, const float* __restrict__ beta2, float eps, T* __restrict__ normed,
     int width) {
-  __shared__ float scratch[16];
+  __shared__ __attribute__((aligned(16))) float scratch[16];
   const int64_t t = blockIdx.x;
   float* row = h + t * width;
   float x[HELD], v[HELD], scale[HELD], shift[HELD], scale2[HELD], shift2[HELD];

@@ -23,16 +23,21 @@
 // The kernel waits on memory alone (two trips at few rows: the operands, then the store's way out; the bytes at
 // many).  Nothing that is optional stands behind a branch in front of the loads, which would make them wait
 // for what was asked for before: a row of 4 x 768 without and with it, 8 rows 3.3 / 3.85 us, 2,048 rows 13.4 / 15.3.
+// The arguments in front of `normed` come with the launch, and the waves' sums meet behind one barrier: 8 rows of 4 x 768
+// in a decode step 3.3 -> 2.8 us.
+#define HS_READS 1          // normed is wanted
+#define HS_WAVES(form) ((form) >> 1)
 template <typename TOut, int STREAMS, bool writes>
 __global__ __launch_bounds__(HS_THREADS) void hyper_step_kernel(
     float* __restrict__ X, const float* __restrict__ y, const float* __restrict__ mix,
     const float* __restrict__ out_w, const float* __restrict__ in_w,
-    const float* __restrict__ gamma, float eps, TOut* __restrict__ normed,
-    float* __restrict__ zero, int width) {
+    const float* __restrict__ gamma, int width, int form, TOut* __restrict__ normed,
+    float* __restrict__ zero, float eps) {
   extern __shared__ float s_u[];
-  __shared__ float red[16];
+  __shared__ __attribute__((aligned(16))) float red[16];
   const int t = blockIdx.x;
-  const bool reads = normed != nullptr;
+  const bool reads = form & HS_READS;
+  const int waves = HS_WAVES(form), threads = waves * 64;
   float* row = X + (int64_t)t * STREAMS * width;
   // the few weights: every thread reads them itself (the same addresses in all lanes: scalar loads),
   // without a branch, which would make the copies' loads wait for them: where nothing is read the row
@@ -76,7 +81,7 @@ __global__ __launch_bounds__(HS_THREADS) void hyper_step_kernel(
     if (zero != nullptr) zero[(int64_t)t * width + col] = 0.f;
     return uu;
   };
-  if (width <= (int)blockDim.x) {
+  if (width <= threads) {
     // a thread per column: u and the norm's scale stay in registers, and the scale's load
     // leaves with the others instead of behind the sum of squares
     const int col = threadIdx.x;
@@ -84,12 +89,12 @@ __global__ __launch_bounds__(HS_THREADS) void hyper_step_kernel(
     const float g = (reads && active) ? gamma[col] : 0.f;
     const float uu = active ? column(col) : 0.f;
     if (!reads) return;
-    const float total = block_sum(uu * uu, red);
+    const float total = block_total(uu * uu, red, waves);
     const float inv = 1.0f / sqrtf(total / (float)width + eps);
     if (active) normed[(int64_t)t * width + col] = from_float<TOut>(uu * inv * g);
     return;
   }
-  for (int col = threadIdx.x; col < width; col += blockDim.x) {
+  for (int col = threadIdx.x; col < width; col += threads) {
     const float uu = column(col);
     if (reads) {
       s_u[col] = uu;
@@ -97,10 +102,10 @@ __global__ __launch_bounds__(HS_THREADS) void hyper_step_kernel(
     }
   }
   if (!reads) return;
-  const float total = block_sum(sumsq, red);
+  const float total = block_total(sumsq, red, waves);
   const float inv = 1.0f / sqrtf(total / (float)width + eps);
   // (a thread reads back the columns that it wrote itself)
-  for (int col = threadIdx.x; col < width; col += blockDim.x)
+  for (int col = threadIdx.x; col < width; col += threads)
     normed[(int64_t)t * width + col] = from_float<TOut>(s_u[col] * inv * gamma[col]);
 }
 
@@ -125,7 +130,8 @@ extern "C" int ps_hyper_step(float* x, const float* y, const float* mix, const f
   if (tokens > 256 && threads > 256) threads = 256;
 #define PS_LAUNCH_HSW(TOut, S, WRITES)                                                            \
   hipLaunchKernelGGL((hyper_step_kernel<TOut, S, WRITES>), dim3(tokens), dim3(threads), lds, s, x, \
-                     y, mix, out_w, in_w, gamma, eps, (TOut*)normed, zero, width)
+                     y, mix, out_w, in_w, gamma, width, (threads / 64) << 1 | (normed != nullptr ? HS_READS : 0),     \
+                     (TOut*)normed, zero, eps)
 #define PS_LAUNCH_HS(TOut, S)                       \
   do {                                              \
     if (y != nullptr) PS_LAUNCH_HSW(TOut, S, true); \
