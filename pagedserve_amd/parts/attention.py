@@ -649,7 +649,7 @@ class Attention(Mixer):
           ranges of 4-wave blocks, four blocks to a unit, where every head has bfloat16 keys of its own
           (``own_keys``; 16 over 2,000 keys 25.3 and 22.6, 12 over 4,000 38.6 and 31.0; heads that share keys find them in the cache: 20 of 12 heads over 4
           18.1 and 22.0; in float 39.6 and 42.3, so there from 4,096 on, just under a pair per unit, as before);
-        * fewer pairs: up to 512 keys that a block of 16 waves takes in one turn that block (one request of 12
+        * fewer pairs: up to 1,024 keys that a block of 16 waves takes in one turn that block (one request of 12
           heads over 200 and 400 keys 4.3 and 5.8, in ranges 6.0 and 6.5), beyond ranges of a turn of 4-wave blocks or
           more until three blocks come to a unit, up to 16 ranges, 32 over 64 turns (8 of 12 heads over 800 and 2,000
           keys 9.4 and 14.5, in one and two blocks of 16 waves 10.5 and 16.7; one over 4,000 keys in 16 and 32 ranges
@@ -680,7 +680,7 @@ class Attention(Mixer):
         if 2 * pairs > units:
             return (4 * units // pairs, 4) if visible >= 16 * turn and own_keys else (1, 16)
         if visible <= (2048 if 4 * pairs >= units else 8192):
-            if visible <= min(4 * turn, 512):
+            if visible <= min(4 * turn, 1024):
                 return 1, 16
             return max(1, min(3 * units // pairs, visible // turn, 32 if visible >= 64 * turn else 16)), 4
         if pairs >= units // 4:
