@@ -102,7 +102,7 @@ __global__ __launch_bounds__(256) void gemm_nt_f32_rows_kernel(
     float* __restrict__ c, int m, int n, int k, int lda, int ldc) {
   constexpr int AHEAD = 4 / COLS;
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // the same in every lane: scalar
   const int col0 = (blockIdx.x * 4 + wave) * COLS;
   if (col0 >= n) return;
   // (9 to 16 rows: the second eight are another block's)
@@ -115,31 +115,50 @@ __global__ __launch_bounds__(256) void gemm_nt_f32_rows_kernel(
   const float* a_row[MR];
 #pragma unroll
   for (int r = 0; r < MR; ++r) a_row[r] = a + (int64_t)(r < m ? r : m - 1) * lda;
+  // the output (row `own_row`, column col0 + own_j) that this lane finishes; its bias and residual value travel with
+  // the first operands
+  static_assert(COLS * MR <= 64, "one output per lane");
+  const int own_j = lane / MR, own_row = lane - own_j * MR;
+  const bool owns = own_j < COLS && own_row < m && col0 + own_j < n;
+  float* dst = c + (owns ? (int64_t)own_row * ldc + col0 + own_j : col0);
+  float own_bias = 0.f, before = 0.f;
   float acc[COLS][MR];
 #pragma unroll
   for (int j = 0; j < COLS; ++j)
 #pragma unroll
     for (int r = 0; r < MR; ++r) acc[j][r] = 0.f;
-  for (int k0 = lane * 4; k0 < k; k0 += 256 * AHEAD) {
-    float4 wv[AHEAD][COLS];
+  for (int k0 = lane * 4; k0 - lane * 4 < k; k0 += 256 * AHEAD) {
+    // (unconditional, from a place that exists: nothing waits for a branch; a row's values of the next step are
+    // asked for in front of this step's sums)
+    float4 wv[AHEAD][COLS], av[2][MR];
+    auto place = [&](int u) { return k0 + 256 * u < k ? k0 + 256 * u : 0; };
+    auto load_rows = [&](int u) {
+#pragma unroll
+      for (int r = 0; r < MR; ++r) av[u & 1][r] = *reinterpret_cast<const float4*>(a_row[r] + place(u));
+    };
 #pragma unroll
     for (int u = 0; u < AHEAD; ++u)
 #pragma unroll
-      for (int j = 0; j < COLS; ++j)
-        wv[u][j] = k0 + 256 * u < k ? *reinterpret_cast<const float4*>(w_row[j] + k0 + 256 * u)
-                                    : make_float4(0.f, 0.f, 0.f, 0.f);
+      for (int j = 0; j < COLS; ++j) wv[u][j] = *reinterpret_cast<const float4*>(w_row[j] + place(u));
+    load_rows(0);
+    if (k0 < 256) {
+      if (bias != nullptr) own_bias = bias[owns ? col0 + own_j : col0];
+      if (EPI == PS_EPI_RESIDUAL) before = *dst;
+    }
 #pragma unroll
     for (int u = 0; u < AHEAD; ++u) {
-      if (k0 + 256 * u >= k) break;
+      if (u + 1 < AHEAD) load_rows(u + 1);
+      if (k0 + 256 * u < k) {
 #pragma unroll
-      for (int r = 0; r < MR; ++r) {
-        const float4 av = *reinterpret_cast<const float4*>(a_row[r] + k0 + 256 * u);
+        for (int r = 0; r < MR; ++r) {
+          const float4 x = av[u & 1][r];
 #pragma unroll
-        for (int j = 0; j < COLS; ++j) {
-          acc[j][r] = fmaf(av.x, wv[u][j].x, acc[j][r]);
-          acc[j][r] = fmaf(av.y, wv[u][j].y, acc[j][r]);
-          acc[j][r] = fmaf(av.z, wv[u][j].z, acc[j][r]);
-          acc[j][r] = fmaf(av.w, wv[u][j].w, acc[j][r]);
+          for (int j = 0; j < COLS; ++j) {
+            acc[j][r] = fmaf(x.x, wv[u][j].x, acc[j][r]);
+            acc[j][r] = fmaf(x.y, wv[u][j].y, acc[j][r]);
+            acc[j][r] = fmaf(x.z, wv[u][j].z, acc[j][r]);
+            acc[j][r] = fmaf(x.w, wv[u][j].w, acc[j][r]);
+          }
         }
       }
     }
@@ -153,16 +172,10 @@ __global__ __launch_bounds__(256) void gemm_nt_f32_rows_kernel(
       const float total = wave_sum(acc[j][r]);
       if (lane == j * MR + r) mine = total;
     }
-  static_assert(COLS * MR <= 64, "one output per lane");
-  const int j = lane / MR;
-  const int r = lane - j * MR;
-  const int col = col0 + j;
-  if (j >= COLS || r >= m || col >= n) return;
-  float v = mine;
-  if (bias != nullptr) v += bias[col];
+  if (!owns) return;
+  float v = mine + own_bias;
   v = apply_activation<EPI>(v);
-  float* dst = c + (int64_t)r * ldc + col;
-  if (EPI == PS_EPI_RESIDUAL) v += *dst;
+  if (EPI == PS_EPI_RESIDUAL) v += before;
   *dst = v;
 }
 

@@ -34,44 +34,92 @@ __device__ inline float sum_in_pairs(float (&v)[N]) {
   return v[0];
 }
 
+// What the epilogue needs beside the sums (bias, residual values, page slots), asked for behind the weights' loads and
+// there when they are: behind the sums each would be a trip of its own (as SkinnyEnds, gemm_skinny.h).  Thread t
+// finishes elements t, t + 64 WAVES, ... of the block's 16 NT columns of 16 MB rows: element i of a 16 x 16 accumulator is
+// weight row (lane / 16) * 4 + i, activation row lane % 16, and 16 consecutive threads finish one run of 16 columns.
+template <int EPI, int MB, int NT, int WAVES>
+struct FloatEnds {
+  static constexpr int ELEMENTS = NT * MB * 256, COUNT = (ELEMENTS + 64 * WAVES - 1) / (64 * WAVES);
+  float bias[COUNT], before[COUNT];
+  int pos[COUNT], item[COUNT], page[COUNT];
+  bool there[COUNT];
+
+  __device__ static inline int column(int e) { return (e >> 8) / MB * 16 + (e & 15); }
+  __device__ static inline int row(int e) { return (e >> 8) % MB * 16 + ((e >> 4) & 15); }
+  __device__ inline void ask(const float* __restrict__ bias_row, const float* c, int m, int n, int ldc, int n0, int row0,
+                             int split, int k_splits, const KvScatter& scatter) {
+#pragma unroll
+    for (int it = 0; it < COUNT; ++it) {
+      const int e = threadIdx.x + it * 64 * WAVES;
+      const int col = n0 + column(e) < n ? n0 + column(e) : n - 1;
+      const int at = row0 + row(e) < m ? row0 + row(e) : m - 1;
+      bias[it] = 0.f;
+      if (bias_row != nullptr && split == 0) bias[it] = bias_row[col];
+      if (EPI == PS_EPI_RESIDUAL) {
+        before[it] = 0.f;
+        if (k_splits == 1) before[it] = c[(int64_t)at * ldc + col];
+      }
+      if (EPI == PS_EPI_NONE && scatter.k_pool != nullptr) {
+        pos[it] = scatter.tok_pos[at];
+        item[it] = scatter.tok_item[at];
+      }
+    }
+  }
+  __device__ inline void ask_pages(const KvScatter& scatter, int n0) {
+    if (EPI != PS_EPI_NONE || scatter.k_pool == nullptr || n0 + 16 * NT <= scatter.q_cols) return;
+#pragma unroll
+    for (int it = 0; it < COUNT; ++it) {
+      const int logical = scatter.page_shift >= 0 ? (pos[it] >> scatter.page_shift) : pos[it] / scatter.page_size;
+      // a row without a page reads the first entry in its place
+      there[it] = logical < scatter.table_width;
+      page[it] = scatter.tables[there[it] ? (int64_t)item[it] * scatter.table_width + logical : 0];
+    }
+  }
+};
+
 // Sum the waves' partial tiles in a fixed order and finish the block's 16 NT columns of 16 MB rows.
 template <int EPI, int MB, int NT, int WAVES>
-__device__ inline void skinny_f32_epilogue(float (&partial)[NT][WAVES][MB][4][64], const float* bias, float* c,
-                                           int m, int n, int ldc, int n0, int row0, int split,
-                                           int k_splits, const KvScatter& scatter) {
-  // element i of a 16 x 16 accumulator: weight row (lane / 16) * 4 + i, activation row lane % 16;
-  // 16 consecutive threads finish one run of 16 columns
-  for (int e = threadIdx.x; e < NT * MB * 256; e += 64 * WAVES) {
-    const int col_in = e & 15;
-    const int row_in = (e >> 4) & 15;
-    const int b = (e >> 8) % MB;
-    const int j = (e >> 8) / MB;
-    const int col = n0 + j * 16 + col_in;
-    const int row = row0 + b * 16 + row_in;
-    if (col >= n || row >= m) continue;
-    const int i = col_in & 3;
-    const int at = (col_in >> 2) * 16 + row_in;
+__device__ inline void skinny_f32_epilogue(float (&partial)[NT][WAVES][MB][4][64],
+                                           const FloatEnds<EPI, MB, NT, WAVES>& ends, float* c,
+                                           int m, int n, int ldc, int n0, int row0, int k_splits,
+                                           const KvScatter& scatter) {
+  typedef FloatEnds<EPI, MB, NT, WAVES> Ends;
+#pragma unroll
+  for (int it = 0; it < Ends::COUNT; ++it) {
+    const int e = threadIdx.x + it * 64 * WAVES;
+    const int col = n0 + Ends::column(e);
+    const int row = row0 + Ends::row(e);
+    if (e >= Ends::ELEMENTS || col >= n || row >= m) continue;
+    const int j = (e >> 8) / MB, b = (e >> 8) % MB;
+    const int i = e & 3;
+    const int at = ((e & 15) >> 2) * 16 + ((e >> 4) & 15);
     float of_wave[WAVES];
 #pragma unroll
     for (int p = 0; p < WAVES; ++p) of_wave[p] = partial[j][p][b][i][at];
-    float v = sum_in_pairs(of_wave);
-    if (bias != nullptr && split == 0) v += bias[col];
+    float v = sum_in_pairs(of_wave) + ends.bias[it];
     float* dst = c + (int64_t)row * ldc + col;
     if (EPI == PS_EPI_RESIDUAL) {
       if (k_splits > 1) unsafeAtomicAdd(dst, v);
-      else *dst += v;
+      else *dst = ends.before[it] + v;
     } else {
       v = apply_activation<EPI>(v);
       *dst = v;
-      if (EPI == PS_EPI_NONE) kv_scatter_store<float>(scatter, row, col, v);
+      if (EPI == PS_EPI_NONE && scatter.k_pool != nullptr && col >= scatter.q_cols) {
+        int64_t offset;
+        float* pool = kv_scatter_col<float>(scatter, col, &offset);
+        if (ends.there[it] && ends.page[it] >= 0 && ends.page[it] < scatter.num_pages)
+          pool[offset + kv_page_slot(scatter, ends.pos[it], ends.page[it])] = v;
+      }
     }
   }
 }
 
+// (the arguments in front of the scatter come with the launch)
 template <int EPI, int MB, int NT, int UNROLL, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void gemm_nt_skinny_f32_kernel(
     const float* __restrict__ a, const float* __restrict__ w, const float* __restrict__ bias,
-    float* __restrict__ c, int m, int n, int k, int lda, int ldc, int k_chunk, int k_splits,
+    float* __restrict__ c, int m, int n, int k, int lda, int k_chunk, int ldc, int k_splits,
     KvScatter scatter) {
   __shared__ float partial[NT][WAVES][MB][4][64];
   const int lane = threadIdx.x & 63;
@@ -107,10 +155,8 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_nt_skinny_f32_kernel(
 #pragma unroll
       for (int i = 0; i < 4 * SETS; ++i) acc[j][b][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // wave `wave` takes the steps wave, wave + WAVES, ... of the block's range; UNROLL of them are
-  // asked for together
-  for (int k0 = k_begin + wave * SF_STEP; k0 < k_end; k0 += WAVES * UNROLL * SF_STEP) {
-    f32x4 wf[UNROLL][NT][2], xf[UNROLL][MB][2];
+  f32x4 wf[UNROLL][NT][2], xf[UNROLL][MB][2];
+  auto load = [&](int k0) {
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u)
 #pragma unroll
@@ -127,6 +173,8 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_nt_skinny_f32_kernel(
       }
     // (without this the compiler asks for a few at a time, to use fewer registers)
     __builtin_amdgcn_sched_barrier(0);
+  };
+  auto multiply = [&](int k0) {
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u)
 #pragma unroll
@@ -147,7 +195,21 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_nt_skinny_f32_kernel(
               acc[j][b][(2 * u + h) % SETS * 4 + i] = __builtin_amdgcn_mfma_f32_16x16x4f32(
                   wf[u][j][h][i], xf[u][b][h][i], acc[j][b][(2 * u + h) % SETS * 4 + i], 0, 0, 0);
       }
+  };
+  // wave `wave` takes the steps wave, wave + WAVES, ... of the block's range; UNROLL of them are
+  // asked for together, the first ones in front of what the epilogue needs.  (A wave without a step asks for the range's
+  // first values and multiplies by zeros.)
+  FloatEnds<EPI, MB, NT, WAVES> ends;
+  int k0 = k_begin + wave * SF_STEP;
+  load(k0);
+  if (EPI == PS_EPI_NONE && scatter.k_pool != nullptr) read_scatter(scatter);
+  ends.ask(bias, c, m, n, ldc, n0, row0, split, k_splits, scatter);
+  multiply(k0);
+  for (k0 += WAVES * UNROLL * SF_STEP; k0 < k_end; k0 += WAVES * UNROLL * SF_STEP) {
+    load(k0);
+    multiply(k0);
   }
+  ends.ask_pages(scatter, n0);
 #pragma unroll
   for (int j = 0; j < NT; ++j)
 #pragma unroll
@@ -161,18 +223,24 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_nt_skinny_f32_kernel(
       }
   __syncthreads();
 
-  skinny_f32_epilogue<EPI, MB, NT, WAVES>(partial, bias, c, m, n, ldc, n0, row0, split, k_splits, scatter);
+  skinny_f32_epilogue<EPI, MB, NT, WAVES>(partial, ends, c, m, n, ldc, n0, row0, k_splits, scatter);
 }
 
 // The same for up to 16 rows with the norm of its input fused in front (whole k in one round of loads): while the
 // weights travel, each wave normalises up to two rows in registers (as norm_wave_kernel, elementwise.hip)
 // and leaves them in LDS, where the product reads its column operand.  One launch and one trip to memory
 // instead of two launches, in us: 1 x 2304 x 768 7.4 -> 5.3, 8 x 2304 x 768 8.7 -> 5.9, 16 x 2304 x 768
-// 11.6 -> 6.7, 8 x 4096 x 1024 16.9 -> 8.7.
+// 11.6 -> 6.7, 8 x 4096 x 1024 16.9 -> 8.7.  (The arguments in front of the bias come with the launch.)
+#define SF_ROW_BITS 16  // of the number of rows; behind it
+#define SF_RMS 1
+#define SF_SHIFT 2      // (without a shift the argument is gamma)
 template <int EPI, int UNROLL>
 __global__ __launch_bounds__(512) void gemm_nt_skinny_norm_f32_kernel(
-    const NormPrologue norm, const float* __restrict__ w, const float* __restrict__ bias,
-    float* __restrict__ c, int m, int n, int k, int ldc, KvScatter scatter) {
+    const float* __restrict__ h_rows, const float* __restrict__ gamma, const float* __restrict__ shift,
+    const float* __restrict__ w, const int* __restrict__ rows_of, int ldh, int rows_and_flags, int n, int k,
+    const float* __restrict__ bias, float* __restrict__ c, int ldc, float eps, KvScatter scatter) {
+  const int m = rows_and_flags & ((1 << SF_ROW_BITS) - 1);
+  const bool rms = (rows_and_flags >> SF_ROW_BITS) & SF_RMS, shifts = (rows_and_flags >> SF_ROW_BITS) & SF_SHIFT;
   constexpr int WAVES = 8;
   constexpr int MOST = WAVES * UNROLL * SF_STEP;     // the longest k
   constexpr int STRIDE = MOST + 4;                   // floats; the next row is four banks further
@@ -187,13 +255,11 @@ __global__ __launch_bounds__(512) void gemm_nt_skinny_norm_f32_kernel(
   const float* w_row = w + (int64_t)(n0 + sub < n ? n0 + sub : n - 1) * k;
   // The rows and the norm's scale and shift are asked for in front of the weights: a wave's loads come back in
   // the order of issue, and the norm works while the weights travel.
-  const bool shifts = !norm.rms && norm.beta != nullptr;
-  const float* shift = shifts ? norm.beta : norm.gamma;
   const bool two = m > WAVES;                        // a second row per wave
   float v[2][PIECES][4], g[PIECES][4], b[PIECES][4];
   auto load_row = [&](int half) {
     const int r = wave + half * WAVES < m ? wave + half * WAVES : m - 1;
-    const float* src = norm.h + (int64_t)(norm.rows ? norm.rows[r] : r) * norm.ldh;
+    const float* src = h_rows + (int64_t)(rows_of ? rows_of[r] : r) * ldh;
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) {
       const int col = (lane + i * 64) * 4;
@@ -201,12 +267,13 @@ __global__ __launch_bounds__(512) void gemm_nt_skinny_norm_f32_kernel(
     }
   };
   f32x4 wf[UNROLL][2];
+  FloatEnds<EPI, 1, 1, WAVES> ends;
   auto load_scale = [&] {
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) {
       const int col = (lane + i * 64) * 4;
       const int safe = col < k ? col : k - 4;
-      *reinterpret_cast<float4*>(g[i]) = *reinterpret_cast<const float4*>(norm.gamma + safe);
+      *reinterpret_cast<float4*>(g[i]) = *reinterpret_cast<const float4*>(gamma + safe);
       *reinterpret_cast<float4*>(b[i]) = *reinterpret_cast<const float4*>(shift + safe);
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -219,13 +286,16 @@ __global__ __launch_bounds__(512) void gemm_nt_skinny_norm_f32_kernel(
         const int kk = (u * WAVES + wave) * SF_STEP + h * 16 + group * 4;
         wf[u][h] = *reinterpret_cast<const f32x4*>(w_row + (kk < k ? kk : 0));
       }
+    read_arguments(bias, c, ldc, eps);
+    if (EPI == PS_EPI_NONE && scatter.k_pool != nullptr) read_scatter(scatter);
+    ends.ask(bias, c, m, n, ldc, n0, 0, 0, 1, scatter);
     __builtin_amdgcn_sched_barrier(0);
   };
   auto finish_row = [&](int half) {
     const int r = wave + half * WAVES;
     if (r >= m) return;
     float mean = 0.f;
-    if (!norm.rms) {
+    if (!rms) {
       float sum = 0.f;
 #pragma unroll
       for (int i = 0; i < PIECES; ++i)
@@ -240,7 +310,7 @@ __global__ __launch_bounds__(512) void gemm_nt_skinny_norm_f32_kernel(
         v[half][i][j] = (lane + i * 64) * 4 < k ? v[half][i][j] - mean : 0.f;
         sq = fmaf(v[half][i][j], v[half][i][j], sq);
       }
-    const float inv_std = 1.0f / sqrtf(wave_sum(sq) / (float)k + norm.eps);
+    const float inv_std = 1.0f / sqrtf(wave_sum(sq) / (float)k + eps);
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) {
       const int col = (lane + i * 64) * 4;
@@ -269,6 +339,7 @@ __global__ __launch_bounds__(512) void gemm_nt_skinny_norm_f32_kernel(
   } else {
     load_weights();
   }
+  ends.ask_pages(scatter, n0);
 #pragma unroll
   for (int u = 0; u < UNROLL; ++u)
 #pragma unroll
@@ -300,7 +371,7 @@ __global__ __launch_bounds__(512) void gemm_nt_skinny_norm_f32_kernel(
     partial[0][wave][0][i][lane] = sum_in_pairs(sums);
   }
   __syncthreads();
-  skinny_f32_epilogue<EPI, 1, 1, WAVES>(partial, bias, c, m, n, ldc, n0, 0, 0, 1, scatter);
+  skinny_f32_epilogue<EPI, 1, 1, WAVES>(partial, ends, c, m, n, ldc, n0, 0, 1, scatter);
 }
 
 // --------------------------------------------------------------------------------- host
@@ -345,9 +416,12 @@ bool ps_norm_gemm_f32_fusable(const void* w, const NormPrologue& norm, int m, in
 
 int ps_norm_gemm_f32_fused(const NormPrologue& norm, const void* w, const float* bias, void* c, int m,
                            int n, int k, int ldc, int epilogue, const KvScatter& scatter, hipStream_t s) {
+  const bool shift = norm.rms == 0 && norm.beta != nullptr;
+  const int rows_and_flags = m | ((norm.rms ? SF_RMS : 0) | (shift ? SF_SHIFT : 0)) << SF_ROW_BITS;
 #define PS_LAUNCH_SNF(EPI, UNROLL)                                                                     \
   hipLaunchKernelGGL((gemm_nt_skinny_norm_f32_kernel<EPI, UNROLL>), dim3((n + 15) / 16), dim3(512), 0, \
-                     s, norm, (const float*)w, bias, (float*)c, m, n, k, ldc, scatter)
+                     s, norm.h, norm.gamma, shift ? norm.beta : norm.gamma, (const float*)w, norm.rows, norm.ldh, \
+                     rows_and_flags, n, k, bias, (float*)c, ldc, norm.eps, scatter)
 #define PS_SNF_CASE(EPI)                           \
   case EPI:                                        \
     if (k <= 8 * 3 * SF_STEP) PS_LAUNCH_SNF(EPI, 3); \
@@ -375,7 +449,7 @@ static int launch_skinny_f32(const void* a, const void* w, const float* bias, vo
   hipLaunchKernelGGL((gemm_nt_skinny_f32_kernel<EPI, MB, NT, UNROLL, WAVES>),                       \
                      dim3((n + 16 * NT - 1) / (16 * NT), k_splits, (row_blocks + MB - 1) / MB),     \
                      dim3(64 * WAVES), 0, s, (const float*)a, (const float*)w, bias, (float*)c, m,  \
-                     n, k, lda, ldc, k_chunk, k_splits, scatter)
+                     n, k, lda, k_chunk, ldc, k_splits, scatter)
   if (EPI == PS_EPI_RESIDUAL && m > 16) {
     // ranges of one round of four waves' loads (32 x 768 x 3072: 7.2 us with ranges of 384, 8.7 with 768)
     k_splits = (k + 4 * 3 * SF_STEP - 1) / (4 * 3 * SF_STEP);
