@@ -32,8 +32,11 @@
 // of up to 256 x 128, against the same: 4096 x 1600 x 6400 98 / 131, 2048 x 3072 x 768 18.0 / 19.9, 2048 x 2304 x 768
 // 13.9 / 16.7, 2048 x 3072 x 1024 20 / 24, 544 x 4096 x 1024 13.6 / 14.9, 544 x 3072 x 1024 9.9 / 11.7.  In a
 // prefill that lasts 0.2 s the card's power sets the clock and 4096 x 6400 x 1600 is level (104 / 102).  What is
-// left beside the products is the ends of the tiles, 10 us a round, in which a unit that holds one block
-// multiplies nothing.
+// left beside the products is the ends of the tiles, in which a unit that holds one block multiplies nothing.  They
+// waited for memory one trip after the other: for the arguments behind the preloaded ones in front of the first load,
+// then, all products done, for the bias, the rows added to and the pages.  Tile numbers now come of the preloaded
+// arguments and the rest is asked for in the last two stages: 4096 x 6400 x 1600 107 to 101 us in that prefill, 4096 x
+// 1600 x 1600 and 6400 (their mean) 62.1 to 58.0, 544 x 4096 x 1024 14.4 to 13.9.
 #pragma once
 #include <type_traits>
 
@@ -64,10 +67,14 @@ __device__ __forceinline__ void gl_wait_and_sync() {
 }
 
 // The columns of a wave in slices of SLICE fragments: the region of LDS that a slice is turned through is smaller.
+// `first`: what has been asked for of the first slice; `pages`, `tail`: the rows' pages, as whole slices and as a
+// narrower last one hold them.
 template <int FM, int FN, int SLICE, int FIRST, typename TOut, int EPI>
 __device__ __forceinline__ void gl_store(f32x16 (&acc)[FM][FN], float* region, int lane, int row, int col,
                                          int m, int n, int ldc, TOut* c, const float* bias,
-                                         const KvScatter& scatter) {
+                                         const KvScatter& scatter, const TileEnds<FM, SLICE, TOut, EPI>& first,
+                                         const TilePages<FM, SLICE>& pages,
+                                         const TilePages<FM, FN % SLICE ? FN % SLICE : SLICE>& tail) {
   if constexpr (FIRST < FN) {
     constexpr int COUNT = FIRST + SLICE <= FN ? SLICE : FN - FIRST;
     f32x16 slice[FM][COUNT];
@@ -75,17 +82,27 @@ __device__ __forceinline__ void gl_store(f32x16 (&acc)[FM][FN], float* region, i
     for (int i = 0; i < FM; ++i)
 #pragma unroll
       for (int j = 0; j < COUNT; ++j) slice[i][j] = acc[i][FIRST + j];
-    store_wave_tile<FM, COUNT, TOut, EPI>(slice, region, lane, row, col + FIRST * 32, m, n, ldc, c, bias, 0, 1,
-                                             scatter);
-    gl_store<FM, FN, SLICE, FIRST + COUNT, TOut, EPI>(acc, region, lane, row, col, m, n, ldc, c, bias, scatter);
+    auto store = [&](const auto& ends, const auto& rows) {
+      store_wave_tile<FM, COUNT, TOut, EPI>(slice, region, lane, row, col + FIRST * 32, m, n, ldc, c, bias, 0, 1,
+                                            scatter, ends, rows);
+    };
+    if constexpr (FIRST == 0) {
+      store(first, pages);
+    } else {
+      TileEnds<FM, COUNT, TOut, EPI> ends;
+      ends.ask(lane, row, col + FIRST * 32, m, n, ldc, c, bias, 0, tile_by_column<TOut, EPI>(c, ldc, 1, scatter));
+      if constexpr (COUNT == SLICE) store(ends, pages);
+      else store(ends, tail);
+    }
+    gl_store<FM, FN, SLICE, FIRST + COUNT, TOut, EPI>(acc, region, lane, row, col, m, n, ldc, c, bias, scatter,
+                                                      first, pages, tail);
   }
 }
 
 template <int FM, int FN, int ROW, int RING, typename TOut, int EPI>
 __global__ __launch_bounds__(512) void gemm_nt_bf16_large_kernel(
-    const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, const float* __restrict__ bias,
-    TOut* __restrict__ c, int m, int n, int k, int lda, int ldc, int tiles_m, int tiles_n, int panel,
-    KvScatter scatter) {
+    const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, int m, int n, int k, int lda, int panel, int ldc,
+    TOut* __restrict__ c, const float* __restrict__ bias, KvScatter scatter) {
   constexpr int WAVES = GL_WAVES_M * GL_WAVES_N;
   constexpr int BM = 32 * FM * GL_WAVES_M, BN = 32 * FN * GL_WAVES_N;
   static_assert(ROW == 64 || ROW == 128, "rows of half a line or of a whole one");
@@ -106,7 +123,8 @@ __global__ __launch_bounds__(512) void gemm_nt_bf16_large_kernel(
   const int wave_m = wave % GL_WAVES_M, wave_n = wave / GL_WAVES_M;
   // every XCD works on a contiguous run of tiles (see gemm_tiled.hip): panels of `panel` rows of tiles, walked
   // column by column, so that what runs at one time on an XCD is about as many rows as columns
-  const int per_xcd = gridDim.x / 8;
+  const int tiles_m = (m + BM - 1) / BM, tiles_n = (n + BN - 1) / BN;
+  const int per_xcd = tiles_m * tiles_n / 8;
   int tile = blockIdx.x;
   if (blockIdx.x < per_xcd * 8) tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
   const int first_row = tile / (panel * tiles_n) * panel;
@@ -215,20 +233,44 @@ __global__ __launch_bounds__(512) void gemm_nt_bf16_large_kernel(
   for (; stage + RING < stages; ++stage) {
     gl_for<0, SUB>([&](auto which) { step(stage, which, Yes{}, Full{}); });
   }
-  // the last RING stages; the first of them still asks for the other parts of the last one
+  // the last RING stages; the first of them still asks for the other parts of the last one.  The last two ask for what
+  // the ends need from memory: the rows' positions in front of the wait for the last stage, which leaves nothing on
+  // its way, and behind it the pages and, where there are registers for it, the first slice's bias and rows.
+  constexpr int SLICE = FN > 1 && FN < 5 ? 2 : 1;      // (FN = 5 has registers for one fragment's residual rows)
+  constexpr bool EARLY = FM * FN <= 4 || EPI != PS_EPI_RESIDUAL;
+  const int row_base = m0 + wave_m * FM * 32, col_base = n0 + wave_n * FN * 32;
+  const bool by_column = tile_by_column<TOut, EPI>(c, ldc, 1, scatter);
+  TileEnds<FM, SLICE, TOut, EPI> ends;
+  TilePages<FM, SLICE> pages;
+  constexpr int REST = FN % SLICE;
+  TilePages<FM, REST ? REST : SLICE> tail;
+  const bool paged = EPI == PS_EPI_NONE && !by_column && pages.wanted(scatter, col_base + FN * 32);
   gl_for<0, RING>([&](auto index) {
     constexpr int T = decltype(index)::value;
+    if constexpr (T == RING - 2) {
+      if (paged) {
+        pages.ask_rows(scatter, lane, row_base, m);
+        if constexpr (REST) tail.ask_rows(scatter, lane, row_base, m);
+      }
+    }
+    if constexpr (T == RING - 1) {
+      if (paged) {
+        pages.ask_pages(scatter);
+        if constexpr (REST) tail.ask_pages(scatter);
+      }
+      if constexpr (EARLY) ends.ask(lane, row_base, col_base, m, n, ldc, c, bias, 0, by_column);
+    }
     gl_for<0, SUB - 1>([&](auto which) { step(stage + T, which, std::integral_constant<bool, T == 0>{}, Full{}); });
     step(stage + T, Last{}, No{},
          std::integral_constant<int, T == RING - 1 ? -1 : (RING - 2 - T > 0 ? RING - 2 - T : 0)>{});
   });
 
-  // ---- epilogue: no load or read is on its way, and every wave is past its last operand
-  constexpr int SLICE = FN > 1 && FN < 5 ? 2 : 1;      // (FN = 5 has registers for one fragment's residual rows)
+  // ---- epilogue: no load of a stage and no read is on its way, and every wave is past its last operand
   static_assert(WAVES * 32 * (SLICE * 32 + 8) * 4 <= RING * STAGE_BYTES, "the epilogue reuses the stages");
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  if constexpr (!EARLY) ends.ask(lane, row_base, col_base, m, n, ldc, c, bias, 0, by_column);
   gl_store<FM, FN, SLICE, 0, TOut, EPI>(acc, reinterpret_cast<float*>(lds) + wave * 32 * (SLICE * 32 + 8), lane,
-                                    m0 + wave_m * FM * 32, n0 + wave_n * FN * 32, m, n, ldc, c, bias, scatter);
+                                        row_base, col_base, m, n, ldc, c, bias, scatter, ends, pages, tail);
 }
 
 // --------------------------------------------------------------------------------- host
@@ -250,8 +292,7 @@ static int launch_large(const void* a, const void* w, const float* bias, void* c
   dim3 grid(tiles_m * tiles_n);
 #define PS_LAUNCH_GL(EPI)                                                                                       \
   hipLaunchKernelGGL((gemm_nt_bf16_large_kernel<FM, FN, ROW, RING, TOut, EPI>), grid, dim3(512), 0, s,          \
-                     (const bf16_t*)a, (const bf16_t*)w, bias, (TOut*)c, m, n, k, lda, ldc, tiles_m, tiles_n,   \
-                     panel, scatter)
+                     (const bf16_t*)a, (const bf16_t*)w, m, n, k, lda, panel, ldc, (TOut*)c, bias, scatter)
   switch (epilogue) {
     case PS_EPI_NONE: PS_LAUNCH_GL(PS_EPI_NONE); break;
     case PS_EPI_GELU_TANH: PS_LAUNCH_GL(PS_EPI_GELU_TANH); break;

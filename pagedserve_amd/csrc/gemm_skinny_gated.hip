@@ -8,7 +8,8 @@
 // kernel, so the result has the same bits as the two launches.
 //
 // Bound by the trip of the weights from memory.  In us, two launches and this one, with weights from memory: 8 x (2 x
-// 3072) x 768 6.7 and 4.4 (4.2 since row scale and arguments are read beside the weights), 64 rows 10.7 and 6.9, 8 x (2 x 6400) x 1600 14.0 and 12.1, 8 x (2 x 512) x 256 4.4 and 2.8.
+// 3072) x 768 6.7 and 4.4 (4.2 since row scale and arguments are read beside the weights), 64 rows 10.7 and 6.9,
+// 8 x (2 x 6400) x 1600 14.0 and 12.1, 8 x (2 x 512) x 256 4.4 and 2.8.
 #include <type_traits>
 
 #include "gemm_skinny.h"

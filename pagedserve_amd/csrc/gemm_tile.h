@@ -72,44 +72,148 @@ __device__ inline void store8(bf16_t* out, const float* v) {
   *reinterpret_cast<uint4*>(out) = packed;
 }
 
+// How a wave's 32-column blocks leave for memory.  Element e of a 32 x 32 accumulator is row (e / 4) * 8 + (lane / 32)
+// * 4 + e % 4, column lane % 32: a lane holds one column.  Each wave turns 32 rows at a time through a region of LDS of
+// its own, after which a lane holds eight consecutive columns of one row: bias and activation are applied there and
+// rows leave in pieces of 16 or 32 bytes, eight (or more) lanes to a row.
+template <int WM, int WN>
+struct TilePieces {
+  static constexpr int STRIDE = WN * 32 + 8;      // floats of LDS; 4 rows further is 32 banks further
+  static constexpr int CHUNKS = WN * 4;           // pieces of eight columns per row
+  static constexpr int ROWS = 64 / CHUNKS;        // rows per pass of the wave
+  static constexpr int PASSES = 32 / ROWS;
+  static constexpr int COUNT = WM * PASSES;       // pieces of a lane
+  // (the last piece that lies in m rows, for those beyond)
+  __device__ static int row(int lane, int row_base, int piece, int m) {
+    const int at = row_base + piece / PASSES * 32 + piece % PASSES * ROWS + lane / CHUNKS;
+    return at < m ? at : m - 1;
+  }
+};
+
+// Pieces of eight columns cannot be stored: rows that are not aligned, heads that are no whole pieces (eight key or
+// value columns lie in one head; then n is whole pieces too), and partial sums of a split k.
+template <typename TOut, int EPI>
+__device__ inline bool tile_by_column(const TOut* c, int ldc, int k_splits, const KvScatter& scatter) {
+  const bool vec_c = ldc % (16 / (int)sizeof(TOut)) == 0 && (reinterpret_cast<uintptr_t>(c) & 15u) == 0;
+  const bool whole_kv = EPI != PS_EPI_NONE || scatter.k_pool == nullptr ||
+                        ((scatter.head_dim | scatter.q_cols | scatter.kv_cols) & 7) == 0;
+  return !vec_c || !whole_kv || k_splits > 1;
+}
+
+// First column of a lane's pieces.  The piece that the end of the rows lies in begins further left where that is
+// aligned and within the wave's columns (float rows of whole fours): both pieces then write the same values to the
+// columns that they share.
+template <typename TOut>
+__device__ inline bool tile_reaches_back(int col_base, int n) {
+  return sizeof(TOut) == 4 && (n & 3) == 0 && n - col_base >= 8;
+}
+template <int WN, typename TOut>
+__device__ inline int tile_first_col(int lane, int col_base, int n) {
+  const int first = col_base + lane % (WN * 4) * 8;
+  return tile_reaches_back<TOut>(col_base, n) && first < n && first + 8 > n ? n - 8 : first;
+}
+
+// The pages of a wave's rows: two dependent reads for each.  They are the same for all its columns, so that a kernel
+// asks for all of them at once (where a row's check in front of its read made one trip per row and slice of columns),
+// and before its last products: with this 4096 x 4800 x 1600 with 3200 key and value columns, 256 x 320 to a tile, went
+// from 70.4 to 64.0 us in a prefill, 2048 x 2304 x 768 from 17.8 to 16.0, 544 x 3072 x 1024 from 10.2 to 9.2.
+template <int WM, int WN>
+struct TilePages {
+  using Pieces = TilePieces<WM, WN>;
+  int pos[Pieces::COUNT], page[Pieces::COUNT];
+  // `wanted` (the same for the whole wave): some of its columns are keys or values
+  __device__ static bool wanted(const KvScatter& s, int col_end) {
+    return s.k_pool != nullptr && s.table_width > 0 && col_end > s.q_cols;
+  }
+  __device__ void ask_rows(const KvScatter& s, int lane, int row_base, int m) {
+#pragma unroll
+    for (int p = 0; p < Pieces::COUNT; ++p) {
+      const int row = Pieces::row(lane, row_base, p, m);
+      pos[p] = s.tok_pos[row];
+      page[p] = s.tok_item[row];
+    }
+  }
+  __device__ void ask_pages(const KvScatter& s) {
+    int64_t entry[Pieces::COUNT];
+#pragma unroll
+    for (int p = 0; p < Pieces::COUNT; ++p) entry[p] = (int64_t)page[p] * s.table_width;
+    int logical[Pieces::COUNT];
+    if (s.page_shift >= 0) {
+#pragma unroll
+      for (int p = 0; p < Pieces::COUNT; ++p) logical[p] = pos[p] >> s.page_shift;
+    } else {
+#pragma unroll
+      for (int p = 0; p < Pieces::COUNT; ++p) logical[p] = pos[p] / s.page_size;
+    }
+#pragma unroll
+    for (int p = 0; p < Pieces::COUNT; ++p) page[p] = s.tables[logical[p] < s.table_width ? entry[p] + logical[p] : 0];
+#pragma unroll
+    for (int p = 0; p < Pieces::COUNT; ++p) pos[p] = logical[p] < s.table_width ? pos[p] : -1;
+  }
+  __device__ bool holds(const KvScatter& s, int p) const {
+    return s.table_width > 0 && pos[p] >= 0 && page[p] >= 0 && page[p] < s.num_pages;
+  }
+};
+
+// What a wave's whole pieces need from memory: bias, and the rows that are added to.  The bias is read without a
+// branch, as zeros from memory where there is none: behind a branch, or in front of a choice, the compiler waits for it.
+static __device__ const float tile_no_bias[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
+typedef __attribute__((__vector_size__(4 * sizeof(float)), aligned(4))) float f32x4_any;
+typedef const __attribute__((address_space(1))) f32x4* global_f32x4_t;
+typedef const __attribute__((address_space(1))) f32x4_any* global_f32x4_any_t;
+template <int WM, int WN, typename TOut, int EPI>
+struct TileEnds {
+  using Pieces = TilePieces<WM, WN>;
+  static constexpr bool RESIDUAL = EPI == PS_EPI_RESIDUAL;
+  f32x4 bias[2], old[RESIDUAL ? Pieces::COUNT : 1][2];
+  __device__ void ask(int lane, int row_base, int col_base, int m, int n, int ldc, const TOut* c, const float* b,
+                      int split, bool by_column) {
+    const int col0 = tile_first_col<WN, TOut>(lane, col_base, n);
+    const bool full = col0 + 8 <= n;
+    const bool biased = b != nullptr && split == 0 && n >= 8;
+    const float* from = biased ? b : tile_no_bias;
+    const int col = biased && full ? col0 : 0;
+    // (through pointers that the compiler does not know: it would choose between values instead, and move the reads of
+    // c to where they are used)
+    const float* rows = reinterpret_cast<const float*>(c);
+    asm volatile("" : "+v"(from), "+v"(rows));
+    bias[0] = *(global_f32x4_any_t)(from + col);
+    bias[1] = *(global_f32x4_any_t)(from + col + 4);
+    if (RESIDUAL && !by_column && full) {
+#pragma unroll
+      for (int p = 0; p < (RESIDUAL ? Pieces::COUNT : 0); ++p) {
+        const float* sum = rows + (int64_t)Pieces::row(lane, row_base, p, m) * ldc + col0;
+        old[p][0] = *(global_f32x4_t)sum;
+        old[p][1] = *(global_f32x4_t)(sum + 4);
+      }
+    }
+  }
+};
+
 // The accumulators acc[WM][WN] of one wave (32 x 32 each, rows row_base + 32 i ..., columns
 // col_base + 32 j ...) to C, through `region`, an area of LDS of 32 x (32 WN + 8) floats that
 // belongs to this wave alone: bias, activation, residual add into the float stream, key/value
 // columns into cache pages.  `split` / `k_splits`: partial sums of a k range are added with
-// atomics, the bias by split 0 only.
+// atomics, the bias by split 0 only.  `ends`, `pages`: what the caller has asked for (the pages
+// where TilePages::wanted says so).
 template <int WM, int WN, typename TOut, int EPI>
 __device__ inline void store_wave_tile(f32x16 (&acc)[WM][WN], float* region, int lane, int row_base,
                                        int col_base, int m, int n, int ldc, TOut* __restrict__ c,
                                        const float* __restrict__ bias, int split, int k_splits,
-                                       const KvScatter& scatter) {
-  // ---- epilogue.  Element e of a 32 x 32 accumulator is row (e / 4) * 8 + (lane / 32) * 4 +
-  // e % 4, column lane % 32: a lane holds one column.  Each wave turns 32 rows at a time
-  // through a region of LDS of its own, after which a lane holds eight consecutive columns of
-  // one row: bias and activation are applied there and rows leave in pieces of 16 or 32
-  // bytes, eight (or more) lanes to a row.
-  constexpr int EP_STRIDE = WN * 32 + 8;          // floats; 4 rows further is 32 banks further
-  constexpr int EP_CHUNKS = WN * 4;               // pieces of eight columns per row
-  constexpr int EP_ROWS = 64 / EP_CHUNKS;         // rows per pass of the wave
+                                       const KvScatter& scatter, const TileEnds<WM, WN, TOut, EPI>& ends,
+                                       const TilePages<WM, WN>& pages) {
+  using Pieces = TilePieces<WM, WN>;
+  constexpr int EP_STRIDE = Pieces::STRIDE, EP_ROWS = Pieces::ROWS, PASSES = Pieces::PASSES;
   // The callers read operands by assembly and wait for them just in front of this.  What is worked out of the lane here
   // must not be moved in front of that wait, into a register that such a read may still be filling.
   asm volatile("" : "+v"(lane));
-  const int chunk = lane % EP_CHUNKS;
-  const int row_in_pass = lane / EP_CHUNKS;
-  // The piece that the end of the rows lies in begins further left where that is aligned and within the wave's columns
-  // (float rows of whole fours): both pieces then write the same values to the columns that they share.
-  const bool reaches_back = sizeof(TOut) == 4 && (n & 3) == 0 && n - col_base >= 8;
-  const int first = col_base + chunk * 8;
-  const int col0 = reaches_back && first < n && first + 8 > n ? n - 8 : first;
-  const bool vec_c = ldc % (16 / (int)sizeof(TOut)) == 0 && (reinterpret_cast<uintptr_t>(c) & 15u) == 0;
-  constexpr bool PLAIN = EPI == PS_EPI_NONE;
+  const int row_in_pass = lane / Pieces::CHUNKS;
+  const bool reaches_back = tile_reaches_back<TOut>(col_base, n);
+  const int col0 = tile_first_col<WN, TOut>(lane, col_base, n);
+  constexpr bool PLAIN = EPI == PS_EPI_NONE, RESIDUAL = EPI == PS_EPI_RESIDUAL;
   const bool full = col0 + 8 <= n;
-  // eight key or value columns lie in one head (then n is whole pieces too)
-  const bool whole_kv = !PLAIN || scatter.k_pool == nullptr ||
-                        ((scatter.head_dim | scatter.q_cols | scatter.kv_cols) & 7) == 0;
-  const bool by_column = !vec_c || !whole_kv || k_splits > 1;
-  float b[8];
-#pragma unroll
-  for (int q = 0; q < 8; ++q) b[q] = (bias && split == 0 && col0 + q < n) ? bias[col0 + q] : 0.f;
+  const bool by_column = tile_by_column<TOut, EPI>(c, ldc, k_splits, scatter);
   // otherwise the columns behind the last whole piece go eight rows at a time
   const bool ends_inside =
       !reaches_back && (n & 7) != 0 && (n & ~7) >= col_base && (n & ~7) < col_base + WN * 32;
@@ -120,40 +224,6 @@ __device__ inline void store_wave_tile(f32x16 (&acc)[WM][WN], float* region, int
   int64_t pool_offset = 0;
   if (PLAIN && !by_column && scatter.k_pool != nullptr && full && col0 >= scatter.q_cols)
     pool = kv_scatter_col<TOut>(scatter, col0, &pool_offset);
-
-  // What the whole pieces need from memory is asked for before the first of them: the residual rows, and
-  // where each token's keys and values lie (two dependent reads a row).  One trip each, not one per pass.
-  constexpr int PASSES = 32 / EP_ROWS;
-  constexpr bool RESIDUAL = EPI == PS_EPI_RESIDUAL;
-  float4 old[RESIDUAL ? WM : 1][RESIDUAL ? PASSES : 1][2];
-  if (RESIDUAL && !by_column && full) {
-#pragma unroll
-    for (int i = 0; i < WM; ++i)
-#pragma unroll
-      for (int pass = 0; pass < PASSES; ++pass) {
-        const int row = row_base + i * 32 + pass * EP_ROWS + row_in_pass;
-        const float* sum = reinterpret_cast<const float*>(c) + (int64_t)(row < m ? row : m - 1) * ldc + col0;
-        old[RESIDUAL ? i : 0][RESIDUAL ? pass : 0][0] = *reinterpret_cast<const float4*>(sum);
-        old[RESIDUAL ? i : 0][RESIDUAL ? pass : 0][1] = *reinterpret_cast<const float4*>(sum + 4);
-      }
-  }
-  int64_t slots[PLAIN ? WM : 1][PLAIN ? PASSES : 1];
-  if (PLAIN && pool != nullptr) {
-    int pos[PLAIN ? WM : 1][PLAIN ? PASSES : 1], item[PLAIN ? WM : 1][PLAIN ? PASSES : 1];
-#pragma unroll
-    for (int i = 0; i < (PLAIN ? WM : 0); ++i)
-#pragma unroll
-      for (int pass = 0; pass < PASSES; ++pass) {
-        const int row = row_base + i * 32 + pass * EP_ROWS + row_in_pass;
-        pos[i][pass] = scatter.tok_pos[row < m ? row : m - 1];
-        item[i][pass] = scatter.tok_item[row < m ? row : m - 1];
-      }
-#pragma unroll
-    for (int i = 0; i < (PLAIN ? WM : 0); ++i)
-#pragma unroll
-      for (int pass = 0; pass < PASSES; ++pass)
-        slots[i][pass] = kv_scatter_slot(scatter, pos[i][pass], &item[i][pass]);
-  }
 
 #pragma unroll
   for (int i = 0; i < WM; ++i) {
@@ -201,20 +271,21 @@ __device__ inline void store_wave_tile(f32x16 (&acc)[WM][WN], float* region, int
       if (row >= m || !full) continue;
       float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
 #pragma unroll
-      for (int q = 0; q < 8; ++q) v[q] = finish_value<EPI, TOut>(v[q] + b[q]);
+      for (int q = 0; q < 8; ++q) v[q] = finish_value<EPI, TOut>(v[q] + ends.bias[q / 4][q % 4]);
       TOut* out = c + (int64_t)row * ldc + col0;
       if constexpr (RESIDUAL) {
         float* sum = reinterpret_cast<float*>(out);
-        float4 o0 = old[i][pass][0], o1 = old[i][pass][1];
-        o0.x += v[0]; o0.y += v[1]; o0.z += v[2]; o0.w += v[3];
-        o1.x += v[4]; o1.y += v[5]; o1.z += v[6]; o1.w += v[7];
-        *reinterpret_cast<float4*>(sum) = o0;
-        *reinterpret_cast<float4*>(sum + 4) = o1;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] += ends.old[i * PASSES + pass][q / 4][q % 4];
+        store8(sum, v);
       } else {
         // (eight key or value columns that go to their page and that nobody reads from c)
         if (!(PLAIN && pool != nullptr && scatter.cache_only)) store8(out, v);
-        if constexpr (PLAIN)
-          if (pool != nullptr && slots[i][pass] >= 0) store8(pool + slots[i][pass] + pool_offset, v);
+        if constexpr (PLAIN) {
+          const int p = i * PASSES + pass;
+          if (pool != nullptr && pages.holds(scatter, p))
+            store8(pool + kv_page_slot(scatter, pages.pos[p], pages.page[p]) + pool_offset, v);
+        }
       }
     }
     if (ends_inside) {
@@ -232,4 +303,22 @@ __device__ inline void store_wave_tile(f32x16 (&acc)[WM][WN], float* region, int
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }
+}
+
+// The same for a kernel that has asked for nothing yet.
+template <int WM, int WN, typename TOut, int EPI>
+__device__ inline void store_wave_tile(f32x16 (&acc)[WM][WN], float* region, int lane, int row_base,
+                                       int col_base, int m, int n, int ldc, TOut* __restrict__ c,
+                                       const float* __restrict__ bias, int split, int k_splits,
+                                       const KvScatter& scatter) {
+  asm volatile("" : "+v"(lane));
+  const bool by_column = tile_by_column<TOut, EPI>(c, ldc, k_splits, scatter);
+  TileEnds<WM, WN, TOut, EPI> ends;
+  TilePages<WM, WN> pages;
+  const bool paged = EPI == PS_EPI_NONE && !by_column && pages.wanted(scatter, col_base + WN * 32);
+  if (paged) pages.ask_rows(scatter, lane, row_base, m);
+  ends.ask(lane, row_base, col_base, m, n, ldc, c, bias, split, by_column);
+  if (paged) pages.ask_pages(scatter);
+  store_wave_tile<WM, WN, TOut, EPI>(acc, region, lane, row_base, col_base, m, n, ldc, c, bias, split, k_splits,
+                                     scatter, ends, pages);
 }

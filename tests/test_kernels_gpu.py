@@ -1672,6 +1672,42 @@ def test_linear_of_many_rows_with_scatter(m, heads, kv_heads, k, tile):
     assert torch.equal(v_pool.view(torch.int16), pools[1].view(torch.int16))
 
 
+@pytest.mark.parametrize("dtype,m,heads,kv_heads,k", [
+    (torch.bfloat16, 70, 4, 2, 128), (torch.bfloat16, 300, 4, 2, 64), (torch.bfloat16, 545, 32, 16, 832),
+    (torch.bfloat16, 1030, 32, 16, 832), (torch.bfloat16, 2050, 25, 25, 832), (torch.float32, 70, 4, 2, 128),
+    (torch.float32, 700, 8, 4, 64)])
+@pytest.mark.parametrize("page_size", [16, 12])
+def test_linear_of_many_rows_leaves_out_rows_without_a_page(dtype, m, heads, kv_heads, k, page_size):
+    """Rows whose position lies behind the table's last column, or whose entry there is no page, change no page; and a
+    bias that begins at any float.  In tiles of each kind (one fragment, one and a half slices, pairs of k tiles)."""
+    from pagedserve_amd.ops import kernels
+
+    head_dim = 64
+    q_cols, kv_cols = heads * head_dim, kv_heads * head_dim
+    n = q_cols + 2 * kv_cols
+    k_pool, v_pool, tables = _paged_fixture(dtype, [m, 40], kv_heads, head_dim, page_size, 410)
+    tables[0, 1], tables[0, 3] = -1, k_pool.shape[0]
+    tok_item = torch.tensor([1] * 30 + [0] * (m - 30), dtype=torch.int32, device="cuda")
+    tok_pos = torch.tensor(list(range(10, 40)) + list(range(30, m)), dtype=torch.int32, device="cuda")
+    tok_pos[m - 7:] += tables.shape[1] * page_size
+    x, w = _rand((m, k), dtype, 411), _rand((n, k), dtype, 412, 1.0 / math.sqrt(k))
+    bias = _rand((n + 1,), torch.float32, 413)[1:]
+    out, pools = torch.empty((m, n), dtype=dtype, device="cuda"), (k_pool.clone(), v_pool.clone())
+    kernels.linear(x, w, bias, out, packed=kernels.pack_decode_weight(w),
+                   scatter=(k_pool, v_pool, tok_item, tok_pos, tables, q_cols, kv_cols))
+    torch.testing.assert_close(out.double(), x.double() @ w.double().t() + bias.double(), atol=1e-4,
+                               rtol=4e-3 if dtype == torch.bfloat16 else 1e-5)
+    logical = (tok_pos // page_size).long()
+    entry = tables[tok_item.long(), logical.clamp(max=tables.shape[1] - 1)].long()
+    kept = (logical < tables.shape[1]) & (entry >= 0) & (entry < k_pool.shape[0])
+    assert 0 < int(kept.sum()) < m - 7
+    for pool, first in zip(pools, (q_cols, q_cols + kv_cols)):
+        columns = out[kept, first:first + kv_cols].view(-1, kv_heads, head_dim)
+        pool[entry[kept], :, (tok_pos[kept] % page_size).long()] = columns
+    for pool, expected in zip((k_pool, v_pool), pools):      # (NaN where no token lies)
+        torch.testing.assert_close(pool, expected, atol=0, rtol=0, equal_nan=True)
+
+
 def test_linear_takes_the_large_product_for_thousands_of_rows():
     """Through ``kernels.linear``: rows and columns that fill the chip with tiles of 256 x 192, with the key/value
     scatter behind the product, against float64 and a scatter of its own."""
