@@ -195,8 +195,8 @@ __global__ __launch_bounds__(256) void norm_wave_kernel(
 // waves share a row and meet through LDS: one where rows are many, four where they are few and what
 // counts is the one trip to memory (then a thread holds one or two pieces).  Measured, in us, single
 // values per lane before and now: 64 x 768 3.3 / 2.85, 544 x 1024 3.7 / 3.1, 2048 x 768 4.5 / 4.2, 4096 x
-// 1600 11.9 / 10.6; with one barrier to a sum 64 x 768 in a decode step 3.0 -> 2.4.  Short rows, a handful of values per lane either way, stay with norm_wave_kernel (launch_norm
-// says up to where).
+// 1600 11.9 / 10.6; with one barrier to a sum 64 x 768 in a decode step 3.0 -> 2.4.  Short rows, a handful of values per
+// lane either way, stay with norm_wave_kernel (launch_norm says up to where).
 template <typename T>
 __device__ inline void store4(T* out, const float* v);
 template <>
@@ -208,6 +208,15 @@ __device__ inline void store4<bf16_t>(bf16_t* out, const float* v) {
   *reinterpret_cast<uint2*>(out) = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
 }
 
+// In the packed order a line of 128 bytes holds 8 columns of 8 rows.  Blocks of those rows on different XCDs, each with
+// an L2 of its own, would each write a sixteenth of it to memory: consecutive block ids run on different XCDs, so that
+// every eighth block takes a row of the same 16 (64 x 768 in a decode step 2.6 us, in the order of the rows 3.95).
+__device__ inline int norm_packed_row(int block) {
+  const int xcd = block & 7, slot = block >> 3;
+  return ((slot >> 4) * 8 + xcd) * 16 + (slot & 15);
+}
+static int norm_packed_blocks(int rows) { return (rows + 127) / 128 * 128; }
+
 template <typename T, bool RMS, int PIECES, int WAVES>
 __global__ __launch_bounds__(256) void norm_vec_kernel(
     const float* __restrict__ x, const int* __restrict__ rows, const float* __restrict__ gamma,
@@ -215,8 +224,9 @@ __global__ __launch_bounds__(256) void norm_vec_kernel(
     int packed) {
   __shared__ __attribute__((aligned(16))) float scratch[2][WAVES];    // a place for each of the two sums
   const int at = WAVES == 1 ? threadIdx.x & 63 : threadIdx.x;
-  const int r = WAVES == 1 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
-  if (WAVES == 1 && r >= n_rows) return;
+  int r = WAVES == 1 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
+  if (WAVES > 1 && packed) r = norm_packed_row(blockIdx.x);
+  if (r >= n_rows) return;
   const float* src = x + (int64_t)(rows ? rows[r] : r) * width;
   // loads are unconditional, as above; without a shift gamma stands in for it
   const float* shift = (!RMS && beta != nullptr) ? beta : gamma;
@@ -356,7 +366,8 @@ static void launch_norm(const float* x, const int* rows, const float* gamma, con
   if (width % 4 == 0 && width >= (n_rows <= NORM_FEW_ROWS ? NORM_FEW_WIDTH : NORM_MANY_WIDTH) && width <= 2048 &&
       (all & 15u) == 0) {
 #define PS_LAUNCH_NV(PIECES, WAVES)                                                               \
-  hipLaunchKernelGGL((norm_vec_kernel<T, RMS, PIECES, WAVES>), WAVES == 1 ? grid : dim3(n_rows),  \
+  hipLaunchKernelGGL((norm_vec_kernel<T, RMS, PIECES, WAVES>),                                    \
+                     WAVES == 1 ? grid : dim3(packed ? norm_packed_blocks(n_rows) : n_rows),      \
                      dim3(256), 0, s, x, rows, gamma, beta, (T*)out, n_rows, width, eps, packed)
     if (n_rows <= NORM_FEW_ROWS) {
       if (width <= 1024) PS_LAUNCH_NV(1, 4);
