@@ -226,6 +226,12 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_nt_skinny_f32_kernel(
   skinny_f32_epilogue<EPI, MB, NT, WAVES>(partial, ends, c, m, n, ldc, n0, row0, k_splits, scatter);
 }
 
+// A value of the lane N places on within its run of 16.
+template <int N>
+__device__ inline float row_turned(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x120 + N, 0xf, 0xf, false));
+}
+
 // The same for up to 16 rows with the norm of its input fused in front (whole k in one round of loads): while the
 // weights travel, each wave normalises up to two rows in registers (as norm_wave_kernel, elementwise.hip)
 // and leaves them in LDS, where the product reads its column operand.  One launch and one trip to memory
@@ -374,6 +380,189 @@ __global__ __launch_bounds__(512) void gemm_nt_skinny_norm_f32_kernel(
   skinny_f32_epilogue<EPI, 1, 1, WAVES>(partial, ends, c, m, n, ldc, n0, 0, 1, scatter);
 }
 
+// The same for up to eight rows.  Instructions of 16 x 16 spend half of their time and more on rows that are not there
+// (0.55 of 5.4 us, 8 x 3072 x 768), and blocks of 16 columns leave 112 units without one at 2304 columns.  Here four
+// waves take a quarter of k each and blocks have 4 GROUPS columns: an instruction of 4 x 4 multiplies four columns by
+// four rows in 16 places of k, whose sums meet at the end.  A lane's 16 bytes are those of column lane % 4 and k piece
+// lane / 4, so that a load takes 256 bytes of four rows of W.  Up to four rows, or eight, which use W's operand twice.
+// Bound by the launch and the trip of the weights from memory (without them 3.7 us).  In us, 16 x 16 and this one: 1 x
+// 2304 x 768 5.1 / 4.35, 4 rows 4.95 / 4.25, 8 rows 5.5 / 4.9, 1 x 3072 x 768 5.35 / 4.6, 8 rows 5.7 / 5.1.  In blocks of
+// 16 columns 8 x 2304 x 768 takes 5.5, 8 x 3072 x 768 5.5: 12 wherever that is no more blocks than units.
+#define SF_FEW_ROWS 8
+#define SF_FEW_PIECE 64      // values of k that the 16 places take
+template <int EPI, int PIECES, int GROUPS, int ROWS>
+__global__ __launch_bounds__(256) void gemm_nt_few_norm_f32_kernel(
+    const float* __restrict__ h_rows, const float* __restrict__ gamma, const float* __restrict__ shift,
+    const float* __restrict__ w, const int* __restrict__ rows_of, int ldh, int rows_and_flags, int n, int k,
+    const float* __restrict__ bias, float* __restrict__ c, int ldc, float eps, KvScatter scatter) {
+  const int m = rows_and_flags & ((1 << SF_ROW_BITS) - 1);
+  const bool rms = (rows_and_flags >> SF_ROW_BITS) & SF_RMS, shifts = (rows_and_flags >> SF_ROW_BITS) & SF_SHIFT;
+  constexpr int WAVES = 4, SETS = ROWS / 4, HELD = ROWS / WAVES;     // rows that a wave normalises
+  constexpr int MOST = WAVES * PIECES * SF_FEW_PIECE;                // the longest k
+  constexpr int STRIDE = MOST + 8;                   // the four rows of two places then lie in 32 different banks
+  constexpr int COLS = 4 * GROUPS, ELEMENTS = COLS * ROWS;
+  static_assert(ROWS == 4 || ROWS == 8, "one or two sets of four rows");
+  static_assert(ELEMENTS <= 64 * WAVES && MOST % 256 == 0, "a thread finishes one element, a wave reads whole rows");
+  __shared__ __attribute__((aligned(16))) float rows[ROWS * STRIDE];
+  __shared__ float partial[4 * WAVES][ELEMENTS];     // of a wave's four runs of 16 lanes
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // the same in every lane: scalar
+  const int n0 = blockIdx.x * COLS;
+  const int sub = lane & 3, place = lane >> 2;
+  // (rows, scale, shift and weights in this order, as above)
+  constexpr int PARTS = MOST / 256;
+  float v[HELD][PARTS][4], g[PARTS][4], b[PARTS][4];
+  f32x4 wf[PIECES][GROUPS];
+  int src_row[HELD];
+#pragma unroll
+  for (int half = 0; half < HELD; ++half) {
+    const int r = wave + half * WAVES < m ? wave + half * WAVES : m - 1;
+    src_row[half] = rows_of ? scalar_load(rows_of + r) : r;
+  }
+#pragma unroll
+  for (int half = 0; half < HELD; ++half) {
+    const float* src = h_rows + (int64_t)src_row[half] * ldh;
+#pragma unroll
+    for (int i = 0; i < PARTS; ++i) {
+      const int col = (lane + i * 64) * 4;
+      *reinterpret_cast<float4*>(v[half][i]) = *reinterpret_cast<const float4*>(src + (col < k ? col : k - 4));
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < PARTS; ++i) {
+    const int col = (lane + i * 64) * 4;
+    const int safe = col < k ? col : k - 4;
+    *reinterpret_cast<float4*>(g[i]) = *reinterpret_cast<const float4*>(gamma + safe);
+    *reinterpret_cast<float4*>(b[i]) = *reinterpret_cast<const float4*>(shift + safe);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int p = 0; p < PIECES; ++p)
+#pragma unroll
+    for (int j = 0; j < GROUPS; ++j) {
+      const int col = n0 + j * 4 + sub < n ? n0 + j * 4 + sub : n - 1;
+      const int kk = (p * WAVES + wave) * SF_FEW_PIECE + place * 4;
+      wf[p][j] = *reinterpret_cast<const f32x4*>(w + (int64_t)col * k + (kk < k ? kk : 0));
+    }
+  read_arguments(bias, c, ldc, eps);
+  if (EPI == PS_EPI_NONE && scatter.k_pool != nullptr) read_scatter(scatter);
+  // what the epilogue needs: element e is column e % COLS of row e / COLS
+  const int element = threadIdx.x;
+  const int out_col = n0 + element % COLS, out_row = element / COLS;
+  const int col_read = out_col < n ? out_col : n - 1, row_read = out_row < m ? out_row : m - 1;
+  const bool scatters = EPI == PS_EPI_NONE && scatter.k_pool != nullptr;
+  float own_bias = 0.f;
+  int pos = 0, item = 0, page = -1;
+  bool there = false;
+  if (bias != nullptr) own_bias = bias[col_read];
+  if (scatters) {
+    pos = scatter.tok_pos[row_read];
+    item = scatter.tok_item[row_read];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  float mean[HELD], inv_std[HELD];      // (a wave's rows side by side: their sums do not wait for each other)
+#pragma unroll
+  for (int half = 0; half < HELD; ++half) mean[half] = 0.f;
+  if (!rms) {
+#pragma unroll
+    for (int half = 0; half < HELD; ++half) {
+      float sum = 0.f;
+#pragma unroll
+      for (int i = 0; i < PARTS; ++i)
+        if ((lane + i * 64) * 4 < k) sum += (v[half][i][0] + v[half][i][1]) + (v[half][i][2] + v[half][i][3]);
+      mean[half] = sum;
+    }
+#pragma unroll
+    for (int half = 0; half < HELD; ++half) mean[half] = wave_sum(mean[half]) / (float)k;
+  }
+#pragma unroll
+  for (int half = 0; half < HELD; ++half) {
+    float sq = 0.f;
+#pragma unroll
+    for (int i = 0; i < PARTS; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        v[half][i][j] = (lane + i * 64) * 4 < k ? v[half][i][j] - mean[half] : 0.f;
+        sq = fmaf(v[half][i][j], v[half][i][j], sq);
+      }
+    inv_std[half] = sq;
+  }
+#pragma unroll
+  for (int half = 0; half < HELD; ++half) inv_std[half] = 1.0f / sqrtf(wave_sum(inv_std[half]) / (float)k + eps);
+  // (rows beyond m are the last one again, places beyond k zeros)
+#pragma unroll
+  for (int half = 0; half < HELD; ++half)
+#pragma unroll
+    for (int i = 0; i < PARTS; ++i) {
+      const int col = (lane + i * 64) * 4;
+      f32x4 y;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        y[j] = shifts ? fmaf(v[half][i][j] * inv_std[half], g[i][j], b[i][j]) : v[half][i][j] * inv_std[half] * g[i][j];
+      if (col >= k) y = f32x4{0.f, 0.f, 0.f, 0.f};
+      *reinterpret_cast<f32x4*>(rows + (wave + half * WAVES) * STRIDE + col) = y;
+    }
+  __syncthreads();
+
+  // an accumulator for each of a lane's four values of k: chains of PIECES
+  f32x4 acc[GROUPS][SETS][4];
+#pragma unroll
+  for (int j = 0; j < GROUPS; ++j)
+#pragma unroll
+    for (int t = 0; t < SETS; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[j][t][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int p = 0; p < PIECES; ++p) {
+    const int kk = (p * WAVES + wave) * SF_FEW_PIECE + place * 4;
+    f32x4 x[SETS];
+#pragma unroll
+    for (int t = 0; t < SETS; ++t) x[t] = *reinterpret_cast<const f32x4*>(rows + (t * 4 + sub) * STRIDE + kk);
+#pragma unroll
+    for (int j = 0; j < GROUPS; ++j) {
+      f32x4 weights = wf[p][j];
+      asm volatile("" : "+v"(weights));      // (or the choice below is made, and waited for, in front of the norm)
+      if (kk >= k) weights = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int t = 0; t < SETS; ++t)
+          acc[j][t][i] = __builtin_amdgcn_mfma_f32_4x4x1f32(weights[i], x[t][i], acc[j][t][i], 0, 0, 0);
+    }
+  }
+  if (scatters && n0 + COLS > scatter.q_cols) {
+    const int logical = scatter.page_shift >= 0 ? (pos >> scatter.page_shift) : pos / scatter.page_size;
+    // a row without a page reads the first entry in its place
+    there = logical < scatter.table_width;
+    page = scatter.tables[there ? (int64_t)item * scatter.table_width + logical : 0];
+  }
+  // lane l holds columns 4 j .. 4 j + 3 of row 4 t + l % 4 for place l / 4
+#pragma unroll
+  for (int j = 0; j < GROUPS; ++j)
+#pragma unroll
+    for (int t = 0; t < SETS; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float sum = (acc[j][t][0][i] + acc[j][t][1][i]) + (acc[j][t][2][i] + acc[j][t][3][i]);
+        sum += row_turned<4>(sum);
+        sum += row_turned<8>(sum);
+        if ((lane & 15) < 4) partial[wave * 4 + (lane >> 4)][(t * 4 + sub) * COLS + j * 4 + i] = sum;
+      }
+  __syncthreads();
+  if (element >= ELEMENTS || out_col >= n || out_row >= m) return;
+  float of_run[4 * WAVES];
+#pragma unroll
+  for (int p = 0; p < 4 * WAVES; ++p) of_run[p] = partial[p][element];
+  const float value = apply_activation<EPI>(sum_in_pairs(of_run) + own_bias);
+  c[(int64_t)out_row * ldc + out_col] = value;
+  if (scatters && out_col >= scatter.q_cols) {
+    int64_t offset;
+    float* pool = kv_scatter_col<float>(scatter, out_col, &offset);
+    if (there && page >= 0 && page < scatter.num_pages) pool[offset + kv_page_slot(scatter, pos, page)] = value;
+  }
+}
+
 // --------------------------------------------------------------------------------- host
 // Whether this kernel takes the product (a row of either operand in pieces of 16 bytes), and is the
 // fastest that does.  The lines, with weights from memory, in us:
@@ -418,14 +607,28 @@ int ps_norm_gemm_f32_fused(const NormPrologue& norm, const void* w, const float*
                            int n, int k, int ldc, int epilogue, const KvScatter& scatter, hipStream_t s) {
   const bool shift = norm.rms == 0 && norm.beta != nullptr;
   const int rows_and_flags = m | ((norm.rms ? SF_RMS : 0) | (shift ? SF_SHIFT : 0)) << SF_ROW_BITS;
+  const bool narrow = n <= 12 * ps_compute_units();      // blocks of 12 columns are at most one to a unit
 #define PS_LAUNCH_SNF(EPI, UNROLL)                                                                     \
   hipLaunchKernelGGL((gemm_nt_skinny_norm_f32_kernel<EPI, UNROLL>), dim3((n + 15) / 16), dim3(512), 0, \
                      s, norm.h, norm.gamma, shift ? norm.beta : norm.gamma, (const float*)w, norm.rows, norm.ldh, \
                      rows_and_flags, n, k, bias, (float*)c, ldc, norm.eps, scatter)
-#define PS_SNF_CASE(EPI)                           \
-  case EPI:                                        \
-    if (k <= 8 * 3 * SF_STEP) PS_LAUNCH_SNF(EPI, 3); \
-    else PS_LAUNCH_SNF(EPI, 4);                    \
+#define PS_LAUNCH_FNF(EPI, PIECES, GROUPS, ROWS)                                                                    \
+  hipLaunchKernelGGL((gemm_nt_few_norm_f32_kernel<EPI, PIECES, GROUPS, ROWS>), dim3((n + 4 * GROUPS - 1) / (4 * GROUPS)), \
+                     dim3(256), 0, s, norm.h, norm.gamma, shift ? norm.beta : norm.gamma, (const float*)w, norm.rows,  \
+                     norm.ldh, rows_and_flags, n, k, bias, (float*)c, ldc, norm.eps, scatter)
+#define PS_FNF_ROWS(EPI, PIECES, GROUPS)               \
+  do {                                                 \
+    if (m <= 4) PS_LAUNCH_FNF(EPI, PIECES, GROUPS, 4); \
+    else PS_LAUNCH_FNF(EPI, PIECES, GROUPS, 8);        \
+  } while (0)
+#define PS_SNF_CASE(EPI)                                                         \
+  case EPI:                                                                      \
+    if (m <= SF_FEW_ROWS && narrow && k <= 768) PS_FNF_ROWS(EPI, 3, 3);          \
+    else if (m <= SF_FEW_ROWS && narrow) PS_FNF_ROWS(EPI, 4, 3);                 \
+    else if (m <= SF_FEW_ROWS && k <= 768) PS_FNF_ROWS(EPI, 3, 4);               \
+    else if (m <= SF_FEW_ROWS) PS_FNF_ROWS(EPI, 4, 4);                           \
+    else if (k <= 8 * 3 * SF_STEP) PS_LAUNCH_SNF(EPI, 3);                        \
+    else PS_LAUNCH_SNF(EPI, 4);                                                  \
     break
   switch (epilogue) {
     PS_SNF_CASE(PS_EPI_NONE);
@@ -435,6 +638,8 @@ int ps_norm_gemm_f32_fused(const NormPrologue& norm, const void* w, const float*
     default: ps_set_error("ps_linear: unknown epilogue %d", epilogue); return 1;
   }
 #undef PS_SNF_CASE
+#undef PS_FNF_ROWS
+#undef PS_LAUNCH_FNF
 #undef PS_LAUNCH_SNF
   PS_CHECK_LAUNCH("ps_linear(skinny, norm, float)");
   return 0;

@@ -39,12 +39,13 @@ HIPCC_FLAGS = [
 ]
 # Per source: matrix products that accumulate in ordinary vector registers.  Kernels that go on
 # computing with the results (softmax, wide epilogues) then need no copies from the
-# accumulation registers; the skinny decode products are better off without.
+# accumulation registers; the skinny bfloat16 products are better off without.
 EXTRA_FLAGS = {
     "attention_prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "attention_mixed.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "attention_tiled_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "gemm_tiled.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "gemm_skinny_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 
 

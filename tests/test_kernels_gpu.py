@@ -249,6 +249,42 @@ def test_norm_in_front_of_a_product_of_float_rows(m, n, k, rms):
                                    atol=2e-6 * math.sqrt(k) / 8 + 8e-6, rtol=8e-6)
 
 
+@pytest.mark.parametrize("m,heads,kv_heads,k", [(1, 1, 1, 256), (4, 7, 2, 768), (5, 5, 3, 772), (8, 33, 11, 1020),
+                                                (3, 100, 15, 1024), (8, 99, 16, 764), (9, 7, 2, 768)])
+def test_norm_product_of_few_float_rows_writes_its_pages(m, heads, kv_heads, k):
+    """A norm, a product of up to four, eight and more float rows and its key/value scatter in one launch: heads of 25
+    columns (which end inside a block's 12 or 16), a k that is no whole piece, a row without a page and one whose
+    largest weight is infinite."""
+    from pagedserve_amd.ops import kernels
+
+    head_dim, page_size = 25, 8
+    q_cols, kv_cols = heads * head_dim, kv_heads * head_dim
+    n = q_cols + 2 * kv_cols
+    k_pool, v_pool, tables = _paged_fixture(torch.float32, [m + 20], kv_heads, head_dim, page_size, 420)
+    k_pool.zero_(), v_pool.zero_()
+    tok_item = torch.zeros(m, dtype=torch.int32, device="cuda")
+    tok_pos = torch.arange(20, m + 20, dtype=torch.int32, device="cuda")
+    if m > 1:
+        tok_pos[m - 1] = tables.shape[1] * page_size
+    h, gamma = _rand((m, k), torch.float32, 421, 2.0) + 0.5, 1.0 + _rand((k,), torch.float32, 422, 0.2)
+    beta, bias = _rand((k,), torch.float32, 423, 0.2), _rand((n,), torch.float32, 424)
+    w = _rand((n, k), torch.float32, 425, 1.0 / math.sqrt(k))
+    w[3, 0] = math.inf
+    out, scratch = torch.full((m, n), float("nan"), device="cuda"), torch.empty((m, k), device="cuda")
+    kernels.linear(kernels.PendingNorm(h, gamma, beta, 1e-5, False, scratch), w, bias, out,
+                   scatter=(k_pool, v_pool, tok_item, tok_pos, tables, q_cols, kv_cols))
+    normed = F.layer_norm(h.double(), (k,), gamma.double(), beta.double(), 1e-5)
+    # (the bounds of test_norm_in_front_of_a_product_of_float_rows)
+    torch.testing.assert_close(out.double(), normed @ w.double().t() + bias.double(),
+                               atol=2e-6 * math.sqrt(k) / 8 + 8e-6, rtol=8e-6)
+    kept = tok_pos < tables.shape[1] * page_size
+    pools = torch.zeros_like(k_pool), torch.zeros_like(v_pool)
+    for pool, first in zip(pools, (q_cols, q_cols + kv_cols)):
+        columns = out[kept, first:first + kv_cols].view(-1, kv_heads, head_dim)
+        pool[tables[0, (tok_pos[kept] // page_size).long()].long(), :, (tok_pos[kept] % page_size).long()] = columns
+    assert torch.equal(k_pool, pools[0]) and torch.equal(v_pool, pools[1])
+
+
 @pytest.mark.parametrize("m,n,k,norm", [(5, 2304, 768, False), (16, 2304, 768, False), (16, 17000, 768, False), (8, 4096, 1024, False),
                                         (16, 2100, 1600, False), (1, 2304, 768, True), (16, 2304, 768, True), (8, 4096, 1024, True),
                                         (16, 1536, 512, True)])
