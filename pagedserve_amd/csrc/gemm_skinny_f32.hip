@@ -563,6 +563,75 @@ __global__ __launch_bounds__(256) void gemm_nt_few_norm_f32_kernel(
   }
 }
 
+// Up to eight rows added to, without a norm in front, four columns to a block: the operands as in
+// gemm_nt_few_norm_f32_kernel, the rows' straight from memory, all asked for at once, and each block reads them once
+// (the waves of the plain kernel, gemm_simple.hip, read all of them each: that, and not the weights, is what a unit then
+// waits for).  Where it is taken (few_rows_take) both sides are measured.
+template <int PIECES, int ROWS>
+__global__ __launch_bounds__(256) void gemm_nt_few_f32_kernel(
+    const float* __restrict__ a, const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ c,
+    int m, int n, int k, int lda, int ldc) {
+  constexpr int WAVES = 4, SETS = ROWS / 4, ELEMENTS = 4 * ROWS;
+  __shared__ float partial[4 * WAVES][ELEMENTS];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // the same in every lane: scalar
+  const int n0 = blockIdx.x * 4;
+  const int sub = lane & 3, place = lane >> 2;
+  const float* w_row = w + (int64_t)(n0 + sub < n ? n0 + sub : n - 1) * k;
+  const float* a_row[SETS];
+#pragma unroll
+  for (int t = 0; t < SETS; ++t) a_row[t] = a + (int64_t)(t * 4 + sub < m ? t * 4 + sub : m - 1) * lda;
+  f32x4 wf[PIECES], xf[PIECES][SETS];
+#pragma unroll
+  for (int p = 0; p < PIECES; ++p) {
+    const int kk = (p * WAVES + wave) * SF_FEW_PIECE + place * 4;
+    const int at = kk < k ? kk : 0;
+    wf[p] = *reinterpret_cast<const f32x4*>(w_row + at);
+#pragma unroll
+    for (int t = 0; t < SETS; ++t) xf[p][t] = *reinterpret_cast<const f32x4*>(a_row[t] + at);
+  }
+  const int element = threadIdx.x;
+  const int out_col = n0 + (element & 3), out_row = element >> 2;
+  float* dst = c + (int64_t)(out_row < m ? out_row : m - 1) * ldc + (out_col < n ? out_col : n - 1);
+  const float before = *dst;
+  float own_bias = 0.f;
+  if (bias != nullptr) own_bias = bias[out_col < n ? out_col : n - 1];
+  __builtin_amdgcn_sched_barrier(0);
+  f32x4 acc[SETS][4];
+#pragma unroll
+  for (int t = 0; t < SETS; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[t][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int p = 0; p < PIECES; ++p) {
+    const bool beyond = (p * WAVES + wave) * SF_FEW_PIECE + place * 4 >= k;
+    if (beyond) wf[p] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < SETS; ++t)
+      if (beyond) xf[p][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int t = 0; t < SETS; ++t)
+        acc[t][i] = __builtin_amdgcn_mfma_f32_4x4x1f32(wf[p][i], xf[p][t][i], acc[t][i], 0, 0, 0);
+  }
+#pragma unroll
+  for (int t = 0; t < SETS; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float sum = (acc[t][0][i] + acc[t][1][i]) + (acc[t][2][i] + acc[t][3][i]);
+      sum += row_turned<4>(sum);
+      sum += row_turned<8>(sum);
+      if ((lane & 15) < 4) partial[wave * 4 + (lane >> 4)][(t * 4 + sub) * 4 + i] = sum;
+    }
+  __syncthreads();
+  if (element >= ELEMENTS || out_col >= n || out_row >= m) return;
+  float of_run[4 * WAVES];
+#pragma unroll
+  for (int p = 0; p < 4 * WAVES; ++p) of_run[p] = partial[p][element];
+  *dst = before + (sum_in_pairs(of_run) + own_bias);
+}
+
 // --------------------------------------------------------------------------------- host
 // Whether this kernel takes the product (a row of either operand in pieces of 16 bytes), and is the
 // fastest that does.  The lines, with weights from memory, in us:
@@ -579,11 +648,21 @@ __global__ __launch_bounds__(256) void gemm_nt_few_norm_f32_kernel(
 //   the output head beyond 16 rows (32 x 50257 x 768 71 against 68).
 // - A k that is no multiple of 32, which the tiled kernel does not take, up to 768 rows: there it
 //   meets the one that does (gemm_mfma.hip).
+// (few_rows_take) Rows added to, four columns to a block.  In us with weights from memory, before and with it: up to
+// four rows where k is long, 1 x 768 x 3072 5.5 / 4.2, 4 rows 5.55 / 5.15, 1 x 1600 x 1600 6.3 / 4.8, 4 x 1024 x 4096 6.75 /
+// 6.5, but 4 x 1024 x 1024 3.15 / 3.2; five to eight where it is not, 5 x 512 x 512 3.15 / 2.75, 5 x 768 x 768 3.4 / 3.1,
+// 8 x 1024 x 1024 3.8 / 3.75, but 8 x 1600 x 1600 7.0 / 8.3 and 5 x 768 x 3072, whose k is split, 4.85 / 6.2.
+static bool few_rows_take(int m, int n, int k, int epilogue) {
+  if (epilogue != PS_EPI_RESIDUAL || m > 8 || n > 8 * ps_compute_units()) return false;
+  return m <= 4 ? k > 1024 && k <= 4096 : k >= 512 && k <= 1024;
+}
+
 bool ps_gemm_nt_f32_skinny_takes(const void* a, const void* w, int m, int n, int k, int lda,
                                  int epilogue) {
   if (k % 4 != 0 || lda % 4 != 0 || (reinterpret_cast<uintptr_t>(a) & 15u) != 0 ||
       (reinterpret_cast<uintptr_t>(w) & 15u) != 0)
     return false;
+  if (few_rows_take(m, n, k, epilogue)) return true;
   const bool residual = epilogue == PS_EPI_RESIDUAL;
   const int64_t weights = (int64_t)n * k;
   if (m <= 4) return residual && k >= 4096;
@@ -681,6 +760,21 @@ static int launch_skinny_f32(const void* a, const void* w, const float* bias, vo
 int ps_gemm_nt_f32_skinny(const void* a, const void* w, const float* bias, void* c, int m, int n,
                           int k, int lda, int ldc, int epilogue, const KvScatter& scatter,
                           hipStream_t s) {
+  if (few_rows_take(m, n, k, epilogue)) {
+#define PS_LAUNCH_FEW(PIECES, ROWS)                                                                       \
+  hipLaunchKernelGGL((gemm_nt_few_f32_kernel<PIECES, ROWS>), dim3((n + 3) / 4), dim3(256), 0, s,          \
+                     (const float*)a, (const float*)w, bias, (float*)c, m, n, k, lda, ldc)
+    if (m > 4) {
+      if (k <= 512) PS_LAUNCH_FEW(2, 8);
+      else if (k <= 768) PS_LAUNCH_FEW(3, 8);
+      else PS_LAUNCH_FEW(4, 8);
+    } else if (k <= 2048) PS_LAUNCH_FEW(8, 4);
+    else if (k <= 3072) PS_LAUNCH_FEW(12, 4);
+    else PS_LAUNCH_FEW(16, 4);
+#undef PS_LAUNCH_FEW
+    PS_CHECK_LAUNCH("ps_linear(few rows, float)");
+    return 0;
+  }
 #define PS_SKINNY_CASE(EPI) \
   case EPI: return launch_skinny_f32<EPI>(a, w, bias, c, m, n, k, lda, ldc, scatter, s)
   switch (epilogue) {

@@ -285,6 +285,24 @@ def test_norm_product_of_few_float_rows_writes_its_pages(m, heads, kv_heads, k):
     assert torch.equal(k_pool, pools[0]) and torch.equal(v_pool, pools[1])
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1028), (4, 1601, 1600), (3, 50, 2052), (4, 768, 3076), (2, 30, 4096), (4, 40, 4100),
+                                   (5, 33, 512), (8, 2048, 516), (7, 767, 768), (6, 9, 772), (8, 2049, 1024), (5, 40, 1028)])
+def test_few_float_rows_added_to(m, n, k):
+    """Sums of a block's four columns over 16 places of k, on both sides of where that kernel is taken: remainders of
+    columns, pieces and rows; rows of C that are longer than n keep what lies behind it."""
+    from pagedserve_amd.ops import kernels
+
+    x, w = _rand((m, k + 4), torch.float32, 430)[:, :k], _rand((n, k), torch.float32, 431, 1.0 / math.sqrt(k))
+    bias, whole = _rand((n,), torch.float32, 432), _rand((m + 1, n + 3), torch.float32, 433)
+    for b in (None, bias):
+        before, out = whole.clone(), whole[:m, :n]
+        kernels.linear(x, w, b, out, epilogue="residual")
+        expected = before[:m, :n].double() + x.double() @ w.double().t() + (0.0 if b is None else b.double())
+        # (the bound of test_gemm_of_float_rows)
+        torch.testing.assert_close(out.double(), expected, atol=2e-6 * math.sqrt(k) / 8 + 4e-6, rtol=4e-6)
+        assert torch.equal(whole[:, n:], before[:, n:]) and torch.equal(whole[m:], before[m:])
+
+
 @pytest.mark.parametrize("m,n,k,norm", [(5, 2304, 768, False), (16, 2304, 768, False), (16, 17000, 768, False), (8, 4096, 1024, False),
                                         (16, 2100, 1600, False), (1, 2304, 768, True), (16, 2304, 768, True), (8, 4096, 1024, True),
                                         (16, 1536, 512, True)])
