@@ -29,8 +29,10 @@
 
 #define ADS_KEYS 64
 #define ADS_HEADS 16
+#define ADS_DIMS 256          // of a head at most
 #define ADS_PROW (ADS_KEYS + 8)
 #define ADS_LOADS 8           // 16-byte pieces of a tile per thread: 64 keys x 32 pieces / 256
+#define ADS_QUERIES 2         // and of the queries: 16 heads x 32 pieces / 256
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
@@ -40,29 +42,31 @@ int ps_attention_reduce(const float* partial, void* out, int64_t out_stride, con
                         void* stream);
 
 struct AdsArgs {
-  const bf16_t* q;
-  int64_t q_stride;
   const bf16_t* k_pool;
   const bf16_t* v_pool;
   float* partial;
-  const int* tok_list;
-  const int* tok_item;
-  const int* tok_pos;
-  const int* tables;
-  int table_width, heads, kv_heads, head_dim, page_size, num_pages;
+  int heads, kv_heads, page_size, num_pages;
   float scale_log2;
   int window, splits;
   float softcap_log2;
-  int page_shift, pieces_shift;     // log2 of the page size and of head_dim / 8, or -1
+  int page_shift;                   // log2 of the page size, or -1
+  uint32_t pieces_magic;            // i / (head_dim / 8) is i * this >> 20, i < 2,048
+  int group, parts;                 // query heads of a key/value head, and blocks that they are dealt to
   const float* logistic;            // (common.h: AttnExtras)
   float logistic_norm;
 };
 
 // dynamic LDS: keys [64][D + 8] bf16 | values the same (absent when they are the keys) |
 // queries [16][D + 8] bf16 | p [16][64 + 8] bf16 | scores [16][64] float | m, l, factor [16] float
-__global__ __launch_bounds__(256) void attention_decode_shared_kernel(const AdsArgs a) {
+// What a block needs first stands in front and comes with the launch.  A step of few keys to a range is bound by its
+// chain of dependent trips: position, page, rows.  The queries travel beside the first tile's (8 tokens of 12 heads of
+// 256 in 8 ranges 10.25 -> 9.95 us; what is left in front of the rows is their addresses' arithmetic).
+__global__ __launch_bounds__(256) void attention_decode_shared_kernel(
+    const int* __restrict__ tok_pos, const int* __restrict__ tables, const int* __restrict__ tok_list,
+    const int* __restrict__ tok_item, const bf16_t* __restrict__ q, int64_t q_stride, int table_width, int head_dim,
+    const AdsArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char ads_lds[];
-  const int D = a.head_dim;
+  const int D = head_dim;
   const int row = D + 8;                         // bf16 per cached row in LDS
   const bool same = a.v_pool == a.k_pool;
   bf16_t* s_k = reinterpret_cast<bf16_t*>(ads_lds);
@@ -75,17 +79,19 @@ __global__ __launch_bounds__(256) void attention_decode_shared_kernel(const AdsA
   float* s_f = s_l + ADS_HEADS;
 
   const int n = blockIdx.x;
-  const int group = a.heads / a.kv_heads;        // query heads per key/value head
-  const int parts = (group + ADS_HEADS - 1) / ADS_HEADS;
+  const int t = tok_list ? scalar_load(tok_list + n) : n;
+  const int pos = scalar_load(tok_pos + t);
+  const int item = tok_item ? scalar_load(tok_item + t) : t;
+  read_arguments(a.k_pool, a.v_pool, a.partial, a.heads, a.kv_heads, a.page_size, a.num_pages, a.scale_log2, a.window,
+                 a.splits, a.page_shift, a.pieces_magic, a.group, a.parts);
+  const int group = a.group, parts = a.parts;
   const int kv_head = blockIdx.y / parts;
   const int head0 = kv_head * group + (blockIdx.y % parts) * ADS_HEADS;
   const int nh = min(ADS_HEADS, kv_head * group + group - head0);
   const int split = blockIdx.z;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
-  const int t = a.tok_list ? a.tok_list[n] : n;
-  const int pos = a.tok_pos[t];
-  const int* table = a.tables + (int64_t)(a.tok_item ? a.tok_item[t] : t) * a.table_width;
+  const int* table = tables + (int64_t)item * table_width;
   const int first_key = first_visible_key(pos, a.window);
   const int end_key = pos + 1;
   int chunk = (end_key - first_key + a.splits - 1) / a.splits;
@@ -94,15 +100,19 @@ __global__ __launch_bounds__(256) void attention_decode_shared_kernel(const AdsA
   const int range_end = min(range_begin + chunk, end_key);
   const int pieces = D / 8;                      // 16-byte pieces of a cached row
 
-  // the heads' queries as they are; rows of heads that the block does not have are zero
-  for (int i = tid; i < ADS_HEADS * pieces; i += 256) {
-    const int h = i / pieces, piece = i - h * pieces;
-    uint4 v = make_uint4(0, 0, 0, 0);
-    if (h < nh) {
-      const bf16_t* src = a.q + (int64_t)t * a.q_stride + (int64_t)(head0 + h) * D + piece * 8;
-      v = *reinterpret_cast<const uint4*>(src);
-    }
-    *reinterpret_cast<uint4*>(s_q + h * row + piece * 8) = v;
+  // the heads' queries as they are; rows of heads that the block does not have are zero.  They wait in registers until
+  // the first tile's rows are asked for.
+  uint4 queries[ADS_QUERIES];
+  auto query_place = [&](int u, int* h, int* piece) {
+    const int i = tid + 256 * u;
+    *h = (int)(((uint32_t)i * a.pieces_magic) >> 20);
+    *piece = i - *h * pieces;
+  };
+#pragma unroll
+  for (int u = 0; u < ADS_QUERIES; ++u) {
+    int h, piece;
+    query_place(u, &h, &piece);
+    queries[u] = *reinterpret_cast<const uint4*>(q + (int64_t)t * q_stride + (int64_t)(head0 + (h < nh ? h : 0)) * D + piece * 8);
   }
   for (int i = tid; i < ADS_HEADS * ADS_PROW / 2; i += 256) reinterpret_cast<uint32_t*>(s_p)[i] = 0u;
   if (tid < ADS_HEADS) {
@@ -117,82 +127,141 @@ __global__ __launch_bounds__(256) void attention_decode_shared_kernel(const AdsA
   for (int j = 0; j < 4; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int d_tiles = (D + 15) / 16;
 
-  for (int base = range_begin; base < range_end; base += ADS_KEYS) {
-    __syncthreads();                             // the tile before is done with (and s_q is there)
-    {
-      // a thread's pieces of the tile: first every page number, then every row, then LDS, so
-      // that the trips to memory overlap
-      int key[ADS_LOADS], piece[ADS_LOADS], page[ADS_LOADS];
-      bool live[ADS_LOADS];
-      uint4 kv[ADS_LOADS], vv[ADS_LOADS];
+  auto there = [&](int base, int key) { return key < ADS_KEYS && base + key < range_end; };
+  auto kept_bits = [](const uint4& v, uint32_t keep) {
+    return make_uint4(v.x & keep, v.y & keep, v.z & keep, v.w & keep);
+  };
+  auto put_queries = [&] {
+#pragma unroll
+    for (int u = 0; u < ADS_QUERIES; ++u) {
+      int h, piece;
+      query_place(u, &h, &piece);
+      if (h < ADS_HEADS)
+        *reinterpret_cast<uint4*>(s_q + h * row + piece * 8) = kept_bits(queries[u], h < nh ? 0xFFFFFFFFu : 0u);
+    }
+  };
+  // a thread's pieces of a tile: first every page number, then every row, then LDS, so that the trips to memory
+  // overlap; the next tile's travel while this one is worked on
+  int key[ADS_LOADS], piece[ADS_LOADS];
+  uint4 kv[ADS_LOADS], vv[ADS_LOADS];
+#pragma unroll
+  for (int u = 0; u < ADS_LOADS; ++u) {
+    const int i = tid + 256 * u;
+    key[u] = (int)(((uint32_t)i * a.pieces_magic) >> 20);
+    piece[u] = i - key[u] * pieces;
+  }
+  auto load_tile = [&](int base) {
+    // (keys beyond the range, or the tile, are read as the range's first and left out below)
+    int page[ADS_LOADS], within[ADS_LOADS];
+    if (a.page_shift >= 0) {
 #pragma unroll
       for (int u = 0; u < ADS_LOADS; ++u) {
-        const int i = tid + 256 * u;
-        key[u] = a.pieces_shift >= 0 ? i >> a.pieces_shift : i / pieces;
-        piece[u] = i - key[u] * pieces;
-        const int p = base + key[u];
-        live[u] = key[u] < ADS_KEYS && p < range_end;
-        const int logical = a.page_shift >= 0 ? p >> a.page_shift : p / a.page_size;
-        page[u] = table[live[u] ? logical : 0];
+        const int p = there(base, key[u]) ? base + key[u] : range_begin;
+        page[u] = p >> a.page_shift;
+        within[u] = p & (a.page_size - 1);
       }
+    } else {
 #pragma unroll
       for (int u = 0; u < ADS_LOADS; ++u) {
-        const int p = base + key[u];
-        const int within = a.page_shift >= 0 ? p & (a.page_size - 1) : p % a.page_size;
-        const int safe = min(max(page[u], 0), a.num_pages - 1);
-        const int64_t at = (((int64_t)safe * a.kv_heads + kv_head) * a.page_size + within) * D + piece[u] * 8;
-        kv[u] = live[u] ? *reinterpret_cast<const uint4*>(a.k_pool + at) : make_uint4(0, 0, 0, 0);
-        if (!same) vv[u] = live[u] ? *reinterpret_cast<const uint4*>(a.v_pool + at) : make_uint4(0, 0, 0, 0);
-      }
-#pragma unroll
-      for (int u = 0; u < ADS_LOADS; ++u) {
-        if (key[u] < ADS_KEYS) {
-          *reinterpret_cast<uint4*>(s_k + key[u] * row + piece[u] * 8) = kv[u];
-          if (!same) *reinterpret_cast<uint4*>(s_v + key[u] * row + piece[u] * 8) = vv[u];
-        }
+        const int p = there(base, key[u]) ? base + key[u] : range_begin;
+        page[u] = p / a.page_size;
+        within[u] = p - page[u] * a.page_size;
       }
     }
+#pragma unroll
+    for (int u = 0; u < ADS_LOADS; ++u) page[u] = table[page[u]];
+#pragma unroll
+    for (int u = 0; u < ADS_LOADS; ++u) {
+      const int safe = min(max(page[u], 0), a.num_pages - 1);
+      const int64_t at = (((int64_t)safe * a.kv_heads + kv_head) * a.page_size + within[u]) * D + piece[u] * 8;
+      kv[u] = *reinterpret_cast<const uint4*>(a.k_pool + at);
+      if (!same) vv[u] = *reinterpret_cast<const uint4*>(a.v_pool + at);
+    }
+  };
+  if (range_begin < range_end) {
+    load_tile(range_begin);
+    put_queries();
+  }
+  for (int base = range_begin; base < range_end; base += ADS_KEYS) {
+    if (base > range_begin) __syncthreads();     // the tile before is done with
+#pragma unroll
+    for (int u = 0; u < ADS_LOADS; ++u) {
+      if (key[u] < ADS_KEYS) {
+        const uint32_t keep = there(base, key[u]) ? 0xFFFFFFFFu : 0u;
+        *reinterpret_cast<uint4*>(s_k + key[u] * row + piece[u] * 8) = kept_bits(kv[u], keep);
+        if (!same) *reinterpret_cast<uint4*>(s_v + key[u] * row + piece[u] * 8) = kept_bits(vv[u], keep);
+      }
+    }
+    if (base + ADS_KEYS < range_end) load_tile(base + ADS_KEYS);
     __syncthreads();
     {
       // S[key 16 wave + 4 g + i][head r]
       f32x4 sc = f32x4{0.f, 0.f, 0.f, 0.f};
       const bf16_t* kr = s_k + (16 * wave + r) * row + 8 * g;
       const bf16_t* qr = s_q + r * row + 8 * g;
-      for (int d0 = 0; d0 < D; d0 += 32) {
-        uint4 kf = make_uint4(0, 0, 0, 0), qf = make_uint4(0, 0, 0, 0);
-        if (d0 + 8 * g < D) {
-          kf = *reinterpret_cast<const uint4*>(kr + d0);
-          qf = *reinterpret_cast<const uint4*>(qr + d0);
-        }
-        sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(&kf),
-                                                     *reinterpret_cast<const bf16x8*>(&qf), sc, 0, 0, 0);
+      // (eight pieces at most, asked for together: one trip to LDS)
+      uint4 kf[ADS_DIMS / 32], qf[ADS_DIMS / 32];
+#pragma unroll
+      for (int d = 0; d < ADS_DIMS / 32; ++d) {
+        const int at = 32 * d + 8 * g < D ? 32 * d : 0;
+        kf[d] = *reinterpret_cast<const uint4*>(kr + at);
+        qf[d] = *reinterpret_cast<const uint4*>(qr + at);
+      }
+#pragma unroll
+      for (int d = 0; d < ADS_DIMS / 32; ++d) {
+        if (32 * d >= D) break;
+        const uint32_t keep = 32 * d + 8 * g < D ? 0xFFFFFFFFu : 0u;
+        const uint4 ko = kept_bits(kf[d], keep), qo = kept_bits(qf[d], keep);
+        sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(&ko),
+                                                     *reinterpret_cast<const bf16x8*>(&qo), sc, 0, 0, 0);
       }
       *reinterpret_cast<float4*>(s_s + r * ADS_KEYS + 16 * wave + 4 * g) =
           make_float4(sc[0] * a.scale_log2, sc[1] * a.scale_log2, sc[2] * a.scale_log2, sc[3] * a.scale_log2);
     }
     __syncthreads();
+    // a wave's up to four heads side by side: their maxima and sums do not wait for each other
+    constexpr int OWN = ADS_HEADS / 4;
     const bool visible = base + lane < range_end;
-    for (int h = wave; h < nh; h += 4) {
-      float s = s_s[h * ADS_KEYS + lane];
-      if (a.softcap_log2 > 0.f) s = capped_score_fast(s, a.softcap_log2);
-      if (!visible) s = -INFINITY;
-      if (a.logistic != nullptr) {
-        const float p = visible ? logistic_weight_fast(s + a.logistic[head0 + h] * 1.4426950408889634f) : 0.f;
+    float score[OWN];
+#pragma unroll
+    for (int u = 0; u < OWN; ++u) {
+      score[u] = s_s[(wave + 4 * u) * ADS_KEYS + lane];
+      if (a.softcap_log2 > 0.f) score[u] = capped_score_fast(score[u], a.softcap_log2);
+      if (!visible) score[u] = -INFINITY;
+    }
+    if (a.logistic != nullptr) {
+#pragma unroll
+      for (int u = 0; u < OWN; ++u) {
+        const int h = wave + 4 * u;
+        if (h >= nh) break;
+        const float p = visible ? logistic_weight_fast(score[u] + a.logistic[head0 + h] * 1.4426950408889634f) : 0.f;
         s_p[h * ADS_PROW + lane] = float_to_bf16(p);
-        continue;
       }
-      const float before = s_m[h];
-      const float m_new = fmaxf(before, wave_max(s));          // (a tile has at least one visible key)
-      const float p = visible ? __builtin_amdgcn_exp2f(s - m_new) : 0.f;
-      // the sum is of the rounded weights, which are what multiplies the values
-      const bf16_t rounded = float_to_bf16(p);
-      const float sum = wave_sum(bf16_to_float(rounded));
-      s_p[h * ADS_PROW + lane] = rounded;
-      if (lane == 0) {
-        const float factor = before == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(before - m_new);
-        s_f[h] = factor;
-        s_l[h] = s_l[h] * factor + sum;
-        s_m[h] = m_new;
+    } else {
+      float before[OWN], m_new[OWN], sum[OWN];
+      bf16_t rounded[OWN];
+#pragma unroll
+      for (int u = 0; u < OWN; ++u) before[u] = s_m[wave + 4 * u];
+#pragma unroll
+      for (int u = 0; u < OWN; ++u)
+        m_new[u] = fmaxf(before[u], wave_max(score[u]));          // (a tile has at least one visible key)
+#pragma unroll
+      for (int u = 0; u < OWN; ++u) {
+        // the sum is of the rounded weights, which are what multiplies the values
+        rounded[u] = float_to_bf16(visible ? __builtin_amdgcn_exp2f(score[u] - m_new[u]) : 0.f);
+        sum[u] = wave_sum(bf16_to_float(rounded[u]));
+      }
+#pragma unroll
+      for (int u = 0; u < OWN; ++u) {
+        const int h = wave + 4 * u;
+        if (h >= nh) break;
+        s_p[h * ADS_PROW + lane] = rounded[u];
+        if (lane == 0) {
+          const float factor = before[u] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(before[u] - m_new[u]);
+          s_f[h] = factor;
+          s_l[h] = s_l[h] * factor + sum[u];
+          s_m[h] = m_new[u];
+        }
       }
     }
     __syncthreads();
@@ -295,12 +364,12 @@ extern "C" int ps_attention_decode_shared(const void* q, int64_t q_stride, const
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(attention_decode_shared_kernel),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)ads_lds_bytes(256, false));
   });
-  const AdsArgs a = {(const bf16_t*)q, q_stride, (const bf16_t*)k_pool, (const bf16_t*)v_pool, partial,
-                     tok_list, tok_item, tok_pos, tables, table_width, heads, kv_heads, head_dim,
-                     page_size, num_pages, scale * 1.4426950408889634f, window, splits,
-                     softcap * 1.4426950408889634f, ads_shift(page_size), ads_shift(head_dim / 8),
-                     logistic, logistic_norm};
-  hipLaunchKernelGGL(attention_decode_shared_kernel, dim3(count, kv_heads * parts, splits), dim3(256), lds, s, a);
+  const AdsArgs a = {(const bf16_t*)k_pool, (const bf16_t*)v_pool, partial, heads, kv_heads, page_size, num_pages,
+                     scale * 1.4426950408889634f, window, splits, softcap * 1.4426950408889634f,
+                     ads_shift(page_size),
+                     (uint32_t)(((1 << 20) + head_dim / 8 - 1) / (head_dim / 8)), group, parts, logistic, logistic_norm};
+  hipLaunchKernelGGL(attention_decode_shared_kernel, dim3(count, kv_heads * parts, splits), dim3(256), lds, s, tok_pos,
+                     tables, tok_list, tok_item, (const bf16_t*)q, q_stride, table_width, head_dim, a);
   PS_CHECK_LAUNCH("ps_attention_decode_shared");
   if (out == nullptr) return 0;      // the records are all that is asked for: the caller merges them
   return ps_attention_reduce(partial, out, out_stride, tok_list, count, heads, head_dim, splits, gate, gate_ld,

@@ -39,25 +39,41 @@ __device__ inline float decay_of<bf16_t>(float rate, float step) { return __buil
 
 // x[t, c] = silu(conv(u)[t, c]): a thread per (token, channel).  Inputs before the step's first
 // token of the item come from the slot (zeros for a new request: the slot was cleared).
-template <typename T>
+// TAPS: their number, so that all of a thread's inputs and weights are asked for at once, from the row or the slot as
+// each lies; 0: any number, one after the other (four: 8 tokens of 768 channels 2.85 -> 2.5 us in a decode step, 2048
+// tokens 11.1 -> 7.3).
+template <typename T, int TAPS>
 __global__ __launch_bounds__(256) void conv_silu_kernel(
-    const float* __restrict__ proj, int64_t ld, int u_col, const float* __restrict__ w,
-    const float* __restrict__ bias, const float* __restrict__ state, int row, int tail,
-    T* __restrict__ x, const int* __restrict__ tok_item, const int* __restrict__ cu_tokens,
-    const int* __restrict__ slots, int channels, int taps, int activation) {
+    const int* __restrict__ tok_item, const int* __restrict__ cu_tokens, const int* __restrict__ slots,
+    const float* __restrict__ proj, const float* __restrict__ state, const float* __restrict__ w,
+    const float* __restrict__ bias, T* __restrict__ x, int64_t ld, int u_col, int row, int tail, int channels, int taps,
+    int activation) {
   const int t = blockIdx.x;
+  const int item = scalar_load(tok_item + t);
+  read_arguments(x, ld, u_col, row, tail, channels, taps, activation);
+  const int first = scalar_load(cu_tokens + item), slot = scalar_load(slots + item);
   const int c = blockIdx.y * 256 + threadIdx.x;
   if (c >= channels) return;
-  const int item = tok_item[t];
-  const int first = cu_tokens[item];
-  const float* kept = state + ((int64_t)slots[item] * channels + c) * row + tail;
+  const int count = TAPS > 0 ? TAPS : taps;
+  const float* kept = state + ((int64_t)slot * channels + c) * row + tail;
+  const float* own = proj + u_col + c;
+  // the input `back` tokens before this one: a token of this step, or one that the slot kept
+  auto place = [&](int j) {
+    const int back = count - 1 - j;
+    const int local = (t - first) - back;
+    return local >= 0 ? own + (int64_t)(t - back) * ld : kept + (count - 1 + local);
+  };
   float sum = bias ? bias[c] : 0.f;
-  for (int j = 0; j < taps; ++j) {
-    const int back = taps - 1 - j;           // the input `back` tokens before this one
-    const int local = (t - first) - back;    // its place among the item's tokens of this step
-    const float u = local >= 0 ? proj[(int64_t)(t - back) * ld + u_col + c]
-                               : kept[taps - 1 + local];
-    sum = fmaf(w[(int64_t)c * taps + j], u, sum);
+  if constexpr (TAPS > 0) {
+    float u[TAPS], weight[TAPS];
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) u[j] = *place(j);
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) weight[j] = w[(int64_t)c * TAPS + j];
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) sum = fmaf(weight[j], u[j], sum);
+  } else {
+    for (int j = 0; j < taps; ++j) sum = fmaf(w[(int64_t)c * taps + j], *place(j), sum);
   }
   x[(int64_t)t * channels + c] = from_float<T>(activation ? silu_f(sum) : sum);
 }
@@ -375,12 +391,20 @@ extern "C" int ps_conv_silu(const float* proj, int64_t ld, int u_col, const floa
   hipStream_t s = (hipStream_t)stream;
   const dim3 grid(tokens, (channels + 255) / 256);
   const int row = states + taps - 1;
-  if (dtype == PS_F32)
-    hipLaunchKernelGGL(conv_silu_kernel<float>, grid, dim3(256), 0, s, proj, ld, u_col, w, bias, state,
-                       row, states, (float*)x, tok_item, cu_tokens, slots, channels, taps, activation);
-  else
-    hipLaunchKernelGGL(conv_silu_kernel<bf16_t>, grid, dim3(256), 0, s, proj, ld, u_col, w, bias, state,
-                       row, states, (bf16_t*)x, tok_item, cu_tokens, slots, channels, taps, activation);
+#define PS_LAUNCH_CS_AS(T, TAPS)                                                                         \
+  hipLaunchKernelGGL((conv_silu_kernel<T, TAPS>), grid, dim3(256), 0, s, tok_item, cu_tokens, slots, proj, \
+                     state, w, bias, (T*)x, ld, u_col, row, states, channels, taps, activation)
+#define PS_LAUNCH_CS(T)                       \
+  do {                                        \
+    if (taps == 2) PS_LAUNCH_CS_AS(T, 2);     \
+    else if (taps == 3) PS_LAUNCH_CS_AS(T, 3); \
+    else if (taps == 4) PS_LAUNCH_CS_AS(T, 4); \
+    else PS_LAUNCH_CS_AS(T, 0);               \
+  } while (0)
+  if (dtype == PS_F32) PS_LAUNCH_CS(float);
+  else PS_LAUNCH_CS(bf16_t);
+#undef PS_LAUNCH_CS
+#undef PS_LAUNCH_CS_AS
   PS_CHECK_LAUNCH("ps_conv_silu");
   return 0;
 }

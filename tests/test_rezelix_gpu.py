@@ -157,6 +157,29 @@ def test_gated_recurrence_per_item_and_in_pieces(channels, blocks, taps):
     assert torch.allclose(half.float(), out, atol=2e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("channels,taps", [(70, 7), (64, 8), (30, 9)])
+def test_single_tokens_of_long_convolutions(channels, taps):
+    """One token of each item, with as many kept inputs as are asked for at once, and one more; an item without
+    tokens between them."""
+    kernels = _kernels()
+    g = torch.Generator().manual_seed(channels)
+    proj, u, gates, lam, r, i = _recurrence_inputs(g, 2, channels, 1)
+    start = torch.randn((3, channels, taps), generator=g)
+    state, out = start.clone().cuda(), torch.empty((2, channels), device="cuda")
+    kernels.lru_scan(proj.cuda(), 3, 3 + channels, u.cuda(), gates.cuda(), channels, lam.cuda(), 8.0, state, out,
+                     _ints([0, 1, 1, 2]), _ints([2, 1, 0]), taps)
+    for row, slot in ((0, 2), (1, 0)):
+        one = slice(row, row + 1)
+        states, final = plain.gated_recurrence(u[one].double(), r[one], i[one], lam.double(), 8.0,
+                                               start[slot, :, 0].double())
+        expected = states * plain.gelu_tanh(proj[one, 3:3 + channels].double())
+        assert torch.allclose(out[one].double().cpu(), expected, atol=2e-5, rtol=2e-5)
+        assert torch.allclose(state[slot, :, 0].double().cpu(), final, atol=2e-5, rtol=2e-5)
+        kept = torch.cat([start[slot, :, 2:], proj[row, 3 + channels:3 + 2 * channels, None]], dim=1)
+        assert torch.equal(state[slot, :, 1:].cpu(), kept)
+    assert torch.equal(state[1].cpu(), start[1])
+
+
 def test_a_channel_that_barely_forgets_keeps_what_it_was_given():
     """A decay next to one: ``sqrt(1 - a^2)`` must not be lost to cancellation, and what the first
     token wrote is still there five hundred tokens on."""
