@@ -442,6 +442,56 @@ def test_recurrent_output_norm_and_gate():
         assert torch.allclose(out.double().cpu(), expected, atol=tol, rtol=tol)
 
 
+@pytest.mark.parametrize("heads,dim,vdim", [(2, 24, 40), (3, 64, 64), (1, 33, 5), (2, 128, 30), (1, 200, 64)])
+@pytest.mark.parametrize("per_head", [False, True])
+def test_single_tokens_like_chunks_of_eight(heads, dim, vdim, per_head):
+    """Steps of one token a request, staged alone, give the bits of steps of up to eight; a request without a token
+    and a slot that nobody holds keep their state."""
+    kernels = _kernels()
+    g = torch.Generator().manual_seed(dim + vdim)
+    q_col, k_col, v_col = 3, 3 + heads * dim, 3 + 2 * heads * dim
+    proj = torch.randn((3, v_col + heads * vdim + 1), generator=g).cuda()
+    alpha, decay = torch.rand((3, heads * dim), generator=g).cuda(), torch.rand(heads, generator=g).cuda()
+    initial = torch.randn((5, heads, dim, vdim), generator=g).cuda()
+    cu = torch.tensor([0, 1, 1, 2, 3], dtype=torch.int32, device="cuda")
+    slots = torch.tensor([4, 0, 1, 3], dtype=torch.int32, device="cuda")
+    got = []
+    for longest in (1, 8):
+        state, out = initial.clone(), torch.full((3, heads * vdim), float("nan"), device="cuda")
+        kernels.gla_scan(proj, (q_col, k_col, v_col), None if per_head else alpha, state, out, cu, slots, heads, dim,
+                         vdim, 0.5, longest=longest, head_decay=decay if per_head else None, silu_inputs=per_head)
+        got.append((state, out))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    assert not torch.isnan(got[0][1]).any()
+    for idle in (0, 2):
+        assert torch.equal(got[0][0][idle], initial[idle])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rank,channels", [(8, 37), (16, 300), (32, 256), (24, 300)])
+def test_decay_of_whole_pieces(dtype, rank, channels):
+    kernels = _kernels()
+    g = torch.Generator().manual_seed(rank)
+    proj = torch.randn((5, 3 + rank), generator=g)
+    w, bias = torch.randn((channels, rank), generator=g).to(dtype), torch.randn(channels, generator=g)
+    alpha = torch.empty((5, channels), device="cuda")
+    kernels.gla_decay(proj.cuda(), 3, w.cuda(), bias.cuda(), 16.0, alpha)
+    expected = plain.decay_of(proj[:, 3:].double() @ w.double().T + bias.double(), 16.0)
+    assert torch.allclose(alpha.double().cpu(), expected, rtol=2e-5, atol=1e-12)
+
+
+@pytest.mark.parametrize("vdim", [5, 64, 100, 256, 300])
+def test_output_norm_of_every_head_size(vdim):
+    kernels = _kernels()
+    g = torch.Generator().manual_seed(vdim)
+    o, gate = torch.randn((3, 2 * vdim), generator=g), torch.randn((3, 2 * vdim), generator=g)
+    weight, out = 1 + 0.2 * torch.randn(vdim, generator=g), torch.empty((3, 2 * vdim), device="cuda")
+    kernels.gla_output(o.cuda(), weight.cuda(), 1e-5, gate.cuda(), out, 2, vdim)
+    expected = (plain.rms_norm(o.double().view(3, 2, vdim), weight.double(), 1e-5).view(3, -1)
+                * gate.double() * torch.sigmoid(gate.double()))
+    assert torch.allclose(out.double().cpu(), expected, atol=1e-5, rtol=1e-5)
+
+
 # ---------------------------------------------------------------- whole models
 def _close(rows, reference, dtype):
     """float32: every position within the tolerance.  bfloat16: the recurrent mixer norms each
