@@ -450,7 +450,7 @@ class Engine:
         for group in range(groups):
             section(f"tables{group}").reshape(items, width)[:] = cache.table_arrays[group][slot_index]
         self._meta_words[turn].to_device(self._meta_device, cursor)
-        self._meta_events[turn].record()
+        self._meta_events[turn].record(self.stream)
         self._meta_pending[turn] = True
         self._last_layout = (offsets, cursor)
 
@@ -497,7 +497,7 @@ class Engine:
             output.host_tokens = self._tokens_host[turn][:rows]
             self._tokens_words[turn].from_device(output.tokens, rows)
             output.ready = self._tokens_ready[turn]
-            output.ready.record()
+            output.ready.record(self.stream)     # (the current one: named, torch need not look it up)
             self._carried_rows = rows
         else:
             self._carried_rows = 0
@@ -651,7 +651,7 @@ class Engine:
         for group in range(len(cache.groups)):
             sections[f"tables{group}"][:] = cache.table_arrays[group][slots]
         self._meta_words[turn].to_device(self._meta_device, plan.used)
-        self._meta_events[turn].record()
+        self._meta_events[turn].record(self.stream)
         self._meta_pending[turn] = True
         plan.graph.launch()
         rows = [(entry.request_id, start) for entry, start in zip(entries, starts)]
