@@ -60,7 +60,7 @@ struct NothingAhead {
 
 // How a launch's pages are walked, worked out on the host: a word that comes with the launch.
 #define AD_SHIFT(form) (((form) & 63) - 1)     // log2 of the page size, -1: no power of two
-#define AD_EVEN 64          // the keys of one load lie in one page, whose values are counted in 31 bits
+#define AD_EVEN 64          // the keys of one load lie in one page, whose bytes are counted in 31 bits
 #define AD_FROM_START 128   // token t is item t and its block walks all keys from the first: the first entries of the
                             // block table are known without the position
 #define AD_HEAD_DIM(form) ((form) >> 16)
@@ -73,7 +73,7 @@ inline int decode_form(int head_dim, int page_size, int kv_heads, bool from_star
     while ((1 << shift) < page_size) ++shift;
   }
   const bool even = shift >= 0 && page_size >= 64 / lanes &&
-                    (int64_t)page_size * kv_heads * head_dim < ((int64_t)1 << 31);
+                    (int64_t)page_size * kv_heads * head_dim < ((int64_t)1 << 29);
   return (shift + 1) | (even ? AD_EVEN : 0) | (from_start ? AD_FROM_START : 0) | (head_dim << 16);
 }
 

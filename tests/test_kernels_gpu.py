@@ -1236,6 +1236,28 @@ def test_attention_decode_pages_of_a_load(dtype, window, head_dim, page_size):
             torch.testing.assert_close(out[:rows].double(), expected, atol=atol, rtol=rtol)
 
 
+def test_attention_decode_page_beyond_32_bits():
+    """Float keys further into their page than 32 bits count bytes (one page of 2^23 keys of 192 values, 6 GiB a pool)."""
+    from pagedserve_amd.ops import kernels
+
+    page_size, head_dim, window = 1 << 23, 192, 40
+    k_pool = torch.empty((1, 1, page_size, head_dim), device="cuda")
+    v_pool = torch.empty((1, 1, page_size, head_dim), device="cuda")
+    last = page_size - 3
+    keys, values = _rand((window, head_dim), torch.float32, 523), _rand((window, head_dim), torch.float32, 524)
+    for pool, rows in ((k_pool, keys), (v_pool, values)):
+        pool[0, 0, :64], pool[0, 0, -64:] = 1.0, 2.0
+        pool[0, 0, last + 1 - window:last + 1] = rows
+    q = _rand((1, head_dim), torch.float32, 525)
+    scale = head_dim ** -0.5
+    weights = torch.softmax(q.double() @ keys.double().T * scale, dim=-1)
+    out = torch.full_like(q, float("nan"))
+    pos = torch.tensor([last], dtype=torch.int32, device="cuda")
+    tables = torch.zeros((1, 1), dtype=torch.int32, device="cuda")
+    kernels.attention_decode(q, k_pool, v_pool, out, None, pos, tables, 1, scale, 1, window=window)
+    torch.testing.assert_close(out.double(), weights @ values.double(), atol=3e-5, rtol=3e-5)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_attention_decode_sixteen_waves(dtype):
     from pagedserve_amd.ops import kernels
