@@ -196,13 +196,16 @@ struct TileEnds {
 // belongs to this wave alone: bias, activation, residual add into the float stream, key/value
 // columns into cache pages.  `split` / `k_splits`: partial sums of a k range are added with
 // atomics, the bias by split 0 only.  `ends`, `pages`: what the caller has asked for (the pages
-// where TilePages::wanted says so).
+// where TilePages::wanted says so).  Inlined whatever it costs: the compiler made it a function of its own behind
+// the GELU of tiles of 128 x 64, its arrays in scratch memory (float rows, us: 2048 x 3072 x 768 92.6, inlined 90.0,
+// 4096 x 3072 x 768 176.7 and 170.8, 2048 x 6400 x 1600 391 and 384).
 template <int WM, int WN, typename TOut, int EPI>
-__device__ inline void store_wave_tile(f32x16 (&acc)[WM][WN], float* region, int lane, int row_base,
-                                       int col_base, int m, int n, int ldc, TOut* __restrict__ c,
-                                       const float* __restrict__ bias, int split, int k_splits,
-                                       const KvScatter& scatter, const TileEnds<WM, WN, TOut, EPI>& ends,
-                                       const TilePages<WM, WN>& pages) {
+__device__ __forceinline__ void store_wave_tile(f32x16 (&acc)[WM][WN], float* region, int lane, int row_base,
+                                                int col_base, int m, int n, int ldc, TOut* __restrict__ c,
+                                                const float* __restrict__ bias, int split, int k_splits,
+                                                const KvScatter& scatter,
+                                                const TileEnds<WM, WN, TOut, EPI>& ends,
+                                                const TilePages<WM, WN>& pages) {
   using Pieces = TilePieces<WM, WN>;
   constexpr int EP_STRIDE = Pieces::STRIDE, EP_ROWS = Pieces::ROWS, PASSES = Pieces::PASSES;
   // The callers read operands by assembly and wait for them just in front of this.  What is worked out of the lane here
@@ -307,10 +310,10 @@ __device__ inline void store_wave_tile(f32x16 (&acc)[WM][WN], float* region, int
 
 // The same for a kernel that has asked for nothing yet.
 template <int WM, int WN, typename TOut, int EPI>
-__device__ inline void store_wave_tile(f32x16 (&acc)[WM][WN], float* region, int lane, int row_base,
-                                       int col_base, int m, int n, int ldc, TOut* __restrict__ c,
-                                       const float* __restrict__ bias, int split, int k_splits,
-                                       const KvScatter& scatter) {
+__device__ __forceinline__ void store_wave_tile(f32x16 (&acc)[WM][WN], float* region, int lane, int row_base,
+                                                int col_base, int m, int n, int ldc, TOut* __restrict__ c,
+                                                const float* __restrict__ bias, int split, int k_splits,
+                                                const KvScatter& scatter) {
   asm volatile("" : "+v"(lane));
   const bool by_column = tile_by_column<TOut, EPI>(c, ldc, k_splits, scatter);
   TileEnds<WM, WN, TOut, EPI> ends;

@@ -1,5 +1,5 @@
 """Looks through the machine code of the built kernel library for registers that are used while a load into them is
-still on its way.
+still on its way, and says what its kernels take of registers, LDS and scratch memory.
 
 The compiler waits for the loads that it knows of.  Loads written in assembly it takes as done where they stand, so that
 nothing but the kernel's own waits, and where the compiler happens to keep the values, stands between a load and the
@@ -148,3 +148,19 @@ def disassemble(image, arch, folder):
         handle.write(image)
     return subprocess.run([disassembler(), "-d", f"--mcpu={arch}", path], check=True, stdout=subprocess.PIPE,
                           text=True).stdout
+
+
+def resources(image, folder):
+    """{symbol of a kernel: {"vgpr": registers, "scratch" and "lds": bytes}} of a code object, from the notes that the
+    compiler leaves in it."""
+    path = os.path.join(str(folder), "kernels.elf")
+    with open(path, "wb") as handle:
+        handle.write(image)
+    notes = subprocess.run([os.path.join(os.path.dirname(disassembler()), "llvm-readelf"), "--notes", path], check=True,
+                           stdout=subprocess.PIPE, text=True).stdout
+    found = {}
+    for part in notes.split("- .agpr_count:")[1:]:
+        fields = dict(re.findall(r"^    \.(\w+):\s+(\S+)$", part, re.M))
+        found[fields["name"]] = {"vgpr": int(fields["vgpr_count"]), "scratch": int(fields["private_segment_fixed_size"]),
+                                 "lds": int(fields["group_segment_fixed_size"])}
+    return found

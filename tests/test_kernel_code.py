@@ -1,4 +1,5 @@
-"""The machine code of the kernels whose loads are written in assembly: no register is used before its load is there."""
+"""The machine code of the kernels whose loads are written in assembly: no register is used before its load is there.
+And what the tiled products take, which decides how many of their blocks a compute unit holds."""
 
 import os
 
@@ -54,4 +55,25 @@ def test_no_register_is_used_before_its_load(kernel, tmp_path):
                 seen += 1
                 assert any(operation.startswith("ds_read") for _, operation, _, _ in code), name
                 assert not kernel_code.early_uses(code), (name, kernel_code.early_uses(code)[:4])
+    assert seen
+
+
+@pytest.mark.skipif(kernel_code.disassembler() is None, reason="no disassembler")
+@pytest.mark.parametrize("kernel", ["gemm_nt_bf16_large_kernel", "gemm_nt_ring_kernel", "gemm_nt_bf16_wide_kernel"])
+def test_tiled_products_call_nothing(kernel, tmp_path):
+    """Their epilogue (gemm_tile.h) holds accumulators, bias, rows and pages in arrays: called and not inlined, it would
+    take them through scratch memory, and would lie where the test above does not look."""
+    path = os.path.join(library.in_tree_dir(), library.LIB_NAME)
+    if not os.path.isfile(path):
+        pytest.skip("the library is not built in the tree")
+    seen = 0
+    for image in kernel_code.code_objects(path, library.ARCH):
+        if kernel.encode() not in image:
+            continue
+        for name, taken in kernel_code.resources(image, tmp_path).items():
+            if kernel in name:
+                seen += 1
+                assert taken["vgpr"] > 0 and taken["scratch"] == 0, (name, taken)
+        for name, code in kernel_code.kernels(kernel_code.disassemble(image, library.ARCH, tmp_path)):
+            assert kernel not in name or not any(operation.startswith("s_swappc") for _, operation, _, _ in code), name
     assert seen
