@@ -140,7 +140,7 @@ __device__ __forceinline__ void attention_decode_block(
   const bool from_start = even && (form & AD_FROM_START);
   if (from_start) ask_entries(tables + (int64_t)t * table_width, wave * KEYS_PER_WAVE);
   Raw8<T> query;
-  query.template load<false>(q + (int64_t)t * q_stride + (int64_t)head * head_dim + lane_dim);
+  query.load_anywhere(q + (int64_t)t * q_stride + (int64_t)head * head_dim + lane_dim);
   const int pos = tok_pos[t];
   const int* table = tables + (int64_t)(direct ? t : tok_item[t]) * table_width;
   read_arguments(pos, k_pool, v_pool, kv_heads, page_size, num_pages, scale_log2, window, extra.sink, extra.gate,

@@ -98,6 +98,12 @@ struct Raw8<float> {
     a = *reinterpret_cast<const float4*>(p);
     b = *reinterpret_cast<const float4*>(p + 4);
   }
+  // from any element of a row on: the compiler is told so, and takes the same instructions (this hardware asks for no alignment)
+  __device__ inline void load_anywhere(const float* p) {
+    typedef __attribute__((__vector_size__(4 * sizeof(float)), aligned(4))) float any_t;
+    a = __builtin_bit_cast(float4, *reinterpret_cast<const any_t*>(p));
+    b = __builtin_bit_cast(float4, *reinterpret_cast<const any_t*>(p + 4));
+  }
   __device__ inline void widen(float* out) const {
     out[0] = a.x; out[1] = a.y; out[2] = a.z; out[3] = a.w;
     out[4] = b.x; out[5] = b.y; out[6] = b.z; out[7] = b.w;
@@ -131,6 +137,10 @@ struct Raw8<bf16_t> {
     } else {
       raw = *reinterpret_cast<const uint4*>(p);
     }
+  }
+  __device__ inline void load_anywhere(const bf16_t* p) {
+    typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)), aligned(2))) uint32_t any_t;
+    raw = __builtin_bit_cast(uint4, *reinterpret_cast<const any_t*>(p));
   }
   __device__ inline void widen(float* out) const {
     const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};

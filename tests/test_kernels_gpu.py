@@ -1236,6 +1236,47 @@ def test_attention_decode_pages_of_a_load(dtype, window, head_dim, page_size):
             torch.testing.assert_close(out[:rows].double(), expected, atol=atol, rtol=rtol)
 
 
+@pytest.mark.parametrize("head_dim,page_size", [(64, 16), (128, 12), (256, 16), (24, 8)])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_attention_decode_queries_from_any_element(dtype, head_dim, page_size):
+    """Query rows that begin at no multiple of 16 bytes, in every place that a row can have: the same bits as rows that
+    do (with the projection the heads' sums are added in any order: some units of the last place of a float)."""
+    from pagedserve_amd.ops import kernels
+
+    heads, contexts = 4, [1, 17, 130, 300, 33, 64, 9, 200]
+    k_pool, v_pool, tables = _paged_fixture(dtype, contexts, heads, head_dim, page_size, 541)
+    aligned = _rand((len(contexts), heads * head_dim), dtype, 542)
+    pos = torch.tensor([c - 1 for c in contexts], dtype=torch.int32, device="cuda")
+    scale = head_dim ** -0.5
+    w = _rand((200, heads * head_dim), dtype, 543, 1.0 / math.sqrt(heads * head_dim))
+    packed = kernels.pack_decode_weight(w) if kernels.decode_linear_supported(
+        dtype, len(contexts), head_dim, w if dtype == torch.bfloat16 else None) else None
+
+    def results(q):
+        for splits, waves in ((1, 4), (1, 16), (3, 4)):
+            partial = torch.full((len(contexts) * heads * splits * (head_dim + 2),), float("nan"), device="cuda")
+            out = torch.full((len(contexts), heads * head_dim), float("nan"), dtype=dtype, device="cuda")
+            kernels.attention_decode(q, k_pool, v_pool, out, None, pos, tables, heads, scale, splits, partial=partial, waves=waves)
+            yield out, 0.0
+            if splits > 1:
+                records = torch.full_like(partial, float("nan"))
+                kernels.attention_decode_partial(q, k_pool, v_pool, records, None, pos, tables, heads, scale, splits)
+                yield records, 0.0
+        if packed is not None:
+            for parts, waves in ((1, 4), (2, 8)):
+                residual = torch.zeros((len(contexts), 200), device="cuda")
+                kernels.attention_decode_linear(q, k_pool, v_pool, pos, tables, heads, scale, w, packed, None, residual, parts, waves)
+                yield residual, 1e-5
+
+    expected = list(results(aligned))
+    for first, behind in ((1, 0), (3, 4), (8, 1)):
+        rows = torch.full((len(contexts), first + heads * head_dim + behind), float("nan"), dtype=dtype, device="cuda")
+        q = rows[:, first:first + heads * head_dim]
+        q.copy_(aligned)
+        for (got, tolerance), (wanted, _) in zip(results(q), expected):
+            torch.testing.assert_close(got, wanted, atol=tolerance / 10, rtol=tolerance)
+
+
 def test_attention_decode_page_beyond_32_bits():
     """Float keys further into their page than 32 bits count bytes (one page of 2^23 keys of 192 values, 6 GiB a pool)."""
     from pagedserve_amd.ops import kernels
