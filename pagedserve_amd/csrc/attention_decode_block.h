@@ -132,9 +132,10 @@ __device__ __forceinline__ void attention_decode_block(
     held = row[lane < table_width ? lane : table_width - 1];
     if (table_width > 64) held1 = row[lane + 64 < table_width ? lane + 64 : table_width - 1];
   }
-  // (of a turn that begins at key `base` no lane beyond the first AD_UNROLL + 1 is asked)
+  // (of a turn that begins at key `base` no lane beyond the first AD_UNROLL + 1 is asked; a token of a negative position,
+  // which sees no key, has ranges that begin in front of the table)
   auto ask_entries = [&](const int* row, int base) {
-    const int entry = (base >> page_shift) + (lane < AD_UNROLL ? lane : AD_UNROLL);
+    const int entry = ((base > 0 ? base : 0) >> page_shift) + (lane < AD_UNROLL ? lane : AD_UNROLL);
     held = row[entry < table_width ? entry : table_width - 1];
   };
   const bool from_start = even && (form & AD_FROM_START);

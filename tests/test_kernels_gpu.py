@@ -1277,6 +1277,27 @@ def test_attention_decode_queries_from_any_element(dtype, head_dim, page_size):
             torch.testing.assert_close(got, wanted, atol=tolerance / 10, rtol=tolerance)
 
 
+@pytest.mark.parametrize("page_size", [16, 12])
+@pytest.mark.parametrize("window", [0, 20])
+def test_attention_decode_tokens_in_front_of_their_table(page_size, window):
+    """Tokens of negative positions see no key, and their key ranges begin in front of the block table: no entry is read
+    there, and the tokens beside them are as ever."""
+    from pagedserve_amd.ops import kernels
+
+    heads, head_dim, contexts = 3, 64, [300, 41, 1, 200, 130, 17]
+    k_pool, v_pool, tables = _paged_fixture(torch.bfloat16, contexts, heads, head_dim, page_size, 551)
+    q = _rand((len(contexts), heads * head_dim), torch.bfloat16, 552)
+    pos = torch.tensor([c - 1 for c in contexts], dtype=torch.int32, device="cuda")
+    for splits in (1, 2, 5):
+        partial = torch.full((len(contexts) * heads * splits * (head_dim + 2),), float("nan"), device="cuda")
+        expected, got = (torch.full_like(q, float("nan")) for _ in range(2))
+        kernels.attention_decode(q, k_pool, v_pool, expected, None, pos, tables, heads, 0.125, splits, partial=partial, window=window)
+        moved = pos.clone()
+        moved[0], moved[2], moved[4] = -300, -1, -70_000
+        kernels.attention_decode(q, k_pool, v_pool, got, None, moved, tables, heads, 0.125, splits, partial=partial, window=window)
+        assert torch.equal(got[1::2], expected[1::2]) and bool(torch.isfinite(expected).all())
+
+
 def test_attention_decode_page_beyond_32_bits():
     """Float keys further into their page than 32 bits count bytes (one page of 2^23 keys of 192 values, 6 GiB a pool)."""
     from pagedserve_amd.ops import kernels
