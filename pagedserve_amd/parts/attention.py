@@ -633,9 +633,13 @@ class Attention(Mixer):
         """(ranges per request, waves per block) of the decode kernel, by the number of (token,
         head) pairs per compute unit and the keys that a query sees (us in brackets: bfloat16, keys from memory):
 
-        * up to 128 keys (a turn of 4 waves, if that is more), and from three and a half pairs per unit:
-          one block of 4 waves per pair (8 requests of 8 heads of 128 over 20 keys: 3.7, in blocks of 16
-          waves 4.4, in two ranges 5.9);
+        * up to 128 keys (a turn of 4 waves, if that is more; of heads wider than 128 a turn, 32 keys), and from
+          three and a half pairs per unit: one block of 4 waves per pair (8 requests of 8 heads of 128 over 20 keys:
+          3.7, in blocks of 16 waves 4.4, in two ranges 5.9).  The keys are the context class's bound: of heads of 128,
+          whose turn is 64 keys, 4 waves are ahead within the first (8 of 8 over 16, 32 and 64 keys 3.3, 3.4 and 4.1,
+          in 16 waves 4.1, 4.1 and 4.5) and behind in the second (128 keys 5.9 and 5.4); of heads of 256 they are ahead by less
+          and behind by more (8 of 8 over 16, 32, 64 and 128 keys 3.5, 4.2, 6.1 and 9.4, in 16 waves 4.1, 4.8, 5.6 and
+          7.1; in float 12.5 and 10.2 over 128; 32 of 8 12.0 and 10.5);
         * from one and a half: the same at short contexts; from 2,048 keys on a handful of long
           blocks per unit would leave units idle towards the end, so the keys are cut into
           ranges until six blocks come to a unit;
@@ -663,7 +667,7 @@ class Attention(Mixer):
         pairs = count * self.heads
         units = kernels.compute_units()
         turn = kernels.decode_keys_per_block(self.head_dim, 4)      # keys that 4 waves take at once: 128 of 64 values
-        if visible <= max(128, turn) or 2 * pairs >= 7 * units:
+        if visible <= (max(128, turn) if self.head_dim <= 128 else turn) or 2 * pairs >= 7 * units:
             return 1, 4
         if pairs >= units + units // 2:
             # (32 requests of 12 heads at 8,192 keys: 126 instead of 172 us; none under 2,048 keys)

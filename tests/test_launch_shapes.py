@@ -77,6 +77,13 @@ def test_documented_cases(monkeypatch):
     assert _part(16)._merged_splits(8, 400) == 4 and _part(16)._merged_splits(12, 400) == 0
     assert _part(25)._merged_splits(2, 1024) == 8 and _part(25)._merged_splits(4, 1024) == 0
     assert _part(25)._merged_splits(4, 400) == 4
+    # one block of four waves up to 128 keys, of heads wider than 128 up to a turn, 32 keys
+    for head_dim, most in ((64, 128), (128, 128), (136, 32), (256, 32)):
+        for count in (1, 8, 21):
+            assert _part(12, head_dim)._splits(count, most) == (1, 4)
+            assert _part(12, head_dim)._splits(count, most + 1) == (1, 16)
+            assert _part(12, head_dim)._splits(count, 128) == (1, 4 if head_dim <= 128 else 16)
+        assert _part(12, head_dim)._splits(22, 128) == (1, 4)      # more than a pair per unit
     # a window bounds the keys that a query sees
     assert _part(12, window=256)._splits(32, 8192) == (1, 4)
 
