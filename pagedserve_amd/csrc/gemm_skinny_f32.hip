@@ -638,7 +638,8 @@ __global__ __launch_bounds__(256) void gemm_nt_few_f32_kernel(
 // - Up to 16 rows one dot product per wave and column (gemm_simple.hip) is ahead while the weights
 //   are few (8 x 768 x 768 4.2 against 4.7, 16 x 768 x 768 5.0 against 5.9, 16 x 64 x 256 3.1 against 5.3, 16 x
 //   1024 x 1024 5.6 against 6.8, 16 x 320 x 1280 4.7 against 5.6), and up to 8 level at very many columns; up to 4 rows
-//   always but where k is long and can be split (4 x 1024 x 4096 8.6 against 7.1).  Nine rows and more with the
+//   always but where k is long and can be split (4 x 1024 x 4096 8.6 against 7.1), or where rows are added to (see
+//   few_rows_take).  Nine rows and more with the
 //   plain epilogue come here all the same: with a key/value scatter behind it the other kernel needs a second launch
 //   (2.5), and a product is the same bits with and without (16 x 192 x 64 3.3 here, 2.8 there).
 // - Residual epilogue, k split: 200 x 768 x 3072 24.3 against 25.2 for the tiled kernel, 300 rows 33 against
@@ -648,13 +649,25 @@ __global__ __launch_bounds__(256) void gemm_nt_few_f32_kernel(
 //   the output head beyond 16 rows (32 x 50257 x 768 71 against 68).
 // - A k that is no multiple of 32, which the tiled kernel does not take, up to 768 rows: there it
 //   meets the one that does (gemm_mfma.hip).
-// (few_rows_take) Rows added to, four columns to a block.  In us with weights from memory, before and with it: up to
-// four rows where k is long, 1 x 768 x 3072 5.5 / 4.2, 4 rows 5.55 / 5.15, 1 x 1600 x 1600 6.3 / 4.8, 4 x 1024 x 4096 6.75 /
-// 6.5, but 4 x 1024 x 1024 3.15 / 3.2; five to eight where it is not, 5 x 512 x 512 3.15 / 2.75, 5 x 768 x 768 3.4 / 3.1,
-// 8 x 1024 x 1024 3.8 / 3.75, but 8 x 1600 x 1600 7.0 / 8.3 and 5 x 768 x 3072, whose k is split, 4.85 / 6.2.
+// (few_rows_take) Rows added to, four columns to a block.  In us with weights from memory, the kernels that would take
+// them otherwise and this one:
+// - Up to three rows of a k above 1024, where the other is a dot product per wave: 1 x 256 x 1280 3.4 / 3.2, 1 x 1024 x
+//   3072 6.05 / 4.75, 2 x 1600 x 1600 6.55 / 5.35, 2 x 2048 x 3584 10.9 / 9.75, 3 x 1600 x 1600 6.55 / 5.75, 3 x 1280 x 3584 9.4 / 9.75.
+// - Four rows where a block's rounds of loads are nearly full: 4 x 256 x 1280 3.4 / 3.9, 4 x 1600 x 1280 5.5 / 6.2, but 4 x 1024 x
+//   1600 4.55 / 4.4, 4 x 1600 x 1600 6.6 / 6.25, 4 x 2048 x 3072 9.8 / 9.35; 4 x 1280 x 3584 9.6 / 10.7.
+// - k = 4096, up to four rows: the other splits k, and its blocks are many however few the columns are.  Where the last round
+//   of this kernel's blocks leaves half of the units empty it is behind, of three or four rows a quarter: 1 x 512 x 4096 4.5 / 5.4, 4 rows 4.85 / 6.6, 2 x
+//   1280 x 4096 7.55 / 8.8, 4 x 1600 x 4096 9.8 / 11.05, but 1 x 1600 x 4096 9.25 / 8.7, 2 x 768 x 4096 6.55 / 6.35, 1 x 1024 x 4096 6.85 / 6.0, 4 rows 7.4 / 7.45,
+//   1 x 2048 x 4096 11.5 / 8.85, 4 rows 12.4 / 12.05.
+// - Five to eight rows of 512 to 1024: 5 x 512 x 512 3.2 / 2.75, 5 x 2048 x 1024 5.85 / 4.85, 8 x 1024 x 1024 4.05 / 4.0, 8 x 2048 x
+//   768 5.35 / 4.7, 8 x 256 x 1024 3.45 / 3.6; beyond, 8 x 1600 x 1600 7.0 / 8.3 and 5 x 768 x 3072, whose k is split, 4.85 / 6.2.
 static bool few_rows_take(int m, int n, int k, int epilogue) {
-  if (epilogue != PS_EPI_RESIDUAL || m > 8 || n > 8 * ps_compute_units()) return false;
-  return m <= 4 ? k > 1024 && k <= 4096 : k >= 512 && k <= 1024;
+  const int units = ps_compute_units();
+  if (epilogue != PS_EPI_RESIDUAL || m > 8 || n > 8 * units) return false;
+  if (m > 4) return k >= 512 && k <= 1024;
+  const int last_round = ((n + 3) / 4 - 1) % units + 1;
+  if (k == 4096) return m <= 2 ? 2 * last_round > units : 4 * last_round >= 3 * units;
+  return m < 4 ? k > 1024 && k < 4096 : k >= 1536 && k <= 3072;
 }
 
 bool ps_gemm_nt_f32_skinny_takes(const void* a, const void* w, int m, int n, int k, int lda,

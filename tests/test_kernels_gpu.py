@@ -286,7 +286,9 @@ def test_norm_product_of_few_float_rows_writes_its_pages(m, heads, kv_heads, k):
 
 
 @pytest.mark.parametrize("m,n,k", [(1, 1, 1028), (4, 1601, 1600), (3, 50, 2052), (4, 768, 3076), (2, 30, 4096), (4, 40, 4100),
-                                   (5, 33, 512), (8, 2048, 516), (7, 767, 768), (6, 9, 772), (8, 2049, 1024), (5, 40, 1028)])
+                                   (5, 33, 512), (8, 2048, 516), (7, 767, 768), (6, 9, 772), (8, 2049, 1024), (5, 40, 1028),
+                                   (3, 767, 3076), (3, 33, 4092), (4, 33, 1532), (4, 33, 1536), (4, 31, 3072), (4, 764, 4096),
+                                   (4, 765, 4096), (1, 1025, 4096)])
 def test_few_float_rows_added_to(m, n, k):
     """Sums of a block's four columns over 16 places of k, on both sides of where that kernel is taken: remainders of
     columns, pieces and rows; rows of C that are longer than n keep what lies behind it."""
