@@ -183,7 +183,11 @@ __global__ __launch_bounds__(256) void gemm_nt_ring_kernel(
   // stage, positions and items once it has landed (what they are read by lies further back in the arguments).  With
   // this, and tile numbers of the preloaded arguments: 64 x 4800 x 1600 9.6 to 8.7 us, 448 x 1600 x 1600 added to rows
   // 21.2 to 19.8 (mean of that and k = 6400), 544 x 1024 x 1024 8.2 to 7.4.
-  constexpr bool EARLY = WM * WN == 1;
+  // (Not for float rows added to in two stages: of their blocks registers and not LDS set how many share a unit, and the rows
+  // held through the loop take those of the fourth, 135 instead of 111.  us, early and late: 96 x 50257 x 768 141 / 132, 1500
+  // x 2304 x 768 61.8 / 60.0, 1024 x 4096 x 1024 88.6 / 85.4, 2048 x 1600 x 1600 113.3 / 113.6, twelve shapes 0.983.  Without
+  // rows it is four blocks instead of five, and as fast: the twelve plain 1.000 late, with GELU 1.009.)
+  constexpr bool EARLY = WM * WN == 1 && !(sizeof(T) == 4 && STAGES == 2 && EPI == PS_EPI_RESIDUAL);
   const int row_base = m0 + wave_m * WM * 32, col_base = n0 + wave_n * WN * 32;
   TileEnds<WM, WN, TOut, EPI> ends;
   TilePages<WM, WN> pages;

@@ -77,3 +77,22 @@ def test_tiled_products_call_nothing(kernel, tmp_path):
         for name, code in kernel_code.kernels(kernel_code.disassemble(image, library.ARCH, tmp_path)):
             assert kernel not in name or not any(operation.startswith("s_swappc") for _, operation, _, _ in code), name
     assert seen
+
+
+@pytest.mark.skipif(kernel_code.disassembler() is None, reason="no disassembler")
+def test_float_rows_added_to_share_a_unit(tmp_path):
+    """Tiles of 64 x 64 in two stages are taken where many blocks share a compute unit, four at least: 160 KB of LDS hold
+    five, the registers of a SIMD, 512 to a lane, four waves of up to 128."""
+    path = os.path.join(library.in_tree_dir(), library.LIB_NAME)
+    if not os.path.isfile(path):
+        pytest.skip("the library is not built in the tree")
+    kernel, form = "gemm_nt_ring_kernel", "If" + "".join(f"Li{i}E" for i in (1, 1, 2))    # float, 1 x 1, two stages
+    seen = 0
+    for image in kernel_code.code_objects(path, library.ARCH):
+        if kernel.encode() not in image:
+            continue
+        for name, taken in kernel_code.resources(image, tmp_path).items():
+            if kernel + form in name:
+                seen += 1
+                assert taken["vgpr"] <= 128 and taken["lds"] <= 160 * 1024 // 4, (name, taken)
+    assert seen == 5
