@@ -209,8 +209,8 @@ int ps_attention_merge_linear(const float* partial, int64_t partial_floats, cons
 // Decode attention and output projection in one launch, for up to 64 tokens of items 0 .. count - 1
 // (token t is item t) and heads of 64 or 128, bfloat16:  residual[t, :] += context of token t  W^T +
 // bias, W [n, heads * head_dim] in its packed copy.  One block per (token, head, part of the
-// columns): `parts` parts, each of which repeats the attention; `waves` (4, 8 or 16) to a block.  weights_first: heads of
-// 64 in blocks of 4 or 16 waves ask for W in front of the keys and not behind the first of them.
+// columns): `parts` parts, each of which repeats the attention; `waves` (4 or 8; 16 are run as 8) to a block.
+// weights_first: heads of 64 in blocks of 4 waves ask for W in front of the keys and not behind the first of them.
 int ps_attention_decode_linear(const void* q, int64_t q_stride, const void* k_pool,
                                const void* v_pool, const int* tok_pos, const int* tables,
                                int table_width, int count, int heads, int kv_heads, int head_dim,

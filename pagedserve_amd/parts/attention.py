@@ -382,7 +382,7 @@ class Attention(Mixer):
                                                 self.scale, self.out_weight, self.out_packed, self.out_bias, residual,
                                                 *shape, window=self.span, sink=sink, gate=gates,
                                                 softcap=self.score_cap, logistic=self.logistic,
-                                                weights_first=self._weights_first(*shape, ctx.max_kv_len))
+                                                weights_first=self._weights_first(shape[1], ctx.max_kv_len))
                 return
         merged_splits = 0
         if residual is not None and gates is None and singles == tokens and kernels.merge_linear_supported(
@@ -519,10 +519,10 @@ class Attention(Mixer):
           four or more (4 requests of 12 heads over 100 keys in 5 and 12 parts 3.9 and 5.6), else until two or three of them
           share a unit (16 over 60 keys in 1, 2 and 3 parts 5.9, 5.9 and 5.6).
         * Beyond, eight waves take up to 512 keys in one round of loads (8 of 12 heads over 250 and 540 keys in two parts
-          6.2 and 8.5, with four waves 6.5 and 10.0).  Parts until the blocks come to one per unit, but four from 1,024
-          keys on, which every part reads again (one request of 25 heads over 900 keys in 8, 4 and 3 parts 13.2, 10.9
-          and 10.7, two launches 12.6).  What asks for sixteen waves (longer contexts, blocks without parts, more
-          columns than eight waves hold) is run as eight as well, see attention_decode_linear.hip.
+          6.2 and 8.5, with four waves 6.5 and 10.0), and more of them in several: sixteen waves have too few registers
+          for keys and weights of a turn (see attention_decode_linear.hip).  Parts until the blocks come to one per
+          unit, but four from 1,024 keys on, which every part reads again (one request of 25 heads over 900 keys in 8, 4
+          and 3 parts 13.2, 10.9 and 10.7, two launches 12.6).
         * Between one and one and a half pairs per unit, up to 512 keys, 256 of wider heads: four waves, two parts (24
           requests of 12 heads over 270 keys 15.5 / 12.7; over 1,000 keys 23.6 / 24.5; of 12 heads of 128 over one
           key/value head within 128 and over 250 keys 14.0 / 11.4 and 14.2 / 15.9).
@@ -557,24 +557,22 @@ class Attention(Mixer):
         else:
             if keys > 1024 and (2 * pairs < units or keys >= 4096):
                 return None
-            parts = min(4 if visible > 512 else 8, units // pairs)
-            waves = 8 if parts > 1 and visible <= 512 and -(-tiles // parts) <= 32 else 16
+            parts, waves = min(4 if visible > 512 else 8, units // pairs), 8
         parts = min(parts, tiles)
         if self.width * self.head_dim * 2 > 131072 * parts:
             return None
         return parts, waves
 
-    def _weights_first(self, parts: int, waves: int, max_kv_len: int) -> bool:
+    def _weights_first(self, waves: int, max_kv_len: int) -> bool:
         """Whether the blocks of that kernel ask for their weights in front of the keys, not behind the first of them.  A
         wave's loads come back in the order of issue: in front, the weights hold back the block table and the
         first keys; behind, the keys of a wave's second turn.  (Keys and weights from memory, behind and in front,
         heads of 64, four waves: one request of 12 heads over 60 keys 3.55 / 3.85; where a wave takes several turns and
         the blocks come to more than one per unit, 24 over 250 and 400 keys 10.4 / 10.1 and 13.5 / 12.7.)  Blocks of
-        more waves, which hold more of a block's keys in one turn, ask for them behind whatever is said here."""
-        visible = self._visible(max_kv_len)
-        if waves == 16 and parts > 1:
-            return visible <= 512 or self.width > 768 * parts
-        return (waves == 4 and visible > 128) or (waves == 16 and visible > 512)
+        eight waves, which hold more of a block's keys in one turn, always ask for them behind, and so do heads of 128
+        (8 of them over 60 keys, four waves, with 1 and 16 requests 4.0 / 4.3 and 7.2 / 8.0; eight waves, 8 requests over 250
+        and 500 keys 7.7 / 8.2 and 11.3 / 11.0; 187 shapes 1.034 in front)."""
+        return self.head_dim == 64 and waves == 4 and self._visible(max_kv_len) > 128
 
     def _range_records(self, ctx):
         """Scratch for one record per (token, head, key range): always asked for at its largest

@@ -107,15 +107,13 @@ def test_attention_and_projection_in_one_launch(monkeypatch):
     for keys in (1, 20, 64, 127, 128):
         assert _part(12)._one_launch_decode(1, keys) == (12, 4) and _part(12)._one_launch_decode(16, keys) == (3, 4)
     assert _part(12, window=64)._one_launch_decode(8, 1024) == (7, 4)
-    assert _part(12)._one_launch_decode(8, 512) == (2, 8) and _part(12)._one_launch_decode(16, 1024) == (1, 16)
-    assert _part(12)._one_launch_decode(1, 1024) == (4, 16) and _part(12)._one_launch_decode(1, 2048) is None
+    assert _part(12)._one_launch_decode(8, 512) == (2, 8) and _part(12)._one_launch_decode(16, 1024) == (1, 8)
+    assert _part(12)._one_launch_decode(1, 1024) == (4, 8) and _part(12)._one_launch_decode(1, 2048) is None
     assert _part(12)._one_launch_decode(24, 512) == (2, 4) and _part(12)._one_launch_decode(24, 1024) is None
-    # the weights in front of the keys where a wave takes several turns over them
-    assert not _part(12)._weights_first(3, 4, 128) and _part(12)._weights_first(2, 4, 256)
-    assert not _part(12, window=64)._weights_first(7, 4, 1024) and not _part(12)._weights_first(2, 8, 512)
-    assert not _part(12)._weights_first(1, 16, 512) and _part(12)._weights_first(1, 16, 1024)
-    assert _part(25)._weights_first(3, 16, 256) and not _part(12)._weights_first(2, 16, 1024)
-    assert _part(25)._weights_first(2, 16, 1024) and not _part(25)._weights_first(4, 16, 1024)
+    # the weights in front of the keys where a wave of blocks of four takes several turns over them
+    assert not _part(12)._weights_first(4, 128) and _part(12)._weights_first(4, 129)
+    assert not _part(12, window=64)._weights_first(4, 1024) and not _part(6, 128)._weights_first(4, 256)
+    assert not _part(12)._weights_first(8, 512) and not _part(12)._weights_first(8, 1024)
     # wide models
     for keys in (128, 256, 512):
         for count in (5, 6, 7, 8):
@@ -123,7 +121,7 @@ def test_attention_and_projection_in_one_launch(monkeypatch):
         assert _part(25)._one_launch_decode(1, keys) and _part(25)._one_launch_decode(4, keys)
         assert _part(20)._one_launch_decode(6, keys) and _part(20)._one_launch_decode(7, keys) is None
         assert _part(16, 128)._one_launch_decode(3, keys) and _part(16, 128)._one_launch_decode(4, keys) is None
-    assert _part(25)._one_launch_decode(3, 256) == (3, 16)      # 34 tiles of columns in a part: two rounds of eight waves
+    assert _part(25)._one_launch_decode(3, 256) == (3, 8)       # 34 tiles of columns in a part: two rounds of eight waves
     assert _part(20)._one_launch_decode(3, 256) == (4, 8)
     assert _part(12)._one_launch_decode(24, 512) and _part(6, 128)._one_launch_decode(48, 128)
     assert _part(6, 128)._one_launch_decode(48, 256) is None
@@ -138,7 +136,7 @@ def test_attention_and_projection_in_one_launch(monkeypatch):
                         for keys in (1, 64, 128, 200, 256, 512, 1024, 2048, 8192):
                             shape = part._one_launch_decode(count, keys)
                             if shape is not None:
-                                assert 1 <= shape[0] <= -(-part.width // 16) and shape[1] in (4, 8, 16)
+                                assert 1 <= shape[0] <= -(-part.width // 16) and shape[1] in (4, 8)
 
 
 def test_query_tiles_of_the_prefill_attention(monkeypatch):
