@@ -661,6 +661,8 @@ __global__ __launch_bounds__(256) void gemm_nt_few_f32_kernel(
 //   1 x 2048 x 4096 11.5 / 8.85, 4 rows 12.4 / 12.05.
 // - Five to eight rows of 512 to 1024: 5 x 512 x 512 3.2 / 2.75, 5 x 2048 x 1024 5.85 / 4.85, 8 x 1024 x 1024 4.05 / 4.0, 8 x 2048 x
 //   768 5.35 / 4.7, 8 x 256 x 1024 3.45 / 3.6; beyond, 8 x 1600 x 1600 7.0 / 8.3 and 5 x 768 x 3072, whose k is split, 4.85 / 6.2.
+// - Up to 2,048 columns, two rounds of blocks, the line of eight rows (8 x 2304 x 768 4.9 / 5.6, 8 x 4096 x 1024 6.8 / 8.3).  Up to
+//   three rows would gain from it further on (1 x 2304 x 2048 8.7 / 6.3, 3 x 4096 x 2048 11.4 / 9.0, 4 x 6400 x 1600 12.85 / 15.1).
 static bool few_rows_take(int m, int n, int k, int epilogue) {
   const int units = ps_compute_units();
   if (epilogue != PS_EPI_RESIDUAL || m > 8 || n > 8 * units) return false;

@@ -78,8 +78,9 @@ __global__ __launch_bounds__(256) void gla_decay_pieces_kernel(
 // take four waves to 16 columns, which stage q, k and decays for all of them; blocks of one wave and 4
 // columns staged them four times as often, 57 KB of LDS each, two to a compute unit.  5 prompts of 400 tokens at
 // 12 heads of 64: 151 -> 44 us, 16 of 128: 45 -> 27, one of 2,000: 350 -> 193.  Chunks of 32 let one block into
-// a unit instead of three (16 prompts of 128 45 us, 5 of 400 49).  Steps of single tokens take one wave and 4
-// columns (16 with many blocks), in chunks of 8.
+// a unit instead of three (16 prompts of 128 45 us, 5 of 400 49).  Steps of up to eight
+// tokens an item take one wave: 16 columns in chunks of 8 where that gives blocks enough, else 4, in chunks of 8 or,
+// of single tokens, of one.
 #define GLA_LONG 16   // tokens of a chunk of a prompt
 
 template <int RPL, int COLS, int GLA_CHUNK, int WAVES, bool HEAD_DECAY>
@@ -416,8 +417,8 @@ extern "C" int ps_gla_scan(const float* proj, int64_t ld, int q_col, int k_col, 
   PS_REQUIRE(heads <= 65535 && (value_dim + 3) / 4 <= 65535, "ps_gla_scan: grid too large");
   if (items == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
-  // items of a few tokens at most (decode steps): chunks of 8, which cost less to stage, and blocks of one wave,
-  // narrow ones while wide ones would leave the chip's SIMDs (four to a compute unit) idle
+  // items of a few tokens at most (decode steps): chunks of 8 or fewer, which cost less to stage, and blocks of one
+  // wave, narrow ones while wide ones would leave the chip's SIMDs (four to a compute unit) idle
   const int64_t wide_blocks = (int64_t)items * heads * ((value_dim + 15) / 16);
   const bool narrow = wide_blocks < 2 * (int64_t)ps_compute_units();
   const bool brief = longest > 0 && longest <= 8;
