@@ -421,8 +421,8 @@ class Attention(Mixer):
         elif singles:
             # one-token items: keys of a request are cut into ranges so that few requests
             # still fill the chip
-            splits, waves = self._splits(singles, ctx.max_kv_len,
-                                         self.heads == self.kv_heads and self.dtype == torch.bfloat16)
+            splits, waves = self._splits(singles, ctx.max_kv_len, self.heads == self.kv_heads,
+                                         self.dtype == torch.bfloat16)
             partial = None
             if splits > 1:
                 partial = self._range_records(ctx)
@@ -627,9 +627,11 @@ class Attention(Mixer):
         room = 1 + 6 * units // (count * self.heads)
         return max(1, min(wanted, most, room, 64))
 
-    def _splits(self, count: int, max_kv_len: int, own_keys: bool = False):
+    def _splits(self, count: int, max_kv_len: int, own_keys: bool = False, bfloat16: bool = False):
         """(ranges per request, waves per block) of the decode kernel, by the number of (token,
-        head) pairs per compute unit and the keys that a query sees (us in brackets: bfloat16, keys from memory):
+        head) pairs per compute unit, the keys that a query sees and whether every head has keys of its own (``own_keys``;
+        heads that share keys find them in the cache); us in brackets: bfloat16, keys from memory.  A turn is what 4 waves take
+        at once, 128 keys of 64 values:
 
         * up to 128 keys (a turn of 4 waves, if that is more; of heads wider than 128 a turn, 32 keys), and from
           three and a half pairs per unit: one block of 4 waves per pair (8 requests of 8 heads of 128 over 20 keys:
@@ -641,22 +643,29 @@ class Attention(Mixer):
         * from one and a half: the same at short contexts; from 2,048 keys on a handful of long
           blocks per unit would leave units idle towards the end, so the keys are cut into
           ranges until six blocks come to a unit;
-        * between one and one and a half: up to 512 keys the same (24 requests of 12 heads at 400
-          keys 10.6, in two ranges 12.2); beyond, blocks of 16 waves would come two to some units and
+        * between one and one and a half: up to 512 keys and eight turns the same (24 requests of 12 heads at 400
+          keys 10.6, in two ranges 12.2; 20 of 16 heads of 256 over 4 at 512 31.6 and 27.6); beyond, blocks of 16 waves would come two to some units and
           one to the others, and one block of 4 waves is long (24 over 1,500 and 2,000 keys 27.0 and 33.6):
           ranges of 4-wave blocks, four blocks to a unit (24.6 and 31.3 with the launch that merges them),
           six over thousands of keys;
         * between half a pair and one: one block of 16 waves takes a whole request's keys and no
           second launch is needed; from 16 turns of four waves on (2,048 keys of 64 values) that is behind
           ranges of 4-wave blocks, four blocks to a unit, where every head has bfloat16 keys of its own
-          (``own_keys``; 16 over 2,000 keys 25.3 and 22.6, 12 over 4,000 38.6 and 31.0; heads that share keys find them in the cache: 20 of 12 heads over 4
-          18.1 and 22.0; in float 39.6 and 42.3, so there from 4,096 on, just under a pair per unit, as before);
-        * fewer pairs: up to 1,024 keys that a block of 16 waves takes in one turn that block (one request of 12
+          (16 over 2,000 keys 25.3 and 22.6, 12 over 4,000 38.6 and 31.0; 20 of 12 heads over 4
+          18.1 and 22.0; in float 39.6 and 42.3, so there from 4,096 on, just under a pair per unit);
+        * fewer pairs: up to four turns within 1,024 keys one block of 16 waves (one request of 12
           heads over 200 and 400 keys 4.3 and 5.8, in ranges 6.0 and 6.5), beyond ranges of a turn of 4-wave blocks or
-          more until three blocks come to a unit, up to 16 ranges, 32 over 64 turns (8 of 12 heads over 800 and 2,000
-          keys 9.4 and 14.5, in one and two blocks of 16 waves 10.5 and 16.7; one over 4,000 keys in 16 and 32 ranges
-          10.1 and 10.5).  That holds to 8,192 keys and, from a quarter of a pair per unit on, to 2,048; beyond,
-          ranges until four blocks come to a unit, or two or three blocks of 16 waves.
+          more until three blocks come to a unit, up to 16 ranges (8 of 12 heads over 2,000 keys 14.5, in two blocks of 16
+          waves 16.7), 32 over 64 turns or, up to a sixteenth of a pair per unit, with keys of their own (one of 16 over
+          4,096 keys in 16 and 32 ranges 8.9 and 8.4), 64 over 128 turns of up to 8 pairs (8
+          heads of 256 over 8,192 keys in 32 and 64 ranges 23.6 and 18.4).  A rest of a turn is a range of its own (8 heads over
+          800 keys in 6 and 7 ranges 6.3 and 5.9).  That holds to 8,192 keys and, from a quarter of a pair per unit on, to
+          2,048; beyond, ranges until four blocks come to a unit, or two or three blocks of 16 waves;
+        * from that quarter on, up to 2,048 keys, one block of 16 waves also up to seven turns (6 of 12 heads over 800 keys
+          8.2, in six and seven ranges 9.0 and 8.2), or eight where some ranges would be of two (8 of 16 in float over 800
+          keys 14.9, in six ranges 16.1; but 8 of 12, whose eight ranges are of one, over 1,024 keys 10.4 and 9.5); heads that share
+          keys blocks of 16 waves of eight turns or more (6 of 16 over 4 at 1,024 and 1,500 keys 8.6 and 11.0, in eight
+          ranges 10.8 and 13.6).
 
         Never more ranges than the keys of the longest request can feed, and never more than
         six blocks per unit beside one per pair (the scratch for the records is sized for
@@ -664,7 +673,8 @@ class Attention(Mixer):
         visible = self._visible(max_kv_len)
         pairs = count * self.heads
         units = kernels.compute_units()
-        turn = kernels.decode_keys_per_block(self.head_dim, 4)      # keys that 4 waves take at once: 128 of 64 values
+        turn = kernels.decode_keys_per_block(self.head_dim, 4)
+        most = max(1, -(-visible // turn))
         if visible <= (max(128, turn) if self.head_dim <= 128 else turn) or 2 * pairs >= 7 * units:
             return 1, 4
         if pairs >= units + units // 2:
@@ -673,22 +683,31 @@ class Attention(Mixer):
         if pairs > units:
             # (four blocks to a unit, six over thousands of keys)
             blocks = (6 if visible >= 4096 else 4) * units
-            return (max(1, min(-(-blocks // pairs), visible // 256)) if visible > 512 else 1), 4
+            return (max(1, min(-(-blocks // pairs), visible // 256)) if visible > 512 or most > 8 else 1), 4
         if 4 * pairs >= 3 * units and visible >= 4096:
             # nearly a pair per unit over thousands of keys: six blocks of 4 waves to a unit are
             # ahead of one block of 16 waves per pair (17 requests of 12 heads at 4,096 keys:
             # 41.4 against 44.2 us, at 16,384 keys 141 against 155)
             return min(-(-6 * units // pairs), 64), 4
         if 2 * pairs > units:
-            return (4 * units // pairs, 4) if visible >= 16 * turn and own_keys else (1, 16)
+            return (4 * units // pairs, 4) if visible >= 16 * turn and own_keys and bfloat16 else (1, 16)
         if visible <= (2048 if 4 * pairs >= units else 8192):
             if visible <= min(4 * turn, 1024):
                 return 1, 16
-            return max(1, min(3 * units // pairs, visible // turn, 32 if visible >= 64 * turn else 16)), 4
+            ranges = 3 * units // pairs
+            if 4 * pairs >= units:
+                if not own_keys:
+                    return max(1, min(units // pairs, visible // (8 * turn))), 16
+                if most <= 7 or ranges < most <= 8:
+                    return 1, 16
+            if visible >= 128 * turn and 64 * pairs <= 2 * units:
+                limit = 64
+            else:
+                limit = 32 if visible >= 64 * turn or (own_keys and 16 * pairs <= units) else 16
+            return max(1, min(ranges, most, limit)), 4
         if pairs >= units // 4:
             # contexts of many thousand keys: two or three such blocks per request, as
             # long as every block still has a compute unit of its own
             return max(1, min(units // pairs, visible // 1024)), 16
-        most = max(1, -(-visible // turn))
         wanted = max(1, -(-4 * units // pairs))
         return min(most, wanted, 64), 4

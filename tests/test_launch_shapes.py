@@ -23,10 +23,11 @@ def test_ranges_fit_the_scratch_and_the_kernel(monkeypatch, units):
                 part = _part(heads, head_dim, window)
                 for count in list(range(1, 70)) + [100, 128, 256, 300]:
                     for context in (1, 17, 100, 256, 300, 1000, 1024, 2048, 4096, 8192, 16384, 1 << 20):
-                        splits, waves = part._splits(count, context)
-                        assert 1 <= splits <= 64 and waves in (4, 16)
-                        # what Attention._range_records holds: six blocks per unit beside one per pair
-                        assert count * heads * splits <= 6 * units + count * heads
+                        for own_keys, bfloat16 in ((False, False), (True, False), (False, True), (True, True)):
+                            splits, waves = part._splits(count, context, own_keys, bfloat16)
+                            assert 1 <= splits <= 64 and waves in (4, 16)
+                            # what Attention._range_records holds: six blocks per unit beside one per pair
+                            assert count * heads * splits <= 6 * units + count * heads
                         merged = part._merged_splits(count, context)
                         assert 0 <= merged <= 64
                         assert count * heads * merged <= 6 * units + count * heads
@@ -86,6 +87,23 @@ def test_documented_cases(monkeypatch):
         assert _part(12, head_dim)._splits(22, 128) == (1, 4)      # more than a pair per unit
     # a window bounds the keys that a query sees
     assert _part(12, window=256)._splits(32, 8192) == (1, 4)
+    # few pairs, beyond four turns of keys: ranges of a turn, its rest one of its own
+    assert _part(8)._splits(1, 512) == (1, 16)
+    assert _part(8)._splits(1, 800) == (7, 4) and _part(8)._splits(1, 1024) == (8, 4) and _part(8)._splits(1, 1025) == (9, 4)
+    assert _part(16)._splits(1, 4096) == (16, 4) and _part(16)._splits(1, 4096, True) == (32, 4)
+    assert _part(16)._splits(2, 4096, True) == (16, 4) and _part(16)._splits(2, 8192, True) == (24, 4)
+    assert _part(8, 256)._splits(1, 4096) == (64, 4) and _part(9, 256)._splits(1, 4096) == (32, 4)
+    # from a quarter of a pair per unit to half of one: one block of 16 waves a little longer, and where keys are shared
+    assert _part(12)._splits(6, 896, True) == (1, 16) and _part(12)._splits(6, 897, True) == (8, 4)
+    assert _part(16)._splits(8, 1024, True) == (1, 16) and _part(16)._splits(8, 1025, True) == (6, 4)
+    assert _part(16)._splits(6, 1024) == (1, 16) and _part(16)._splits(6, 2047) == (1, 16)
+    assert _part(16)._splits(6, 2048) == (2, 16) and _part(16, 256)._splits(4, 768) == (3, 16)
+    # between half a pair and one: ranges over long contexts of bfloat16 keys that are not shared
+    assert _part(12)._splits(16, 2048, True, True) == (5, 4) and _part(12)._splits(16, 2048, True) == (1, 16)
+    assert _part(12)._splits(16, 2048, False, True) == (1, 16)
+    # more than one: from eight turns on
+    assert _part(16, 256)._splits(20, 256) == (1, 4) and _part(16, 256)._splits(20, 512) == (2, 4)
+    assert _part(16)._splits(20, 512) == (1, 4) and _part(16)._splits(20, 513) == (2, 4)
 
 
 def test_tiles_of_short_portions_in_32_bit(monkeypatch):
