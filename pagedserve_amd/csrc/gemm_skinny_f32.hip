@@ -197,14 +197,16 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_nt_skinny_f32_kernel(
       }
   };
   // wave `wave` takes the steps wave, wave + WAVES, ... of the block's range; UNROLL of them are
-  // asked for together, the first ones in front of what the epilogue needs.  (A wave without a step asks for the range's
-  // first values and multiplies by zeros.)
+  // asked for together, the first ones in front of what the epilogue needs.  (A wave without a step, of a short k, asks
+  // for nothing and leaves the matrix cores to the others: 32 x 192 x 64 7.05 us when it multiplied zeros, now 3.8, 16 x
+  // 320 x 96 4.95 and 3.5.)
   FloatEnds<EPI, MB, NT, WAVES> ends;
   int k0 = k_begin + wave * SF_STEP;
-  load(k0);
+  const bool works = k0 < k_end;
+  if (works) load(k0);
   if (EPI == PS_EPI_NONE && scatter.k_pool != nullptr) read_scatter(scatter);
   ends.ask(bias, c, m, n, ldc, n0, row0, split, k_splits, scatter);
-  multiply(k0);
+  if (works) multiply(k0);
   for (k0 += WAVES * UNROLL * SF_STEP; k0 < k_end; k0 += WAVES * UNROLL * SF_STEP) {
     load(k0);
     multiply(k0);

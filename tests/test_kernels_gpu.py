@@ -285,6 +285,28 @@ def test_norm_product_of_few_float_rows_writes_its_pages(m, heads, kv_heads, k):
     assert torch.equal(k_pool, pools[0]) and torch.equal(v_pool, pools[1])
 
 
+@pytest.mark.parametrize("m,n,k", [(9, 20, 4), (16, 192, 64), (17, 33, 32), (32, 320, 96), (48, 50, 100), (64, 192, 36), (33, 47, 260),
+                                   (1, 3100, 252), (4, 4801, 1600), (8, 3100, 260), (16, 3073, 1284), (3, 1540, 1028)])
+@pytest.mark.parametrize("epilogue", ["none", "gelu_tanh", "residual"])
+def test_float_rows_of_any_k(m, n, k, epilogue):
+    """Fewer steps of k than a block has waves, and a k that ends inside a lane's round of loads: one to four columns to a
+    wave, one and two sets of eight rows."""
+    from pagedserve_amd.ops import kernels
+
+    x = _rand((m, k), torch.float32, 561)
+    w = _rand((n, k), torch.float32, 562, 1.0 / math.sqrt(k))
+    bias, start = _rand((n,), torch.float32, 563), _rand((m, n), torch.float32, 564)
+    out = start.clone()
+    kernels.linear(x, w, bias, out, epilogue=epilogue)
+    expected = x.double() @ w.double().t() + bias.double()
+    if epilogue == "gelu_tanh":
+        expected = torch.nn.functional.gelu(expected, approximate="tanh")
+    elif epilogue == "residual":
+        expected += start.double()
+    # sums of size 1 of up to 1,600 products in 32 bits: some units of 6e-8
+    torch.testing.assert_close(out.double(), expected, atol=2e-6, rtol=2e-6)
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 1, 1028), (4, 1601, 1600), (3, 50, 2052), (4, 768, 3076), (2, 30, 4096), (4, 40, 4100),
                                    (5, 33, 512), (8, 2048, 516), (7, 767, 768), (6, 9, 772), (8, 2049, 1024), (5, 40, 1028),
                                    (3, 767, 3076), (3, 33, 4092), (4, 33, 1532), (4, 33, 1536), (4, 31, 3072), (4, 764, 4096),
