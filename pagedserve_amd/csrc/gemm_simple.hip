@@ -115,8 +115,8 @@ __global__ __launch_bounds__(256) void gemm_nt_f32_rows_kernel(
   const float* a_row[MR];
 #pragma unroll
   for (int r = 0; r < MR; ++r) a_row[r] = a + (int64_t)(r < m ? r : m - 1) * lda;
-  // the output (row `own_row`, column col0 + own_j) that this lane finishes; its bias and residual value travel with
-  // the first operands
+  // the output (row `own_row`, column col0 + own_j) that this lane finishes; its bias and residual value travel in front
+  // of the first operands
   static_assert(COLS * MR <= 64, "one output per lane");
   const int own_j = lane / MR, own_row = lane - own_j * MR;
   const bool owns = own_j < COLS && own_row < m && col0 + own_j < n;
@@ -127,37 +127,52 @@ __global__ __launch_bounds__(256) void gemm_nt_f32_rows_kernel(
   for (int j = 0; j < COLS; ++j)
 #pragma unroll
     for (int r = 0; r < MR; ++r) acc[j][r] = 0.f;
-  for (int k0 = lane * 4; k0 - lane * 4 < k; k0 += 256 * AHEAD) {
-    // (unconditional, from a place that exists: nothing waits for a branch; a row's values of the next step are
-    // asked for in front of this step's sums)
-    float4 wv[AHEAD][COLS], av[2][MR];
-    auto place = [&](int u) { return k0 + 256 * u < k ? k0 + 256 * u : 0; };
-    auto load_rows = [&](int u) {
+  if (bias != nullptr) own_bias = bias[owns ? col0 + own_j : col0];
+  if (EPI == PS_EPI_RESIDUAL) before = *dst;
+  // Lanes beyond k ask for nothing.  (Asking for a place that exists in their stead, so that nothing stands behind a branch,
+  // takes longer, us: 1 x 4800 x 1600 12.3, so 10.2, 4 x 6400 x 1600 12.8 and 10.7, 1 x 512 x 256 2.5 and 2.4; but eight rows of
+  // four columns to a wave have loads enough on their way only like that: the head, 8 x 50257 x 768, 35.8 and 47.4.)
+  if constexpr (MR == 8 && COLS == 4) {
+    for (int k0 = lane * 4; k0 - lane * 4 < k; k0 += 256) {
+      const int at = k0 < k ? k0 : 0;
+      float4 wv[COLS], av[MR];
 #pragma unroll
-      for (int r = 0; r < MR; ++r) av[u & 1][r] = *reinterpret_cast<const float4*>(a_row[r] + place(u));
-    };
+      for (int j = 0; j < COLS; ++j) wv[j] = *reinterpret_cast<const float4*>(w_row[j] + at);
 #pragma unroll
-    for (int u = 0; u < AHEAD; ++u)
+      for (int r = 0; r < MR; ++r) av[r] = *reinterpret_cast<const float4*>(a_row[r] + at);
+      if (k0 < k) {
 #pragma unroll
-      for (int j = 0; j < COLS; ++j) wv[u][j] = *reinterpret_cast<const float4*>(w_row[j] + place(u));
-    load_rows(0);
-    if (k0 < 256) {
-      if (bias != nullptr) own_bias = bias[owns ? col0 + own_j : col0];
-      if (EPI == PS_EPI_RESIDUAL) before = *dst;
-    }
-#pragma unroll
-    for (int u = 0; u < AHEAD; ++u) {
-      if (u + 1 < AHEAD) load_rows(u + 1);
-      if (k0 + 256 * u < k) {
-#pragma unroll
-        for (int r = 0; r < MR; ++r) {
-          const float4 x = av[u & 1][r];
+        for (int r = 0; r < MR; ++r)
 #pragma unroll
           for (int j = 0; j < COLS; ++j) {
-            acc[j][r] = fmaf(x.x, wv[u][j].x, acc[j][r]);
-            acc[j][r] = fmaf(x.y, wv[u][j].y, acc[j][r]);
-            acc[j][r] = fmaf(x.z, wv[u][j].z, acc[j][r]);
-            acc[j][r] = fmaf(x.w, wv[u][j].w, acc[j][r]);
+            acc[j][r] = fmaf(av[r].x, wv[j].x, acc[j][r]);
+            acc[j][r] = fmaf(av[r].y, wv[j].y, acc[j][r]);
+            acc[j][r] = fmaf(av[r].z, wv[j].z, acc[j][r]);
+            acc[j][r] = fmaf(av[r].w, wv[j].w, acc[j][r]);
+          }
+      }
+    }
+  } else {
+    for (int k0 = lane * 4; k0 < k; k0 += 256 * AHEAD) {
+      float4 wv[AHEAD][COLS];
+#pragma unroll
+      for (int u = 0; u < AHEAD; ++u)
+#pragma unroll
+        for (int j = 0; j < COLS; ++j)
+          wv[u][j] = k0 + 256 * u < k ? *reinterpret_cast<const float4*>(w_row[j] + k0 + 256 * u)
+                                      : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+      for (int u = 0; u < AHEAD; ++u) {
+        if (k0 + 256 * u >= k) break;
+#pragma unroll
+        for (int r = 0; r < MR; ++r) {
+          const float4 av = *reinterpret_cast<const float4*>(a_row[r] + k0 + 256 * u);
+#pragma unroll
+          for (int j = 0; j < COLS; ++j) {
+            acc[j][r] = fmaf(av.x, wv[u][j].x, acc[j][r]);
+            acc[j][r] = fmaf(av.y, wv[u][j].y, acc[j][r]);
+            acc[j][r] = fmaf(av.z, wv[u][j].z, acc[j][r]);
+            acc[j][r] = fmaf(av.w, wv[u][j].w, acc[j][r]);
           }
         }
       }
