@@ -323,8 +323,12 @@ __device__ inline void skinny_top_choice(float (*partial)[SK_WAVES][MB][4][64], 
 #define SK_W_PACKED 4   // w is the packed copy
 #define SK_K_SPLIT 8    // k is split over blocks: C is added to with atomics
 #define SK_ROW_BITS 16  // in front of these flags stands the number of rows
+// Waves to a SIMD that the registers must leave room for: two for rows added to by two tiles of columns, whose blocks share a
+// unit (a round of 5 steps of 64 rows takes too many for that).  48 x 6400 x 1600 added to rows 16.8 us with 276 registers, 12.8
+// with 248, 65 x 1600 x 6400 15.9 and 12.8, 96 rows 17.7 and 14.5.
+#define SK_SHARED(EPI, MB, NT, UNROLL) (NT == 2 && EPI == PS_EPI_RESIDUAL && MB * UNROLL <= 16 ? 2 : 1)
 template <typename TOut, int EPI, int MB, int NT, int UNROLL>
-__global__ __launch_bounds__(64 * SK_WAVES) void gemm_nt_skinny_kernel(
+__global__ __launch_bounds__(64 * SK_WAVES, SK_SHARED(EPI, MB, NT, UNROLL)) void gemm_nt_skinny_kernel(
     const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, const int* __restrict__ tok_pos,
     const int* __restrict__ tok_item, int rows_and_flags, int n, int k, int lda, int k_chunk,
     const float* __restrict__ bias, TOut* __restrict__ c, int ldc, KvScatter scatter, TopChoice top) {
@@ -364,9 +368,10 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_nt_skinny_kernel(
 
   const uint4 zero = {0u, 0u, 0u, 0u};
   uint4 wf[UNROLL][NT][2], xf[UNROLL][MB][2];
-  // the steps k0, k0 + 4 x 64, ... of a wave
+  // the steps k0, k0 + 4 x 64, ... of a wave; `whole`: all of them are there
+  auto whole = [&](int k0) { return w_packed && k0 + (UNROLL - 1) * SK_WAVES * 64 + 64 <= k_end; };
   auto load = [&](int k0) {
-    if (w_packed && k0 + (UNROLL - 1) * SK_WAVES * 64 + 64 <= k_end) {
+    if (whole(k0)) {
       // packed copy: the 16 x 64 tile of step s lies in the order in which the lanes hold it,
       // first the halves of the first product, then those of the second (1 KB each)
       const int tiles = (n + 15) / 16;
@@ -410,8 +415,8 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_nt_skinny_kernel(
       const int kk = ku + group * 16;
       const bool first = kk < k_end;
       const bool second = kk + 8 < k_end;
-      // unconditional loads from a clamped offset, zeroed afterwards: loads under a branch
-      // would not be issued together
+      // unconditional loads from a clamped offset, zeroed where they are used: loads under a branch
+      // would not be issued together, and zeroed here they would be waited for in front of what the ends need
       const int o0 = first ? ku : k_begin - group * 16;
       const int o1 = second ? ku + 8 : k_begin - group * 16;
       // (packed: k is a multiple of 64, so a step is whole or absent)
@@ -429,13 +434,20 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_nt_skinny_kernel(
         xf[u][b][0] = *reinterpret_cast<const uint4*>(a_ptr[b] + q0);
         xf[u][b][1] = *reinterpret_cast<const uint4*>(a_ptr[b] + q1);
       }
-      if (!first) {
+    }
+  };
+  // of a step that ends inside it
+  auto trim = [&](int k0) {
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      const int kk = k0 + u * SK_WAVES * 64 + group * 16;
+      if (kk >= k_end) {
 #pragma unroll
         for (int j = 0; j < NT; ++j) wf[u][j][0] = zero;
 #pragma unroll
         for (int b = 0; b < MB; ++b) xf[u][b][0] = zero;
       }
-      if (!second) {
+      if (kk + 8 >= k_end) {
 #pragma unroll
         for (int j = 0; j < NT; ++j) wf[u][j][1] = zero;
 #pragma unroll
@@ -448,12 +460,18 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_nt_skinny_kernel(
   if (k0 < k_end) load(k0);
   read_arguments(bias, c, ldc);
   if (EPI == PS_EPI_NONE && tok_pos != nullptr) read_scatter(scatter);
+  // (two tiles of columns, whose k is split, need no more than the bias, and its place in registers: see SK_SHARED)
+  constexpr bool LATE = NT == 2 && EPI == PS_EPI_RESIDUAL;
+  auto ask_ends = [&] {
 #pragma unroll
-  for (int j = 0; j < NT; ++j) {
-    ends[j].ask(bias, c, m, n, ldc, n0 + j * 16, row0, split, k_splits, scatter, tok_pos, layouts & SK_C_PACKED);
-    ends[j].ask_pages(scatter, tok_pos, n0 + j * 16);
-  }
+    for (int j = 0; j < NT; ++j) {
+      ends[j].ask(bias, c, m, n, ldc, n0 + j * 16, row0, split, k_splits, scatter, tok_pos, layouts & SK_C_PACKED);
+      ends[j].ask_pages(scatter, tok_pos, n0 + j * 16);
+    }
+  };
+  if constexpr (!LATE) ask_ends();
   while (k0 < k_end) {
+    if (!whole(k0)) trim(k0);
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u)
 #pragma unroll
@@ -468,6 +486,7 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_nt_skinny_kernel(
     k0 += SK_WAVES * UNROLL * 64;
     if (k0 < k_end) load(k0);
   }
+  if constexpr (LATE) ask_ends();
 
 #pragma unroll
   for (int j = 0; j < NT; ++j)

@@ -96,3 +96,24 @@ def test_float_rows_added_to_share_a_unit(tmp_path):
                 seen += 1
                 assert taken["vgpr"] <= 128 and taken["lds"] <= 160 * 1024 // 4, (name, taken)
     assert seen == 5
+
+
+@pytest.mark.skipif(kernel_code.disassembler() is None, reason="no disassembler")
+def test_rows_added_to_by_two_tiles_of_columns_share_a_unit(tmp_path):
+    """The skinny bfloat16 product of rows added to, two tiles of columns to a block: two of its blocks share a compute unit,
+    256 registers to a lane each, but where 5 steps of 64 rows travel at once."""
+    path = os.path.join(library.in_tree_dir(), library.LIB_NAME)
+    if not os.path.isfile(path):
+        pytest.skip("the library is not built in the tree")
+    kernel = "gemm_nt_skinny_kernel"
+    forms = {f"Li3ELi{rows}ELi2ELi{steps}E": (rows, steps) for rows in (2, 3, 4) for steps in (2, 3, 4, 5)}
+    seen = set()
+    for image in kernel_code.code_objects(path, library.ARCH):
+        if kernel.encode() not in image:
+            continue
+        for name, taken in kernel_code.resources(image, tmp_path).items():
+            for form in forms if kernel in name else ():
+                if form in name:
+                    seen.add(form)
+                    assert taken["scratch"] == 0 and (taken["vgpr"] <= 256 or forms[form] == (4, 5)), (name, taken)
+    assert len(seen) == len(forms)
