@@ -69,7 +69,8 @@ struct BlPiece<float> {
 // WT waves along the tokens x WC along the columns (WT * WC = 4), CT tiles of 16 columns a wave.  STEPS of 32 values of
 // k are asked for at once, from a place that exists where a lane's lies beyond k, with bias and gate behind them: few
 // tokens wait for trips to memory and for nothing else, and this makes them one (8 tokens, 12 blocks of 64 x 128 in
-// bfloat16 5.9 -> 4.2 us in a decode step, of 128 x 64 in float 3.5 -> 3.05).
+// bfloat16 5.9 -> 4.2 us in a decode step, of 128 x 64 in float 3.5 -> 3.05).  Six where that is all of k: 8 tokens, 12 blocks
+// of 64 x 192 3.16 us, in rounds of four 3.58, of one 3.4; beyond, four.
 template <typename TX, typename TO, int WT, int WC, int CT, int STEPS>
 __global__ __launch_bounds__(256) void block_linear_mfma_kernel(
     const TX* __restrict__ x, int64_t x_ld, const bf16_t* __restrict__ w, int x_step, int n, int k, int tokens,
@@ -248,6 +249,7 @@ extern "C" int ps_block_linear(const void* x, int x_dtype, int64_t x_ld, int x_s
   do {                                                         \
     if (!few) PS_LAUNCH_BLM_AS(TX, TO, 4, 1, 4, 1);            \
     else if (k <= 64) PS_LAUNCH_BLM_AS(TX, TO, 1, 4, 1, 2);    \
+    else if (k > 128 && k <= 192) PS_LAUNCH_BLM_AS(TX, TO, 1, 4, 1, 6);  \
     else PS_LAUNCH_BLM_AS(TX, TO, 1, 4, 1, 4);                 \
   } while (0)
     if (x_dtype == PS_F32) {

@@ -86,6 +86,35 @@ def test_block_diagonal_product(blocks, n, k, x_step, out_step, tokens):
             assert float(out[tokens:].abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("n,k", [(4, 8), (20, 40), (68, 64), (64, 72), (16, 128), (200, 136), (64, 192), (12, 200), (36, 264)])
+@pytest.mark.parametrize("tokens", [1, 5, 16, 17, 70])
+@pytest.mark.parametrize("x_dtype", [torch.float32, torch.bfloat16])
+def test_block_diagonal_product_on_the_matrix_cores(n, k, tokens, x_dtype):
+    """Aligned rows of whole pieces against bfloat16 weights: a k of one round of loads, of a piece more, and ends of
+    columns and tokens inside their tiles; NaN behind what belongs to a block."""
+    kernels = _kernels()
+    g = torch.Generator().manual_seed(n * 1000 + k)
+    blocks, x_step, out_step = 3, k + 8, n + 4
+    x = torch.randn((tokens, blocks, x_step), generator=g)
+    x[:, :, k:] = float("nan")
+    x = x.to(x_dtype)
+    w = (torch.randn((blocks, n, k), generator=g) / k ** 0.5).to(torch.bfloat16)
+    bias, gate = torch.randn(blocks * n, generator=g), torch.randn((tokens, blocks * n), generator=g) * 2
+    # (float rows are split into two bfloat16 parts, which leaves 2^-17 of them)
+    plain_product = torch.stack([x[:, b, :k].double() @ w[b].double().T for b in range(blocks)], 1)
+    for out_dtype in (torch.float32, torch.bfloat16):
+        for with_bias, with_gate in ((False, False), (True, True)):
+            expected = plain_product
+            if with_bias:
+                expected = (expected + bias.view(blocks, n).double()) * torch.sigmoid(gate.view(tokens, blocks, n).double())
+            out = torch.full((tokens + 2, blocks, out_step), 3.0, dtype=out_dtype, device="cuda")
+            kernels.block_linear(x.view(tokens, -1).cuda(), x_step, w.cuda(), bias.cuda() if with_bias else None,
+                                 out.view(tokens + 2, -1), out_step, gate=gate.cuda() if with_gate else None)
+            tol = 2e-4 if out_dtype == torch.float32 else 2e-2
+            assert torch.allclose(out[:tokens, :, :n].double().cpu(), expected, atol=tol, rtol=tol)
+            assert bool((out[:, :, n:] == 3).all()) and bool((out[tokens:] == 3).all())
+
+
 def _recurrence_inputs(g, total, channels, blocks):
     size = channels // blocks
     proj = torch.randn((total, 2 * channels + 3), generator=g)
