@@ -72,6 +72,7 @@ __global__ __launch_bounds__(1024) void attention_prepare_kernel(
       if (!weighted) wa = wb = 1.f;
     }
   };
+  const bool normed = q_gamma != nullptr || k_gamma != nullptr;
   auto load_pair = [&](const int i) -> Pair {
     Pair p;
     p.is_q = i < q_pairs;
@@ -86,13 +87,16 @@ __global__ __launch_bounds__(1024) void attention_prepare_kernel(
     p.has_a = at >= 0 && at < own;
     p.has_b = at + 1 >= 0 && at + 1 < own;
     p.weighted = gamma != nullptr;
-    const float* weights = p.weighted ? gamma : row + (p.is_q ? q_col : k_col);
     const float* src = row + (p.is_q ? q_col : k_col) + p.head * own;
     const int place_a = p.has_a ? at : 0, place_b = p.has_b ? at + 1 : 0;
     p.a = src[place_a];
     p.b = src[place_b];
-    p.wa = weights[p.head * own + place_a];
-    p.wb = weights[p.head * own + place_b];
+    p.wa = p.wb = 1.f;
+    if (normed) {      // (the same in every lane)
+      const float* weights = p.weighted ? gamma : row + (p.is_q ? q_col : k_col);
+      p.wa = weights[p.head * own + place_a];
+      p.wb = weights[p.head * own + place_b];
+    }
     return p;
   };
   const int pairs = q_pairs + k_pairs;
