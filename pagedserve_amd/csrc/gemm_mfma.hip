@@ -368,10 +368,9 @@ __global__ __launch_bounds__(64 * SK_WAVES, SK_SHARED(EPI, MB, NT, UNROLL)) void
 
   const uint4 zero = {0u, 0u, 0u, 0u};
   uint4 wf[UNROLL][NT][2], xf[UNROLL][MB][2];
-  // the steps k0, k0 + 4 x 64, ... of a wave; `whole`: all of them are there
-  auto whole = [&](int k0) { return w_packed && k0 + (UNROLL - 1) * SK_WAVES * 64 + 64 <= k_end; };
+  // the steps k0, k0 + 4 x 64, ... of a wave
   auto load = [&](int k0) {
-    if (whole(k0)) {
+    if (w_packed && k0 + (UNROLL - 1) * SK_WAVES * 64 + 64 <= k_end) {
       // packed copy: the 16 x 64 tile of step s lies in the order in which the lanes hold it,
       // first the halves of the first product, then those of the second (1 KB each)
       const int tiles = (n + 15) / 16;
@@ -415,8 +414,8 @@ __global__ __launch_bounds__(64 * SK_WAVES, SK_SHARED(EPI, MB, NT, UNROLL)) void
       const int kk = ku + group * 16;
       const bool first = kk < k_end;
       const bool second = kk + 8 < k_end;
-      // unconditional loads from a clamped offset, zeroed where they are used: loads under a branch
-      // would not be issued together, and zeroed here they would be waited for in front of what the ends need
+      // unconditional loads from a clamped offset, zeroed afterwards: loads under a branch
+      // would not be issued together
       const int o0 = first ? ku : k_begin - group * 16;
       const int o1 = second ? ku + 8 : k_begin - group * 16;
       // (packed: k is a multiple of 64, so a step is whole or absent)
@@ -434,20 +433,13 @@ __global__ __launch_bounds__(64 * SK_WAVES, SK_SHARED(EPI, MB, NT, UNROLL)) void
         xf[u][b][0] = *reinterpret_cast<const uint4*>(a_ptr[b] + q0);
         xf[u][b][1] = *reinterpret_cast<const uint4*>(a_ptr[b] + q1);
       }
-    }
-  };
-  // of a step that ends inside it
-  auto trim = [&](int k0) {
-#pragma unroll
-    for (int u = 0; u < UNROLL; ++u) {
-      const int kk = k0 + u * SK_WAVES * 64 + group * 16;
-      if (kk >= k_end) {
+      if (!first) {
 #pragma unroll
         for (int j = 0; j < NT; ++j) wf[u][j][0] = zero;
 #pragma unroll
         for (int b = 0; b < MB; ++b) xf[u][b][0] = zero;
       }
-      if (kk + 8 >= k_end) {
+      if (!second) {
 #pragma unroll
         for (int j = 0; j < NT; ++j) wf[u][j][1] = zero;
 #pragma unroll
@@ -471,7 +463,6 @@ __global__ __launch_bounds__(64 * SK_WAVES, SK_SHARED(EPI, MB, NT, UNROLL)) void
   };
   if constexpr (!LATE) ask_ends();
   while (k0 < k_end) {
-    if (!whole(k0)) trim(k0);
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u)
 #pragma unroll
