@@ -123,8 +123,7 @@ __global__ __launch_bounds__(256) void gemm_nt_ring_kernel(
                                        (lds_ptr_t)(stage + dst[j]), 16, 0, 0);
   };
 
-  // (128 x 128 tiles have registers for two accumulators of a float sum)
-  constexpr int ACCS = sizeof(T) == 2 ? 1 : (WM * WN == 4 ? 2 : 4);
+  constexpr int ACCS = sizeof(T) == 2 ? 1 : 4;
   f32x16 sums[WM][WN][ACCS];
 #pragma unroll
   for (int i = 0; i < WM; ++i)
@@ -317,10 +316,9 @@ __global__ __launch_bounds__(256) void gemm_nt_ring_kernel(
     for (int j = 0; j < WN; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e)
-        acc[i][j][e] = ACCS == 1   ? sums[i][j][0][e]
-                       : ACCS == 2 ? sums[i][j][0][e] + sums[i][j][1 % ACCS][e]
-                                   : (sums[i][j][0][e] + sums[i][j][1 % ACCS][e]) +
-                                         (sums[i][j][2 % ACCS][e] + sums[i][j][3 % ACCS][e]);
+        acc[i][j][e] = ACCS == 1 ? sums[i][j][0][e]
+                                 : (sums[i][j][0][e] + sums[i][j][1 % ACCS][e]) +
+                                       (sums[i][j][2 % ACCS][e] + sums[i][j][3 % ACCS][e]);
   if constexpr (RUNS) {
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[0][0][e] += total[e];
@@ -469,18 +467,12 @@ int ps_gemm_nt_bf16_tiled(const void* a, const void* w, const float* bias, void*
   return launch_tiled_bf16<bf16_t>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
 }
 
-// The same product in true 32-bit.  Its matrix instructions take sixteen times as long per value of
-// k, so that small tiles keep the matrix cores as busy as large ones would and balance better over
-// the compute units: 64 x 64 (three stages, or two where more than two blocks share a unit: 100 x 4800 x
-// 1600 36 us with three and 44 with two, 2048 x 4096 x 1024 162 and 155), or 64 x 32 where those leave
-// half of the units without a block (100 x 2304 x 768 11.9 against 18.5).  Only many rounds of blocks
-// make larger tiles worth their uneven last round: 128 x 64 from six of 64 x 64 per unit (2048 x 4800 x
-// 1600 272 against 282) and more than one row of them (128 x 50257 x 768 129 against 110, 128 x 50257 x 1600 237 against
-// 209), 128 x 128 from four of its own (4096 x 4096 x 1024 283 against 300; with three, 4096 x 3072 x 768, 200 against 175).  With weights from memory, the kernel that did this before (128 x 128
-// tiles; below 96 rows the plain kernel) and this one, in us: 2048 x 2304 x 768 110 / 75, 2048 x 3072 x
-// 768 120 / 95 (102 TFLOP/s; the library's 4096-cubed product reaches 139), 300 x 2304 x 768 65 / 19,
-// 544 x 768 x 768 35 / 12, 330 x 1024 x 4096 60 / 43, 64 x 50257 x 768 201 / 67, 96 x 50257 x 768 116 / 109, 4096 x 3072 x
-// 768 172 / 174.
+// The same product in true 32-bit goes to gemm_even_f32.hip.  What that leaves, a k of up to 96 or rows very far apart, takes
+// 64 x 64 in two stages.
+bool ps_gemm_nt_f32_even_takes(int m, int n, int k, int lda);
+int ps_gemm_nt_f32_even(const void* a, const void* w, const float* bias, void* c, int m, int n, int k, int lda, int ldc,
+                        int epilogue, const KvScatter& scatter, hipStream_t s);
+
 bool ps_gemm_nt_f32_tiled_supported(const void* a, const void* w, int m, int k, int lda) {
   return m > 16 && k % (TB_ROW / 4) == 0 && lda % 4 == 0 &&
          (reinterpret_cast<uintptr_t>(a) & 15u) == 0 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
@@ -489,16 +481,7 @@ bool ps_gemm_nt_f32_tiled_supported(const void* a, const void* w, int m, int k, 
 int ps_gemm_nt_f32_tiled(const void* a, const void* w, const float* bias, void* c, int m, int n,
                          int k, int lda, int ldc, int epilogue, const KvScatter& scatter,
                          hipStream_t s) {
-  const int64_t tiles_64 = (int64_t)((m + 63) / 64) * ((n + 63) / 64);
-  const int units = ps_compute_units();
-  const bool splits_k = epilogue == PS_EPI_RESIDUAL && k > 1024;
-  if (2 * tiles_64 <= units && !splits_k)
-    return launch_variant<float, 1, 1, 4, float, 2>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
-  if (tiles_64 <= 2 * units)
-    return launch_variant<float, 1, 1, 3, float>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
-  if ((int64_t)((m + 127) / 128) * ((n + 127) / 128) >= 4 * units)
-    return launch_variant<float, 2, 2, 2, float>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
-  if (tiles_64 >= 6 * units && m > 128)
-    return launch_variant<float, 2, 1, 2, float>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
+  if (ps_gemm_nt_f32_even_takes(m, n, k, lda))
+    return ps_gemm_nt_f32_even(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
   return launch_variant<float, 1, 1, 2, float>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
 }

@@ -117,3 +117,28 @@ def test_rows_added_to_by_two_tiles_of_columns_share_a_unit(tmp_path):
                     seen.add(form)
                     assert taken["scratch"] == 0 and (taken["vgpr"] <= 256 or forms[form] == (4, 5)), (name, taken)
     assert len(seen) == len(forms)
+
+
+@pytest.mark.skipif(kernel_code.disassembler() is None, reason="no disassembler")
+def test_float_products_in_even_tiles_wait_for_their_operands(tmp_path):
+    """Every instance: no register is used before its read from LDS is there, nothing goes through scratch memory, and as
+    many blocks share a compute unit as the rule that picks a tile counts on (two, or three of 32 x 64)."""
+    path = os.path.join(library.in_tree_dir(), library.LIB_NAME)
+    if not os.path.isfile(path):
+        pytest.skip("the library is not built in the tree")
+    kernel = "gemm_nt_even_f32_kernel"
+    resident = {"Li1ELi2ELi1ELi4E": 3, "Li1ELi3ELi1ELi4E": 2, "Li1ELi4ELi1ELi3E": 2, "Li1ELi5ELi1ELi3E": 2, "Li2ELi2ELi3ELi3E": 2}
+    seen = []
+    for image in kernel_code.code_objects(path, library.ARCH):
+        if kernel.encode() not in image:
+            continue
+        for name, taken in kernel_code.resources(image, tmp_path).items():
+            for form, blocks in resident.items():
+                if kernel + "I" + form in name:
+                    seen.append(form)
+                    assert taken["scratch"] == 0 and taken["lds"] * blocks <= 160 * 1024, (name, taken)
+                    assert (taken["vgpr"] + 7) // 8 * 8 * blocks <= 512, (name, taken)
+        for name, code in kernel_code.kernels(kernel_code.disassemble(image, library.ARCH, tmp_path)):
+            if kernel in name:
+                assert not kernel_code.early_uses(code), (name, kernel_code.early_uses(code)[:4])
+    assert len(seen) == 6 * len(resident)
