@@ -699,7 +699,12 @@ bool ps_gemm_nt_mfma_skinny(const void* a, const void* w, int m, int n, int k, i
   return skinny_k || !ps_gemm_nt_bf16_tiled_supported(a, w, m, k, lda);
 }
 
-// What takes a bfloat16 product that the skinny kernel does not: a tile's number of the large one, the wide one, or
+bool ps_gemm_nt_k_waves_takes(const void* a, const void* w, int m, int n, int k, int lda, int ldc);
+bool ps_gemm_nt_k_waves_choice(int m, int n, int k, int c_dtype, int epilogue, bool few, int* best_tile, int* best_ranges);
+int ps_gemm_nt_k_waves_tile(const void* a, const void* w, const float* bias, void* c, int m, int n, int k, int lda, int ldc,
+                            int c_dtype, int epilogue, int tile, int ranges, const KvScatter& scatter, hipStream_t s);
+
+// What takes a bfloat16 product that neither the skinny kernel nor the one of gemm_k_waves_bf16.hip does: a tile's number of the large one, the wide one, or
 // 0: the ring kernel or, where its operands do not suit that, the plain tiles.
 #define WIDE_PRODUCT 1
 static int choice_of_many_rows(const void* a, const void* w, const void* wp, int m, int n, int k, int lda,
@@ -720,7 +725,12 @@ int ps_gemm_nt_mfma(const void* a, const void* w, const float* bias, void* c, in
                     const KvScatter& scatter, const void* w_packed, int layouts,
                     const TopChoice& top, hipStream_t s) {
   const bf16_t* wp = (const bf16_t*)w_packed;
-  if (ps_gemm_nt_mfma_skinny(a, w, m, n, k, lda, dtype, epilogue)) {
+  const bool few = ps_gemm_nt_mfma_skinny(a, w, m, n, k, lda, dtype, epilogue);
+  int tile, ranges;
+  if (dtype == PS_BF16 && m > 64 && layouts == 0 && top.keys == nullptr && ps_gemm_nt_k_waves_takes(a, w, m, n, k, lda, ldc) &&
+      ps_gemm_nt_k_waves_choice(m, n, k, c_dtype, epilogue, few, &tile, &ranges))
+    return ps_gemm_nt_k_waves_tile(a, w, bias, c, m, n, k, lda, ldc, c_dtype, epilogue, tile, ranges, scatter, s);
+  if (few) {
     if (c_dtype == PS_F32)
       return launch_skinny<float>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, wp, layouts,
                                   top, s);

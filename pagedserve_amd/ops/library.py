@@ -49,6 +49,7 @@ EXTRA_FLAGS = {
     "attention_tiled_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "gemm_tiled.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "gemm_skinny_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "gemm_k_waves_bf16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "gemm_even_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 

@@ -142,3 +142,23 @@ def test_float_products_in_even_tiles_wait_for_their_operands(tmp_path):
             if kernel in name:
                 assert not kernel_code.early_uses(code), (name, kernel_code.early_uses(code)[:4])
     assert len(seen) == 6 * len(resident)
+
+
+@pytest.mark.skipif(kernel_code.disassembler() is None, reason="no disassembler")
+def test_products_whose_waves_split_k_wait_for_their_operands(tmp_path):
+    """Every instance: no register is used before its read from LDS is there, nothing goes through scratch memory."""
+    path = os.path.join(library.in_tree_dir(), library.LIB_NAME)
+    if not os.path.isfile(path):
+        pytest.skip("the library is not built in the tree")
+    kernel, seen = "gemm_nt_k_waves_kernel", 0
+    for image in kernel_code.code_objects(path, library.ARCH):
+        if kernel.encode() not in image:
+            continue
+        for name, taken in kernel_code.resources(image, tmp_path).items():
+            if kernel in name:
+                assert taken["scratch"] == 0, (name, taken)
+        for name, code in kernel_code.kernels(kernel_code.disassemble(image, library.ARCH, tmp_path)):
+            if kernel in name:
+                seen += 1
+                assert not kernel_code.early_uses(code), (name, kernel_code.early_uses(code)[:4])
+    assert seen == 4 * 9

@@ -1791,6 +1791,78 @@ def test_float_products_of_many_rows_fill_the_cache(m, k, heads, kv_heads, head_
     _assert_product(v_pool, expected_v, "none")
 
 
+@pytest.mark.parametrize("m,n,k", [(33, 70, 384), (64, 96, 512), (130, 200, 768), (97, 1027, 576), (300, 388, 1600)])
+@pytest.mark.parametrize("tile", range(4))
+@pytest.mark.parametrize("epilogue,dtype", LARGE_EPILOGUES)
+def test_products_whose_waves_split_k(m, n, k, tile, epilogue, dtype):
+    """Each tile: as few stages as the longest ring holds, even and odd counts beyond it, blocks that begin at every place
+    of their k, rows and columns that end inside a tile, output rows in pieces and in single values, input rows apart
+    from one another, ranges of k whose sums are added by atomics; nothing beside the output."""
+    import ctypes
+
+    from pagedserve_amd.ops import kernels, library
+
+    lib = library.load_library()
+    fn = lib.ps_gemm_nt_k_waves
+    fn.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 9 + [ctypes.c_void_p]
+    a = _rand((m, k + 8), torch.bfloat16, 430, 1.0)[:, :k]
+    w = _rand((n, k), torch.bfloat16, 431, 1.0 / math.sqrt(k))
+    bias = _rand((n,), torch.float32, 432)
+    product = a.double() @ w.double().t() + bias.double()
+    c_dtype = 0 if dtype == torch.float32 else 1
+    for ranges in (1, 2, 3) if epilogue == "residual" and k >= 1600 else (1,):
+        for pad in (0, 1, 4):
+            before = _rand((m + 1, n + pad), torch.float32, 433).to(dtype)
+            out = before.clone()
+            status = fn(a.data_ptr(), w.data_ptr(), bias.data_ptr(), out.data_ptr(), m, n, k, a.stride(0), out.stride(0), c_dtype,
+                        kernels.EPILOGUES[epilogue], tile, ranges, torch.cuda.current_stream().cuda_stream)
+            assert status == 0, lib.ps_last_error().decode()
+            expected = before[:m, :n].double() + product if epilogue == "residual" else _activated(product, epilogue)
+            _assert_product(out[:m, :n], expected, epilogue)
+            assert torch.equal(out[m], before[m]) and torch.equal(out[:, n:], before[:, n:])
+    for bad_k, bad_lda, ranges in ((320, a.stride(0), 1), (k - 32, a.stride(0), 1), (k, a.stride(0) + 4, 1), (k, a.stride(0), 0)):
+        assert fn(a.data_ptr(), w.data_ptr(), bias.data_ptr(), out.data_ptr(), m, n, bad_k, bad_lda, out.stride(0), c_dtype,
+                  kernels.EPILOGUES[epilogue], tile, ranges, None) != 0
+
+
+@pytest.mark.parametrize("m,k", [(70, 512), (257, 768), (544, 512)])
+@pytest.mark.parametrize("heads,kv_heads,head_dim,page_size", [(3, 2, 8, 16), (5, 1, 7, 4), (12, 12, 64, 16), (2, 1, 6, 5)])
+@pytest.mark.parametrize("scatter_only", [False, True])
+def test_products_whose_waves_split_k_fill_the_cache(m, k, heads, kv_heads, head_dim, page_size, scatter_only):
+    """Key and value columns go into their pages, in pieces of four and one by one; a row beyond its block table and a page
+    that is none are left out."""
+    from pagedserve_amd.ops import kernels
+
+    q_cols, kv_cols = heads * head_dim, kv_heads * head_dim
+    n = q_cols + 2 * kv_cols
+    k_pool, v_pool, tables = _paged_fixture(torch.bfloat16, [m + 20], kv_heads, head_dim, page_size, 440)
+    k_pool.fill_(-3.0), v_pool.fill_(-3.0)
+    x = _rand((m, k), torch.bfloat16, 434, 1.0)
+    w = _rand((n, k), torch.bfloat16, 435, 1.0 / math.sqrt(k))
+    bias = _rand((n,), torch.float32, 436)
+    tok_item = torch.zeros(m, dtype=torch.int32, device="cuda")
+    tok_pos = torch.arange(3, m + 3, dtype=torch.int32, device="cuda")
+    tok_pos[m - 2] = tables.shape[1] * page_size       # beyond the table
+    tables = tables.clone()
+    tables[0, 1] = -1
+    out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+    kernels.linear(x, w, bias, out, scatter=(k_pool, v_pool, tok_item, tok_pos, tables, q_cols, kv_cols),
+                   scatter_only=scatter_only)
+    product = x.double() @ w.double().t() + bias.double()
+    columns = q_cols if scatter_only else n
+    _assert_product(out[:, :columns], product[:, :columns], "none")
+    expected_k, expected_v = torch.full_like(k_pool, -3.0).double(), torch.full_like(v_pool, -3.0).double()
+    for row in range(m):
+        position = int(tok_pos[row])
+        page = int(tables[0, position // page_size]) if position // page_size < tables.shape[1] else -1
+        if page < 0:
+            continue
+        expected_k[page, :, position % page_size] = product[row, q_cols:q_cols + kv_cols].view(kv_heads, head_dim)
+        expected_v[page, :, position % page_size] = product[row, q_cols + kv_cols:].view(kv_heads, head_dim)
+    _assert_product(k_pool, expected_k, "none")
+    _assert_product(v_pool, expected_v, "none")
+
+
 def _gelu_tanh_bits(u):
     """``u / (1 + exp(-2 z))``, ``2 z = 2 sqrt(2 / pi) (u + 0.044715 u^3)``, in float as the tiled products round it:
     every product and the division once, the cube's last product and sum together, ``exp`` as a power of two.  (A product
