@@ -99,10 +99,12 @@ __device__ __forceinline__ void gl_store(f32x16 (&acc)[FM][FN], float* region, i
   }
 }
 
+// What a block of 8 waves does: tile `block` of `blocks` of C.  `lds`: RING stages.
 template <int FM, int FN, int ROW, int RING, typename TOut, int EPI>
-__global__ __launch_bounds__(512) void gemm_nt_bf16_large_kernel(
-    const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, int m, int n, int k, int lda, int panel, int ldc,
-    TOut* __restrict__ c, const float* __restrict__ bias, KvScatter scatter) {
+__device__ __forceinline__ void gl_tile(unsigned char* lds, const int block, const int blocks, const bf16_t* __restrict__ a,
+                                        const bf16_t* __restrict__ w, const int m, const int n, const int k, const int lda,
+                                        const int panel, const int ldc, TOut* __restrict__ c,
+                                        const float* __restrict__ bias, const KvScatter& scatter) {
   constexpr int WAVES = GL_WAVES_M * GL_WAVES_N;
   constexpr int BM = 32 * FM * GL_WAVES_M, BN = 32 * FN * GL_WAVES_N;
   static_assert(ROW == 64 || ROW == 128, "rows of half a line or of a whole one");
@@ -115,7 +117,6 @@ __global__ __launch_bounds__(512) void gemm_nt_bf16_large_kernel(
   constexpr int FIRST_PART = (LOADS + SUB - 1) / SUB;    // part p: the loads from p LOADS / SUB on, rounded up
   constexpr int READS = FM + FN, PRODUCTS = FM * FN;
   static_assert((RING - 1) * LOADS + FIRST_PART < 64, "the load counter has six bits");
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[RING * STAGE_BYTES];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -124,9 +125,9 @@ __global__ __launch_bounds__(512) void gemm_nt_bf16_large_kernel(
   // every XCD works on a contiguous run of tiles (see gemm_tiled.hip): panels of `panel` rows of tiles, walked
   // column by column, so that what runs at one time on an XCD is about as many rows as columns
   const int tiles_m = (m + BM - 1) / BM, tiles_n = (n + BN - 1) / BN;
-  const int per_xcd = tiles_m * tiles_n / 8;
-  int tile = blockIdx.x;
-  if (blockIdx.x < per_xcd * 8) tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  const int per_xcd = blocks / 8;
+  int tile = block;
+  if (block < per_xcd * 8) tile = (block & 7) * per_xcd + (block >> 3);
   const int first_row = tile / (panel * tiles_n) * panel;
   const int within = tile - first_row * tiles_n;
   const int panel_rows = min(panel, tiles_m - first_row);
@@ -271,6 +272,19 @@ __global__ __launch_bounds__(512) void gemm_nt_bf16_large_kernel(
   if constexpr (!EARLY) ends.ask(lane, row_base, col_base, m, n, ldc, c, bias, 0, by_column);
   gl_store<FM, FN, SLICE, 0, TOut, EPI>(acc, reinterpret_cast<float*>(lds) + wave * 32 * (SLICE * 32 + 8), lane,
                                         row_base, col_base, m, n, ldc, c, bias, scatter, ends, pages, tail);
+}
+
+template <int FM, int FN, int ROW>
+constexpr int gl_stage_bytes() { return 32 * (FM * GL_WAVES_M + FN * GL_WAVES_N) * ROW; }
+
+template <int FM, int FN, int ROW, int RING, typename TOut, int EPI>
+__global__ __launch_bounds__(512) void gemm_nt_bf16_large_kernel(
+    const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, int m, int n, int k, int lda, int panel, int ldc,
+    TOut* __restrict__ c, const float* __restrict__ bias, KvScatter scatter) {
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[RING * gl_stage_bytes<FM, FN, ROW>()];
+  constexpr int BM = 32 * FM * GL_WAVES_M, BN = 32 * FN * GL_WAVES_N;
+  gl_tile<FM, FN, ROW, RING, TOut, EPI>(lds, blockIdx.x, ((m + BM - 1) / BM) * ((n + BN - 1) / BN), a, w, m, n, k, lda, panel,
+                                        ldc, c, bias, scatter);
 }
 
 // --------------------------------------------------------------------------------- host

@@ -110,6 +110,10 @@ static bool large_takes(const void* a, const void* w, int m, int n, int k, int l
          (reinterpret_cast<uintptr_t>(a) & 15u) == 0 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
 }
 
+bool ps_gemm_nt_bf16_large_operands(const void* a, const void* w, int m, int n, int k, int lda) {
+  return large_takes(a, w, m, n, k, lda);
+}
+
 int ps_gemm_nt_bf16_large_shape(const void* a, const void* w, int m, int n, int k, int lda, int c_dtype, int epilogue,
                                 bool wide) {
   return large_takes(a, w, m, n, k, lda) ? shape_for(m, n, k, c_dtype, epilogue, wide) : 0;

@@ -704,6 +704,10 @@ bool ps_gemm_nt_k_waves_choice(int m, int n, int k, int c_dtype, int epilogue, b
 int ps_gemm_nt_k_waves_tile(const void* a, const void* w, const float* bias, void* c, int m, int n, int k, int lda, int ldc,
                             int c_dtype, int epilogue, int tile, int ranges, const KvScatter& scatter, hipStream_t s);
 
+int ps_gemm_nt_bf16_two_sizes_columns(int m, int n, int k, int c_dtype, int epilogue, const KvScatter& scatter);
+int ps_gemm_nt_bf16_two_sizes(const void* a, const void* w, const float* bias, void* c, int m, int n, int k, int lda, int ldc,
+                              int epilogue, int first_columns, hipStream_t s);
+
 // What takes a bfloat16 product that neither the skinny kernel nor the one of gemm_k_waves_bf16.hip does: a tile's number of the large one, the wide one, or
 // 0: the ring kernel or, where its operands do not suit that, the plain tiles.
 #define WIDE_PRODUCT 1
@@ -743,8 +747,12 @@ int ps_gemm_nt_mfma(const void* a, const void* w, const float* bias, void* c, in
     return 1;
   }
   const int choice = dtype == PS_BF16 ? choice_of_many_rows(a, w, wp, m, n, k, lda, c_dtype, epilogue) : 0;
-  if (choice > WIDE_PRODUCT)
+  if (choice > WIDE_PRODUCT) {
+    const int first_columns = ps_gemm_nt_bf16_two_sizes_columns(m, n, k, c_dtype, epilogue, scatter);
+    if (first_columns > 0)
+      return ps_gemm_nt_bf16_two_sizes(a, w, bias, c, m, n, k, lda, ldc, epilogue, first_columns, s);
     return ps_gemm_nt_bf16_large(a, w, bias, c, m, n, k, lda, ldc, c_dtype, epilogue, scatter, choice, s);
+  }
   if (choice == WIDE_PRODUCT)
     return ps_gemm_nt_bf16_wide(a, wp, bias, c, m, n, k, lda, ldc, c_dtype, epilogue, scatter, 0, s);
   if (dtype == PS_BF16 && ps_gemm_nt_bf16_tiled_supported(a, w, m, k, lda))

@@ -1863,6 +1863,38 @@ def test_products_whose_waves_split_k_fill_the_cache(m, k, heads, kv_heads, head
     _assert_product(v_pool, expected_v, "none")
 
 
+@pytest.mark.parametrize("m,n,k,first", [(300, 400, 512, 320), (1, 321, 512, 320), (700, 1001, 576, 640), (2100, 1360, 1600, 320)])
+@pytest.mark.parametrize("epilogue", ["none", "gelu_tanh", "gelu_erf", "relu2"])
+def test_products_in_two_sizes_of_tiles(m, n, k, first, epilogue):
+    """Columns in tiles of 256 x 320 and the rest in 128 x 192, in one launch: the bits of one size, rows and columns that
+    end inside a tile, nothing beside the output."""
+    import ctypes
+
+    from pagedserve_amd.ops import kernels, library
+
+    lib = library.load_library()
+    fn, one = lib.ps_gemm_nt_two_sizes, lib.ps_gemm_nt_large
+    fn.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 7 + [ctypes.c_void_p]
+    one.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 8 + [ctypes.c_void_p]
+    a = _rand((m, k + 8), torch.bfloat16, 450, 1.0)[:, :k]
+    w = _rand((n, k), torch.bfloat16, 451, 1.0 / math.sqrt(k))
+    bias = _rand((n,), torch.float32, 452)
+    expected = _activated(a.double() @ w.double().t() + bias.double(), epilogue)
+    stream = torch.cuda.current_stream().cuda_stream
+    for pad in (0, 3, 8):
+        before = _rand((m + 1, n + pad), torch.float32, 453).bfloat16()
+        out, same = before.clone(), before.clone()
+        sizes = (m, n, k, a.stride(0), out.stride(0))
+        operands = (a.data_ptr(), w.data_ptr(), bias.data_ptr())
+        assert fn(*operands, out.data_ptr(), *sizes, kernels.EPILOGUES[epilogue], first, stream) == 0, lib.ps_last_error().decode()
+        assert one(*operands, same.data_ptr(), *sizes, 1, kernels.EPILOGUES[epilogue], 4, stream) == 0
+        assert torch.equal(out, same)
+        _assert_product(out[:m, :n], expected, epilogue)
+        assert torch.equal(out[m], before[m]) and torch.equal(out[:, n:], before[:, n:])
+    for bad_first in (0, 300, n // 320 * 320 + 320):
+        assert fn(*operands, out.data_ptr(), *sizes, kernels.EPILOGUES[epilogue], bad_first, None) != 0
+
+
 def _gelu_tanh_bits(u):
     """``u / (1 + exp(-2 z))``, ``2 z = 2 sqrt(2 / pi) (u + 0.044715 u^3)``, in float as the tiled products round it:
     every product and the division once, the cube's last product and sum together, ``exp`` as a power of two.  (A product
