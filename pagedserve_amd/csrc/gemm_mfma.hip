@@ -718,6 +718,7 @@ static int choice_of_many_rows(const void* a, const void* w, const void* wp, int
   return shape != 0 ? shape : (wide ? WIDE_PRODUCT : 0);
 }
 
+// (for the products that gemm_k_waves_bf16.hip leaves, and in one size of tiles)
 extern "C" int ps_linear_choice(int m, int n, int k, int c_dtype, int epilogue, int packed) {
   const void* aligned = reinterpret_cast<const void*>((uintptr_t)256);
   if (ps_gemm_nt_mfma_skinny(aligned, aligned, m, n, k, k, PS_BF16, epilogue)) return 0;

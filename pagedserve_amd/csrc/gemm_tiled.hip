@@ -408,6 +408,9 @@ static int launch_variant(const void* a, const void* w, const float* bias, void*
   return 0;
 }
 
+// (Products of more than 64 rows with a k of 512 and more whose small tiles come to one round of blocks go to
+// gemm_k_waves_bf16.hip first: what is measured here on such shapes is this kernel's part of that comparison.)
+//
 // Tile shapes by the number of blocks they give against the chip's compute units: a product
 // of this size is over in a few microseconds, so filling them counts for more than the reuse
 // inside a large tile.  (More than 128 rows with a k of 768 and more come here where 64 x 64 tiles or two rounds of
