@@ -7,7 +7,8 @@
 // multiplies one of a stage's four steps of 16 values, so that every operand is read once: 3 cycles a row of the tile
 // instead of 4, and tiles that are no square of squares, 32 x 96 and 64 x 96, cost their rows and no more (measured: 430
 // cycles a stage for 64 x 64, 510 for 64 x 96).  At the end the four waves' sums meet in LDS, 32 rows at a time, where a
-// thread takes four columns of a row and adds them in a fixed order.
+// thread takes four columns of a row and adds them in a fixed order.  (Four chains of a quarter of k: error against float64 0.64e-7
+// for a k of 768, 1.7e-7 for 6,400, in one chain 1.13 and 3.6e-7.)
 //
 // With one block to a unit nothing hides its ends, so they are straight code: C and bias are buffers (what lies outside reads
 // as zero and is not written), and what cannot go in pieces of four columns takes another branch in a loop of its own.
