@@ -6,7 +6,7 @@
 // which begin as the units become free.  Every output keeps its bits: both kinds of tiles add up k in the same order.
 //
 // With weights from memory, one size of tiles and two, us: 4096 x 6400 x 1600 with GELU 100 / 91 (two launches 93), 8192 x
-// 6400 x 1600 186 / 175, 2048 x 12800 x 1600 92 / 83.  In a batch of 64 prompts of 768 and 12 steps (GPT-2 XL) 105 to 97 a layer
+// 6400 x 1600 186 / 175, 2048 x 12800 x 1600 92 / 83.  In a batch of 64 prompts of 768 and 12 steps (GPT-2 XL) 105 to 93 a layer
 // and budget of 4,096 tokens.
 #include "gemm_large_bf16.h"
 
