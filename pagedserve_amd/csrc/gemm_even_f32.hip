@@ -394,14 +394,18 @@ static float even_time(int m, int n, int k, int tile, int ranges, int units) {
   return 1.05f * area + stages * (0.109f * area * fullest + 0.08f * ceilf(fullest / t.resident)) + added;
 }
 
-// Ranges of k only where C is added to anyway.
+// Ranges of k only where C is added to anyway, over a k of more than 1,024 and with at most one and a half tiles of 64 x 64 to
+// a unit.  Elsewhere sums keep an order that does not change from call to call; ranges would gain there (us, one range and
+// several: 224 x 768 x 768 10.1 / 7.7, 160 x 1024 x 1024 12.1 / 8.3, 256 x 1024 x 1024 12.4 / 10.1, 1024 x 1600 x 6400 199 / 178).
 static void choose_even(int m, int n, int k, int epilogue, int* best_tile, int* best_ranges) {
   const int units = ps_compute_units();
+  const int64_t tiles_64 = (int64_t)((m + 63) / 64) * ((n + 63) / 64);
+  const int most = epilogue == PS_EPI_RESIDUAL && k > 1024 && 2 * tiles_64 <= 3 * units ? 12 : 1;
   float least = INFINITY;
   *best_tile = 0;
   *best_ranges = 1;
   for (int tile = 0; tile < GE_TILES; ++tile)
-    for (int ranges = 1; ranges == 1 || (epilogue == PS_EPI_RESIDUAL && ranges <= 12); ++ranges) {
+    for (int ranges = 1; ranges <= most; ++ranges) {
       const int stages = (k / GE_BK + ranges - 1) / ranges;
       const int shortest = k / GE_BK - (ranges - 1) * stages;
       if (ranges > 1 && shortest * GE_BK < GE_SHORTEST_RANGE) continue;
@@ -424,6 +428,14 @@ int ps_gemm_nt_f32_even(const void* a, const void* w, const float* bias, void* c
   int tile, ranges;
   choose_even(m, n, k, epilogue, &tile, &ranges);
   return launch_even_tile(a, w, bias, c, m, n, k, lda, ldc, epilogue, tile, ranges, scatter, s);
+}
+
+// The tile and number of ranges that a product gets, tile + 16 * ranges, -1: not this kernel; for tests.
+extern "C" int ps_gemm_nt_even_choice(int m, int n, int k, int epilogue) {
+  if (!ps_gemm_nt_f32_even_takes(m, n, k, k)) return -1;
+  int tile, ranges;
+  choose_even(m, n, k, epilogue, &tile, &ranges);
+  return tile + 16 * ranges;
 }
 
 // The product in a given tile and number of ranges, for tests and measurements.

@@ -1752,6 +1752,22 @@ def test_float_products_in_even_tiles(m, n, k, tile, epilogue):
                   kernels.EPILOGUES[epilogue], tile, ranges, None) != 0
 
 
+@pytest.mark.parametrize("m,n,k", [(256, 768, 768), (160, 1024, 1024), (400, 512, 1024), (2100, 768, 3072)])
+def test_float_rows_added_to_repeat_themselves(m, n, k):
+    """Float rows added to over a k of up to 1,024, or in more tiles than ranges of k are for: the same bits on every call."""
+    from pagedserve_amd.ops import kernels
+
+    x, w = _rand((m, k), torch.float32, 397, 1.0), _rand((n, k), torch.float32, 398, 1.0 / math.sqrt(k))
+    before = _rand((m, n), torch.float32, 399)
+    first = before.clone()
+    kernels.linear(x, w, None, first, epilogue="residual")
+    torch.testing.assert_close(first.double(), before.double() + x.double() @ w.double().t(), atol=1e-4, rtol=1e-5)
+    for _ in range(12):
+        again = before.clone()
+        kernels.linear(x, w, None, again, epilogue="residual")
+        assert torch.equal(again, first)
+
+
 @pytest.mark.parametrize("m,k", [(70, 128), (200, 768), (97, 96)])
 @pytest.mark.parametrize("heads,kv_heads,head_dim,page_size", [(3, 2, 8, 16), (5, 1, 7, 4), (12, 12, 64, 16), (2, 1, 6, 5)])
 @pytest.mark.parametrize("scatter_only", [False, True])
