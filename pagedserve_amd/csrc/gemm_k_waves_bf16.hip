@@ -9,6 +9,10 @@
 // cycles a stage for 64 x 64, 510 for 64 x 96).  At the end the four waves' sums meet in LDS, 32 rows at a time, where a
 // thread takes four columns of a row and adds them in a fixed order.  (Four chains of a quarter of k: error against float64 0.64e-7
 // for a k of 768, 1.7e-7 for 6,400, in one chain 1.13 and 3.6e-7.)
+// Every tile of every size adds a row's products in the same order, so that equal rows of a product give equal bits wherever they
+// lie.  Blocks of an XCD that begin their k 256 bytes apart, round and round, ask for fewer rows of one channel at a time, but
+// lose that: 667 products took 1.002 of the time on average (256 x 5120 x 1280 11.2 us and 12.2, 1024 x 1280 x 5120 29.7 and 32.5, but
+// x 1024 x 4096 16.0 and 15.2); begun by the tile's column, which would keep it, 1.003 of what k from its start takes.
 //
 // With one block to a unit nothing hides its ends, so they are straight code: C and bias are buffers (what lies outside reads
 // as zero and is not written), and what cannot go in pieces of four columns takes another branch in a loop of its own.
@@ -101,14 +105,6 @@ __global__ __launch_bounds__(64 * KW_WAVES, 2) void gemm_nt_k_waves_kernel(
   const int m0 = (row_major ? outer : inner) * BM;
   const int n0 = (row_major ? inner : outer) * BN;
 
-  // The blocks of an XCD begin their k 256 bytes apart, round and round.  With all of them at one place the rows that
-  // they ask for at a time lie on few channels of the caches and of memory wherever a row is a large power of two of bytes,
-  // or nearly: 0.83 to 0.92 of the time for 2,048 to 6,400 columns of a k of 1,024 to 1,600, 0.93 to 0.97 for k of 4,096 and
-  // 5,120, level to 1.03 for k of 768 and 3,072.
-  uint32_t first = ((blockIdx.x >> 3) & 15) * 2;
-  if (first >= (uint32_t)stages) first -= stages;
-  if (first >= (uint32_t)stages) first = 0;
-
   // ---- loads: lane l of an instruction fills slot l % 8 of row l / 8 of its eight rows.  Rows beyond m or n are fetched
   // from the last valid one (they feed outputs that are never stored).
   const __amdgpu_buffer_rsrc_t from_a = kw_operand(a + (int64_t)m0 * lda + k_begin, min(BM, m - m0), lda, stages * TB_BK);
@@ -141,9 +137,7 @@ __global__ __launch_bounds__(64 * KW_WAVES, 2) void gemm_nt_k_waves_kernel(
   const uint32_t reads_at = (uint32_t)(uintptr_t)(lds_ptr_t)lds + (lane & 31) * TB_ROW +
                             (uint32_t)(((2 * wave + (lane >> 5)) ^ ((lane >> 1) & 7)) << 4);
   u32x4_t operands[2][READS];
-  uint32_t here = 0, k_next = first * TB_ROW;      // the stage that is multiplied, in the ring; the stage that is asked for
-  const uint32_t k_end = (uint32_t)stages * TB_ROW;
-  auto beyond = [&](uint32_t at) { return at + TB_ROW < k_end ? at + TB_ROW : 0u; };
+  uint32_t here = 0, k_next = 0;      // the stage that is multiplied, in the ring; the stage that is asked for
   auto around = [](uint32_t at) { return at + STAGE_BYTES < RING * STAGE_BYTES ? at + STAGE_BYTES : 0u; };
   auto arrived = [](u32x4_t* of) {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -184,7 +178,7 @@ __global__ __launch_bounds__(64 * KW_WAVES, 2) void gemm_nt_k_waves_kernel(
       });
     if constexpr (NEXT) arrived(operands[TO]);
     here = next;
-    if constexpr (LOAD) k_next = beyond(k_next);
+    if constexpr (LOAD) k_next += TB_ROW;
   };
   using Yes = std::true_type;
   using No = std::false_type;
@@ -194,7 +188,7 @@ __global__ __launch_bounds__(64 * KW_WAVES, 2) void gemm_nt_k_waves_kernel(
 
   kw_for<0, RING>([&](auto stage) {      // (the host sends no product of fewer stages)
     kw_for<0, LOADS>([&](auto index) { load(k_next, decltype(stage)::value * STAGE_BYTES, index); });
-    k_next = beyond(k_next);
+    k_next += TB_ROW;
   });
   kw_wait_and_sync<(RING - 1) * LOADS>();
   kw_for<0, READS>([&](auto index) {

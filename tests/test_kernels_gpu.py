@@ -1841,6 +1841,25 @@ def test_products_whose_waves_split_k(m, n, k, tile, epilogue, dtype):
                   kernels.EPILOGUES[epilogue], tile, ranges, None) != 0
 
 
+@pytest.mark.parametrize("n,k,epilogue", [(768, 768, "residual"), (768, 3072, "residual"), (1024, 1024, "residual"), (1001, 576, "none"),
+                                          (2304, 768, "none"), (3072, 768, "gelu_tanh"), (4800, 1600, "none")])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_equal_rows_of_a_product_give_equal_bits(n, k, epilogue, dtype):
+    """The same hundred rows four times, in tiles of different rows and columns: the same bits wherever they lie."""
+    from pagedserve_amd.ops import kernels
+
+    rows, w = _rand((100, k), dtype, 437, 1.0), _rand((n, k), dtype, 438, 1.0 / math.sqrt(k))
+    bias, before = _rand((n,), torch.float32, 439), _rand((100, n), torch.float32, 440)
+    if dtype == torch.float32 and epilogue == "residual" and k > 1024:
+        pytest.skip("float sums of ranges of k are added by atomics")
+    out = torch.cat([before if epilogue == "residual" else before.to(dtype)] * 4)
+    kernels.linear(torch.cat([rows] * 4), w, bias, out, epilogue=epilogue)
+    for place in (100, 200, 300):
+        assert torch.equal(out[place:place + 100], out[:100])
+    product = rows.double() @ w.double().t() + bias.double()
+    _assert_product(out[:100], before.double() + product if epilogue == "residual" else _activated(product, epilogue), epilogue)
+
+
 @pytest.mark.parametrize("m,k", [(70, 512), (257, 768), (544, 512)])
 @pytest.mark.parametrize("heads,kv_heads,head_dim,page_size", [(3, 2, 8, 16), (5, 1, 7, 4), (12, 12, 64, 16), (2, 1, 6, 5)])
 @pytest.mark.parametrize("scatter_only", [False, True])
