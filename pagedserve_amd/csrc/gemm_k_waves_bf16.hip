@@ -12,7 +12,7 @@
 // Every tile of every size adds a row's products in the same order, so that equal rows of a product give equal bits wherever they
 // lie.  Blocks of an XCD that begin their k 256 bytes apart, round and round, ask for fewer rows of one channel at a time, but
 // lose that: 667 products took 1.002 of the time on average (256 x 5120 x 1280 11.2 us and 12.2, 1024 x 1280 x 5120 29.7 and 32.5, but
-// x 1024 x 4096 16.0 and 15.2); begun by the tile's column, which would keep it, 1.003 of what k from its start takes.
+// 1024 x 1024 x 4096 16.3 and 15.5); begun by the tile's column, which would keep it, 1.003 of what k from its start takes.
 //
 // With one block to a unit nothing hides its ends, so they are straight code: C and bias are buffers (what lies outside reads
 // as zero and is not written), and what cannot go in pieces of four columns takes another branch in a loop of its own.
