@@ -471,10 +471,17 @@ int ps_gemm_nt_bf16_tiled(const void* a, const void* w, const float* bias, void*
 }
 
 // The same product in true 32-bit goes to gemm_even_f32.hip.  What that leaves, a k of up to 96 or rows very far apart, takes
-// 64 x 64 in two stages.
+// 64 x 64 in two stages, or 64 x 32 by pairs of k tiles where 64 x 64 would leave half of the units without a block: 129 x 192 x
+// 64 3.8 against 4.5 us, 300 x 1000 x 64 4.0 and 4.8, 500 x 512 x 96 4.5 and 5.2, 500 x 256 x 64 with GELU 5.5 and 6.0.  (Beyond,
+// three stages up to two blocks to a unit 0.97 to 1.04 of it, 128 x 64 tiles behind: 2048 x 3072 x 64 21.8 and 18.0.)
 bool ps_gemm_nt_f32_even_takes(int m, int n, int k, int lda);
 int ps_gemm_nt_f32_even(const void* a, const void* w, const float* bias, void* c, int m, int n, int k, int lda, int ldc,
                         int epilogue, const KvScatter& scatter, hipStream_t s);
+
+extern "C" int ps_gemm_nt_f32_ring_columns(int m, int n, int k) {
+  const int64_t tiles_64 = (int64_t)((m + 63) / 64) * ((n + 63) / 64);
+  return 2 * tiles_64 <= ps_compute_units() && k <= 1024 ? 32 : 64;
+}
 
 bool ps_gemm_nt_f32_tiled_supported(const void* a, const void* w, int m, int k, int lda) {
   return m > 16 && k % (TB_ROW / 4) == 0 && lda % 4 == 0 &&
@@ -486,5 +493,7 @@ int ps_gemm_nt_f32_tiled(const void* a, const void* w, const float* bias, void* 
                          hipStream_t s) {
   if (ps_gemm_nt_f32_even_takes(m, n, k, lda))
     return ps_gemm_nt_f32_even(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
+  if (ps_gemm_nt_f32_ring_columns(m, n, k) == 32)
+    return launch_variant<float, 1, 1, 4, float, 2>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
   return launch_variant<float, 1, 1, 2, float>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
 }

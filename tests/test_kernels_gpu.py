@@ -1752,6 +1752,27 @@ def test_float_products_in_even_tiles(m, n, k, tile, epilogue):
                   kernels.EPILOGUES[epilogue], tile, ranges, None) != 0
 
 
+@pytest.mark.parametrize("m,n,k", [(65, 5, 32), (129, 192, 64), (300, 385, 96), (70, 1001, 96), (513, 1024, 64)])
+@pytest.mark.parametrize("epilogue", ["none", "gelu_tanh", "gelu_erf", "relu2", "residual"])
+def test_float_products_of_a_short_k(m, n, k, epilogue):
+    """Through ``kernels.linear``, k of one to three tiles, which the even tiles leave: pairs of k tiles and, with more rows and
+    columns, one by one; rows and columns that end inside a tile, rows that do not allow 16-byte stores, nothing beside
+    the output."""
+    from pagedserve_amd.ops import kernels
+
+    x = _rand((m, k + 8), torch.float32, 400, 1.0)[:, :k]
+    w = _rand((n, k), torch.float32, 401, 1.0 / math.sqrt(k))
+    bias = _rand((n,), torch.float32, 402)
+    product = x.double() @ w.double().t() + bias.double()
+    for pad in (0, 1, 4):
+        before = _rand((m + 1, n + pad), torch.float32, 403)
+        out = before.clone()
+        kernels.linear(x, w, bias, out[:m, :n], epilogue=epilogue)
+        expected = before[:m, :n].double() + product if epilogue == "residual" else _activated(product, epilogue)
+        _assert_product(out[:m, :n], expected, epilogue)
+        assert torch.equal(out[m], before[m]) and torch.equal(out[:, n:], before[:, n:])
+
+
 @pytest.mark.parametrize("m,n,k", [(256, 768, 768), (160, 1024, 1024), (400, 512, 1024), (2100, 768, 3072)])
 def test_float_rows_added_to_repeat_themselves(m, n, k):
     """Float rows added to over a k of up to 1,024, or in more tiles than ranges of k are for: the same bits on every call."""

@@ -30,3 +30,12 @@ def test_ranges_of_k_of_float_products(lib, m, n, k, ranges):
     64 x 64 for one and a half to a unit at most."""
     assert _even(lib, m, n, k, "residual")[1] == ranges
     assert _even(lib, m, n, k, "none")[1] == _even(lib, m, n, k, "gelu_tanh")[1] == 1
+
+
+@pytest.mark.parametrize("m,n,k,columns", [
+    (65, 192, 64, 32), (129, 192, 64, 32), (300, 1000, 96, 32), (2048, 256, 32, 32), (500, 1024, 64, 32),        # 128 tiles of 64 x 64
+    (513, 1024, 64, 64), (2049, 256, 32, 64), (4096, 4096, 64, 64)])
+def test_tiles_of_float_products_of_a_short_k(lib, m, n, k, columns):
+    """A k of up to 96: 64 x 32 by pairs of k tiles where tiles of 64 x 64 come to half of the units at most."""
+    assert lib.ps_gemm_nt_even_choice(m, n, k, kernels.EPILOGUES["none"]) == -1
+    assert lib.ps_gemm_nt_f32_ring_columns(m, n, k) == columns
