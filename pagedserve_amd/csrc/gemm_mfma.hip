@@ -708,21 +708,45 @@ int ps_gemm_nt_bf16_two_sizes_columns(int m, int n, int k, int c_dtype, int epil
 int ps_gemm_nt_bf16_two_sizes(const void* a, const void* w, const float* bias, void* c, int m, int n, int k, int lda, int ldc,
                               int epilogue, int first_columns, hipStream_t s);
 
-// What takes a bfloat16 product that neither the skinny kernel nor the one of gemm_k_waves_bf16.hip does: a tile's number of the large one, the wide one, or
-// 0: the ring kernel or, where its operands do not suit that, the plain tiles.
-#define WIDE_PRODUCT 1
-static int choice_of_many_rows(const void* a, const void* w, const void* wp, int m, int n, int k, int lda,
-                               int c_dtype, int epilogue) {
+// Which kernel takes a product of bfloat16 operands that the matrix cores take; `tile`: the number of its tile, or the columns that
+// go in the first size of tiles.
+enum BfKernel { BF_FEW_ROWS, BF_K_WAVES, BF_TWO_SIZES, BF_LARGE, BF_WIDE, BF_RING, BF_PLAIN };
+struct BfRoute {
+  BfKernel kernel;
+  int tile, ranges;
+};
+
+// `own_order`: rows and tokens in the way of the kernel for few rows (packed rows, choice of tokens).
+static BfRoute bf_route(const void* a, const void* w, const void* wp, int m, int n, int k, int lda, int ldc, int c_dtype,
+                        int epilogue, const KvScatter& scatter, bool own_order) {
+  BfRoute route = {BF_FEW_ROWS, 0, 1};
+  const bool few = ps_gemm_nt_mfma_skinny(a, w, m, n, k, lda, PS_BF16, epilogue);
+  if (m > 64 && !own_order && ps_gemm_nt_k_waves_takes(a, w, m, n, k, lda, ldc) &&
+      ps_gemm_nt_k_waves_choice(m, n, k, c_dtype, epilogue, few, &route.tile, &route.ranges)) {
+    route.kernel = BF_K_WAVES;
+    return route;
+  }
+  if (few) return route;
   const bool wide = ps_gemm_nt_bf16_wide_supported(a, wp, m, n, k, lda);
   const int shape = ps_gemm_nt_bf16_large_shape(a, w, m, n, k, lda, c_dtype, epilogue, wide);
-  return shape != 0 ? shape : (wide ? WIDE_PRODUCT : 0);
+  if (shape != 0) {
+    const int first_columns = ps_gemm_nt_bf16_two_sizes_columns(m, n, k, c_dtype, epilogue, scatter);
+    route.kernel = first_columns > 0 ? BF_TWO_SIZES : BF_LARGE;
+    route.tile = first_columns > 0 ? first_columns : shape;
+    return route;
+  }
+  route.kernel = wide ? BF_WIDE : ps_gemm_nt_bf16_tiled_supported(a, w, m, k, lda) ? BF_RING : BF_PLAIN;
+  return route;
 }
 
-// (for the products that gemm_k_waves_bf16.hip leaves, and in one size of tiles)
-extern "C" int ps_linear_choice(int m, int n, int k, int c_dtype, int epilogue, int packed) {
-  const void* aligned = reinterpret_cast<const void*>((uintptr_t)256);
-  if (ps_gemm_nt_mfma_skinny(aligned, aligned, m, n, k, k, PS_BF16, epilogue)) return 0;
-  return choice_of_many_rows(aligned, aligned, packed ? aligned : nullptr, m, n, k, k, c_dtype, epilogue);
+extern "C" int ps_linear_choice(int m, int n, int k, int c_dtype, int epilogue, int packed, int scatter, int* tile, int* ranges) {
+  void* aligned = reinterpret_cast<void*>((uintptr_t)256);
+  KvScatter pages = {};
+  if (scatter) pages.k_pool = aligned;
+  const BfRoute route = bf_route(aligned, aligned, packed ? aligned : nullptr, m, n, k, k, n, c_dtype, epilogue, pages, false);
+  *tile = route.tile;
+  *ranges = route.ranges;
+  return (int)route.kernel;
 }
 
 int ps_gemm_nt_mfma(const void* a, const void* w, const float* bias, void* c, int m, int n, int k,
@@ -730,34 +754,35 @@ int ps_gemm_nt_mfma(const void* a, const void* w, const float* bias, void* c, in
                     const KvScatter& scatter, const void* w_packed, int layouts,
                     const TopChoice& top, hipStream_t s) {
   const bf16_t* wp = (const bf16_t*)w_packed;
-  const bool few = ps_gemm_nt_mfma_skinny(a, w, m, n, k, lda, dtype, epilogue);
-  int tile, ranges;
-  if (dtype == PS_BF16 && m > 64 && layouts == 0 && top.keys == nullptr && ps_gemm_nt_k_waves_takes(a, w, m, n, k, lda, ldc) &&
-      ps_gemm_nt_k_waves_choice(m, n, k, c_dtype, epilogue, few, &tile, &ranges))
-    return ps_gemm_nt_k_waves_tile(a, w, bias, c, m, n, k, lda, ldc, c_dtype, epilogue, tile, ranges, scatter, s);
-  if (few) {
-    if (c_dtype == PS_F32)
-      return launch_skinny<float>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, wp, layouts,
-                                  top, s);
-    return launch_skinny<bf16_t>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, wp, layouts,
-                                 top, s);
+  if (dtype == PS_BF16) {
+    const BfRoute route =
+        bf_route(a, w, wp, m, n, k, lda, ldc, c_dtype, epilogue, scatter, layouts != 0 || top.keys != nullptr);
+    if (route.kernel == BF_FEW_ROWS) {
+      if (c_dtype == PS_F32)
+        return launch_skinny<float>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, wp, layouts,
+                                    top, s);
+      return launch_skinny<bf16_t>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, wp, layouts,
+                                   top, s);
+    }
+    if (layouts != 0) {
+      ps_set_error("ps_linear: packed activations go with the skinny product only (m %d, n %d, k %d)",
+                   m, n, k);
+      return 1;
+    }
+    switch (route.kernel) {
+      case BF_K_WAVES:
+        return ps_gemm_nt_k_waves_tile(a, w, bias, c, m, n, k, lda, ldc, c_dtype, epilogue, route.tile, route.ranges, scatter, s);
+      case BF_TWO_SIZES:
+        return ps_gemm_nt_bf16_two_sizes(a, w, bias, c, m, n, k, lda, ldc, epilogue, route.tile, s);
+      case BF_LARGE:
+        return ps_gemm_nt_bf16_large(a, w, bias, c, m, n, k, lda, ldc, c_dtype, epilogue, scatter, route.tile, s);
+      case BF_WIDE:
+        return ps_gemm_nt_bf16_wide(a, wp, bias, c, m, n, k, lda, ldc, c_dtype, epilogue, scatter, 0, s);
+      case BF_RING:
+        return ps_gemm_nt_bf16_tiled(a, w, bias, c, m, n, k, lda, ldc, c_dtype, epilogue, scatter, s);
+      default: break;
+    }
   }
-  if (layouts != 0) {
-    ps_set_error("ps_linear: packed activations go with the skinny product only (m %d, n %d, k %d)",
-                 m, n, k);
-    return 1;
-  }
-  const int choice = dtype == PS_BF16 ? choice_of_many_rows(a, w, wp, m, n, k, lda, c_dtype, epilogue) : 0;
-  if (choice > WIDE_PRODUCT) {
-    const int first_columns = ps_gemm_nt_bf16_two_sizes_columns(m, n, k, c_dtype, epilogue, scatter);
-    if (first_columns > 0)
-      return ps_gemm_nt_bf16_two_sizes(a, w, bias, c, m, n, k, lda, ldc, epilogue, first_columns, s);
-    return ps_gemm_nt_bf16_large(a, w, bias, c, m, n, k, lda, ldc, c_dtype, epilogue, scatter, choice, s);
-  }
-  if (choice == WIDE_PRODUCT)
-    return ps_gemm_nt_bf16_wide(a, wp, bias, c, m, n, k, lda, ldc, c_dtype, epilogue, scatter, 0, s);
-  if (dtype == PS_BF16 && ps_gemm_nt_bf16_tiled_supported(a, w, m, k, lda))
-    return ps_gemm_nt_bf16_tiled(a, w, bias, c, m, n, k, lda, ldc, c_dtype, epilogue, scatter, s);
   if (dtype == PS_F32 && c_dtype == PS_F32)
     return launch_tiled<float, float>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, s);
   if (dtype == PS_BF16 && c_dtype == PS_F32)

@@ -108,9 +108,11 @@ typedef struct PsLinearArgs {
 
 int ps_linear(const PsLinearArgs* args, void* stream);
 int ps_linear_args_size(void);   // sizeof(PsLinearArgs) as this library was built
-// Which kernel takes a bfloat16 product of aligned operands in dense rows, for tests of the dispatch: 1 the wide one
-// (packed: the packed copy is there), a tile's number of the large one (gemm_large_bf16.hip), 0 another.
-int ps_linear_choice(int m, int n, int k, int c_dtype, int epilogue, int packed);
+// Which kernel takes a bfloat16 product of aligned operands in dense rows, for tests of the dispatch: 0 the one for few rows,
+// 1 the one whose waves split k (tile: its number, ranges: of k), 2 two sizes of tiles (tile: the columns in the first one), 3
+// the large one (tile: its number, gemm_large_bf16.hip), 4 the wide one (packed: the packed copy is there), 5 the ring of
+// stages, 6 plain tiles.  scatter: keys and values go into their pages.
+int ps_linear_choice(int m, int n, int k, int c_dtype, int epilogue, int packed, int scatter, int* tile, int* ranges);
 
 // Store keys and values of the step's tokens into their pages.
 //   k, v: [tokens, kv_heads * head_dim] with row stride `stride`;

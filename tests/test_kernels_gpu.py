@@ -1554,17 +1554,27 @@ def test_linear_takes_the_wide_product_for_long_k():
     assert torch.equal(v_pool.view(torch.int16), v_ref.view(torch.int16))
 
 
-def _linear_choice(m, n, k, dtype, epilogue="none", packed=True):
-    """Which kernel takes a bfloat16 product: 0, 1 (the wide one) or a tile of the large one."""
+K_WAVES = ("k waves", 3, 1)      # tiles of 64 x 96, one range of k
+
+
+def _linear_choice(m, n, k, dtype, epilogue="none", packed=True, scatter=False):
+    """Which kernel takes a bfloat16 product: a tile's number of the large one, 1 (the wide one), 0 (another), the columns in
+    the first of two sizes of tiles, or ("k waves", tile, ranges of k)."""
+    import ctypes
+
     from pagedserve_amd.ops import kernels, library
 
-    return library.load_library().ps_linear_choice(m, n, k, 0 if dtype == torch.float32 else 1, kernels.EPILOGUES[epilogue],
-                                                   1 if packed else 0)
+    tile, ranges = ctypes.c_int(), ctypes.c_int()
+    kernel = library.load_library().ps_linear_choice(
+        m, n, k, 0 if dtype == torch.float32 else 1, kernels.EPILOGUES[epilogue], 1 if packed else 0, 1 if scatter else 0,
+        ctypes.byref(tile), ctypes.byref(ranges))
+    return {1: ("k waves", tile.value, ranges.value), 2: tile.value, 3: tile.value, 4: 1}.get(kernel, 0)
 
 
 @pytest.mark.parametrize("m,n,k,plain,floats", [
+    (544, 2304, 768, K_WAVES, K_WAVES),                                                                          # waves that split k
     (1293, 1536, 768, 0, 0), (1300, 3072, 1024, 1, 1), (1540, 2560, 1024, 1, 1), (320, 12800, 1600, 1, 1),     # twice, 1.5
-    (515, 3072, 1024, 11, 0), (544, 2304, 768, 11, 0), (284, 4800, 1600, 11, 11),                              # 128 x 64
+    (515, 3072, 1024, 11, 0), (580, 3072, 1280, 11, 11),                                                       # 128 x 64
     (544, 4096, 1024, 12, 0), (626, 3840, 1280, 12, 12), (1295, 2560, 1024, 12, 12),                           # 1.33 and 1
     (785, 8192, 1024, 22, 1), (2596, 4096, 1024, 3, 1), (2048, 3840, 1280, 22, 22), (2048, 3904, 768, 22, 22),
     (3292, 3072, 1024, 3, 3), (2048, 4096, 1024, 22, 22), (1568, 1280, 5120, 12, 12), (1294, 1536, 2048, 12, 12), (1300, 3072, 4096, 1, 1),
@@ -2038,10 +2048,10 @@ def test_scatter_of_heads_that_are_no_whole_pieces(heads, kv_heads, head_dim, m,
 
 
 @pytest.mark.parametrize("m,heads,kv_heads,k,tile", [
-    (261, 32, 16, 832, 11), (545, 32, 16, 832, 12), (1030, 32, 16, 832, 13), (2040, 32, 16, 832, 22), (2040, 32, 16, 800, 2),
+    (261, 32, 16, 832, K_WAVES), (322, 32, 16, 832, 11), (545, 32, 16, 832, 12), (1030, 32, 16, 832, 13), (2040, 32, 16, 832, 22), (2040, 32, 16, 800, 2),
     (2050, 25, 25, 832, 3), (3000, 32, 16, 832, 4), (3500, 25, 25, 832, 5), (2050, 32, 16, 832, 0)])
 def test_linear_of_many_rows_with_scatter(m, heads, kv_heads, k, tile):
-    """Through ``kernels.linear``: products that go to each of the large kernel's tiles, and one that goes past it, with
+    """Through ``kernels.linear``: products that go to each of the large kernel's tiles, and two that go past it, with
     the key/value scatter behind the product, against float64 and a scatter of its own."""
     from pagedserve_amd.ops import kernels
 
@@ -2049,7 +2059,7 @@ def test_linear_of_many_rows_with_scatter(m, heads, kv_heads, k, tile):
     q_cols, kv_cols = heads * head_dim, kv_heads * head_dim
     n = q_cols + 2 * kv_cols
     if kernels.compute_units() == 256:
-        assert _linear_choice(m, n, k, torch.bfloat16) == tile
+        assert _linear_choice(m, n, k, torch.bfloat16, scatter=True) == tile
     k_pool, v_pool, tables = _paged_fixture(torch.bfloat16, [m + 40, 60], kv_heads, head_dim, page_size, 360)
     tok_item = torch.tensor([1] * 50 + [0] * (m - 50), dtype=torch.int32, device="cuda")
     tok_pos = torch.tensor(list(range(10, 60)) + list(range(90, m + 40)), dtype=torch.int32, device="cuda")

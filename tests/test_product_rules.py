@@ -1,6 +1,8 @@
 """Which kernel takes a matrix product: the rules' lines, which are drawn for 256 compute units (what the library
 assumes without a device)."""
 
+import ctypes
+
 import pytest
 import torch
 
@@ -12,6 +14,53 @@ def lib():
     if torch.cuda.is_available() and kernels.compute_units() != 256:
         pytest.skip("the lines are drawn for 256 compute units")
     return library.load_library()
+
+
+FEW, K_WAVES, TWO_SIZES, LARGE, WIDE, RING, PLAIN = range(7)
+
+
+def _choice(lib, m, n, k, outputs="bfloat16", epilogue="none", packed=True, scatter=False):
+    """(kernel, tile or columns of the first size, ranges of k) of a product of bfloat16 operands."""
+    tile, ranges = ctypes.c_int(), ctypes.c_int()
+    kernel = lib.ps_linear_choice(m, n, k, 0 if outputs == "float32" else 1, kernels.EPILOGUES[epilogue], int(packed), int(scatter),
+                                  ctypes.byref(tile), ctypes.byref(ranges))
+    return kernel, tile.value, ranges.value
+
+
+@pytest.mark.parametrize("m,n,k,plain,floats,added", [
+    (64, 2304, 768, None, None, None), (65, 2304, 768, 0, 0, None),                       # 65 rows; few rows added to: 97
+    (97, 2304, 448, None, None, None), (97, 2304, 512, 0, 0, 0), (97, 2304, 544, None, None, None),      # whole stages, eight of them
+    (224, 2304, 768, 0, 0, 0), (225, 2304, 768, 1, 1, 1), (320, 2304, 768, 1, 1, 1),      # one round of 32 x 64, 32 x 96,
+    (321, 2304, 768, 2, 2, 2), (448, 2304, 768, 2, 2, 2), (449, 2304, 768, 3, 3, 3),      # 64 x 64,
+    (576, 2304, 768, 3, 3, 3), (577, 2304, 768, None, 3, 3), (640, 2304, 768, None, 3, 3), (641, 2304, 768, None, None, None),
+    (448, 3072, 1024, 3, 3, 3), (449, 3072, 1024, None, 3, 3), (284, 4800, 1600, None, 3, 3),      # 7/8 of the units (bfloat16), all
+    (2048, 768, 3072, None, 3, 3), (2049, 768, 3072, None, None, None)])
+def test_who_splits_k_over_its_waves(lib, m, n, k, plain, floats, added):
+    """The tile of a product whose waves split k, None where it goes elsewhere: both sides of the rule's lines."""
+    for outputs, epilogue, tile in (("bfloat16", "none", plain), ("bfloat16", "gelu_tanh", plain), ("float32", "none", floats),
+                                    ("float32", "residual", added)):
+        choice = _choice(lib, m, n, k, outputs, epilogue)
+        assert choice == (K_WAVES, tile, 1) if tile is not None else choice[0] != K_WAVES
+
+
+@pytest.mark.parametrize("m,n,k,columns", [
+    (3840, 6400, 1600, 0), (3841, 6400, 1600, 5120), (4096, 6400, 1600, 5120), (4097, 6400, 1600, 0),
+    (7680, 6400, 1600, 0), (7681, 6400, 1600, 5120), (8192, 6400, 1600, 5120), (8193, 6400, 1600, 0),
+    (2048, 12800, 1600, 10240), (4096, 6400, 1536, 5120), (4096, 6400, 1472, 0), (1023, 12800, 1600, 0)])
+def test_who_takes_two_sizes_of_tiles(lib, m, n, k, columns):
+    """The columns of the first size, 0: one size; bfloat16 outputs that nothing is added to, without key/value scatter."""
+    choice = _choice(lib, m, n, k)
+    assert choice[:2] == (TWO_SIZES, columns) if columns else choice[0] != TWO_SIZES
+    assert _choice(lib, m, n, k, epilogue="gelu_tanh") == choice
+    assert _choice(lib, m, n, k, scatter=True)[0] != TWO_SIZES
+    assert _choice(lib, m, n, k, "float32")[0] != TWO_SIZES and _choice(lib, m, n, k, "float32", "residual")[0] != TWO_SIZES
+
+
+@pytest.mark.parametrize("m,n,k,tile", [(17, 2304, 768, 0), (544, 2304, 768, 0), (193, 3072, 1024, 1), (544, 1024, 4096, 1),
+                                        (1163, 1600, 1600, 2), (2048, 3072, 768, 0), (2500, 3072, 1024, 3), (1200, 4800, 1600, 4)])
+def test_tiles_of_float_products(lib, m, n, k, tile):
+    """32 x 64, 48 x 64, 64 x 64, 80 x 64 or 64 x 96, by the fitted time."""
+    assert _even(lib, m, n, k, "residual" if k > n else "none")[0] == tile
 
 
 def _even(lib, m, n, k, epilogue):
