@@ -423,7 +423,22 @@ bool ps_gemm_nt_k_waves_takes(const void* a, const void* w, int m, int n, int k,
          ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(w)) & 15u) == 0;
 }
 
+// Rows added to that the kernel for few rows would take: from how many outputs on this one is ahead.  Its blocks read k in one round
+// of loads and this one's walk it, so that it is behind until the other one's blocks outnumber what the units hold at a time.
+// Of 2,389 products (97 to 224 rows, 64 to 2,048 columns, k of 512 to 8,192, in pieces) 981 were more than 3 % slower here, up to
+// twice as slow; of those that this rule takes 13, up to 1.08, and they take 0.79 of the time on average.  us there and here:
+// 128 x 512 x 768 3.5 / 4.1, 128 x 512 x 1024 3.8 / 4.7, 160 x 64 x 5120 3.7 / 7.3, but 144 x 512 x 1024 4.9 / 4.5, 128 x 768 x 3072 8.8 / 7.2;
+// 128 x 768 x 1536 5.2 / 5.7 (two ranges of 768 there, which its waves read in three steps and not four).
+static bool ahead_of_few_rows(int m, int n, int k) {
+  const int64_t outputs = (int64_t)m * n;
+  if (k <= 576) return true;
+  if (k < 2048) return outputs >= (k > 1408 && k <= 1536 ? 100000 : 70000);
+  return outputs * k >= 210000000;
+}
+
 // Which tile and number of ranges a product takes, false: not this kernel.  `few`: it would go to the kernel for few rows.
+// `pieces`: rows of C in aligned pieces of four columns; in single values the ends of rows added to cost 3 us more here, which
+// few rows do not make up for (100 x 321 x 768 3.8 / 8.3, 130 x 1030 x 1600 9.2 / 9.5).
 //
 // One round of blocks: with more than one to a unit this kernel shares LDS as the others do and has longer ends (two rounds of
 // 64 x 96 at 2048 x 2304 x 768 16.5 us, 13.9 in tiles of 128 x 192).  Where only larger tiles than 64 x 96 come to one round,
@@ -435,8 +450,10 @@ bool ps_gemm_nt_k_waves_takes(const void* a, const void* w, int m, int n, int k,
 // rows of them (160 x 6400 x 1600 11.9 and 12.5).
 // Ranges of k only where the kernel for few rows adds ranges by atomics too: beyond, sums keep an order that does not
 // change from call to call (256 x 1024 x 4096 15.1 us, in two ranges 11.8, before 16.4).
-bool ps_gemm_nt_k_waves_choice(int m, int n, int k, int c_dtype, int epilogue, bool few, int* best_tile, int* best_ranges) {
+bool ps_gemm_nt_k_waves_choice(int m, int n, int k, int c_dtype, int epilogue, bool few, bool pieces, int* best_tile,
+                               int* best_ranges) {
   if (m <= (few ? 96 : 64) || k < 512) return false;
+  if (few && !(pieces && ahead_of_few_rows(m, n, k))) return false;
   const int units = ps_compute_units(), most = few && epilogue == PS_EPI_RESIDUAL && k > 1024 ? 6 : 1;
   float least = INFINITY;
   for (int tile = 0; tile < KW_TILES; ++tile) {

@@ -692,6 +692,8 @@ bool ps_gemm_nt_mfma_skinny(const void* a, const void* w, int m, int n, int k, i
   // 16.6, 192 rows 16.7 against 18.3; 128 x 1600 x 6400 21.3 against 27.2, 160 rows 27.5 against
   // 26.9; with a short k 128 x 768 x 768 4.6 against 5.8, 192 x 1024 x 1024 6.5 against 6.8, 96 x
   // 1600 x 1600 9.2 against 9.3, 112 rows 10.6 against 9.4).
+  // (Against the tiled kernel; above 96 rows gemm_k_waves_bf16.hip takes what it is ahead at, 70,000 outputs and more or a k
+  // of up to 576: 128 x 768 x 768, 128 x 768 x 3072 and 128 x 1024 x 4096 go there.)
   if (m > 64)
     return epilogue == PS_EPI_RESIDUAL && m <= 224 && n < 64 * 256 &&
            (int64_t)m * n <= (k >= 2048 ? 200000 : 160000);
@@ -700,7 +702,8 @@ bool ps_gemm_nt_mfma_skinny(const void* a, const void* w, int m, int n, int k, i
 }
 
 bool ps_gemm_nt_k_waves_takes(const void* a, const void* w, int m, int n, int k, int lda, int ldc);
-bool ps_gemm_nt_k_waves_choice(int m, int n, int k, int c_dtype, int epilogue, bool few, int* best_tile, int* best_ranges);
+bool ps_gemm_nt_k_waves_choice(int m, int n, int k, int c_dtype, int epilogue, bool few, bool pieces, int* best_tile,
+                               int* best_ranges);
 int ps_gemm_nt_k_waves_tile(const void* a, const void* w, const float* bias, void* c, int m, int n, int k, int lda, int ldc,
                             int c_dtype, int epilogue, int tile, int ranges, const KvScatter& scatter, hipStream_t s);
 
@@ -717,12 +720,14 @@ struct BfRoute {
 };
 
 // `own_order`: rows and tokens in the way of the kernel for few rows (packed rows, choice of tokens).
-static BfRoute bf_route(const void* a, const void* w, const void* wp, int m, int n, int k, int lda, int ldc, int c_dtype,
+static BfRoute bf_route(const void* a, const void* w, const void* wp, const void* c, int m, int n, int k, int lda, int ldc, int c_dtype,
                         int epilogue, const KvScatter& scatter, bool own_order) {
   BfRoute route = {BF_FEW_ROWS, 0, 1};
   const bool few = ps_gemm_nt_mfma_skinny(a, w, m, n, k, lda, PS_BF16, epilogue);
+  // (rows of C in aligned pieces of four columns)
+  const bool pieces = ((ldc | n) & 3) == 0 && (reinterpret_cast<uintptr_t>(c) & (c_dtype == PS_F32 ? 15u : 7u)) == 0;
   if (m > 64 && !own_order && ps_gemm_nt_k_waves_takes(a, w, m, n, k, lda, ldc) &&
-      ps_gemm_nt_k_waves_choice(m, n, k, c_dtype, epilogue, few, &route.tile, &route.ranges)) {
+      ps_gemm_nt_k_waves_choice(m, n, k, c_dtype, epilogue, few, pieces, &route.tile, &route.ranges)) {
     route.kernel = BF_K_WAVES;
     return route;
   }
@@ -743,7 +748,7 @@ extern "C" int ps_linear_choice(int m, int n, int k, int c_dtype, int epilogue, 
   void* aligned = reinterpret_cast<void*>((uintptr_t)256);
   KvScatter pages = {};
   if (scatter) pages.k_pool = aligned;
-  const BfRoute route = bf_route(aligned, aligned, packed ? aligned : nullptr, m, n, k, k, n, c_dtype, epilogue, pages, false);
+  const BfRoute route = bf_route(aligned, aligned, packed ? aligned : nullptr, aligned, m, n, k, k, n, c_dtype, epilogue, pages, false);
   *tile = route.tile;
   *ranges = route.ranges;
   return (int)route.kernel;
@@ -756,7 +761,7 @@ int ps_gemm_nt_mfma(const void* a, const void* w, const float* bias, void* c, in
   const bf16_t* wp = (const bf16_t*)w_packed;
   if (dtype == PS_BF16) {
     const BfRoute route =
-        bf_route(a, w, wp, m, n, k, lda, ldc, c_dtype, epilogue, scatter, layouts != 0 || top.keys != nullptr);
+        bf_route(a, w, wp, c, m, n, k, lda, ldc, c_dtype, epilogue, scatter, layouts != 0 || top.keys != nullptr);
     if (route.kernel == BF_FEW_ROWS) {
       if (c_dtype == PS_F32)
         return launch_skinny<float>(a, w, bias, c, m, n, k, lda, ldc, epilogue, scatter, wp, layouts,

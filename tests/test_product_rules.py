@@ -43,6 +43,19 @@ def test_who_splits_k_over_its_waves(lib, m, n, k, plain, floats, added):
         assert choice == (K_WAVES, tile, 1) if tile is not None else choice[0] != K_WAVES
 
 
+@pytest.mark.parametrize("m,n,k,waves", [
+    (96, 512, 512, False), (97, 512, 512, True), (97, 64, 576, True), (97, 320, 640, False),          # a k of up to 576: any outputs
+    (128, 512, 1024, False), (136, 512, 1024, False), (137, 512, 1024, True), (97, 768, 1024, True),  # 70,000 outputs
+    (128, 768, 1536, False), (131, 768, 1536, True), (97, 768, 1408, True), (137, 512, 1600, True),   # a k in two ranges of 768
+    (133, 768, 2048, False), (134, 768, 2048, True), (160, 64, 5120, False), (128, 768, 3072, True),  # 2.1e8 products
+    (97, 1030, 1024, False), (97, 1028, 1024, True), (130, 321, 6400, False)])                        # not in pieces of four
+def test_who_takes_few_rows_added_to(lib, m, n, k, waves):
+    """Rows added to that the kernel for few rows could take: whether they go to the one whose waves split k."""
+    assert _choice(lib, m, n, k, "float32", "residual")[0] == (K_WAVES if waves else FEW)
+    # ranges of k, whose sums are added by atomics, only where the other kernel has them too
+    assert _choice(lib, m, n, k, "float32", "residual")[2] == 1 or k > 1024
+
+
 @pytest.mark.parametrize("m,n,k,columns", [
     (3840, 6400, 1600, 0), (3841, 6400, 1600, 5120), (4096, 6400, 1600, 5120), (4097, 6400, 1600, 0),
     (7680, 6400, 1600, 0), (7681, 6400, 1600, 5120), (8192, 6400, 1600, 5120), (8193, 6400, 1600, 0),
