@@ -446,8 +446,11 @@ static bool ahead_of_few_rows(int m, int n, int k) {
 // 1.28).  Of 230 products in these four tiles all but nine took less than the kernel before (0.74 to 0.88 on average): those
 // nine were 65 rows added to, which the kernel for few rows takes faster (768 x 768 3.2 and 3.9 us; 100 rows level, 160
 // 4.1 and 4.3), and bfloat16 rows in 64 x 96 on nearly all units (500 x 3072 x 1024 8.4 and 9.2, 1400 x 1000 x 2560 15.8 and
-// 18.0; on 216 of them 544 x 2304 x 768 6.9 and 6.1) or in three
-// rows of them (160 x 6400 x 1600 11.9 and 12.5).
+// 18.0; on 216 of them 544 x 2304 x 768 6.9 and 6.1).  Three rows of 64 x 96 over a k of more than 1,024 are behind, whatever
+// the outputs (180 products of 130 to 192 rows 0.88 to 1.10, 1.01 on average; 180 x 6400 x 1600 11.6 and 12.6), over a shorter one
+// ahead (180 products 0.89 on average), as are one or two rows of them where smaller tiles do not come to one round (192 products
+// 0.82 on average, bfloat16 110 x 9600 x 1024 11.4 and 9.5).  In single values rows added
+// to in 64 x 96 are behind on nearly all units too (300 x 4097 x 768 17.8 and 19.7, on 172 of them 200 rows 0.76 to 0.86).
 // Ranges of k only where the kernel for few rows adds ranges by atomics too: beyond, sums keep an order that does not
 // change from call to call (256 x 1024 x 4096 15.1 us, in two ranges 11.8, before 16.4).
 bool ps_gemm_nt_k_waves_choice(int m, int n, int k, int c_dtype, int epilogue, bool few, bool pieces, int* best_tile,
@@ -459,7 +462,9 @@ bool ps_gemm_nt_k_waves_choice(int m, int n, int k, int c_dtype, int epilogue, b
   for (int tile = 0; tile < KW_TILES; ++tile) {
     const auto& t = k_waves_tiles[tile];
     const int64_t tiles = (int64_t)((m + t.rows - 1) / t.rows) * ((n + t.columns - 1) / t.columns);
-    if (c_dtype != PS_F32 && tile == KW_TILES - 1 && (8 * tiles > 7 * units || m <= 3 * t.rows)) continue;
+    if (tile == KW_TILES - 1 && ((c_dtype != PS_F32 && 8 * tiles > 7 * units) || (m > 2 * t.rows && m <= 3 * t.rows && k > 1024) ||
+                                 (epilogue == PS_EPI_RESIDUAL && !pieces && 4 * tiles > 3 * units)))
+      continue;
     for (int ranges = 1; ranges <= most && tiles * ranges <= units; ++ranges) {
       const int stages = (k / TB_BK + ranges - 1) / ranges;
       if (k / TB_BK - (ranges - 1) * stages < 8) break;

@@ -34,7 +34,10 @@ def _choice(lib, m, n, k, outputs="bfloat16", epilogue="none", packed=True, scat
     (321, 2304, 768, 2, 2, 2), (448, 2304, 768, 2, 2, 2), (449, 2304, 768, 3, 3, 3),      # 64 x 64,
     (576, 2304, 768, 3, 3, 3), (577, 2304, 768, None, 3, 3), (640, 2304, 768, None, 3, 3), (641, 2304, 768, None, None, None),
     (448, 3072, 1024, 3, 3, 3), (449, 3072, 1024, None, 3, 3), (284, 4800, 1600, None, 3, 3),      # 7/8 of the units (bfloat16), all
-    (2048, 768, 3072, None, 3, 3), (2049, 768, 3072, None, None, None)])
+    (2048, 768, 3072, None, 3, 3), (2049, 768, 3072, None, None, None),
+    (128, 6400, 1600, 2, 2, 2), (160, 6400, 1600, None, None, None), (192, 6400, 1024, 3, 3, 3), (193, 4800, 1600, 3, 3, 3),   # three rows
+    (110, 9600, 1024, 3, 3, 3),                                                           # of 64 x 96: a k of up to 1,024
+    (260, 4092, 768, 3, 3, 3), (260, 4097, 768, 3, 3, None), (256, 4097, 768, 3, 3, 3)])      # rows in no pieces of four
 def test_who_splits_k_over_its_waves(lib, m, n, k, plain, floats, added):
     """The tile of a product whose waves split k, None where it goes elsewhere: both sides of the rule's lines."""
     for outputs, epilogue, tile in (("bfloat16", "none", plain), ("bfloat16", "gelu_tanh", plain), ("float32", "none", floats),
