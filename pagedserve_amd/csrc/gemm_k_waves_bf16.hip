@@ -436,7 +436,32 @@ static bool ahead_of_few_rows(int m, int n, int k) {
   return outputs * k >= 210000000;
 }
 
+// Products that go elsewhere although their tiles come to one round: those whose rows nearly fill their tiles (rows beyond m are read
+// from one address, so that what is left of a tile costs little here and much in larger tiles).
+//  - 64 x 96 in an odd number of rows of tiles, more than 7/8 full, over a k of 1,024 and more where the large kernel takes 128 x
+//    64: the half of a row of tiles that it wastes is cheap there too.  532 products take 0.95 of the time there, 0.88 to 1.05 (us,
+//    here and there: 293 x 3840 x 1280 11.4 / 10.0, 314 x 4096 x 1024 8.9 / 8.3, 805 x 1600 x 6400 35.5 / 32.5).  Less full they are level, in
+//    an even number, or over a k of up to 960, behind there (544 x 2304 x 768 6.1 / 6.9), as are nine and more rows of tiles over a k of
+//    less than 3,584 (821 x 1472 x 1600 1.18 of the time) or with plain float outputs (150 products 1.04).
+//  - a long k where the ring kernel is left and 257 rows and more: 64 x 64 on up to 9/16 of the units, 19/20 full, which goes in
+//    pairs of 64 x 32 there (33 products of a k of more than 4,096 0.92, 0.81 to 1.02 and one 1.14: 704 x 768 x 5120 25.5 / 21.8; but plain
+//    float outputs 0.99 to 1.26, up to 512 columns 1.04 to 1.35, and a k of 2,048 to 4,096 0.88 to 1.30), and 64 x 96, 49/50 full, that
+//    are up to 9/8 of the units in 64 x 64 and as many on every XCD (39 products of a k of more than 3,456 0.94, 0.87 to 1.08: 1071 x
+//    1024 x 6400 36.7 / 32.2; not as many on every XCD 1.09).  Three and four rows of tiles are 1.0 to 1.3 there.
+// `plain_float`: float outputs that are not added to what is there.
+static bool behind_elsewhere(int tile, int m, int n, int k, bool added, bool plain_float, int large_shape, int units) {
+  const int rows = (m + 63) / 64;
+  const int64_t tiles_64 = (int64_t)rows * ((n + 63) / 64);
+  if (tile == 3 && large_shape == 11)
+    return rows % 2 == 1 && 8 * m > 7 * 64 * rows && k >= (rows > 7 ? 3584 : added ? 1088 : 1024) && !(plain_float && rows > 5);
+  if (large_shape != 0 || m <= 256) return false;
+  if (tile == 2)
+    return k > 4096 && n > 512 && !plain_float && 2 * tiles_64 > units && 16 * tiles_64 <= 9 * units && 20 * m >= 19 * 64 * rows;
+  return tile == 3 && k > 3456 && 8 * tiles_64 <= 9 * units && tiles_64 % 8 == 0 && 50 * m >= 49 * 64 * rows;
+}
+
 // Which tile and number of ranges a product takes, false: not this kernel.  `few`: it would go to the kernel for few rows.
+// `large_shape`: the tile that the large kernel would take it in, 0: none.
 // `pieces`: rows of C in aligned pieces of four columns; in single values the ends of rows added to cost 3 us more here, which
 // few rows do not make up for (100 x 321 x 768 3.8 / 8.3, 130 x 1030 x 1600 9.2 / 9.5).
 //
@@ -453,8 +478,8 @@ static bool ahead_of_few_rows(int m, int n, int k) {
 // to in 64 x 96 are behind on nearly all units too (300 x 4097 x 768 17.8 and 19.7, on 172 of them 200 rows 0.76 to 0.86).
 // Ranges of k only where the kernel for few rows adds ranges by atomics too: beyond, sums keep an order that does not
 // change from call to call (256 x 1024 x 4096 15.1 us, in two ranges 11.8, before 16.4).
-bool ps_gemm_nt_k_waves_choice(int m, int n, int k, int c_dtype, int epilogue, bool few, bool pieces, int* best_tile,
-                               int* best_ranges) {
+bool ps_gemm_nt_k_waves_choice(int m, int n, int k, int c_dtype, int epilogue, bool few, bool pieces, int large_shape,
+                               int* best_tile, int* best_ranges) {
   if (m <= (few ? 96 : 64) || k < 512) return false;
   if (few && !(pieces && ahead_of_few_rows(m, n, k))) return false;
   const int units = ps_compute_units(), most = few && epilogue == PS_EPI_RESIDUAL && k > 1024 ? 6 : 1;
@@ -477,7 +502,8 @@ bool ps_gemm_nt_k_waves_choice(int m, int n, int k, int c_dtype, int epilogue, b
       }
     }
   }
-  return least < INFINITY;
+  return least < INFINITY && (few || !behind_elsewhere(*best_tile, m, n, k, epilogue == PS_EPI_RESIDUAL, c_dtype == PS_F32 && epilogue != PS_EPI_RESIDUAL,
+                                                         large_shape, units));
 }
 
 // The product in a given tile and number of ranges, for tests and measurements.

@@ -702,8 +702,8 @@ bool ps_gemm_nt_mfma_skinny(const void* a, const void* w, int m, int n, int k, i
 }
 
 bool ps_gemm_nt_k_waves_takes(const void* a, const void* w, int m, int n, int k, int lda, int ldc);
-bool ps_gemm_nt_k_waves_choice(int m, int n, int k, int c_dtype, int epilogue, bool few, bool pieces, int* best_tile,
-                               int* best_ranges);
+bool ps_gemm_nt_k_waves_choice(int m, int n, int k, int c_dtype, int epilogue, bool few, bool pieces, int large_shape,
+                               int* best_tile, int* best_ranges);
 int ps_gemm_nt_k_waves_tile(const void* a, const void* w, const float* bias, void* c, int m, int n, int k, int lda, int ldc,
                             int c_dtype, int epilogue, int tile, int ranges, const KvScatter& scatter, hipStream_t s);
 
@@ -726,14 +726,16 @@ static BfRoute bf_route(const void* a, const void* w, const void* wp, const void
   const bool few = ps_gemm_nt_mfma_skinny(a, w, m, n, k, lda, PS_BF16, epilogue);
   // (rows of C in aligned pieces of four columns)
   const bool pieces = ((ldc | n) & 3) == 0 && (reinterpret_cast<uintptr_t>(c) & (c_dtype == PS_F32 ? 15u : 7u)) == 0;
+  const bool wide = !few && ps_gemm_nt_bf16_wide_supported(a, wp, m, n, k, lda);
+  const int shape = few ? 0 : ps_gemm_nt_bf16_large_shape(a, w, m, n, k, lda, c_dtype, epilogue, wide);
   if (m > 64 && !own_order && ps_gemm_nt_k_waves_takes(a, w, m, n, k, lda, ldc) &&
-      ps_gemm_nt_k_waves_choice(m, n, k, c_dtype, epilogue, few, pieces, &route.tile, &route.ranges)) {
+      ps_gemm_nt_k_waves_choice(m, n, k, c_dtype, epilogue, few, pieces, shape, &route.tile, &route.ranges)) {
     route.kernel = BF_K_WAVES;
     return route;
   }
+  route.tile = 0;
+  route.ranges = 1;
   if (few) return route;
-  const bool wide = ps_gemm_nt_bf16_wide_supported(a, wp, m, n, k, lda);
-  const int shape = ps_gemm_nt_bf16_large_shape(a, w, m, n, k, lda, c_dtype, epilogue, wide);
   if (shape != 0) {
     const int first_columns = ps_gemm_nt_bf16_two_sizes_columns(m, n, k, c_dtype, epilogue, scatter);
     route.kernel = first_columns > 0 ? BF_TWO_SIZES : BF_LARGE;

@@ -33,9 +33,9 @@ def _choice(lib, m, n, k, outputs="bfloat16", epilogue="none", packed=True, scat
     (224, 2304, 768, 0, 0, 0), (225, 2304, 768, 1, 1, 1), (320, 2304, 768, 1, 1, 1),      # one round of 32 x 64, 32 x 96,
     (321, 2304, 768, 2, 2, 2), (448, 2304, 768, 2, 2, 2), (449, 2304, 768, 3, 3, 3),      # 64 x 64,
     (576, 2304, 768, 3, 3, 3), (577, 2304, 768, None, 3, 3), (640, 2304, 768, None, 3, 3), (641, 2304, 768, None, None, None),
-    (448, 3072, 1024, 3, 3, 3), (449, 3072, 1024, None, 3, 3), (284, 4800, 1600, None, 3, 3),      # 7/8 of the units (bfloat16), all
+    (392, 3072, 1024, 3, 3, 3), (449, 3072, 1024, None, 3, 3),      # 7/8 of the units (bfloat16), all
     (2048, 768, 3072, None, 3, 3), (2049, 768, 3072, None, None, None),
-    (128, 6400, 1600, 2, 2, 2), (160, 6400, 1600, None, None, None), (192, 6400, 1024, 3, 3, 3), (193, 4800, 1600, 3, 3, 3),   # three rows
+    (128, 6400, 1600, 2, 2, 2), (160, 6400, 1600, None, None, None), (168, 6400, 1024, 3, 3, 3), (193, 4800, 1600, 3, 3, 3),   # three rows
     (110, 9600, 1024, 3, 3, 3),                                                           # of 64 x 96: a k of up to 1,024
     (260, 4092, 768, 3, 3, 3), (260, 4097, 768, 3, 3, None), (256, 4097, 768, 3, 3, 3)])      # rows in no pieces of four
 def test_who_splits_k_over_its_waves(lib, m, n, k, plain, floats, added):
@@ -44,6 +44,25 @@ def test_who_splits_k_over_its_waves(lib, m, n, k, plain, floats, added):
                                     ("float32", "residual", added)):
         choice = _choice(lib, m, n, k, outputs, epilogue)
         assert choice == (K_WAVES, tile, 1) if tile is not None else choice[0] != K_WAVES
+
+
+@pytest.mark.parametrize("m,n,k,plain,floats,added", [
+    (393, 3456, 1024, LARGE, "64x96", "64x96"), (393, 3456, 1088, LARGE, "64x96", LARGE), (392, 3008, 1088, "64x96", "64x96", "64x96"),
+    (576, 2304, 768, "64x96", "64x96", "64x96"), (169, 6400, 1024, LARGE, "64x96", "64x96"), (168, 6400, 1024, "64x96", "64x96", "64x96"),
+    (281, 4800, 1280, LARGE, LARGE, LARGE), (280, 4096, 1280, "64x96", "64x96", "64x96"), (384, 3072, 1280, "64x96", "64x96", "64x96"),
+    (805, 1600, 3520, "64x96", "64x96", "64x96"), (805, 1600, 3584, LARGE, "64x96", "64x96"), (805, 1792, 3584, LARGE, "64x96", LARGE),
+    (704, 768, 4096, "64x64", "64x64", "64x64"), (704, 768, 4160, RING, "64x64", RING), (768, 768, 4160, RING, "64x64", RING),
+    (729, 768, 4160, "64x64", "64x64", "64x64"), (730, 768, 4160, RING, "64x64", RING), (832, 768, 4160, "64x64", "64x64", "64x64"),
+    (1088, 512, 4160, "64x64", "64x64", "64x64"), (250, 2304, 6400, "64x64", "64x64", "64x64"),
+    (1088, 1024, 3456, "64x96", "64x96", "64x96"), (1088, 1024, 3520, RING, RING, RING), (1066, 1024, 3520, "64x96", "64x96", "64x96"),
+    (1472, 768, 5120, "64x96", "64x96", "64x96"), (1536, 768, 5120, RING, RING, RING), (1600, 768, 5120, "64x96", "64x96", "64x96")])
+def test_who_splits_k_over_its_waves_in_full_tiles(lib, m, n, k, plain, floats, added):
+    """Tiles that the rows nearly fill: the kernel of a product that goes elsewhere, the tile of one that stays."""
+    for outputs, epilogue, expected in (("bfloat16", "none", plain), ("bfloat16", "gelu_tanh", plain), ("float32", "none", floats),
+                                        ("float32", "residual", added)):
+        kernel, tile, ranges = _choice(lib, m, n, k, outputs, epilogue)
+        assert (("32x64", "32x96", "64x64", "64x96")[tile] if kernel == K_WAVES else kernel) == expected
+        assert (kernel != LARGE or tile == 11) and ranges == 1
 
 
 @pytest.mark.parametrize("m,n,k,waves", [
