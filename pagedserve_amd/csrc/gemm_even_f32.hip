@@ -5,8 +5,9 @@
 // count: that every SIMD gets about as many products, and that nothing stands between them.
 //
 // Fragments are 16 x 16 (v_mfma_f32_16x16x4_f32, as many products per cycle as 32 x 32 x 2), four waves to a block, so
-// that tiles come in steps of 16 rows and the one that fills the units most evenly is chosen (even_time below).  2048 x
-// 768 is 256 tiles of 64 x 96, 544 x 2304 252 of 80 x 64, where 64 x 64 leaves some units two and others one.
+// that tiles come in steps of 16 rows and one that fills the units evenly is chosen (even_time below): 193 x 3072 is 240 blocks of 48 x
+// 64, 2500 x 3072 six blocks of 80 x 64 to every unit, 2048 x 768 and 544 x 2304 go in 32 x 64, three blocks to a unit and up to three,
+// where 64 x 64 leaves some units two and others one.
 //
 // A wave alone on its SIMD has to issue a product every 32 cycles, seven instructions at most.  With pointers of 64 bits
 // and places in the ring by division a load to LDS took nine by itself and the matrix cores stood still: 544 x 768 x 3072
@@ -21,10 +22,13 @@
 // steps around: no chain is longer than 32 products.  Against float64, over 150 products of 17 to 2,300 rows and k of 256
 // to 6,400: 0.8 to 1.3e-7, where the kernel that took them before was 0.8 to 2.7e-7.
 //
-// With weights from memory, that kernel (tiles of 64 x 64 to 128 x 128) and this one, us: 2048 x 2304 x 768 71 / 60, x 3072
-// with GELU 95 / 85, 2048 x 768 x 768 added to rows 31 / 22.5, x 3072 100 / 78 (124 TFLOP/s), 544 x 2304 x 768 30.2 / 19.1,
-// 544 x 768 x 3072 38.6 / 27.3, 193 x 3072 x 1024 23.6 / 17.0, 1163 x 1600 x 1600 60.8 / 53.6, 299 x 1600 x 6400 74 / 56,
-// 4096 x 4096 x 1024 266 / 268.
+// With weights from memory, each product by itself, that kernel (tiles of 64 x 64 to 128 x 128) and this one, us: 2048 x 2304 x 768 70 /
+// 61, x 3072 with GELU 95 / 85, 2048 x 768 x 768 added to rows 31 / 22, x 3072 94 / 76 (127 TFLOP/s), 544 x 2304 x 768 30 / 22, 544 x
+// 768 x 3072 38 / 31, 193 x 3072 x 1024 23.6 / 17.0, 4101 x 1600 x 1600 211 / 176, 4102 x 3072 x 1024 240 / 204, 4096 x 6400 x 1600 with
+// GELU 728 / 656; the output head, 50257 x 768, at 17 rows 60 / 36, 64 64 / 55, 96 106 / 75, 128 107 / 94.  1,001 products of 17 to 8,192
+// rows take 0.83 of the time, the most 1.05 (6000 x 512 x 128 12.0 / 12.5).  In a pass, between a layer's other launches, the gain is
+// less: 2048 x 2304 x 768 74, x 3072 with GELU 99, the two added to rows 59 on average (97 to 103 TFLOP/s; 77 to 103 and 61 at another
+// time), where the kernel before took 103 for the second.
 #include <type_traits>
 
 #include "common.h"

@@ -13,12 +13,16 @@
 // lie.  Blocks of an XCD that begin their k 256 bytes apart, round and round, ask for fewer rows of one channel at a time, but
 // lose that: 667 products took 1.002 of the time on average (256 x 5120 x 1280 11.2 us and 12.2, 1024 x 1280 x 5120 29.7 and 32.5, but
 // 1024 x 1024 x 4096 16.3 and 15.5); begun by the tile's column, which would keep it, 1.003 of what k from its start takes.
+// Between the other launches of a pass, whose rows have just been written, it costs more: 512 rows of GPT-2 small 8.4 us for the
+// mean of the two products added to rows and 9.6 for QKV, begun apart 7.5 and 8.9, by the column 8.4 and 9.6 in either order of
+// tiles: what helps is that rows of tiles begin apart.
 //
 // With one block to a unit nothing hides its ends, so they are straight code: C and bias are buffers (what lies outside reads
 // as zero and is not written), and what cannot go in pieces of four columns takes another branch in a loop of its own.
 // With branches and single values beside every piece a tile of 64 x 160 spent 1.7 us more in them, in skipped code.
 //
-// Stages hold 64 values of k of every row, four to six in a ring, which two blocks of a unit have room for, in the order of gemm_tiled.hip.  A stage meets the other
+// Stages hold 64 values of k of every row, four to six in a ring, which two blocks of a unit have room for, in the order of
+// gemm_tiled.hip (piece c of row r in slot c ^ ((r >> 1) & 7)).  A stage meets the other
 // waves once: everyone has then read it and the next one has landed; its products run with the next stage's reads and the
 // loads of the stage that takes its place between them.
 //
@@ -502,8 +506,8 @@ bool ps_gemm_nt_k_waves_choice(int m, int n, int k, int c_dtype, int epilogue, b
       }
     }
   }
-  return least < INFINITY && (few || !behind_elsewhere(*best_tile, m, n, k, epilogue == PS_EPI_RESIDUAL, c_dtype == PS_F32 && epilogue != PS_EPI_RESIDUAL,
-                                                         large_shape, units));
+  const bool added = epilogue == PS_EPI_RESIDUAL, plain_float = c_dtype == PS_F32 && !added;
+  return least < INFINITY && (few || !behind_elsewhere(*best_tile, m, n, k, added, plain_float, large_shape, units));
 }
 
 // The product in a given tile and number of ranges, for tests and measurements.

@@ -134,6 +134,8 @@ __global__ __launch_bounds__(256) void gemm_nt_ring_kernel(
 #pragma unroll
         for (int e = 0; e < 16; ++e) sums[i][j][p][e] = 0.f;
 
+  // (Float products come here with a k of up to 96, or with rows more than 2^22 values apart at any k: what follows is for
+  // the latter, measured when this kernel took all of them.)
   // A residual product of 64 x 64 float tiles takes whole k ranges where others would be split over more
   // blocks: every RUN k tiles its accumulators are added to a total and start anew, so that no chain grows
   // longer than the 128 additions that a range of 128 values would have (error of 1024 x 1024 x 1024: 2.9e-7
@@ -182,7 +184,7 @@ __global__ __launch_bounds__(256) void gemm_nt_ring_kernel(
   // stage, positions and items once it has landed (what they are read by lies further back in the arguments).  With
   // this, and tile numbers of the preloaded arguments: 64 x 4800 x 1600 9.6 to 8.7 us, 448 x 1600 x 1600 added to rows
   // 21.2 to 19.8 (mean of that and k = 6400), 544 x 1024 x 1024 8.2 to 7.4.
-  // (Not for float rows added to in two stages: of their blocks registers and not LDS set how many share a unit, and the rows
+  // (Not for float rows added to in two stages, measured while they had any k: of their blocks registers and not LDS set how many share a unit, and the rows
   // held through the loop take those of the fourth, 135 instead of 111.  us, early and late: 96 x 50257 x 768 141 / 132, 1500
   // x 2304 x 768 61.8 / 60.0, 1024 x 4096 x 1024 88.6 / 85.4, 2048 x 1600 x 1600 113.3 / 113.6, twelve shapes 0.983.  Without
   // rows it is four blocks instead of five, and as fast: the twelve plain 1.000 late, with GELU 1.009.)
@@ -374,7 +376,8 @@ static int launch_variant(const void* a, const void* w, const float* bias, void*
   // Few tiles with a long k leave most of the chip idle: where partial sums can be added in
   // place (residual epilogue) k is split over blocks.  Float atomics are slow, so this pays
   // only while the output is small.
-  // float products keep the matrix cores sixteen times as long, so there the adds weigh less: as many
+  // float products (a k of more than 1,024 only where rows lie more than 2^22 values apart, the rest goes to
+  // gemm_even_f32.hip) keep the matrix cores sixteen times as long, so there the adds weigh less: as many
   // ranges of a long k as leave at most three blocks per compute unit (with one range and with this
   // many: 330 x 1024 x 4096 50 and 43 us, 1024 x 768 x 3072 60 and 56; but 1024 x 768 x 768 18 and 28)
   int k_splits = 1;
